@@ -71,6 +71,7 @@ extern "C" int andr_destroy(andr_ctx *ctx) {
   andr_pool_trim(ctx);
   for (auto &kv : ctx->pool.size_of) (void)hipFree(kv.first);  // blocks still held by nobody's buffers
   ctx->pool.size_of.clear();
+  for (void *c : ctx->pinned.chunks) (void)hipHostFree(c);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return ANDR_OK;
@@ -127,6 +128,24 @@ void andr_pool_trim(andr_ctx *ctx) {
   P.free_blocks.clear();
   P.cached = 0;
 }
+
+void *andr_pinned_alloc(andr_ctx *ctx) {
+  andr_pinned &P = ctx->pinned;
+  if (P.free_slots.empty()) {
+    void *c = nullptr;
+    if (hipHostMalloc(&c, ANDR_PINNED_CHUNK * ANDR_PINNED_SLOT, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    P.chunks.push_back(c);
+    for (int i = ANDR_PINNED_CHUNK - 1; i >= 0; --i) P.free_slots.push_back((char *)c + i * ANDR_PINNED_SLOT);
+  }
+  void *s = P.free_slots.back();
+  P.free_slots.pop_back();
+  return s;
+}
+
+void andr_pinned_release(andr_ctx *ctx, void *slot) { ctx->pinned.free_slots.push_back(slot); }
 
 extern "C" const char *andr_last_error(const andr_ctx *ctx) { return ctx ? ctx->err.c_str() : "no context"; }
 

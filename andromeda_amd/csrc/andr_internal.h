@@ -32,11 +32,20 @@ struct andr_pool {
   size_t cached = 0;
 };
 
+// Pinned host memory that kernels write states to for the host to read (hipHostMalloc), handed out in
+// slots; a context allocates it in chunks as its solves need it and keeps it until andr_destroy.
+#define ANDR_PINNED_SLOT ((size_t)4096)
+#define ANDR_PINNED_CHUNK 32 /* slots */
+struct andr_pinned {
+  std::vector<void *> chunks, free_slots;
+};
+
 struct andr_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   std::string err;
   andr_pool pool;
+  andr_pinned pinned;
   // learned quadrature model (BF16 copy lives in the device buffer below)
   bool has_model = false;
   float model_conf = 0.9f;
@@ -65,6 +74,8 @@ int andr_fail(andr_ctx *ctx, int code, const char *fmt, ...);
 void *andr_dev_alloc(andr_ctx *ctx, size_t bytes);  // from the context's cache or the driver; null on failure
 void andr_dev_release(andr_ctx *ctx, void *p);       // back to the context's cache
 void andr_pool_trim(andr_ctx *ctx);                  // return every cached block to the driver
+void *andr_pinned_alloc(andr_ctx *ctx);              // one slot; null on failure
+void andr_pinned_release(andr_ctx *ctx, void *slot);
 
 // RAII device buffer; with a context it draws on the context's memory cache
 template <class T>

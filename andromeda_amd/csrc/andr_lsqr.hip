@@ -2,12 +2,33 @@
 //
 // Every right-hand side follows its own Paige-Saunders recurrence (lsqr_LSQR, src/lib_lsqr.f:470-1207,
 // damp = 0, conlim = 1e8, nconv = 1), but the two products of an iteration -- A v and A^T u -- are
-// formed for all ANDR_NB columns in one pass over A, so the matrix is streamed from HBM twice per
-// iteration for the whole block instead of twice per iteration per right-hand side.
+// formed for all right-hand sides in one pass over A, so the matrix is streamed twice per iteration
+// for the whole block instead of twice per iteration per right-hand side. Several right-hand sides
+// share vectors of ANDR_NB interleaved columns; a single one runs on plain vectors (WD = 1 below),
+// since eight columns for one cost eight times the partial sums and vector traffic.
 //
 // The u and v vectors are kept unnormalised together with their norms (true u = U / beta, true
 // v = V / alpha); the products fold the normalisation into their scale factors, which removes the
 // separate scaling passes of the reference (dscal at :947, :974, :980).
+//
+// An iteration is three launches. A small system (an A of the order of the 256 MB cache) spends its
+// time in the gaps and the latency of small kernels, not in the products, so the recurrences' scalar
+// work and the vector updates ride along in the products' own kernels:
+//   1. k_lsqr_av: the partial products of A V over column segments;
+//   2. k_lsqr_atu: U = sx .* (A V) + sy .* U for its rows from those partials (each column panel for
+//      itself, the first one keeps it), then the partial products of A^T U over row splits. Its blocks
+//      start with the scalars that end the previous iteration (norm of V, plane rotations, stopping
+//      tests), block (0, 0) for good (state B);
+//   3. k_lsqr_v: V = sx .* (A^T U) + sy .* V from those partials, with the update of X and W that the
+//      previous iteration still owes; starts with the scalars after A V (state A).
+// With more than LSQR_FUSE_SEG column segments every panel's own sum over them would cost more than a
+// launch (per row WD * 8 bytes a segment in each column panel against 1 KB of A), and
+// k_lsqr_u forms U once, as for CSR matrices. Measured per iteration with seven launches and
+// eight columns throughout against this: 3120^2, 6 right-hand sides 73 -> 41 us; 4881 x 2717, one
+// 84 -> 44 us; 1587^2, one 57 -> 18 us; 4897^2 in FP32, one 132 -> 40 us.
+//
+// The host reads the states of every LSQR_POLL-th iteration from pinned memory one poll late, so that
+// the device never waits for it; the iterations enqueued past the end return at once.
 #include "andr_internal.h"
 #include "andr_solve.h"
 #include "andr_prof.h"
@@ -28,489 +49,76 @@ __device__ inline double d2norm(double a, double b) {  // lsqr_d2norm (src/lib_l
   return scale * sqrt(x * x + y * y);
 }
 
-// Butterfly reduce-scatter of 64 per-lane values: afterwards lane l holds the wave sum of v[l].
-__device__ inline double wave_reduce_scatter64(double (&v)[64]) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int half = 32; half >= 1; half >>= 1) {
-    const bool hi = (lane & half) != 0;
-#pragma unroll
-    for (int i = 0; i < half; ++i) {
-      const double keep = hi ? v[i + half] : v[i];
-      const double send = hi ? v[i] : v[i + half];
-      v[i] = keep + __shfl_xor(send, half, 64);
-    }
-  }
-  return v[0];
-}
-
-// Y = sx .* (A X) + sy .* Y for NB interleaved columns; one wave per 8 rows.
-// part[wave][k] = sum of the squares of the new Y over the wave's rows.
-template <class ST>
-__global__ __launch_bounds__(256) void k_gemv_n(const ST *__restrict__ A, int64_t lda, int m, int n,
-                                                const double *__restrict__ X, double *__restrict__ Y,
-                                                const double *__restrict__ sx, const double *__restrict__ sy,
-                                                double *__restrict__ part) {
-  const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const int row0 = wave * 8;
-  if (row0 >= m) return;
-  double acc[64];
-#pragma unroll
-  for (int i = 0; i < 64; ++i) acc[i] = 0.0;
-  const ST *arow[8];
-#pragma unroll
-  for (int r = 0; r < 8; ++r) arow[r] = A + (size_t)min(row0 + r, m - 1) * lda;
-  for (int j = lane; j < n; j += 64) {
-    const double4 x0 = *reinterpret_cast<const double4 *>(X + (size_t)j * NB);
-    const double4 x1 = *reinterpret_cast<const double4 *>(X + (size_t)j * NB + 4);
-    const double xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const double a = (double)arow[r][j];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) acc[r * 8 + k] += a * xv[k];
-    }
-  }
-  double s = wave_reduce_scatter64(acc);  // lane l: row row0 + l/8, column l%8
-  const int r = lane >> 3, k = lane & 7;
-  double y = 0.0;
-  if (row0 + r < m) {
-    double *py = Y + (size_t)(row0 + r) * NB + k;
-    y = sx[k] * s + sy[k] * (*py);
-    *py = y;
-  }
-  double y2 = y * y;
-  y2 += __shfl_xor(y2, 8, 64);
-  y2 += __shfl_xor(y2, 16, 64);
-  y2 += __shfl_xor(y2, 32, 64);
-  if (lane < 8) part[(size_t)wave * NB + lane] = y2;
-}
-
-// The same product for FP64 A on the matrix cores (v_mfma_f64_16x16x4f64). A wave owns 16 GN_T rows
-// (GN_T 16-row tiles) over the column segment blockIdx.y; lane (g = lane / 16, c = lane % 16) feeds
-// row c of tile T with columns 16 kb + 4 g + t (t = 0..3, one instruction each) and column c of
-// B = X (right-hand side c; the upper half c >= NB is zero). The result D[g + 4 v][c] sits in
-// register v of lane (g, c). With one segment the update Y = sx .* D + sy .* Y and
-// out[wave][k] = sum of the new Y^2 over the wave's rows are done here; with several the raw
-// segment products go to out = P[segment][row][k] and k_combine_n finishes. The segment length
-// depends on the matrix shape only, and every row's sum runs over its segment in the same order for
-// every GN_T, so the tile count (chosen by the autotuner) never changes a result bit.
-constexpr int GN_SEGLEN = 1024;  // measured on 13500^2 / 24000^2: 4.5 / 4.8 TB/s (1360 / 1104: 4.3 / 4.6)
+typedef double d2n __attribute__((ext_vector_type(2)));
 typedef double d4v __attribute__((ext_vector_type(4)));
+typedef float f4n __attribute__((ext_vector_type(4)));
 
-template <int GN_T, bool SEG, bool VEC>
-__global__ __launch_bounds__(256) void k_gemv_n_mf(const double *__restrict__ A, int64_t lda, int m, int n,
-                                                   const double *__restrict__ X, int seglen, double *__restrict__ Y,
-                                                   const double *__restrict__ sx, const double *__restrict__ sy,
-                                                   double *__restrict__ out) {
-  typedef const double __attribute__((address_space(1))) *gdp;
-  typedef double d2n __attribute__((ext_vector_type(2)));
-  // VEC: the tiles are read in whole 128-byte row segments (lane (rr = lane / 8, p = lane % 8) takes
-  // columns 2 p, 2 p + 1 of row rr of an 8-row half tile: a load covers 8 full lines, where the
-  // matrix-core lane pattern covers 16 half lines, measured 6.9 against 4.6-5.3 TB/s on a 30 GB
-  // matrix) and redistributed to the matrix-core layout through LDS (16 x 16 tile per T, rows padded
-  // to 18 doubles)
-  constexpr int LR = 18;
-  __shared__ __attribute__((aligned(16))) double lt[VEC ? 4 : 1][VEC ? GN_T : 1][16 * LR];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wid;
-  const int row0 = wave * 16 * GN_T;
-  if (row0 >= m) return;  // uniform over the wave; the LDS tiles are per wave
-  const int g = lane >> 4, c = lane & 15;
-  const int rr = lane >> 3, p = lane & 7;
-  const bool hi = c >= NB;
-  const int k0 = blockIdx.y * seglen, kend = min(n, k0 + seglen);
-  gdp arow[GN_T];   // matrix-core pattern: row 16 T + c, columns 4 g ..
-  gdp lrow[GN_T][2];  // row-segment pattern: rows 16 T + rr and 16 T + 8 + rr, columns 2 p ..
-#pragma unroll
-  for (int T = 0; T < GN_T; ++T) {
-    arow[T] = (gdp)(A + (size_t)min(row0 + 16 * T + c, m - 1) * lda + 4 * g);
-    lrow[T][0] = (gdp)(A + (size_t)min(row0 + 16 * T + rr, m - 1) * lda + 2 * p);
-    lrow[T][1] = (gdp)(A + (size_t)min(row0 + 16 * T + 8 + rr, m - 1) * lda + 2 * p);
-  }
-  const gdp xb = (gdp)(X + (size_t)(4 * g) * NB + (c & (NB - 1)));
-  d4v acc[GN_T];
-#pragma unroll
-  for (int T = 0; T < GN_T; ++T) acc[T] = d4v{0.0, 0.0, 0.0, 0.0};
-  // raw operands of one 16-column block: VEC: two row segments per T; otherwise the matrix-core
-  // values themselves
-  auto load = [&](int kb, double (&a)[GN_T][4], double (&x)[4]) {
-#pragma unroll
-    for (int T = 0; T < GN_T; ++T) {
-      if (VEC) {  // the matrix is streamed once: non-temporal, so that X keeps its place in L2
-        const d2n u = __builtin_nontemporal_load((const d2n __attribute__((address_space(1))) *)(lrow[T][0] + 16 * kb));
-        const d2n w = __builtin_nontemporal_load((const d2n __attribute__((address_space(1))) *)(lrow[T][1] + 16 * kb));
-        a[T][0] = u.x;
-        a[T][1] = u.y;
-        a[T][2] = w.x;
-        a[T][3] = w.y;
-      } else {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) a[T][t] = __builtin_nontemporal_load(arow[T] + 16 * kb + t);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t) x[t] = xb[(size_t)(16 * kb + t) * NB];
-  };
-  // VEC: row segments -> LDS -> matrix-core values (in place)
-  auto stage = [&](double (&a)[GN_T][4]) {
-    if (VEC) {
-#pragma unroll
-      for (int T = 0; T < GN_T; ++T) {
-        *(d2n *)&lt[wid][T][rr * LR + 2 * p] = d2n{a[T][0], a[T][1]};
-        *(d2n *)&lt[wid][T][(8 + rr) * LR + 2 * p] = d2n{a[T][2], a[T][3]};
-      }
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int T = 0; T < GN_T; ++T) {
-        const d2n u = *(const d2n *)&lt[wid][T][c * LR + 4 * g];
-        const d2n w = *(const d2n *)&lt[wid][T][c * LR + 4 * g + 2];
-        a[T][0] = u.x;
-        a[T][1] = u.y;
-        a[T][2] = w.x;
-        a[T][3] = w.y;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
-  };
-  auto step = [&](const double (&a)[GN_T][4], const double (&x)[4]) {
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const double b = hi ? 0.0 : x[t];
-#pragma unroll
-      for (int T = 0; T < GN_T; ++T) acc[T] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[T][t], b, acc[T], 0, 0, 0);
-    }
-  };
-  // full 16-column blocks, two register sets in turn: the operands of the next block are requested
-  // before the products of the current one (the last prefetch re-reads the final block)
-  int kb = k0 >> 4;
-  const int kb_end = kend >> 4;
-  if (kb < kb_end) {
-    double a0[GN_T][4], a1[GN_T][4], x0[4], x1[4];
-    load(kb, a0, x0);
-    for (; kb + 1 < kb_end; kb += 2) {
-      load(kb + 1, a1, x1);
-      __builtin_amdgcn_sched_barrier(0);
-      stage(a0);
-      step(a0, x0);
-      __builtin_amdgcn_sched_barrier(0);
-      load(min(kb + 2, kb_end - 1), a0, x0);
-      __builtin_amdgcn_sched_barrier(0);
-      stage(a1);
-      step(a1, x1);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (kb < kb_end) {  // odd count: a0 holds block kb
-      stage(a0);
-      step(a0, x0);
-      ++kb;
-    }
-  }
-  if (16 * kb < kend) {  // last, partial column block (last segment only): masked
-    double a[GN_T][4], x[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int col = 16 * kb + 4 * g + t;
-      const bool in = col < kend;
-      x[t] = in ? X[(size_t)col * NB + (c & (NB - 1))] : 0.0;
-#pragma unroll
-      for (int T = 0; T < GN_T; ++T) a[T][t] = in ? A[(size_t)min(row0 + 16 * T + c, m - 1) * lda + col] : 0.0;
-    }
-    step(a, x);
-  }
-  if (SEG) {
-    double *P = out + (size_t)blockIdx.y * m * NB;
-#pragma unroll
-    for (int T = 0; T < GN_T; ++T)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int r = row0 + 16 * T + g + 4 * v;
-        if (!hi && r < m) P[(size_t)r * NB + c] = acc[T][v];
-      }
-    return;
-  }
-  double ss = 0.0;
-#pragma unroll
-  for (int T = 0; T < GN_T; ++T)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int r = row0 + 16 * T + g + 4 * v;
-      if (!hi && r < m) {
-        double *py = Y + (size_t)r * NB + c;
-        const double y = sx[c] * acc[T][v] + sy[c] * (*py);
-        *py = y;
-        ss += y * y;
-      }
-    }
-  ss += __shfl_xor(ss, 16, 64);  // lanes of equal c
-  ss += __shfl_xor(ss, 32, 64);
-  if (lane < NB) out[(size_t)wave * NB + lane] = ss;
-}
+// ---- scalar state ----------------------------------------------------------------------------
+// State A holds the columns after A V (k_lsqr_v writes it), state B at the end of an iteration
+// (k_lsqr_atu / k_lsqr_u write it): each kernel reads one and its first block writes the other, so
+// no block reads what another one of the same launch writes.
 
-// Y = sx .* sum_s P[s] + sy .* Y for the segmented product; part[block][k] = sum of the new Y^2.
-__global__ __launch_bounds__(256) void k_combine_n(int m, int nseg, const double *__restrict__ P,
-                                                   double *__restrict__ Y, const double *__restrict__ sx,
-                                                   const double *__restrict__ sy, double *__restrict__ part) {
-  __shared__ double red[4 * NB];
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;  // one (row, k) pair per thread
-  const int k = t & 7;
-  double y2 = 0.0;
-  if (t < m * NB) {
-    double s = 0.0;
-    for (int sg = 0; sg < nseg; ++sg) s += P[(size_t)sg * m * NB + t];
-    const double y = sx[k] * s + sy[k] * Y[t];
-    Y[t] = y;
-    y2 = y * y;
-  }
-  y2 += __shfl_xor(y2, 8, 64);
-  y2 += __shfl_xor(y2, 16, 64);
-  y2 += __shfl_xor(y2, 32, 64);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane < 8) red[wid * NB + lane] = y2;
-  __syncthreads();
-  if (threadIdx.x < 8)
-    part[(size_t)blockIdx.x * NB + threadIdx.x] =
-        (red[threadIdx.x] + red[NB + threadIdx.x]) + (red[2 * NB + threadIdx.x] + red[3 * NB + threadIdx.x]);
-}
-
-// P[s][j][k] = sum_{i in split s} A[i][j] Y[i][k]; one column per thread, splits over blockIdx.y.
-template <class ST>
-__global__ __launch_bounds__(256) void k_gemv_t(const ST *__restrict__ A, int64_t lda, int m, int n,
-                                                const double *__restrict__ Y, int rows_per_split,
-                                                double *__restrict__ P) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  const int s = blockIdx.y;
-  const int i0 = s * rows_per_split;
-  const int i1 = min(m, i0 + rows_per_split);
-  double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (j < n) {
-    const ST *col = A + j;
-    int i = i0;
-    for (; i + 4 <= i1; i += 4) {
-      const double a0 = (double)col[(size_t)i * lda], a1 = (double)col[(size_t)(i + 1) * lda];
-      const double a2 = (double)col[(size_t)(i + 2) * lda], a3 = (double)col[(size_t)(i + 3) * lda];
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        acc[k] += a0 * Y[(size_t)i * NB + k] + a1 * Y[(size_t)(i + 1) * NB + k] + a2 * Y[(size_t)(i + 2) * NB + k] +
-                  a3 * Y[(size_t)(i + 3) * NB + k];
-    }
-    for (; i < i1; ++i) {
-      const double a = (double)col[(size_t)i * lda];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) acc[k] += a * Y[(size_t)i * NB + k];
-    }
-    double4 *p = reinterpret_cast<double4 *>(P + ((size_t)s * n + j) * NB);
-    p[0] = make_double4(acc[0], acc[1], acc[2], acc[3]);
-    p[1] = make_double4(acc[4], acc[5], acc[6], acc[7]);
-  }
-}
-
-// The same for FP64 A with even lda on a 16-byte boundary: two columns per thread, so that a load
-// covers 1 KB of a row (64 lanes x 16 B) instead of 512 B.
-__global__ __launch_bounds__(256) void k_gemv_t2(const double *__restrict__ A, int64_t lda, int m, int n,
-                                                 const double *__restrict__ Y, int rows_per_split,
-                                                 double *__restrict__ P) {
-  typedef double d2n __attribute__((ext_vector_type(2)));
-  typedef const d2n __attribute__((address_space(1))) *gd2p;
-  const int j = 2 * (blockIdx.x * blockDim.x + threadIdx.x);
-  const int s = blockIdx.y;
-  const int i0 = s * rows_per_split;
-  const int i1 = min(m, i0 + rows_per_split);
-  if (j >= n) return;
-  d2n acc[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) acc[k] = d2n{0.0, 0.0};
-  // columns j, j + 1 (the second may be the row padding when n is odd: read, never stored)
-  const gd2p col = (gd2p)(A + j);
-  int i = i0;
-  for (; i + 4 <= i1; i += 4) {
-    d2n a[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) a[u] = __builtin_nontemporal_load(col + (size_t)(i + u) * (lda / 2));
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int k = 0; k < 8; ++k) acc[k] += a[u] * Y[(size_t)(i + u) * NB + k];
-  }
-  for (; i < i1; ++i) {
-    const d2n a = __builtin_nontemporal_load(col + (size_t)i * (lda / 2));
-#pragma unroll
-    for (int k = 0; k < 8; ++k) acc[k] += a * Y[(size_t)i * NB + k];
-  }
-  double4 *p = reinterpret_cast<double4 *>(P + ((size_t)s * n + j) * NB);
-  p[0] = make_double4(acc[0].x, acc[1].x, acc[2].x, acc[3].x);
-  p[1] = make_double4(acc[4].x, acc[5].x, acc[6].x, acc[7].x);
-  if (j + 1 < n) {
-    p[2] = make_double4(acc[0].y, acc[1].y, acc[2].y, acc[3].y);
-    p[3] = make_double4(acc[4].y, acc[5].y, acc[6].y, acc[7].y);
-  }
-}
-
-// V = sx .* sum_s P[s] + sy .* V; partV[block][k] = sum V^2, partW[block][k] = sum W^2 (old W).
-__global__ __launch_bounds__(256) void k_combine_t(int n, int nsplit, const double *__restrict__ P,
-                                                   double *__restrict__ V, const double *__restrict__ W,
-                                                   const double *__restrict__ sx, const double *__restrict__ sy,
-                                                   double *__restrict__ partV, double *__restrict__ partW) {
-  __shared__ double red[2 * NB * 4];
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;  // one (j, k) pair per thread
-  const int k = t & 7;
-  double v2 = 0.0, w2 = 0.0;
-  if (t < n * NB) {
-    double s = 0.0;
-    for (int sp = 0; sp < nsplit; ++sp) s += P[(size_t)sp * n * NB + t];
-    const double v = sx[k] * s + sy[k] * V[t];
-    V[t] = v;
-    v2 = v * v;
-    if (W) {
-      const double w = W[t];
-      w2 = w * w;
-    }
-  }
-  // reduce over lanes with equal k (lane & 7)
-  v2 += __shfl_xor(v2, 8, 64);
-  v2 += __shfl_xor(v2, 16, 64);
-  v2 += __shfl_xor(v2, 32, 64);
-  w2 += __shfl_xor(w2, 8, 64);
-  w2 += __shfl_xor(w2, 16, 64);
-  w2 += __shfl_xor(w2, 32, 64);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane < 8) {
-    red[wid * NB + lane] = v2;
-    red[4 * NB + wid * NB + lane] = w2;
-  }
-  __syncthreads();
-  if (threadIdx.x < 8) {
-    double a = 0.0, b = 0.0;
-    for (int w = 0; w < 4; ++w) {
-      a += red[w * NB + threadIdx.x];
-      b += red[4 * NB + w * NB + threadIdx.x];
-    }
-    partV[(size_t)blockIdx.x * NB + threadIdx.x] = a;
-    partW[(size_t)blockIdx.x * NB + threadIdx.x] = b;
-  }
-}
-
-// Column sums of the partials part[i][k], i < np, by a block of 256 threads (32 partial rows per
-// column in flight); thread k < NB receives the sum of column k. Every thread of the block calls it.
-__device__ double block_sum_parts(const double *__restrict__ part, int np, double *red) {
-  const int t = threadIdx.x, k = t & 7;
+// Column sums of the partials part[i][k], i < np, k < WD, by a block of BS threads, in two parts: a
+// thread's share (loads only: eight in flight, as the partials come from another kernel's blocks and
+// each round trip to them is most of a microsecond), then the sum over the block, which thread k < WD
+// receives for column k. Every thread of the block calls them; red holds BS / 64 * WD doubles.
+template <int WD, int BS>
+__device__ inline double thread_parts(const double *__restrict__ part, int np) {
+  const int k = threadIdx.x % WD;
   double s = 0.0;
-  for (int i = t >> 3; i < np; i += 32) s += part[(size_t)i * NB + k];
-  s += __shfl_xor(s, 8, 64);
-  s += __shfl_xor(s, 16, 64);
-  s += __shfl_xor(s, 32, 64);
+  for (int i = threadIdx.x / WD; i < np; i += 8 * (BS / WD)) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int j = i + u * (BS / WD);
+      v[u] = j < np ? part[(size_t)j * WD + k] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += v[u];
+  }
+  return s;
+}
+template <int WD, int BS>
+__device__ inline double block_sum(double s, double *red) {
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int o = WD; o < 64; o <<= 1) s += __shfl_xor(s, o, 64);
   __syncthreads();  // red may still be read from the previous call
-  if ((t & 63) < 8) red[(t >> 6) * NB + (t & 63)] = s;
+  if ((t & 63) < WD) red[(t >> 6) * WD + (t & 63)] = s;
   __syncthreads();
-  return t < NB ? (red[t] + red[NB + t]) + (red[2 * NB + t] + red[3 * NB + t]) : 0.0;
+  double v = 0.0;
+  if (t < WD)
+#pragma unroll
+    for (int w = 0; w < BS / 64; w += 4)
+      v += (red[w * WD + t] + red[(w + 1) * WD + t]) + (red[(w + 2) * WD + t] + red[(w + 3) * WD + t]);
+  return v;
 }
-#define LSQR_SCALAR_THREADS 256
-
-// ---- scalar kernels (one thread per column) -------------------------------------------------
-// start: U = b - A x_s is formed; beta = ||U||, btol = eps ||b|| / ||r0||; set scales for A^T u.
-__global__ void k_lsqr_start(LsqrState *st, const double *partU, int npU, const double *partB, int npB, double eps,
-                             double *sxt, double *syt) {
-  __shared__ double red[4 * NB];
-  const double sr = block_sum_parts(partU, npU, red);
-  const double sb = block_sum_parts(partB, npB, red);
-  const int k = threadIdx.x;
-  if (k >= NB) return;
-  LsqrState &S = st[k];
-  const double nrm_r = sqrt(sr);
-  const double nrm_b = sqrt(sb);
-  S.atol = eps;
-  S.btol = eps * nrm_b / nrm_r;
-  S.ctol = 1.0 / 1.0e8;
-  S.anorm = S.dnorm = S.res2 = S.xnorm = S.xnorm1 = S.z = 0.0;
-  S.cs2 = -1.0;
-  S.sn2 = 0.0;
-  S.itn = 0;
-  S.istop = 0;
-  S.beta = nrm_r;
-  S.alpha = 0.0;
-  if (S.active && S.beta > 0.0) {
-    sxt[k] = 1.0 / S.beta;
-    syt[k] = 0.0;
-  } else {
-    sxt[k] = 0.0;
-    syt[k] = 0.0;
-  }
+template <int WD, int BS>
+__device__ inline double block_sum_parts(const double *__restrict__ part, int np, double *red) {
+  return block_sum<WD, BS>(thread_parts<WD, BS>(part, np), red);
 }
 
-// after the first A^T u: alpha, w = v, the initial recurrence values (src/lib_lsqr.f:952-1008)
-__global__ void k_lsqr_init2(LsqrState *st, const double *partV, int npV, double *sxn, double *syn, double *inv_alpha) {
-  __shared__ double red[4 * NB];
-  const double sv = block_sum_parts(partV, npV, red);
-  const int k = threadIdx.x;
-  if (k >= NB) return;
-  LsqrState &S = st[k];
-  S.alpha = S.beta > 0.0 ? sqrt(sv) : 0.0;
-  inv_alpha[k] = S.alpha > 0.0 ? 1.0 / S.alpha : 0.0;
-  const double arnorm = S.alpha * S.beta;
-  S.rhobar = S.alpha;
-  S.phibar = S.beta;
-  S.bnorm = S.beta;
-  S.rnorm = S.beta;
-  if (arnorm == 0.0) S.active = 0;  // exact solution x = 0 (istop 0)
-  if (S.active) {
-    sxn[k] = 1.0 / S.alpha;
-    syn[k] = -S.alpha / S.beta;
-  } else {
-    sxn[k] = 0.0;
-    syn[k] = 0.0;
-  }
-}
-
-// after U = A v - alpha u: beta, anorm; scales of the A^T product
-__global__ void k_lsqr_mid(LsqrState *st, const double *partU, int npU, double *sxt, double *syt) {
-  __shared__ double red[4 * NB];
-  const double su = block_sum_parts(partU, npU, red);
-  const int k = threadIdx.x;
-  if (k >= NB) return;
-  LsqrState &S = st[k];
+// the end of an iteration from |V|^2 and |W|^2: alpha, the plane rotations and the convergence tests
+// (src/lib_lsqr.f:1015-1152); before the first one the initial recurrence values (:952-1008), whose
+// "update" W = V / alpha has t1 = t2 = 0
+__device__ inline void lsqr_end(LsqrState &S, double sv, double sw) {
   if (!S.active) {
-    sxt[k] = 0.0;
-    syt[k] = 0.0;
+    S.upd = 0;
     return;
   }
-  S.itn += 1;
-  const double beta = sqrt(su);
-  double temp = d2norm(S.alpha, beta);
-  temp = d2norm(temp, 0.0);
-  S.anorm = d2norm(S.anorm, temp);
-  const double alpha_old = S.alpha;
-  S.beta = beta;
-  if (beta > 0.0) {
-    sxt[k] = 1.0 / beta;
-    syt[k] = -beta / alpha_old;
-  } else {
-    sxt[k] = 0.0;
-    syt[k] = 1.0;  // v unchanged
-  }
-}
-
-// after V = A^T u - beta v: alpha, the plane rotations and the convergence tests
-// (src/lib_lsqr.f:1015-1152)
-__global__ void k_lsqr_end(LsqrState *st, const double *partV, const double *partW, int np, double *sxn, double *syn,
-                           double *t1o, double *t2o, double *inv_alpha, int *active_out) {
-  __shared__ double red[4 * NB];
-  const double sv = block_sum_parts(partV, np, red);
-  const double sw = block_sum_parts(partW, np, red);
-  const int k = threadIdx.x;
-  if (k >= NB) return;
-  LsqrState &S = st[k];
-  if (!S.active) {
-    t1o[k] = 0.0;
-    t2o[k] = 1.0;
-    inv_alpha[k] = 0.0;
-    sxn[k] = 0.0;
-    syn[k] = 0.0;
-    active_out[k] = 0;
+  S.upd = 1;  // the update of this iteration still applies (src/lib_lsqr.f:1057-1062)
+  if (S.itn == 0) {
+    S.alpha = S.beta > 0.0 ? sqrt(sv) : 0.0;
+    S.t1 = S.t2 = 0.0;
+    S.inv_alpha = S.alpha > 0.0 ? 1.0 / S.alpha : 0.0;
+    S.rhobar = S.alpha;
+    S.phibar = S.beta;
+    S.bnorm = S.beta;
+    S.rnorm = S.beta;
+    if (S.alpha * S.beta == 0.0) S.active = 0;  // exact solution x = 0 (istop 0)
     return;
   }
+  S.anorm = d2norm(S.anorm, d2norm(S.alpha, S.beta));  // (src/lib_lsqr.f:1009-1014, damp = 0)
   if (S.beta > 0.0) S.alpha = sqrt(sv);
   const double alpha = S.alpha, beta = S.beta;
   const double wnorm = sqrt(sw);
@@ -522,8 +130,9 @@ __global__ void k_lsqr_end(LsqrState *st, const double *partV, const double *par
   const double phi = cs * S.phibar;
   S.phibar = sn * S.phibar;
   const double tau = sn * phi;
-  const double t1 = phi / rho, t2 = -theta / rho, t3 = 1.0 / rho;
-  const double dknorm = t3 * wnorm;
+  S.t1 = phi / rho;
+  S.t2 = -theta / rho;
+  const double dknorm = (1.0 / rho) * wnorm;
   S.dnorm = d2norm(S.dnorm, dknorm);
   const double delta = S.sn2 * rho, gambar = -S.cs2 * rho;
   const double rhs = phi - delta * S.z, zbar = rhs / gambar;
@@ -553,102 +162,732 @@ __global__ void k_lsqr_end(LsqrState *st, const double *partV, const double *par
   if (test2 <= S.atol) istop = 2;
   if (test1 <= rtol) istop = 1;
   S.istop = istop;
-  t1o[k] = t1;
-  t2o[k] = t2;
-  inv_alpha[k] = alpha > 0.0 ? 1.0 / alpha : 1.0;
+  S.inv_alpha = alpha > 0.0 ? 1.0 / alpha : 1.0;
   if (istop != 0) S.active = 0;
-  active_out[k] = 1;  // the update of this iteration still applies (src/lib_lsqr.f:1057-1062)
-  if (S.active) {
-    sxn[k] = 1.0 / alpha;
-    syn[k] = -alpha / beta;
-  } else {
-    sxn[k] = 0.0;
-    syn[k] = 0.0;
+}
+
+// the scales of U = sx .* (A V) + sy .* U alone, which every block needs. A column that stops in this
+// very iteration still gets them: its U and V are not used any more and stay finite.
+__device__ inline void lsqr_u_scales(const LsqrState &S, double sv, double &sx, double &sy) {
+  sx = sy = 0.0;
+  if (!S.active) return;
+  const double alpha = S.beta > 0.0 ? sqrt(sv) : (S.itn == 0 ? 0.0 : S.alpha);
+  if (alpha != 0.0 && S.beta != 0.0) {  // (a NaN passes, as through the recurrences)
+    sx = 1.0 / alpha;
+    sy = -alpha / S.beta;
   }
 }
 
-// x += t1 w ; w = V * inv_alpha + t2 w  (src/lib_lsqr.f:1057-1062); columns with t1 = 0, t2 = 1,
-// inv_alpha = 0 stay unchanged.
-__global__ void k_lsqr_update(int n, double *__restrict__ X, double *__restrict__ W, const double *__restrict__ V,
-                              const double *__restrict__ t1, const double *__restrict__ t2,
-                              const double *__restrict__ inv_alpha, const int *__restrict__ was_active) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * NB) return;
-  const int k = t & 7;
-  if (!was_active[k]) return;
-  const double w = W[t];
-  X[t] += t1[k] * w;
-  W[t] = V[t] * inv_alpha[k] + t2[k] * w;
+template <int WD>
+__device__ inline bool any_active(const LsqrState *st) {
+  int a = 0;
+#pragma unroll
+  for (int k = 0; k < WD; ++k) a |= st[k].active;
+  return a != 0;
 }
 
-__global__ void k_scale_div(int n, const double *__restrict__ X0, const double *__restrict__ q, double *__restrict__ Xs) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * NB) return;
-  Xs[t] = q ? X0[t] / q[t >> 3] : X0[t];
-}
+// What the kernels of one solve share.
+struct LsqrVecs {
+  LsqrState *sa, *sb;
+  const double *pn;             // A V: nseg x m x WD
+  int nseg;
+  const double *uin;            // U before
+  double *uout;                 // U after
+  double *partU;                // |U|^2 per block of the kernel that forms U
+  const double *partV, *partW;  // |V|^2, |W|^2 per block of k_lsqr_v
+  int npv;
+};
 
-__global__ void k_scale_mul_add(int n, const double *__restrict__ q, const double *__restrict__ Xl,
-                                const double *__restrict__ X0, double *__restrict__ X) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * NB) return;
-  X[t] = (q ? q[t >> 3] * Xl[t] : Xl[t]) + X0[t];
-}
-
-__global__ void k_sumsq_parts(int n, const double *__restrict__ Y, double *__restrict__ part) {
-  __shared__ double red[NB * 4];
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  double y2 = 0.0;
-  if (t < n * NB) y2 = Y[t] * Y[t];
-  y2 += __shfl_xor(y2, 8, 64);
-  y2 += __shfl_xor(y2, 16, 64);
-  y2 += __shfl_xor(y2, 32, 64);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane < 8) red[wid * NB + lane] = y2;
+// The scales of U for the kernel that forms it, from a thread's share of the |V|^2 partials:
+// sc[0..WD-1] = sx, sc[WD..] = sy.
+template <int WD, int BS>
+__device__ inline void lsqr_u_prologue(const LsqrVecs &L, double svt, double *red, double *sc) {
+  const double sv = block_sum<WD, BS>(svt, red);
+  if (threadIdx.x < WD) {
+    double sx, sy;
+    lsqr_u_scales(L.sa[threadIdx.x], sv, sx, sy);
+    sc[threadIdx.x] = sx;
+    sc[WD + threadIdx.x] = sy;
+  }
   __syncthreads();
-  if (threadIdx.x < 8) {
-    double a = 0.0;
-    for (int w = 0; w < 4; ++w) a += red[w * NB + threadIdx.x];
-    part[(size_t)blockIdx.x * NB + threadIdx.x] = a;
+}
+// The end of the previous iteration, state A to state B, by a block of its own (the scalar chain of
+// some forty dependent operations would hold up a block that has a share of the product); host: a copy
+// for the host (pinned memory) or null.
+template <int WD, int BS>
+__device__ inline void lsqr_end_block(const LsqrVecs &L, double *red, LsqrState *host) {
+  const double svt = thread_parts<WD, BS>(L.partV, L.npv), swt = thread_parts<WD, BS>(L.partW, L.npv);
+  const double sv = block_sum<WD, BS>(svt, red), sw = block_sum<WD, BS>(swt, red);
+  if (threadIdx.x < WD) {
+    LsqrState S = L.sa[threadIdx.x];
+    lsqr_end(S, sv, sw);
+    L.sb[threadIdx.x] = S;
+    if (host) host[threadIdx.x] = S;
   }
+}
+
+// ---- A V ---------------------------------------------------------------------------------------
+// P[segment][row][k] = A X over the segment's columns, FP64 A on the matrix cores
+// (v_mfma_f64_16x16x4f64), NB interleaved columns. A block owns 16 T rows over the column segment
+// blockIdx.y, its eight waves an eighth of the segment's columns each (wcols, a multiple of 16); their
+// sums meet in LDS, so that a small system fills the chip with one or two segments instead of a dozen
+// partial results per row. Lane (g = lane / 16, c = lane % 16) feeds row c of tile t with columns
+// 16 kb + 4 g + s (s = 0..3, one instruction each) and column c of B = X (right-hand side c; the
+// upper half c >= NB is zero). The result D[g + 4 v][c] sits in register v of lane (g, c).
+// The tiles are read in whole 128-byte row segments and redistributed to the matrix-core layout
+// through LDS (rows padded to 18 doubles): the matrix-core lane pattern itself covers 16 half lines a
+// load, measured 4.6-5.3 against 6.9 TB/s on a 30 GB matrix. VEC: 16-byte loads (lane = row rr =
+// lane / 8 of an 8-row half tile, columns 2 p, 2 p + 1); otherwise (odd row length or an 8-byte base)
+// 8-byte loads, four rows of 16 columns each (3841^2: 46.8 -> 32.7 us).
+// The column split depends on the matrix shape only, and every row's sum runs over its columns in the
+// same order for every T, so the tile count (chosen by size or by the autotuner) never changes a bit.
+constexpr int AV_WAVES = 8;
+constexpr int AV_MAXCOLS = 1024;  // columns per wave at most
+
+// SEP: the waves' sums stay apart, P[segment * AV_WAVES + wave] (BiCGSTAB, whose iterates part from
+// each other by far more than rounding when the sums of a product are formed in another order).
+template <int T, bool VEC, bool SEP>
+__global__ __launch_bounds__(64 * AV_WAVES) void k_lsqr_av(const double *__restrict__ A, int64_t lda, int m, int n,
+                                                           const double *__restrict__ X, int wcols,
+                                                           double *__restrict__ P, const LsqrState *__restrict__ st) {
+  const bool act = !st || any_active<NB>(st);
+  typedef const double __attribute__((address_space(1))) *gdp;
+  constexpr int LR = 18;
+  __shared__ __attribute__((aligned(16))) double lt[AV_WAVES][T][16 * LR];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int row0 = blockIdx.x * 16 * T;
+  const int g = lane >> 4, c = lane & 15;
+  const bool hi = c >= NB;
+  const int k0 = (blockIdx.y * AV_WAVES + wid) * wcols, kend = min(n, k0 + wcols);
+  gdp lrow[T][VEC ? 2 : 4];
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    if (VEC) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        lrow[t][h] = (gdp)(A + (size_t)min(row0 + 16 * t + 8 * h + (lane >> 3), m - 1) * lda + 2 * (lane & 7));
+    } else {
+#pragma unroll
+      for (int h = 0; h < 4; ++h) lrow[t][h] = (gdp)(A + (size_t)min(row0 + 16 * t + 4 * h + g, m - 1) * lda + c);
+    }
+  }
+  const gdp xb = (gdp)(X + (size_t)(4 * g) * NB + (c & (NB - 1)));
+  d4v acc[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t) acc[t] = d4v{0.0, 0.0, 0.0, 0.0};
+  // raw operands of one 16-column block; the matrix is streamed: non-temporal, so that X keeps its place in L2
+  auto load = [&](int kb, double (&a)[T][4], double (&x)[4]) {
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      if constexpr (VEC) {
+        const d2n u = __builtin_nontemporal_load((const d2n __attribute__((address_space(1))) *)(lrow[t][0] + 16 * kb));
+        const d2n w = __builtin_nontemporal_load((const d2n __attribute__((address_space(1))) *)(lrow[t][1] + 16 * kb));
+        a[t][0] = u.x;
+        a[t][1] = u.y;
+        a[t][2] = w.x;
+        a[t][3] = w.y;
+      } else {
+#pragma unroll
+        for (int h = 0; h < 4; ++h) a[t][h] = __builtin_nontemporal_load(lrow[t][h] + 16 * kb);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x[s] = xb[(size_t)(16 * kb + s) * NB];
+  };
+  // row segments -> LDS -> matrix-core values (in place); the tiles are per wave
+  auto stage = [&](double (&a)[T][4]) {
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      double *l = lt[wid][t];
+      if constexpr (VEC) {
+        const int rr = lane >> 3, p = lane & 7;
+        *(d2n *)&l[rr * LR + 2 * p] = d2n{a[t][0], a[t][1]};
+        *(d2n *)&l[(8 + rr) * LR + 2 * p] = d2n{a[t][2], a[t][3]};
+      } else {
+#pragma unroll
+        for (int h = 0; h < 4; ++h) l[(4 * h + g) * LR + c] = a[t][h];
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const d2n u = *(const d2n *)&lt[wid][t][c * LR + 4 * g];
+      const d2n w = *(const d2n *)&lt[wid][t][c * LR + 4 * g + 2];
+      a[t][0] = u.x;
+      a[t][1] = u.y;
+      a[t][2] = w.x;
+      a[t][3] = w.y;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  auto step = [&](const double (&a)[T][4], const double (&x)[4]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const double b = hi ? 0.0 : x[s];
+#pragma unroll
+      for (int t = 0; t < T; ++t) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t][s], b, acc[t], 0, 0, 0);
+    }
+  };
+  // full 16-column blocks, two register sets in turn: the operands of the next block are requested
+  // before the products of the current one (the last prefetch re-reads the final block)
+  int kb = k0 >> 4;
+  const int kb_end = kend >> 4;
+  if (kb < kb_end) {
+    double a0[T][4], a1[T][4], x0[4], x1[4];
+    load(kb, a0, x0);
+    if (!act) return;  // uniform over the grid; the first loads are under way while the state arrives
+    for (; kb + 1 < kb_end; kb += 2) {
+      load(kb + 1, a1, x1);
+      __builtin_amdgcn_sched_barrier(0);
+      stage(a0);
+      step(a0, x0);
+      __builtin_amdgcn_sched_barrier(0);
+      load(min(kb + 2, kb_end - 1), a0, x0);
+      __builtin_amdgcn_sched_barrier(0);
+      stage(a1);
+      step(a1, x1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (kb < kb_end) {  // odd count: a0 holds block kb
+      stage(a0);
+      step(a0, x0);
+      ++kb;
+    }
+  }
+  if (!act) return;
+  if (16 * kb < kend) {  // last, partial column block of the matrix: masked
+    double a[T][4], x[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int col = 16 * kb + 4 * g + s;
+      const bool in = col < kend;
+      x[s] = in ? X[(size_t)col * NB + (c & (NB - 1))] : 0.0;
+#pragma unroll
+      for (int t = 0; t < T; ++t) a[t][s] = in ? A[(size_t)min(row0 + 16 * t + c, m - 1) * lda + col] : 0.0;
+    }
+    step(a, x);
+  }
+  if (SEP) {
+    if (k0 < n) {
+      double *p = P + (size_t)(blockIdx.y * AV_WAVES + wid) * m * NB;
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int r = row0 + 16 * t + g + 4 * v;
+          if (!hi && r < m) p[(size_t)r * NB + c] = acc[t][v];
+        }
+    }
+    return;
+  }
+  // the waves' sums, wave by wave: red[w][row of the block][k] over the staging tiles (16 T x 8 doubles
+  // of the 16 T x 18 of each wave)
+  __syncthreads();
+  double *red = &lt[0][0][0];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (!hi) red[(wid * 16 * T + 16 * t + g + 4 * v) * NB + c] = acc[t][v];
+  __syncthreads();
+  for (int e = threadIdx.x; e < 16 * T * NB; e += 64 * AV_WAVES) {
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < AV_WAVES; ++w) s += red[w * 16 * T * NB + e];
+    if (row0 + e / NB < m) P[((size_t)blockIdx.y * m + row0) * NB + e] = s;
+  }
+}
+
+// P[segment][row] = A x for one right-hand side: a wave owns eight rows over a column segment, 16 bytes
+// per lane and row (1 KB of a row per load), two register sets in turn; bound by the matrix stream.
+template <class ST>
+__global__ __launch_bounds__(256) void k_lsqr_av1(const ST *__restrict__ A, int64_t lda, int m, int n,
+                                                  const double *__restrict__ x, int seglen, double *__restrict__ P,
+                                                  const LsqrState *__restrict__ st) {
+  if (!st->active) return;
+  constexpr int CPL = 16 / sizeof(ST);  // columns per lane and load
+  constexpr int STEP = 64 * CPL;
+  typedef ST vec __attribute__((ext_vector_type(CPL)));
+  typedef const vec __attribute__((address_space(1))) *gvp;
+  const int lane = threadIdx.x & 63;
+  const int row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 8;
+  if (row0 >= m) return;  // no barriers below
+  const int k0 = blockIdx.y * seglen, kend = min(n, k0 + seglen);
+  const ST *row[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) row[r] = A + (size_t)min(row0 + r, m - 1) * lda;
+  double acc[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) acc[r] = 0.0;
+  struct Set {
+    vec a[8];
+    double x[CPL];
+  };
+  auto load = [&](int k, Set &s) {
+    const int j = k + CPL * lane;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) s.a[r] = __builtin_nontemporal_load((gvp)(row[r] + j));
+#pragma unroll
+    for (int q = 0; q < CPL; ++q) s.x[q] = x[j + q];
+  };
+  auto step = [&](const Set &s) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+#pragma unroll
+      for (int q = 0; q < CPL; ++q) acc[r] += (double)s.a[r][q] * s.x[q];
+  };
+  const int nfull = (kend - k0) / STEP;
+  int k = k0;
+  if (nfull > 0) {
+    Set s0, s1;
+    load(k, s0);
+    int i = 0;
+    for (; i + 1 < nfull; i += 2) {
+      load(k + STEP, s1);
+      __builtin_amdgcn_sched_barrier(0);
+      step(s0);
+      __builtin_amdgcn_sched_barrier(0);
+      load(i + 2 < nfull ? k + 2 * STEP : k, s0);
+      __builtin_amdgcn_sched_barrier(0);
+      step(s1);
+      __builtin_amdgcn_sched_barrier(0);
+      k += 2 * STEP;
+    }
+    if (i < nfull) {
+      step(s0);
+      k += STEP;
+    }
+  }
+  for (int j = k + lane; j < kend; j += 64) {  // the last columns of the segment
+    const double xv = x[j];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) acc[r] += (double)row[r][j] * xv;
+  }
+  // reduce-scatter over the lanes: lane l ends with the sum of row l / 8
+#pragma unroll
+  for (int half = 4; half >= 1; half >>= 1) {
+    const bool up = (lane & (8 * half)) != 0;
+#pragma unroll
+    for (int i = 0; i < half; ++i) {
+      const double keep = up ? acc[i + half] : acc[i];
+      const double send = up ? acc[i] : acc[i + half];
+      acc[i] = keep + __shfl_xor(send, 8 * half, 64);
+    }
+  }
+  double s = acc[0];
+  s += __shfl_xor(s, 4, 64);
+  s += __shfl_xor(s, 2, 64);
+  s += __shfl_xor(s, 1, 64);
+  const int r = row0 + (lane >> 3);
+  if ((lane & 7) == 0 && r < m) P[(size_t)blockIdx.y * m + r] = s;
+}
+
+// ---- A^T U -------------------------------------------------------------------------------------
+// P[split][j][k] = sum over the split's rows of A[i][j] U[i][k]. A block owns CW columns over the rows
+// of split blockIdx.y, its eight waves rw rows each; U of the block's rows sits in LDS (read as
+// broadcasts) and the waves' sums meet there in a fixed order, which leaves an eighth of the partial
+// results of a wave-wide split. FORM: U is formed here from the partials of A V (see the head of the
+// file), by every column panel for its own use and by the first one (blockIdx.x = 0) for keeping.
+// A lane holds the columns of one 16-byte load of a row and their sums; the first rows are requested before
+// U is formed. Bound by the matrix stream; 3120^2 with 6 right-hand sides 22.6 -> 20.0 us, and an
+// eighth of the partial results for k_lsqr_v (13.8 -> 4.8 us); 4881 x 2717 with one 24.3 -> 19.4 us.
+constexpr int AT_WAVES = 8, AT_MAXRW = 32;
+constexpr int at_cols(size_t elem) { return 64 * 16 / (int)elem; }  // a 16-byte load per lane
+
+template <class ST, int WD, bool FORM>
+__global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restrict__ A, int64_t lda, int m, int n, int rw,
+                                                            LsqrVecs L, double *__restrict__ P) {
+  constexpr int BS = 64 * AT_WAVES, CW = at_cols(sizeof(ST)), LV = CW / 64;  // columns per lane
+  constexpr int RMAX = AT_WAVES * AT_MAXRW;
+  typedef ST vec __attribute__((ext_vector_type(LV)));
+  typedef const vec __attribute__((address_space(1))) *gvp;
+  __shared__ __attribute__((aligned(16))) double ul[RMAX * WD];
+  __shared__ __attribute__((aligned(16))) double red[AT_WAVES / 2 * CW * WD];
+  __shared__ double sc[2 * WD];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  if (FORM && blockIdx.y == gridDim.y - 1) {  // one block more for the scalars
+    if (blockIdx.x == 0) lsqr_end_block<WD, BS>(L, red, nullptr);
+    return;
+  }
+  const int i0 = blockIdx.y * AT_WAVES * rw, nr = min(AT_WAVES * rw, m - i0);  // nr >= 1
+  // the lane's columns j ..; past the end column 0 is loaded and nothing stored (a load that starts before
+  // the end may reach into the row padding)
+  const int j = blockIdx.x * CW + LV * lane, jc = j < n ? j : 0;
+  const int r0 = wid * rw;  // the wave's rows within the block
+  const int rn = max(0, min(rw, nr - r0));
+  const ST *base = A + (size_t)i0 * lda;
+  constexpr int UN = WD == 1 ? 8 : 4;  // rows per register set
+  struct Set {
+    vec a[UN];
+  };
+  auto load = [&](int r, Set &s) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const ST *row = base + (size_t)min(r0 + min(r + u, max(rn - 1, 0)), nr - 1) * lda;
+      s.a[u] = __builtin_nontemporal_load((gvp)(row + jc));
+    }
+  };
+  Set s0, s1;
+  load(0, s0);  // the first rows are under way while U is formed
+  __builtin_amdgcn_sched_barrier(0);
+  if (FORM) {
+    // everything the block reads before A goes out at once: the state, the norm partials, the sums
+    // over the column segments and the old U
+    constexpr int NE = RMAX * WD / BS > 0 ? RMAX * WD / BS : 1;  // values of U per thread
+    const bool act = any_active<WD>(L.sa);
+    const double svt = thread_parts<WD, BS>(L.partV, L.npv);
+    double se[NE], ue[NE];
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+      const int e = tid + i * BS;
+      se[i] = ue[i] = 0.0;
+      if (e < nr * WD) {
+        const size_t o = (size_t)i0 * WD + e;
+        ue[i] = L.uin[o];
+        for (int sg = 0; sg < L.nseg; ++sg) se[i] += L.pn[(size_t)sg * m * WD + o];
+      }
+    }
+    if (!act) return;  // uniform over the grid
+    lsqr_u_prologue<WD, BS>(L, svt, red, sc);
+    const bool keep = blockIdx.x == 0;
+    const int k = tid % WD;  // the same for all of a thread's values (BS % WD == 0)
+    double y2 = 0.0;
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+      const int e = tid + i * BS;
+      const double u = e < nr * WD ? sc[k] * se[i] + sc[WD + k] * ue[i] : 0.0;
+      if (keep && e < nr * WD) L.uout[(size_t)i0 * WD + e] = u;
+      y2 += u * u;
+      if (e < RMAX * WD) ul[e] = u;
+    }
+    if (keep) {  // uniform over the block
+      const double s = block_sum<WD, BS>(y2, red);
+      if (tid < WD) L.partU[(size_t)blockIdx.y * WD + tid] = s;
+    }
+  } else {
+    if (!any_active<WD>(L.sb)) return;
+    for (int e = tid; e < AT_WAVES * rw * WD; e += BS) ul[e] = e < nr * WD ? L.uin[(size_t)i0 * WD + e] : 0.0;
+  }
+  __syncthreads();
+  double acc[LV][WD];
+#pragma unroll
+  for (int q = 0; q < LV; ++q)
+#pragma unroll
+    for (int k = 0; k < WD; ++k) acc[q][k] = 0.0;
+  auto step = [&](int r, const Set &s) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      double uv[WD];
+#pragma unroll
+      for (int k = 0; k < WD; ++k) uv[k] = ul[(r0 + r + u) * WD + k];  // zero past the last row
+#pragma unroll
+      for (int q = 0; q < LV; ++q) {
+        const double av = (double)s.a[u][q];
+#pragma unroll
+        for (int k = 0; k < WD; ++k) acc[q][k] += av * uv[k];
+      }
+      // (the U of all the rows at once would take the registers of half the waves in flight)
+      if (WD > 1 && u % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // rw is a multiple of 2 UN: two register sets in turn, the last loads repeat the last row
+#pragma unroll 1
+  for (int r = 0; r < rn; r += 2 * UN) {
+    load(r + UN, s1);
+    __builtin_amdgcn_sched_barrier(0);
+    step(r, s0);
+    __builtin_amdgcn_sched_barrier(0);
+    load(r + 2 * UN, s0);
+    __builtin_amdgcn_sched_barrier(0);
+    step(r + UN, s1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // the waves' sums: (0 + 4) (1 + 5) (2 + 6) (3 + 7), then (0 + 2) (1 + 3), then (0 + 1)
+#pragma unroll
+  for (int half = AT_WAVES / 2; half >= 1; half >>= 1) {
+    __syncthreads();
+    if (wid >= half && wid < 2 * half) {
+      double *d = red + (size_t)(wid - half) * CW * WD;
+#pragma unroll
+      for (int q = 0; q < LV; ++q)
+#pragma unroll
+        for (int k = 0; k < WD; ++k) d[(q * WD + k) * 64 + lane] = acc[q][k];
+    }
+    __syncthreads();
+    if (wid < half) {
+      const double *d = red + (size_t)wid * CW * WD;
+#pragma unroll
+      for (int q = 0; q < LV; ++q)
+#pragma unroll
+        for (int k = 0; k < WD; ++k) acc[q][k] += d[(q * WD + k) * 64 + lane];
+    }
+  }
+  if (wid != 0) return;
+#pragma unroll
+  for (int q = 0; q < LV; ++q)
+    if (j + q < n) {
+      double *p = P + ((size_t)blockIdx.y * n + j + q) * WD;
+#pragma unroll
+      for (int k = 0; k < WD; ++k) p[k] = acc[q][k];
+    }
+}
+
+// U formed on its own (many column segments, CSR): U = sx .* sum_s P[s] + sy .* U, |U|^2 per block.
+template <int WD>
+__global__ __launch_bounds__(256) void k_lsqr_u(int m, LsqrVecs L) {
+  __shared__ double red[4 * WD];
+  __shared__ double sc[2 * WD];
+  if (blockIdx.x == gridDim.x - 1) {  // one block more for the scalars
+    lsqr_end_block<WD, 256>(L, red, nullptr);
+    return;
+  }
+  const bool act = any_active<WD>(L.sa);
+  const double svt = thread_parts<WD, 256>(L.partV, L.npv);
+  const int t = blockIdx.x * 256 + threadIdx.x, k = t % WD;
+  double s = 0.0, y2 = 0.0;
+  if (t < m * WD)
+    for (int sg = 0; sg < L.nseg; ++sg) s += L.pn[(size_t)sg * m * WD + t];
+  if (!act) return;  // uniform over the grid
+  lsqr_u_prologue<WD, 256>(L, svt, red, sc);
+  if (t < m * WD) {
+    const double u = sc[k] * s + sc[WD + k] * L.uin[t];
+    L.uout[t] = u;
+    y2 = u * u;
+  }
+  const double sum = block_sum<WD, 256>(y2, red);
+  if (threadIdx.x < WD) L.partU[(size_t)blockIdx.x * WD + threadIdx.x] = sum;
+}
+
+// ---- V, X and W --------------------------------------------------------------------------------
+// V = sx .* sum_s P[s] + sy .* V, with the update of X and W the previous iteration owes (it needs the
+// old V): X += t1 W, W = V / alpha + t2 W; |V|^2 and |W|^2 per block. beta = |U| first. INIT: V = sum_s P[s] / beta, W = 0 before the first iteration.
+// A block's 256 threads are 64 values (j, k) times four quarters of the splits; at most V_MAXBLOCKS
+// blocks, so that the norms are few partials for the kernels that sum them.
+constexpr int V_QUARTERS = 4, V_VALUES = 256 / V_QUARTERS, V_MAXBLOCKS = 512;
+
+template <int WD, bool INIT>
+__global__ __launch_bounds__(256) void k_lsqr_v(int n, int nsplit, const double *__restrict__ P, LsqrState *sa,
+                                                LsqrState *sb, const double *__restrict__ partU, int npu,
+                                                double *__restrict__ V, double *__restrict__ X, double *__restrict__ W,
+                                                double *__restrict__ partV, double *__restrict__ partW) {
+  constexpr int NV = V_VALUES;
+  __shared__ double red[4 * WD];
+  __shared__ double sc[2 * WD], st[3 * WD];
+  __shared__ int su[WD];
+  __shared__ double part[V_QUARTERS][NV];
+  const int tid = threadIdx.x;
+  // k is the same in every turn of the loop below (NV % WD == 0, also times the grid)
+  const int val = tid % NV, q = tid / NV, k = val % WD;
+  struct Turn {
+    double s, v, w, x;  // the quarter's share of the splits; the old V, W, X (first wave)
+  };
+  auto load = [&](int t, Turn &c) {
+    c.s = c.v = c.w = c.x = 0.0;
+    if (t >= n * WD) return;
+    const double *p = P + t;
+    const size_t stride = (size_t)n * WD;
+    for (int sp = q; sp < nsplit; sp += 8 * V_QUARTERS) {
+      double a[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) a[u] = sp + u * V_QUARTERS < nsplit ? p[(sp + u * V_QUARTERS) * stride] : 0.0;
+      c.s += ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+    }
+    if (!INIT && q == 0) {
+      c.v = V[t];
+      c.w = W[t];
+      c.x = X[t];
+    }
+  };
+  // the first turn's loads go out with those of the scalars
+  Turn cur;
+  if (!INIT) {
+    int any = 0;
+#pragma unroll
+    for (int c = 0; c < WD; ++c) any |= sb[c].active | sb[c].upd;
+    const double uut = thread_parts<WD, 256>(partU, npu);
+    load(blockIdx.x * NV + val, cur);
+    if (!any) return;  // uniform over the grid; state A holds the stopped columns already
+    const double uu = block_sum<WD, 256>(uut, red);
+    if (tid < WD) {
+      LsqrState S = sb[tid];
+      st[tid] = S.t1;
+      st[WD + tid] = S.t2;
+      st[2 * WD + tid] = S.inv_alpha;
+      su[tid] = S.upd;
+      double sx = 0.0, sy = 0.0;
+      if (S.active) {
+        const double beta = sqrt(uu);
+        sx = beta > 0.0 ? 1.0 / beta : 0.0;
+        sy = beta > 0.0 ? -beta / S.alpha : 1.0;  // beta = 0: V unchanged
+        S.itn += 1;
+        S.beta = beta;
+      }
+      sc[tid] = sx;
+      sc[WD + tid] = sy;
+      if (blockIdx.x == gridDim.x - 1) sa[tid] = S;
+    }
+  } else {
+    load(blockIdx.x * NV + val, cur);
+    if (tid < WD) sc[tid] = sb[tid].active && sb[tid].beta > 0.0 ? 1.0 / sb[tid].beta : 0.0;
+  }
+  double v2 = 0.0, w2 = 0.0;
+  for (int t0 = blockIdx.x * NV; t0 < n * WD; t0 += gridDim.x * NV) {  // uniform over the block
+    const int t = t0 + val;
+    __syncthreads();  // the scalars are there; the sums of the previous turn are read
+    part[q][val] = cur.s;
+    __syncthreads();
+    const double vold = cur.v, wold = cur.w, xold = cur.x;
+    if (t0 + gridDim.x * NV < n * WD) load(t + gridDim.x * NV, cur);
+    if (q == 0 && t < n * WD) {  // the first wave holds the turn's values
+      const double s = (part[0][val] + part[1][val]) + (part[2][val] + part[3][val]);
+      if (INIT) {
+        const double v = sc[k] * s;
+        V[t] = v;
+        W[t] = 0.0;
+        X[t] = 0.0;
+        v2 += v * v;
+      } else {
+        double w = wold;
+        if (su[k]) {
+          X[t] = xold + st[k] * wold;
+          w = vold * st[2 * WD + k] + st[WD + k] * wold;
+          W[t] = w;
+        }
+        const double v = sc[k] * s + sc[WD + k] * vold;
+        V[t] = v;
+        v2 += v * v;
+        w2 += w * w;
+      }
+    }
+  }
+  if (q != 0) return;
+#pragma unroll
+  for (int o = WD; o < 64; o <<= 1) {
+    v2 += __shfl_xor(v2, o, 64);
+    w2 += __shfl_xor(w2, o, 64);
+  }
+  if (tid < WD) {
+    partV[(size_t)blockIdx.x * WD + tid] = v2;
+    partW[(size_t)blockIdx.x * WD + tid] = w2;
+  }
+}
+
+// ---- start, polls and finish -------------------------------------------------------------------
+// column k of the interleaved X0 (stride NB) as the solve's own start vector, and x_s = x0 / q
+template <int WD>
+__global__ void k_lsqr_x0(int n, const double *__restrict__ X0, const double *__restrict__ q, double *__restrict__ Xs) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n * WD) return;
+  const int j = t / WD, k = t % WD;
+  const double x = X0[(size_t)j * NB + k];
+  Xs[t] = q ? x / q[j] : x;
+}
+
+// U = B - sum_s P[s] (P = A x_s); |U|^2 and |B|^2 per block
+template <int WD>
+__global__ __launch_bounds__(256) void k_lsqr_u0(int m, int nseg, const double *__restrict__ P,
+                                                 const double *__restrict__ B, double *__restrict__ U,
+                                                 double *__restrict__ partU, double *__restrict__ partB) {
+  __shared__ double red[2][4 * WD];
+  const int t = blockIdx.x * 256 + threadIdx.x, k = t % WD;
+  double u2 = 0.0, b2 = 0.0;
+  if (t < m * WD) {
+    const double b = B[(size_t)(t / WD) * NB + k];
+    double s = 0.0;
+    for (int sg = 0; sg < nseg; ++sg) s += P[(size_t)sg * m * WD + t];
+    const double u = b - s;
+    U[t] = u;
+    u2 = u * u;
+    b2 = b * b;
+  }
+#pragma unroll
+  for (int o = WD; o < 64; o <<= 1) {
+    u2 += __shfl_xor(u2, o, 64);
+    b2 += __shfl_xor(b2, o, 64);
+  }
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if (lane < WD) {
+    red[0][wid * WD + lane] = u2;
+    red[1][wid * WD + lane] = b2;
+  }
+  __syncthreads();
+  if (threadIdx.x < WD) {
+    const int c = threadIdx.x;
+    partU[(size_t)blockIdx.x * WD + c] = (red[0][c] + red[0][WD + c]) + (red[0][2 * WD + c] + red[0][3 * WD + c]);
+    partB[(size_t)blockIdx.x * WD + c] = (red[1][c] + red[1][WD + c]) + (red[1][2 * WD + c] + red[1][3 * WD + c]);
+  }
+}
+
+// beta = ||U||, btol = eps ||b|| / ||r0|| (src/lib_lsqr.f:84-100); both states
+template <int WD>
+__global__ __launch_bounds__(256) void k_lsqr_start(LsqrState *sa, LsqrState *sb, const double *partU,
+                                                    const double *partB, int np, double eps, int nrhs, int itnlim) {
+  __shared__ double red[4 * WD];
+  const double sr = block_sum_parts<WD, 256>(partU, np, red);
+  const double sn = block_sum_parts<WD, 256>(partB, np, red);
+  const int k = threadIdx.x;
+  if (k >= WD) return;
+  LsqrState S = {};
+  const double nrm_r = sqrt(sr);
+  const double nrm_b = sqrt(sn);
+  S.atol = eps;
+  S.btol = eps * nrm_b / nrm_r;
+  S.ctol = 1.0 / 1.0e8;
+  S.cs2 = -1.0;
+  S.beta = nrm_r;
+  S.active = k < nrhs ? 1 : 0;
+  S.itnlim = itnlim;
+  sa[k] = S;
+  sb[k] = S;
+}
+
+// the state at the end of the last enqueued iteration, for the host: what the next k_lsqr_atu writes
+template <int WD>
+__global__ __launch_bounds__(256) void k_lsqr_poll(LsqrVecs L, LsqrState *host) {
+  __shared__ double red[4 * WD];
+  lsqr_end_block<WD, 256>(L, red, host);
+}
+
+// x = q .* (x + the owed update) + x0, into the interleaved X
+template <int WD>
+__global__ void k_lsqr_finish(int n, const double *__restrict__ q, const double *__restrict__ Xl,
+                              const double *__restrict__ W, const LsqrState *__restrict__ sb, double *__restrict__ X) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n * WD) return;
+  const int j = t / WD, k = t % WD;
+  const double x = Xl[t] + (sb[k].upd ? sb[k].t1 * W[t] : 0.0);
+  double *px = X + (size_t)j * NB + k;
+  *px = (q ? q[j] * x : x) + *px;
+}
+
+// Y = sum_s P[s]: a product on its own (BiCGSTAB)
+__global__ __launch_bounds__(256) void k_combine_n(int m, int nseg, const double *__restrict__ P,
+                                                   double *__restrict__ Y) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;  // one (row, k) pair per thread
+  if (t >= m * NB) return;
+  double s = 0.0;
+  for (int sg = 0; sg < nseg; ++sg) s += P[(size_t)sg * m * NB + t];
+  Y[t] = s;
 }
 
 // ---- sparse products (CSR) -----------------------------------------------------------------------
-// Row-parallel CSR product over NB interleaved columns, 0-based row pointers and columns: thread
-// (row r, column k). UPDATE: Y = sx .* (A X) + sy .* Y and part[block][k] = sum of the new Y^2 over
-// the block's 32 rows (the layout of k_combine_n); otherwise the raw product goes to Y (A^T U into
-// the split partials of k_combine_t, one split). Each row sums its entries in stored order.
-template <bool UPDATE>
+// y = A x, 0-based row pointers and columns: eight lanes per row take its entries in turn, their sums
+// meet in a fixed order. For one right-hand side (the Fortran seam has one).
 __global__ __launch_bounds__(256) void k_csr_mv(int rows, const int64_t *__restrict__ ia, const int32_t *__restrict__ ja,
-                                                const double *__restrict__ va, const double *__restrict__ X,
-                                                double *__restrict__ Y, const double *__restrict__ sx,
-                                                const double *__restrict__ sy, double *__restrict__ part) {
-  __shared__ double red[4][NB];
+                                                const double *__restrict__ va, const double *__restrict__ x,
+                                                double *__restrict__ y, const LsqrState *__restrict__ st) {
+  if (!st->active) return;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = t >> 3, k = t & 7;
-  double y = 0.0;
-  if (r < rows) {
-    double acc = 0.0;
-    for (int64_t p = ia[r]; p < ia[r + 1]; ++p) acc += va[p] * X[(size_t)ja[p] * NB + k];
-    double *py = Y + (size_t)r * NB + k;
-    if (UPDATE) {
-      y = sx[k] * acc + sy[k] * (*py);
-      *py = y;
-    } else {
-      *py = acc;
-    }
-  }
-  if (UPDATE) {
-    double y2 = y * y;
-    y2 += __shfl_xor(y2, 8, 64);
-    y2 += __shfl_xor(y2, 16, 64);
-    y2 += __shfl_xor(y2, 32, 64);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane < NB) red[wid][lane] = y2;
-    __syncthreads();
-    if (threadIdx.x < NB)
-      part[(size_t)blockIdx.x * NB + threadIdx.x] =
-          (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
-  }
+  const int r = t >> 3, l = t & 7;
+  double acc = 0.0;
+  if (r < rows)
+    for (int64_t p = ia[r] + l; p < ia[r + 1]; p += 8) acc += va[p] * x[ja[p]];
+  acc += __shfl_xor(acc, 1, 64);
+  acc += __shfl_xor(acc, 2, 64);
+  acc += __shfl_xor(acc, 4, 64);
+  if (r < rows && l == 0) y[r] = acc;
 }
 
 // ---- column scaling (lsqr_precon) ------------------------------------------------------------
@@ -715,6 +954,51 @@ int andr_colscale(andr_ctx *ctx, void *A, bool fp32, int64_t lda, int m, int n, 
 
 namespace {
 
+constexpr int LSQR_POLL = 8;  // iterations between reads of the convergence state
+
+// More column segments than this and U is formed by a kernel of its own: in k_lsqr_atu every panel of
+// columns sums them again, WD * 8 bytes a row and segment (L2) against 1 KB of A.
+constexpr int LSQR_FUSE_SEG = 2, LSQR_FUSE_SEG1 = 16;
+
+// How A X splits its columns, a function of the shape alone (so that the tile count never changes the
+// sums): nseg column segments of AV_WAVES * wcols columns. Two segments while there are fewer than 128
+// 64-row tiles, else one wave per SIMD or less would be in flight; no more than AV_MAXCOLS columns per wave.
+struct AvShape {
+  int nseg, wcols;
+};
+AvShape av_shape(int m, int n) {
+  AvShape s;
+  s.nseg = std::max((n + AV_WAVES * AV_MAXCOLS - 1) / (AV_WAVES * AV_MAXCOLS), m < 8192 && n >= 512 ? 2 : 1);
+  s.wcols = ((n + AV_WAVES * s.nseg - 1) / (AV_WAVES * s.nseg) + 15) / 16 * 16;
+  s.nseg = (n + AV_WAVES * s.wcols - 1) / (AV_WAVES * s.wcols);
+  return s;
+}
+// 16-row tiles per block where the autotuner does not choose: two while four leave the chip short of
+// blocks (3120^2: 18.1 us with four, 15.8 with two)
+int av_tiles(int m, int nseg) { return (m + 63) / 64 * nseg < 512 ? 2 : 4; }
+
+// A X into the segment partials P (FP64, NB interleaved columns)
+template <int T, bool SEP>
+void launch_av_t(hipStream_t st, const double *A, int64_t lda, int m, int n, const double *X, AvShape sh, double *P,
+                 const LsqrState *s) {
+  const dim3 blk(64 * AV_WAVES);
+  if (lda % 2 == 0 && ((uintptr_t)A % 16) == 0) {
+    hipLaunchKernelGGL((k_lsqr_av<T, true, SEP>), dim3((m + 16 * T - 1) / (16 * T), sh.nseg), blk, 0, st, A, lda, m, n, X,
+                       sh.wcols, P, s);
+  } else {
+    constexpr int U = T < 4 ? T : 4;  // eight tiles of 8-byte loads do not fit the registers
+    hipLaunchKernelGGL((k_lsqr_av<U, false, SEP>), dim3((m + 16 * U - 1) / (16 * U), sh.nseg), blk, 0, st, A, lda, m, n, X,
+                       sh.wcols, P, s);
+  }
+}
+template <bool SEP>
+void launch_av(hipStream_t st, int tiles, const double *A, int64_t lda, int m, int n, const double *X, AvShape sh,
+               double *P, const LsqrState *s) {
+  if (tiles == 2) launch_av_t<2, SEP>(st, A, lda, m, n, X, sh, P, s);
+  else if (SEP || tiles == 4) launch_av_t<4, SEP>(st, A, lda, m, n, X, sh, P, s);
+  else launch_av_t<8, false>(st, A, lda, m, n, X, sh, P, s);
+}
+
 // One LSQR solve, advanced in blocks of iterations on a stream of its own (several solves of a batch
 // then overlap on the device); the profiling tokens are taken only on the context's stream.
 struct LsqrRun {
@@ -723,54 +1007,47 @@ struct LsqrRun {
   const void *A = nullptr;
   bool fp32 = false;
   int64_t lda = 0;
-  int m = 0, n = 0, nrhs = 0, itnlim = 0, it = 0;
+  int m = 0, n = 0, nrhs = 0, wd = NB, itnlim = 0, it = 0;  // wd: columns of the vectors, 1 or NB
   const double *q = nullptr;
   double *X = nullptr;
   bool done = false;
-  int wavesN = 0, blocksN = 0, ns = 0, rps = 0, blocksC = 0, blocksM = 0;
-  int nsegN = 1, seglenN = 0, partsN = 0;  // A X: column segments and the partial sums it leaves
-  int tilesN = 4;                           // A X: 16-row tiles per wave (autotuned)
-  bool vecN = false;
-  bool quiet = false;  // no profiling records (the no-allocation path: event creation is skipped)
+  AvShape av{1, 16};  // A X: column segments (one right-hand side: of av.wcols columns)
+  int tilesN = 4;     // A X: 16-row tiles per block (autotuned)
+  int rw = 8, splits = 1;  // A^T U: rows per wave, row splits
+  int blocksV = 0, partsU = 0;
+  bool fuse = false;  // U is formed in the A^T U kernel
+  int cur = 0;        // U of the last iteration is U[cur]
   // sparse mode: A and A^T in CSR (0-based, device); A is then unused
   const int64_t *cia = nullptr, *tia = nullptr;
   const int32_t *cja = nullptr, *tja = nullptr;
   const double *cva = nullptr, *tva = nullptr;
   int64_t nnz = 0;
-  double *pn = nullptr;  // A X segment partials when they come from a caller's workspace
-  DevBuf<double> U, V, W, Xl, X0, Xs, P, PN, partU, partV, partW, partB, sc;
-  DevBuf<LsqrState> S;
-  DevBuf<int> act;
+  DevBuf<double> U[2], V, W, Xl, Xs, P, PN, partU, partB, partV, partW;
+  DevBuf<LsqrState> S;  // state A, state B
   LsqrState hs[NB];
-  double *sxn = nullptr, *syn = nullptr, *sxt = nullptr, *syt = nullptr, *t1 = nullptr, *t2 = nullptr, *ia = nullptr;
+  LsqrState *slot = nullptr;  // two polls' states, pinned host memory of the context
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  int polls = 0, read = 0;  // polls enqueued and read
   double abytes = 0, vbytes = 0, aflops = 0;
 
-  int tok(const char *name, double bytes) {
-    return st == ctx->stream && !quiet ? andr_prof_begin(ctx, name, bytes, aflops) : -1;
-  }
-  template <int T, bool SEG>
-  void launch_mf_t(const double *Xin, double *Y, const double *sx, const double *sy, double *out) {
-    const dim3 grid((m + 64 * T - 1) / (64 * T), nsegN);  // four waves of 16 T rows per block
-    if (vecN)
-      hipLaunchKernelGGL((k_gemv_n_mf<T, SEG, true>), grid, dim3(256), 0, st, (const double *)A, lda, m, n, Xin,
-                         seglenN, Y, sx, sy, out);
-    else
-      hipLaunchKernelGGL((k_gemv_n_mf<T, SEG, false>), grid, dim3(256), 0, st, (const double *)A, lda, m, n, Xin,
-                         seglenN, Y, sx, sy, out);
-  }
-  void launch_mf(int tiles, bool seg, const double *Xin, double *Y, const double *sx, const double *sy, double *out) {
-    switch (tiles * 2 + (seg ? 1 : 0)) {
-      case 4: launch_mf_t<2, false>(Xin, Y, sx, sy, out); break;
-      case 5: launch_mf_t<2, true>(Xin, Y, sx, sy, out); break;
-      case 16: launch_mf_t<8, false>(Xin, Y, sx, sy, out); break;
-      case 17: launch_mf_t<8, true>(Xin, Y, sx, sy, out); break;
-      case 9: launch_mf_t<4, true>(Xin, Y, sx, sy, out); break;
-      default: launch_mf_t<4, false>(Xin, Y, sx, sy, out); break;
+  LsqrRun() = default;
+  LsqrRun(const LsqrRun &) = delete;
+  LsqrRun &operator=(const LsqrRun &) = delete;
+  ~LsqrRun() {
+    if (slot) {
+      (void)hipStreamSynchronize(st);  // nothing in flight writes the slot or the workspaces any more
+      andr_pinned_release(ctx, slot);
     }
+    for (auto e : ev)
+      if (e) (void)hipEventDestroy(e);
   }
+  int tok(const char *name, double bytes) { return st == ctx->stream ? andr_prof_begin(ctx, name, bytes, aflops) : -1; }
+  LsqrState *sa() const { return S.p; }
+  LsqrState *sb() const { return S.p + NB; }
+
   // Autotuner of the FP64 product: on the first large system of a (log2 m, log2 n) bucket, time the
-  // segmented product with 2, 4 and 8 tiles per wave on the actual matrix (its output goes to the
-  // segment partials only) and keep the fastest for the bucket. The choice does not change results.
+  // product with 2, 4 and 8 tiles per block on the actual matrix (its output goes to the segment
+  // partials only) and keep the fastest for the bucket. The choice does not change results.
   int tune_tiles() {
     const std::pair<int, int> key{ilog2c(m), ilog2c(n)};
     auto it = ctx->tune_gemv_n.find(key);
@@ -785,11 +1062,12 @@ struct LsqrRun {
     int best = 4;
     float best_ms = 1e30f;
     for (int tiles : {2, 4, 8}) {
-      launch_mf(tiles, true, V.p, U.p, sxn, syn, PN.p);  // warm-up
+      auto launch = [&]() { launch_av<false>(st, tiles, (const double *)A, lda, m, n, Xs.p, av, PN.p, nullptr); };
+      launch();  // warm-up
       float ms = 1e30f;
       for (int rep = 0; rep < 2; ++rep) {
         (void)hipEventRecord(e0, st);
-        launch_mf(tiles, true, V.p, U.p, sxn, syn, PN.p);
+        launch();
         (void)hipEventRecord(e1, st);
         (void)hipEventSynchronize(e1);
         float t = 0.f;
@@ -814,37 +1092,49 @@ struct LsqrRun {
     return b;
   }
 
-  void gemv_n(const double *Xin, double *Y, const double *sx, const double *sy, double *part) {
-    const int t = tok("lsqr_gemv_n", abytes + vbytes + (double)m * NB * 8.0);
+  LsqrVecs vecs() {
+    return {sa(), sb(), PN.p, av.nseg, U[cur].p, U[cur ^ 1].p, partU.p, partV.p, partW.p, blocksV};
+  }
+  // A Xin into the segment partials
+  void gemv_n(const double *Xin) {
+    const int t = tok("lsqr_gemv_n", abytes + vbytes + (double)av.nseg * m * wd * 8.0);
     if (cia) {
-      hipLaunchKernelGGL(k_csr_mv<true>, dim3(blocksM), dim3(256), 0, st, m, cia, cja, cva, Xin, Y, sx, sy, part);
-    } else if (fp32) {
-      hipLaunchKernelGGL(k_gemv_n<float>, dim3(blocksN), dim3(256), 0, st, (const float *)A, lda, m, n, Xin, Y, sx, sy,
-                         part);
+      hipLaunchKernelGGL(k_csr_mv, dim3((m + 31) / 32), dim3(256), 0, st, m, cia, cja, cva, Xin, PN.p, sb());
+    } else if (wd == 1) {
+      const dim3 grid((m + 31) / 32, av.nseg);
+      if (fp32)
+        hipLaunchKernelGGL(k_lsqr_av1<float>, grid, dim3(256), 0, st, (const float *)A, lda, m, n, Xin, av.wcols, PN.p, sb());
+      else
+        hipLaunchKernelGGL(k_lsqr_av1<double>, grid, dim3(256), 0, st, (const double *)A, lda, m, n, Xin, av.wcols, PN.p, sb());
     } else {
-      double *segp = pn ? pn : PN.p;
-      launch_mf(tilesN, nsegN > 1, Xin, Y, sx, sy, nsegN > 1 ? segp : part);
-      if (nsegN > 1) hipLaunchKernelGGL(k_combine_n, dim3(blocksM), dim3(256), 0, st, m, nsegN, segp, Y, sx, sy, part);
+      launch_av<false>(st, tilesN, (const double *)A, lda, m, n, Xin, av, PN.p, sb());
     }
     andr_prof_end(ctx, t);
   }
-  void gemv_t(const double *Y) {
-    const int t = tok("lsqr_gemv_t", abytes + vbytes + (double)ns * n * NB * 8.0);
-    dim3 g((n + 255) / 256, ns);
-    if (cia)
-      hipLaunchKernelGGL(k_csr_mv<false>, dim3(blocksC), dim3(256), 0, st, n, tia, tja, tva, Y, P.p,
-                         (const double *)nullptr, (const double *)nullptr, (double *)nullptr);
-    else if (fp32)
-      hipLaunchKernelGGL(k_gemv_t<float>, g, dim3(256), 0, st, (const float *)A, lda, m, n, Y, rps, P.p);
-    else if (vecN && (n % 2 == 0 || n < lda))  // column pairs: an odd last column reads the row padding
-      hipLaunchKernelGGL(k_gemv_t2, dim3((n + 511) / 512, ns), dim3(256), 0, st, (const double *)A, lda, m, n, Y, rps,
-                         P.p);
-    else
-      hipLaunchKernelGGL(k_gemv_t<double>, g, dim3(256), 0, st, (const double *)A, lda, m, n, Y, rps, P.p);
+  // A^T U into the split partials; form: U from the segment partials first (into U[cur ^ 1])
+  void gemv_t(const LsqrVecs &L, bool form) {
+    const int t = tok("lsqr_gemv_t", abytes + vbytes + (double)splits * n * wd * 8.0);
+    const int cols = at_cols(fp32 ? 4 : 8);
+    const dim3 grid((n + cols - 1) / cols, splits + (form ? 1 : 0)), blk(64 * AT_WAVES);
+    if (cia) {
+      hipLaunchKernelGGL(k_csr_mv, dim3((n + 31) / 32), dim3(256), 0, st, n, tia, tja, tva, L.uin, P.p, sb());
+    } else if (wd == 1) {
+      if (fp32) {
+        if (form) hipLaunchKernelGGL((k_lsqr_atu<float, 1, true>), grid, blk, 0, st, (const float *)A, lda, m, n, rw, L, P.p);
+        else hipLaunchKernelGGL((k_lsqr_atu<float, 1, false>), grid, blk, 0, st, (const float *)A, lda, m, n, rw, L, P.p);
+      } else {
+        if (form) hipLaunchKernelGGL((k_lsqr_atu<double, 1, true>), grid, blk, 0, st, (const double *)A, lda, m, n, rw, L, P.p);
+        else hipLaunchKernelGGL((k_lsqr_atu<double, 1, false>), grid, blk, 0, st, (const double *)A, lda, m, n, rw, L, P.p);
+      }
+    } else if (form) {
+      hipLaunchKernelGGL((k_lsqr_atu<double, NB, true>), grid, blk, 0, st, (const double *)A, lda, m, n, rw, L, P.p);
+    } else {
+      hipLaunchKernelGGL((k_lsqr_atu<double, NB, false>), grid, blk, 0, st, (const double *)A, lda, m, n, rw, L, P.p);
+    }
     andr_prof_end(ctx, t);
   }
 
-  // workspace, initial state, x_s = x0 / q, U = b - A x_s, V = A^T U, W = V / alpha
+  // workspace, initial state, x_s = x0 / q, U = b - A x_s, V = A^T U / beta
   int begin(andr_ctx *c, hipStream_t stream, const void *A_, bool fp32_, int64_t lda_, int m_, int n_,
             const double *q_, const double *B, double *X_, int nrhs_, int maxit, double eps) {
     ctx = c;
@@ -859,123 +1149,128 @@ struct LsqrRun {
     nrhs = nrhs_;
     if (nrhs < 1 || nrhs > NB) return andr_fail(ctx, ANDR_ERR_ARG, "nrhs must be 1..%d", NB);
     if (m < 1 || n < 1) return andr_fail(ctx, ANDR_ERR_ARG, "empty system");
-    if (cia) {  // CSR products: one thread per (row, column); partials per block of 32 rows
-      nsegN = 1;
-      partsN = (m * NB + 255) / 256;
-    } else if (fp32) {  // VALU product: one wave per 8 rows
-      wavesN = (m + 7) / 8;
-      blocksN = (wavesN + 3) / 4;
-      partsN = wavesN;
-    } else {  // matrix-core product over column segments; room for the most partials
-      // segments of GN_SEGLEN columns, shorter (down to 256) when that leaves fewer than 2048 waves
-      // of 64 rows; a function of the shape only, so that the tile count never changes the sums
-      const int64_t rw = (m + 63) / 64;
-      seglenN = GN_SEGLEN;
-      if (rw * ((n + GN_SEGLEN - 1) / GN_SEGLEN) < 2048)
-        seglenN = (int)std::max<int64_t>(256, ((int64_t)n * rw / 2048 + 15) / 16 * 16);
-      nsegN = (n + seglenN - 1) / seglenN;
-      partsN = std::max((m + 31) / 32, (m * NB + 255) / 256);
-      vecN = lda % 2 == 0 && ((uintptr_t)A % 16) == 0;
+    wd = nrhs == 1 ? 1 : NB;
+    if ((fp32 || cia) && wd != 1) return andr_fail(ctx, ANDR_ERR_ARG, "FP32 and sparse systems take one right-hand side");
+    if (!cia && (lda % (fp32 ? 4 : 2) || ((uintptr_t)A % 16)))
+      return andr_fail(ctx, ANDR_ERR_ARG, "rows of the system matrix must start on 16-byte boundaries");
+    if (cia) {
+      av = {1, n};
+    } else if (wd == 1) {
+      // a wave per eight rows: segments (of whole 1 KB loads) while there are fewer than 2048 waves
+      const int rowwaves = (m + 7) / 8;
+        const int want = std::min(std::max(1, (2048 + rowwaves - 1) / rowwaves), std::max(1, n / 256));
+      av.wcols = ((n + want - 1) / want + 255) / 256 * 256;
+      av.nseg = (n + av.wcols - 1) / av.wcols;
+    } else {
+      av = av_shape(m, n);
     }
-    ns = cia ? 1 : splits_for(m, n);
-    rps = (m + ns - 1) / ns;
-    blocksC = (n * NB + 255) / 256;
-    blocksM = (m * NB + 255) / 256;
-    if (U.alloc((size_t)m * NB, ctx) || V.alloc((size_t)n * NB, ctx) || W.alloc((size_t)n * NB, ctx) ||
-        Xl.alloc((size_t)n * NB, ctx) || X0.alloc((size_t)n * NB, ctx) || Xs.alloc((size_t)n * NB, ctx) ||
-        P.alloc((size_t)ns * n * NB, ctx) || PN.alloc(nsegN > 1 ? (size_t)nsegN * m * NB : 0, ctx) ||
-        partU.alloc((size_t)partsN * NB, ctx) ||
-        partV.alloc((size_t)blocksC * NB, ctx) || partW.alloc((size_t)blocksC * NB, ctx) ||
-        partB.alloc((size_t)blocksM * NB, ctx) || sc.alloc(8 * NB, ctx) || S.alloc(NB, ctx) || act.alloc(NB, ctx))
+    fuse = !cia && av.nseg <= (wd == 1 ? LSQR_FUSE_SEG1 : LSQR_FUSE_SEG);
+    const int cols = at_cols(fp32 ? 4 : 8), panels = (n + cols - 1) / cols;
+    // Rows per wave of A^T U: the fewest (16, the finest split that keeps two register sets busy) whose
+    // blocks run at once, two on each CU; a second, nearly empty round of blocks costs more than the
+    // longer waves (3120^2, 6 right-hand sides: 650 blocks of 16 rows a wave 25.2 us, 425 of 24 20.0).
+    rw = 16;
+    while (rw < AT_MAXRW && panels * ((m + AT_WAVES * rw - 1) / (AT_WAVES * rw) + 1) > 512) rw += wd == 1 ? 16 : 8;
+    splits = cia ? 1 : (m + AT_WAVES * rw - 1) / (AT_WAVES * rw);
+    blocksV = std::min((n * wd + V_VALUES - 1) / V_VALUES, V_MAXBLOCKS);
+    const int blocksM = (m * wd + 255) / 256;
+    partsU = fuse ? splits : blocksM;
+    if (U[0].alloc((size_t)m * wd, ctx) || U[1].alloc((size_t)m * wd, ctx) || V.alloc((size_t)n * wd, ctx) ||
+        W.alloc((size_t)n * wd, ctx) || Xl.alloc((size_t)n * wd, ctx) || Xs.alloc((size_t)n * wd, ctx) ||
+        P.alloc((size_t)splits * n * wd, ctx) || PN.alloc((size_t)av.nseg * m * wd, ctx) ||
+        partU.alloc((size_t)std::max(partsU, blocksM) * wd, ctx) || partB.alloc((size_t)blocksM * wd, ctx) ||
+        partV.alloc((size_t)blocksV * wd, ctx) || partW.alloc((size_t)blocksV * wd, ctx) || S.alloc(2 * NB, ctx))
       return andr_fail(ctx, ANDR_ERR_ALLOC, "LSQR workspace (m=%d n=%d)", m, n);
-    sxn = sc.p;
-    syn = sc.p + NB;
-    sxt = sc.p + 2 * NB;
-    syt = sc.p + 3 * NB;
-    t1 = sc.p + 4 * NB;
-    t2 = sc.p + 5 * NB;
-    ia = sc.p + 6 * NB;
+    static_assert(2 * NB * sizeof(LsqrState) <= ANDR_PINNED_SLOT, "two polls' states in a pinned slot");
+    slot = (LsqrState *)andr_pinned_alloc(ctx);
+    if (!slot) return andr_fail(ctx, ANDR_ERR_ALLOC, "pinned memory for the LSQR states");
+    for (auto &e : ev) ANDR_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     std::memset(hs, 0, sizeof(hs));
     itnlim = maxit > 0 ? maxit : 10 * (m + n + 50);
-    for (int k = 0; k < NB; ++k) {
-      hs[k].active = k < nrhs ? 1 : 0;
-      hs[k].itnlim = itnlim;
-    }
-    double hsc[8 * NB];
-    for (int k = 0; k < NB; ++k) {
-      hsc[k] = -1.0;       // sxn: U = -A x_s + U
-      hsc[NB + k] = 1.0;   // syn
-      hsc[2 * NB + k] = hsc[3 * NB + k] = hsc[4 * NB + k] = hsc[5 * NB + k] = hsc[6 * NB + k] = 0.0;
-      hsc[7 * NB + k] = 1.0;
-    }
-    ANDR_HIP(ctx, hipMemcpyAsync(S.p, hs, sizeof(hs), hipMemcpyHostToDevice, st));
-    ANDR_HIP(ctx, hipMemcpyAsync(sc.p, hsc, sizeof(hsc), hipMemcpyHostToDevice, st));
-    ANDR_HIP(ctx, hipMemcpyAsync(X0.p, X, sizeof(double) * n * NB, hipMemcpyDeviceToDevice, st));
-    ANDR_HIP(ctx, hipMemcpyAsync(U.p, B, sizeof(double) * m * NB, hipMemcpyDeviceToDevice, st));
-    ANDR_HIP(ctx, hipMemsetAsync(V.p, 0, sizeof(double) * n * NB, st));
-    ANDR_HIP(ctx, hipMemsetAsync(Xl.p, 0, sizeof(double) * n * NB, st));
-    ANDR_HIP(ctx, hipMemsetAsync(W.p, 0, sizeof(double) * n * NB, st));
-    if (!fp32 && !cia) {
-      tilesN = ctx->autotune ? 4 : ctx->gemv_n_tiles;
-      if (nsegN > 1 && ctx->autotune && (double)m * n * 8.0 >= 2.56e8) {
+    abytes = cia ? (double)nnz * 12.0 + (double)(m + 1) * 8.0 : (double)m * n * (fp32 ? 4.0 : 8.0);
+    vbytes = ((double)m + n) * wd * 8.0;
+    aflops = 2.0 * m * n * nrhs;
+    return wd == 1 ? start<1>(B, eps) : start<NB>(B, eps);
+  }
+  template <int WD>
+  int start(const double *B, double eps) {
+    const int blocksM = (m * WD + 255) / 256;
+    hipLaunchKernelGGL(k_lsqr_x0<WD>, dim3((n * WD + 255) / 256), dim3(256), 0, st, n, X, q, Xs.p);
+    if (wd == NB) {
+      tilesN = ctx->autotune ? av_tiles(m, av.nseg) : ctx->gemv_n_tiles;
+      if (ctx->autotune && (double)m * n * 8.0 >= 2.56e8) {
         const int rc = tune_tiles();
         if (rc) return rc;
       }
-      partsN = nsegN == 1 ? (m + 16 * tilesN - 1) / (16 * tilesN) : blocksM;  // one per wave, or per block
     }
-    abytes = cia ? (double)nnz * 12.0 + (double)(m + 1) * 8.0 : (double)m * n * (fp32 ? 4.0 : 8.0);
-    vbytes = ((double)m + n) * NB * 8.0;
-    aflops = 2.0 * m * n * nrhs;
-    // x_s = x0 / q ; U = b - A x_s ; ||U||, ||b||
-    hipLaunchKernelGGL(k_scale_div, dim3(blocksC), dim3(256), 0, st, n, X0.p, q, Xs.p);
-    gemv_n(Xs.p, U.p, sxn, syn, partU.p);
-    hipLaunchKernelGGL(k_sumsq_parts, dim3(blocksM), dim3(256), 0, st, m, B, partB.p);
-    hipLaunchKernelGGL(k_lsqr_start, dim3(1), dim3(LSQR_SCALAR_THREADS), 0, st, S.p, partU.p, partsN, partB.p, blocksM, eps, sxt, syt);
-    // V = A^T u
-    gemv_t(U.p);
-    hipLaunchKernelGGL(k_combine_t, dim3(blocksC), dim3(256), 0, st, n, ns, P.p, V.p, (const double *)nullptr, sxt, syt,
-                       partV.p, partW.p);
-    hipLaunchKernelGGL(k_lsqr_init2, dim3(1), dim3(LSQR_SCALAR_THREADS), 0, st, S.p, partV.p, blocksC, sxn, syn, ia);
-    // w = v / alpha  (X update with t1 = 0, t2 = 0, W = V * inv_alpha)
-    int allon[NB];
-    for (int k = 0; k < NB; ++k) allon[k] = 1;
-    ANDR_HIP(ctx, hipMemcpyAsync(act.p, allon, sizeof(allon), hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_lsqr_update, dim3(blocksC), dim3(256), 0, st, n, Xl.p, W.p, V.p, t1, t2, ia, act.p);
+    // the state first: the products look at it
+    hipLaunchKernelGGL(k_lsqr_start<WD>, dim3(1), dim3(256), 0, st, sa(), sb(), partU.p, partB.p, 0, eps, nrhs, itnlim);
+    gemv_n(Xs.p);
+    hipLaunchKernelGGL(k_lsqr_u0<WD>, dim3(blocksM), dim3(256), 0, st, m, av.nseg, PN.p, B, U[0].p, partU.p, partB.p);
+    hipLaunchKernelGGL(k_lsqr_start<WD>, dim3(1), dim3(256), 0, st, sa(), sb(), partU.p, partB.p, blocksM, eps, nrhs,
+                       itnlim);
+    cur = 0;
+    gemv_t(vecs(), false);
+    hipLaunchKernelGGL((k_lsqr_v<WD, true>), dim3(blocksV), dim3(256), 0, st, n, splits, P.p, sa(), sb(),
+                       (const double *)nullptr, 0, V.p, Xl.p, W.p, partV.p, partW.p);
     ANDR_HIP(ctx, hipGetLastError());
     return ANDR_OK;
   }
 
-  // enqueues iterations up to the next multiple of `poll` (or the iteration limit); no host wait
-  void advance(int poll) {
+  // enqueues iterations up to the next multiple of LSQR_POLL (or the iteration limit), then a kernel that
+  // leaves the columns' states in pinned host memory; no host wait
+  int advance() {
+    if (it >= itnlim) return ANDR_OK;
+    if (wd == 1) iterate<1>();
+    else iterate<NB>();
+    ANDR_HIP(ctx, hipGetLastError());
+    ANDR_HIP(ctx, hipEventRecord(ev[polls % 2], st));
+    ++polls;
+    return ANDR_OK;
+  }
+  template <int WD>
+  void iterate() {
     do {
-      gemv_n(V.p, U.p, sxn, syn, partU.p);
-      hipLaunchKernelGGL(k_lsqr_mid, dim3(1), dim3(LSQR_SCALAR_THREADS), 0, st, S.p, partU.p, partsN, sxt, syt);
-      gemv_t(U.p);
-      hipLaunchKernelGGL(k_combine_t, dim3(blocksC), dim3(256), 0, st, n, ns, P.p, V.p, W.p, sxt, syt, partV.p,
-                         partW.p);
-      hipLaunchKernelGGL(k_lsqr_end, dim3(1), dim3(LSQR_SCALAR_THREADS), 0, st, S.p, partV.p, partW.p, blocksC, sxn, syn, t1, t2, ia,
-                         act.p);
-      hipLaunchKernelGGL(k_lsqr_update, dim3(blocksC), dim3(256), 0, st, n, Xl.p, W.p, V.p, t1, t2, ia, act.p);
+      gemv_n(V.p);
+      LsqrVecs L = vecs();
+      if (!fuse) {
+        hipLaunchKernelGGL(k_lsqr_u<WD>, dim3((m * WD + 255) / 256 + 1), dim3(256), 0, st, m, L);
+        L.uin = L.uout;
+      }
+      gemv_t(L, fuse);
+      hipLaunchKernelGGL((k_lsqr_v<WD, false>), dim3(blocksV), dim3(256), 0, st, n, splits, P.p, sa(), sb(), partU.p,
+                         partsU, V.p, Xl.p, W.p, partV.p, partW.p);
+      cur ^= 1;
       ++it;
-    } while (it % poll != 0 && it < itnlim);
+    } while (it % LSQR_POLL != 0 && it < itnlim);
+    hipLaunchKernelGGL(k_lsqr_poll<WD>, dim3(1), dim3(256), 0, st, vecs(), slot + (polls % 2) * NB);
   }
 
-  // reads the per-column states; done when no column is active or the limit is reached
+  // waits for the oldest poll that was not read yet; done when no column is active or the limit is
+  // reached. The device meanwhile works on the iterations after it, which are no-ops (the kernels
+  // return on a stopped state) when that poll turns out to be the last.
   int poll_state() {
-    ANDR_HIP(ctx, hipGetLastError());
-    ANDR_HIP(ctx, hipMemcpyAsync(hs, S.p, sizeof(hs), hipMemcpyDeviceToHost, st));
-    ANDR_HIP(ctx, hipStreamSynchronize(st));
+    ANDR_HIP(ctx, hipEventSynchronize(ev[read % 2]));
+    std::memcpy(hs, slot + (read % 2) * NB, sizeof(LsqrState) * wd);
+    ++read;
     bool any = false;
     for (int k = 0; k < nrhs; ++k) any = any || hs[k].active;
-    done = !any || it >= itnlim;
+    done = !any || (it >= itnlim && read == polls);
     return ANDR_OK;
   }
+  // one round of a solve: iterations ahead of the poll that is waited for
+  int round() {
+    const int rc = advance();
+    return rc ? rc : poll_state();
+  }
 
-  // x = q .* x + x0, iteration counts and stop codes
+  // x = q .* x + x0; iteration counts and stop codes are those of the last poll
   int finish(int *nit, int *istop) {
-    hipLaunchKernelGGL(k_scale_mul_add, dim3(blocksC), dim3(256), 0, st, n, q, Xl.p, X0.p, X);
+    if (wd == 1)
+      hipLaunchKernelGGL(k_lsqr_finish<1>, dim3((n + 255) / 256), dim3(256), 0, st, n, q, Xl.p, W.p, sb(), X);
+    else
+      hipLaunchKernelGGL(k_lsqr_finish<NB>, dim3((n * NB + 255) / 256), dim3(256), 0, st, n, q, Xl.p, W.p, sb(), X);
     ANDR_HIP(ctx, hipGetLastError());
-    ANDR_HIP(ctx, hipMemcpyAsync(hs, S.p, sizeof(hs), hipMemcpyDeviceToHost, st));
     ANDR_HIP(ctx, hipStreamSynchronize(st));
     for (int k = 0; k < nrhs; ++k) {
       if (nit) nit[k] = hs[k].itn;
@@ -985,8 +1280,6 @@ struct LsqrRun {
   }
 };
 
-constexpr int LSQR_POLL = 8;  // iterations between reads of the convergence state
-
 }  // namespace
 
 int andr_lsqr_device(andr_ctx *ctx, const void *A, bool fp32, int64_t lda, int m, int n, const double *q,
@@ -994,10 +1287,9 @@ int andr_lsqr_device(andr_ctx *ctx, const void *A, bool fp32, int64_t lda, int m
   LsqrRun R;
   int rc = R.begin(ctx, ctx->stream, A, fp32, lda, m, n, q, B, X, nrhs, maxit, eps);
   if (rc) return rc;
-  while (!R.done) {
-    R.advance(LSQR_POLL);
-    if ((rc = R.poll_state())) return rc;
-  }
+  if ((rc = R.advance())) return rc;
+  while (!R.done)
+    if ((rc = R.round())) return rc;
   return R.finish(nit, istop);
 }
 
@@ -1014,10 +1306,9 @@ int andr_lsqr_device_csr(andr_ctx *ctx, int m, int n, int64_t nnz, const int64_t
   R.nnz = nnz;
   int rc = R.begin(ctx, ctx->stream, nullptr, false, 0, m, n, q, B, X, nrhs, maxit, eps);
   if (rc) return rc;
-  while (!R.done) {
-    R.advance(LSQR_POLL);
-    if ((rc = R.poll_state())) return rc;
-  }
+  if ((rc = R.advance())) return rc;
+  while (!R.done)
+    if ((rc = R.round())) return rc;
   return R.finish(nit, istop);
 }
 
@@ -1046,10 +1337,12 @@ int andr_lsqr_device_batch(andr_ctx *ctx, int count, const LsqrJob *jobs) {
       rc = runs[i].begin(ctx, streams[i % nst], J.A, J.fp32, J.lda, J.m, J.n, J.q, J.B, J.X, J.nrhs, J.maxit, J.eps);
     }
     // all solves advance together, a block of iterations at a time, each on its stream
+    for (auto &R : runs)
+      if (!rc) rc = R.advance();
     for (bool left = !rc; left && !rc;) {
       left = false;
       for (auto &R : runs)
-        if (!R.done) R.advance(LSQR_POLL);
+        if (!R.done && !rc) rc = R.advance();
       for (auto &R : runs)
         if (!R.done && !rc) {
           rc = R.poll_state();
@@ -1133,8 +1426,8 @@ __global__ void k_bicg_init(int n, const double *__restrict__ B, const double *_
 __global__ void k_bicg_start(BicgState *st, const double *pb, const double *pr, int np, double tol, int nrhs,
                              double *sc) {
   __shared__ double red[4 * NB];
-  const double b2 = block_sum_parts(pb, np, red);
-  const double r2 = block_sum_parts(pr, np, red);
+  const double b2 = block_sum_parts<NB, 256>(pb, np, red);
+  const double r2 = block_sum_parts<NB, 256>(pr, np, red);
   const int k = threadIdx.x;
   if (k >= NB) return;
   BicgState &S = st[k];
@@ -1151,7 +1444,7 @@ __global__ void k_bicg_start(BicgState *st, const double *pb, const double *pr, 
 // rho_new = r_hat . r; beta = (rho_new / rho) (alpha / omega)
 __global__ void k_bicg_beta(BicgState *st, const double *part, int np, double *sc) {
   __shared__ double red[4 * NB];
-  const double rho = block_sum_parts(part, np, red);
+  const double rho = block_sum_parts<NB, 256>(part, np, red);
   const int k = threadIdx.x;
   if (k >= NB) return;
   BicgState &S = st[k];
@@ -1192,7 +1485,7 @@ __global__ void k_bicg_p(int n, const double *__restrict__ R, const double *__re
 // alpha = rho / (r_hat . v)
 __global__ void k_bicg_alpha(BicgState *st, const double *part, int np, double *sc) {
   __shared__ double red[4 * NB];
-  const double rv = block_sum_parts(part, np, red);
+  const double rv = block_sum_parts<NB, 256>(part, np, red);
   const int k = threadIdx.x;
   if (k >= NB) return;
   BicgState &S = st[k];
@@ -1225,8 +1518,8 @@ __global__ void k_bicg_s(int n, double *__restrict__ X, const double *__restrict
 // omega = (t . s) / (t . t)
 __global__ void k_bicg_omega(BicgState *st, const double *pts, const double *ptt, int np, double *sc) {
   __shared__ double red[4 * NB];
-  const double ts = block_sum_parts(pts, np, red);
-  const double tt = block_sum_parts(ptt, np, red);
+  const double ts = block_sum_parts<NB, 256>(pts, np, red);
+  const double tt = block_sum_parts<NB, 256>(ptt, np, red);
   const int k = threadIdx.x;
   if (k >= NB) return;
   BicgState &S = st[k];
@@ -1252,7 +1545,7 @@ __global__ void k_bicg_x(int n, double *__restrict__ X, const double *__restrict
 // convergence: ||r||^2 <= tol^2 ||b||^2; omega = 0 (with r not small) is a breakdown
 __global__ void k_bicg_check(BicgState *st, const double *part, int np, int itnlim) {
   __shared__ double red[4 * NB];
-  const double r2 = block_sum_parts(part, np, red);
+  const double r2 = block_sum_parts<NB, 256>(part, np, red);
   const int k = threadIdx.x;
   if (k >= NB) return;
   BicgState &S = st[k];
@@ -1275,16 +1568,15 @@ namespace {
 // the shape of the BiCGSTAB product A X: column segments and the partial sums they leave (a function
 // of n only, so that the workspace size is known before the call)
 struct BicgLayout {
-  int seglen, nseg, blocksM, partsN;
+  int seglen, nseg, blocksM;
 };
 BicgLayout bicg_layout(int n) {
   BicgLayout L;
-  L.seglen = 1024;
+  L.seglen = AV_MAXCOLS;
   const int64_t rw = (n + 63) / 64;
-  if (rw * ((n + 1023) / 1024) < 2048) L.seglen = (int)std::max<int64_t>(256, ((int64_t)n * rw / 2048 + 15) / 16 * 16);
+  if (rw * ((n + AV_MAXCOLS - 1) / AV_MAXCOLS) < 2048) L.seglen = (int)std::max<int64_t>(256, ((int64_t)n * rw / 2048 + 15) / 16 * 16);
   L.nseg = (n + L.seglen - 1) / L.seglen;
   L.blocksM = (n * NB + 255) / 256;
-  L.partsN = L.nseg == 1 ? (n + 63) / 64 : L.blocksM;
   return L;
 }
 // doubles of each workspace array, in the order they are carved from a caller's region
@@ -1292,13 +1584,13 @@ void bicg_sizes(int n, size_t sz[15]) {
   const BicgLayout L = bicg_layout(n);
   for (int i = 0; i < 7; ++i) sz[i] = (size_t)n * NB;  // r, r_hat, p, v, y, z, t
   sz[7] = n;                                           // dinv
-  sz[8] = (size_t)std::max(L.blocksM, L.partsN) * NB;  // p1
+  sz[8] = (size_t)L.blocksM * NB;                      // p1
   sz[9] = (size_t)L.blocksM * NB;                      // p2
   sz[10] = NB;                                         // one
   sz[11] = NB;                                         // zero
   sz[12] = 6 * NB;                                     // scalars
   sz[13] = (sizeof(BicgState) * NB + 7) / 8;           // per-column states
-  sz[14] = L.nseg > 1 ? (size_t)L.nseg * n * NB : 0;   // A X segment partials
+  sz[14] = (size_t)L.nseg * n * NB;                 // A X segment partials
 }
 __global__ void k_fill(size_t n, double v, double *__restrict__ p) {
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1318,22 +1610,9 @@ int andr_bicgstab_device(andr_ctx *ctx, const double *A, int64_t lda, int n, con
   if (nrhs < 1 || nrhs > NB) return andr_fail(ctx, ANDR_ERR_ARG, "nrhs must be 1..%d", NB);
   if (n < 1) return andr_fail(ctx, ANDR_ERR_ARG, "empty system");
   hipStream_t st = ctx->stream;
-  // the matrix-core product of the LSQR run object (q unused)
   const BicgLayout L = bicg_layout(n);
-  LsqrRun R;
-  R.ctx = ctx;
-  R.st = st;
-  R.A = A;
-  R.fp32 = false;
-  R.lda = lda;
-  R.m = R.n = n;
-  R.seglenN = L.seglen;
-  R.nsegN = L.nseg;
-  R.tilesN = 4;
-  R.vecN = lda % 2 == 0 && ((uintptr_t)A % 16) == 0;
-  R.blocksM = L.blocksM;
-  R.partsN = L.partsN;
-  const int nb = R.blocksM;
+  const int tiles = av_tiles(n, (L.nseg + AV_WAVES - 1) / AV_WAVES);
+  const int nb = L.blocksM;
   // workspace: the context's memory cache, or carved from the caller's region (no allocation)
   DevBuf<double> own[15];
   double *w[15];
@@ -1348,7 +1627,6 @@ int andr_bicgstab_device(andr_ctx *ctx, const double *A, int64_t lda, int n, con
       w[i] = sz[i] ? cur : nullptr;
       cur += (sz[i] + 31) / 32 * 32;
     }
-    R.quiet = true;
   } else {
     for (int i = 0; i < 15; ++i) {
       if (own[i].alloc(sz[i], ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "BiCGSTAB workspace (n=%d)", n);
@@ -1358,45 +1636,45 @@ int andr_bicgstab_device(andr_ctx *ctx, const double *A, int64_t lda, int n, con
   double *Rr = w[0], *Rh = w[1], *P = w[2], *V = w[3], *Yv = w[4], *Z = w[5], *Tt = w[6], *dinv = w[7], *p1 = w[8],
          *p2 = w[9], *one = w[10], *zero = w[11], *sc = w[12];
   BicgState *S = (BicgState *)w[13];
-  R.pn = w[14];
+  double *pn = w[14];
   // constants and cleared outputs by fill kernels (no host copies, no memset nodes): the products
   // write out = 1 * (A in) + 0 * out, so their outputs start finite
   hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, (size_t)NB, 1.0, one);
   hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, (size_t)NB, 0.0, zero);
   hipLaunchKernelGGL(k_fill, dim3((n * NB + 255) / 256), dim3(256), 0, st, (size_t)n * NB, 0.0, V);
   hipLaunchKernelGGL(k_fill, dim3((n * NB + 255) / 256), dim3(256), 0, st, (size_t)n * NB, 0.0, Tt);
-  R.abytes = (double)n * n * 8.0;
-  R.vbytes = 2.0 * n * NB * 8.0;
-  R.aflops = 2.0 * n * n * nrhs;
   const int gb = (n * NB + 255) / 256;
-  auto product = [&](const double *in, double *out) {  // out = A in (its partial squared norms are not used)
-    R.gemv_n(in, out, one, zero, p1);
+  auto product = [&](const double *in, double *out) {  // out = A in; no profiling records with a caller's workspace
+    const int t = ws ? -1 : andr_prof_begin(ctx, "lsqr_gemv_n", (double)n * n * 8.0 + (2.0 + L.nseg) * n * NB * 8.0, 2.0 * n * n * nrhs);
+    launch_av<true>(st, tiles, A, lda, n, n, in, {(L.nseg + AV_WAVES - 1) / AV_WAVES, L.seglen}, pn, nullptr);
+    hipLaunchKernelGGL(k_combine_n, dim3(gb), dim3(256), 0, st, n, L.nseg, pn, out);
+    andr_prof_end(ctx, t);
   };
   hipLaunchKernelGGL(k_bicg_diag, dim3((n + 255) / 256), dim3(256), 0, st, A, lda, n, dinv);
   product(X, V);  // A x0
   hipLaunchKernelGGL(k_bicg_init, dim3(gb), dim3(256), 0, st, n, B, V, Rr, Rh, P, V);
   hipLaunchKernelGGL(k_bicg_dots, dim3(gb), dim3(256), 0, st, n, B, B, Rr, Rr, p1, p2);
-  hipLaunchKernelGGL(k_bicg_start, dim3(1), dim3(LSQR_SCALAR_THREADS), 0, st, S, p1, p2, nb, tol, nrhs, sc);
+  hipLaunchKernelGGL(k_bicg_start, dim3(1), dim3(256), 0, st, S, p1, p2, nb, tol, nrhs, sc);
   const int itnlim = maxit > 0 ? maxit : 1000;
   BicgState hs[NB];
   for (int it = 0; it < itnlim;) {
     for (int inner = 0; inner < 8 && it < itnlim; ++inner, ++it) {
       hipLaunchKernelGGL(k_bicg_dots, dim3(gb), dim3(256), 0, st, n, Rh, Rr, (const double *)nullptr,
                          (const double *)nullptr, p1, p2);
-      hipLaunchKernelGGL(k_bicg_beta, dim3(1), dim3(LSQR_SCALAR_THREADS), 0, st, S, p1, nb, sc);
+      hipLaunchKernelGGL(k_bicg_beta, dim3(1), dim3(256), 0, st, S, p1, nb, sc);
       hipLaunchKernelGGL(k_bicg_p, dim3(gb), dim3(256), 0, st, n, Rr, V, P, Yv, dinv, sc, S);
       product(Yv, V);
       hipLaunchKernelGGL(k_bicg_dots, dim3(gb), dim3(256), 0, st, n, Rh, V, (const double *)nullptr,
                          (const double *)nullptr, p1, p2);
-      hipLaunchKernelGGL(k_bicg_alpha, dim3(1), dim3(LSQR_SCALAR_THREADS), 0, st, S, p1, nb, sc);
+      hipLaunchKernelGGL(k_bicg_alpha, dim3(1), dim3(256), 0, st, S, p1, nb, sc);
       hipLaunchKernelGGL(k_bicg_s, dim3(gb), dim3(256), 0, st, n, X, Yv, Rr, V, Z, dinv, sc);
       product(Z, Tt);
       hipLaunchKernelGGL(k_bicg_dots, dim3(gb), dim3(256), 0, st, n, Tt, Rr, Tt, Tt, p1, p2);
-      hipLaunchKernelGGL(k_bicg_omega, dim3(1), dim3(LSQR_SCALAR_THREADS), 0, st, S, p1, p2, nb, sc);
+      hipLaunchKernelGGL(k_bicg_omega, dim3(1), dim3(256), 0, st, S, p1, p2, nb, sc);
       hipLaunchKernelGGL(k_bicg_x, dim3(gb), dim3(256), 0, st, n, X, Z, Rr, Tt, sc);
       hipLaunchKernelGGL(k_bicg_dots, dim3(gb), dim3(256), 0, st, n, Rr, Rr, (const double *)nullptr,
                          (const double *)nullptr, p1, p2);
-      hipLaunchKernelGGL(k_bicg_check, dim3(1), dim3(LSQR_SCALAR_THREADS), 0, st, S, p1, nb, itnlim);
+      hipLaunchKernelGGL(k_bicg_check, dim3(1), dim3(256), 0, st, S, p1, nb, itnlim);
     }
     ANDR_HIP(ctx, hipGetLastError());
     ANDR_HIP(ctx, hipMemcpyAsync(hs, S, sizeof(hs), hipMemcpyDeviceToHost, st));

@@ -10,9 +10,9 @@
 struct LsqrState {
   double alpha, beta, rhobar, phibar, bnorm, rnorm, anorm, dnorm, xnorm, xnorm1, res2, cs2, sn2, z;
   double atol, btol, ctol;
-  double t1, t2;       // update coefficients of the current iteration
-  double sx, sy;       // scale factors handed to the next product
+  double t1, t2, inv_alpha;  // coefficients of the update of X and W that ends the iteration
   int itn, istop, itnlim, active;
+  int upd;                   // the update is still to be applied
 };
 
 // One dense system of a batch: A is m x n (row-major, leading dimension lda) of type ST.
