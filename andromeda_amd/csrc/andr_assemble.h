@@ -58,5 +58,8 @@ int andr_launch_stokes_surface_pressure(andr_ctx *ctx, DevBody &b, const double 
 #define ANDR_FLOPS_PER_STOKES_EVAL 107.0
 #define ANDR_FLOPS_PER_STOKES_EVAL_SUM 60.0
 #define ANDR_FLOPS_PER_LAPLACE_EVAL 50.0
+// velocity and pressure at a domain point (k_stokes_domain), surface pressure (FMA as 2, rsqrt as 1)
+#define ANDR_FLOPS_PER_DOMAIN_EVAL 92.0
+#define ANDR_FLOPS_PER_SURFACE_EVAL 55.0
 // Dunavant rules (classes 0..6 of the learned form) in the quadrature table
 #define ANDR_DUN_OFF0 297

@@ -785,121 +785,234 @@ __global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int n
 
 // ------------------------------------------------------------------------------------------------
 // Velocity and pressure at points of the flow domain: GetStokesDomainValue (src/lib_Stokes.f90:
-// 3043-3390). One workgroup per point; the threads take elements, integrate each with the mesh's
-// rule (the point is off the boundary, so every pair is regular) and contract the integrals with
-// the nodal velocities u (3 per node) and the element tractions q (3 per element) at once, so that
-// no integral row is stored. out[5 p + 0..2] = velocity, out[5 p + 3] = pressure, out[5 p + 4] =
-// the closure error of the point's integrals (:3255-3300): the T closure -sum_i T_ii = 8 pi and
-// sum_e G n_e = 0 hold inside the domain. osem = 8 pi as the reference forms it.
+// 3043-3390) with Triangle_3DStokesInt (:2341-2446) and StokesKernel (:2450-2544). A workgroup takes a
+// point and a chunk of the elements, integrates each with the mesh's rule (the point is off the boundary,
+// so every pair is regular) and contracts with the boundary data. The contraction is made at the
+// quadrature point, with the velocity u(y) interpolated there and the traction q of the element:
+//   T u = -6 (r.n) (r.u) r / r^5,  G q = q / r + (r.q) r / r^3,
+//   prT u = 4 (3 (r.n) (r.u) / r^2 - n.u) / r^3,  prG q = 2 r.q / r^3
+// instead of forming the 36 moments of the pair first (G 6, T 18, prG 3, prT 9): 14 running sums and some
+// 60 FP64 operations a point instead of 36 sums and 130. r.n is one number per flat element. Bound by
+// FP64 issue: 1501 points x 1000 elements x 126 quadrature points 941 -> 388 us.
+// part[(chunk npts + point) NDV + i]: the sums of a chunk; k_stokes_domain_fin adds the chunks.
 // ------------------------------------------------------------------------------------------------
+constexpr int NDV = 11;  // velocity (3), pressure (2), T closure (3), G n (3)
+
 __global__ __launch_bounds__(256) void k_stokes_domain(BodyGeom g, int qoff, int nq, const double *__restrict__ pts,
-                                                       const double *__restrict__ u, const double *__restrict__ q,
-                                                       double diff, double osem, double *__restrict__ out) {
-  constexpr int NV = 14;  // T u (3), G q (3), prT u, prG q, T closure (3), G n (3)
-  __shared__ double red[NV][4];
+                                                       int npts, int chunk, const double *__restrict__ u,
+                                                       const double *__restrict__ q, double diff,
+                                                       double *__restrict__ part) {
+  __shared__ double red[NDV][4];
   const int ip = blockIdx.x;
   const double s[3] = {pts[3 * ip], pts[3 * ip + 1], pts[3 * ip + 2]};
-  double a[NV];
+  const double idiff = 1.0 / diff;
+  double a[NDV];
 #pragma unroll
-  for (int i = 0; i < NV; ++i) a[i] = 0.0;
-  for (int e = threadIdx.x; e < g.ne; e += blockDim.x) {
-    const int vv[3] = {g.con[3 * e], g.con[3 * e + 1], g.con[3 * e + 2]};
-    const double *x1 = g.xyz + 3 * vv[0], *x2 = g.xyz + 3 * vv[1], *x3 = g.xyz + 3 * vv[2];
-    const double m = g.mul[e];
-    const double nx = m * g.nrm[3 * e], ny = m * g.nrm[3 * e + 1], nz = m * g.nrm[3 * e + 2];
-    double Gs[6], pG[3], Tv[6][3], pT[3][3];
-    stokes_tri_full(s, x1, x2, x3, nx, ny, nz, g.area[e], qoff, nq, Gs, pG, Tv, pT);
+  for (int i = 0; i < NDV; ++i) a[i] = 0.0;
+  const int e1 = min(g.ne, (int)(blockIdx.y + 1) * chunk);
+  for (int e = blockIdx.y * chunk + threadIdx.x; e < e1; e += blockDim.x) {
+    const int v1 = 3 * g.con[3 * e], v2 = 3 * g.con[3 * e + 1], v3 = 3 * g.con[3 * e + 2];
+    const double m = g.mul[e], A = g.area[e];
+    double d[3], xa[3], xb[3], n[3], u0[3], ua[3], ub[3], qe[3];  // r = d + l1 xa + l2 xb, u = u0 + l1 ua + l2 ub
+    double rn = 0.0, un0 = 0.0, una = 0.0, unb = 0.0, rq0 = 0.0, rqa = 0.0, rqb = 0.0;
 #pragma unroll
-    for (int v = 0; v < 3; ++v) {
-      const double ux = u[3 * vv[v]], uy = u[3 * vv[v] + 1], uz = u[3 * vv[v] + 2];
-      a[0] += Tv[0][v] * ux + Tv[1][v] * uy + Tv[2][v] * uz;
-      a[1] += Tv[1][v] * ux + Tv[3][v] * uy + Tv[4][v] * uz;
-      a[2] += Tv[2][v] * ux + Tv[4][v] * uy + Tv[5][v] * uz;
-      a[6] += pT[0][v] * ux + pT[1][v] * uy + pT[2][v] * uz;
-      a[8] += Tv[0][v];
-      a[9] += Tv[3][v];
-      a[10] += Tv[5][v];
+    for (int c = 0; c < 3; ++c) {
+      const double x3 = g.xyz[v3 + c], w3 = u[v3 + c];
+      d[c] = x3 - s[c];
+      xa[c] = g.xyz[v1 + c] - x3;
+      xb[c] = g.xyz[v2 + c] - x3;
+      u0[c] = w3;
+      ua[c] = u[v1 + c] - w3;
+      ub[c] = u[v2 + c] - w3;
+      n[c] = m * g.nrm[3 * e + c];
+      qe[c] = q[3 * e + c];
+      rn += d[c] * n[c];
+      un0 += n[c] * u0[c];
+      una += n[c] * ua[c];
+      unb += n[c] * ub[c];
+      rq0 += d[c] * qe[c];
+      rqa += xa[c] * qe[c];
+      rqb += xb[c] * qe[c];
     }
-    const double qx = q[3 * e], qy = q[3 * e + 1], qz = q[3 * e + 2];
-    a[3] += Gs[0] * qx + Gs[1] * qy + Gs[2] * qz;
-    a[4] += Gs[1] * qx + Gs[3] * qy + Gs[4] * qz;
-    a[5] += Gs[2] * qx + Gs[4] * qy + Gs[5] * qz;
-    a[7] += pG[0] * qx + pG[1] * qy + pG[2] * qz;
-    a[11] += Gs[0] * nx + Gs[1] * ny + Gs[2] * nz;
-    a[12] += Gs[1] * nx + Gs[3] * ny + Gs[4] * nz;
-    a[13] += Gs[2] * nx + Gs[4] * ny + Gs[5] * nz;
-  }
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const double k6 = -6.0 * rn;
+    double s1 = 0.0, sun = 0.0, sru = 0.0, srq = 0.0;
+    double sv[3] = {0.0, 0.0, 0.0}, s3[3] = {0.0, 0.0, 0.0}, s5[3] = {0.0, 0.0, 0.0};
+    for (int p = 0; p < nq; ++p) {
+      const double l1 = c_qd[qoff + p][0], l2 = c_qd[qoff + p][1], w = c_qd[qoff + p][3];
+      const double rx = d[0] + l1 * xa[0] + l2 * xb[0], ry = d[1] + l1 * xa[1] + l2 * xb[1],
+                   rz = d[2] + l1 * xa[2] + l2 * xb[2];
+      const double ux = u0[0] + l1 * ua[0] + l2 * ub[0], uy = u0[1] + l1 * ua[1] + l2 * ub[1],
+                   uz = u0[2] + l1 * ua[2] + l2 * ub[2];
+      const double ir = rsqrt64(rx * rx + ry * ry + rz * rz);
+      const double ir2 = ir * ir, w1 = w * ir, w3 = w1 * ir2, w5 = w3 * ir2;
+      const double cq = w3 * (rq0 + l1 * rqa + l2 * rqb);
+      const double cu = w5 * (rx * ux + ry * uy + rz * uz);
+      const double cv = k6 * cu + idiff * cq;
+      s1 += w1;
+      srq += cq;
+      sru += cu;
+      sun += w3 * (un0 + l1 * una + l2 * unb);
+      sv[0] += cv * rx;
+      sv[1] += cv * ry;
+      sv[2] += cv * rz;
+      s3[0] += w3 * rx;
+      s3[1] += w3 * ry;
+      s3[2] += w3 * rz;
+      s5[0] += w5 * rx * rx;
+      s5[1] += w5 * ry * ry;
+      s5[2] += w5 * rz * rz;
+    }
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
+    for (int c = 0; c < 3; ++c) {
+      a[c] += A * (sv[c] + idiff * qe[c] * s1);
+      a[5 + c] += A * k6 * s5[c];
+      a[8 + c] += A * (n[c] * s1 + rn * s3[c]);
+    }
+    a[3] += A * 4.0 * (3.0 * rn * sru - sun);
+    a[4] += A * 2.0 * srq;
+  }
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+  for (int i = 0; i < NDV; ++i) {
     double v = a[i];
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
     if (lane == 0) red[i][wid] = v;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double t[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) t[i] = (red[i][0] + red[i][1]) + (red[i][2] + red[i][3]);
-    double *o = out + 5 * (size_t)ip;
-    for (int c = 0; c < 3; ++c) o[c] = -(t[c] + t[3 + c] / diff) / osem;
-    o[3] = -(diff * t[6] - t[7]) / osem;
-    double err = -9.99;
-    for (int c = 0; c < 3; ++c) err = fmax(err, fabs(-t[8 + c] / osem - 1.0));
-    for (int c = 0; c < 3; ++c) err = fmax(err, fabs(t[11 + c]));
-    o[4] = err;
+  if (threadIdx.x < NDV) {
+    double t = 0.0;
+    for (int w = 0; w < nw; ++w) t += red[threadIdx.x][w];
+    part[((size_t)blockIdx.y * npts + ip) * NDV + threadIdx.x] = t;
   }
 }
 
+// out[5 p + 0..2] = velocity, out[5 p + 3] = pressure, out[5 p + 4] = the closure error of the point's
+// integrals (src/lib_Stokes.f90:3255-3300): the T closure -sum_i T_ii = 8 pi and sum_e G n_e = 0 hold
+// inside the domain. osem = 8 pi as the reference forms it.
+__global__ void k_stokes_domain_fin(int npts, int nchunk, const double *__restrict__ part, double diff, double osem,
+                                    double *__restrict__ out) {
+  const int ip = blockIdx.x * blockDim.x + threadIdx.x;
+  if (ip >= npts) return;
+  double t[NDV];
+#pragma unroll
+  for (int i = 0; i < NDV; ++i) t[i] = 0.0;
+  for (int c = 0; c < nchunk; ++c)
+#pragma unroll
+    for (int i = 0; i < NDV; ++i) t[i] += part[((size_t)c * npts + ip) * NDV + i];
+  double *o = out + 5 * (size_t)ip;
+  for (int c = 0; c < 3; ++c) o[c] = -t[c] / osem;
+  o[3] = -(diff * t[3] - t[4]) / osem;
+  double err = -9.99;
+  for (int c = 0; c < 3; ++c) err = fmax(err, fabs(-t[5 + c] / osem - 1.0));
+  for (int c = 0; c < 3; ++c) err = fmax(err, fabs(t[8 + c]));
+  o[4] = err;
+}
+
 // Surface pressure at the element centres: pressureStokes (src/lib_Stokes.f90:4-94) with the centroid
-// rows of prT and prG (sdIntRowQStokes, :1562-1897). One workgroup per element r; the pair (r, r)
-// is singular and has no pressure integrals. The row-sum correction of prT (:1851-1863) moves the
-// row sum onto the three nodes of element r; with u_c = the mean of those nodes' velocities
-// (InterpolateToQMesh) the row contracts to sum prT u - rowsum . u_c, so it is not formed:
-// p_r = -2 (diff (sum prT u - rowsum . u_c) - sum prG q) / 8 pi.
-__global__ __launch_bounds__(256) void k_stokes_surface_pressure(BodyGeom g, int qoff, int nq,
+// rows of prT and prG (sdIntRowQStokes, :1562-1897). A workgroup takes element r and a chunk of the
+// elements; the pair (r, r) is singular and has no pressure integrals. The row-sum correction of prT
+// (:1851-1863) moves the row sum onto the three nodes of element r; with u_c = the mean of those nodes'
+// velocities (InterpolateToQMesh) the corrected row is prT applied to u - u_c, which is what is
+// integrated, contracted at the quadrature point as in k_stokes_domain (40 FP64 operations and 3 sums a
+// point; 1000^2 elements x 126 points 431 -> 190 us):
+// p_r = -2 (diff sum prT (u - u_c) - sum prG q) / 8 pi.
+__global__ __launch_bounds__(256) void k_stokes_surface_pressure(BodyGeom g, int qoff, int nq, int chunk,
                                                                  const double *__restrict__ u,
-                                                                 const double *__restrict__ q, double diff,
-                                                                 double osem, double *__restrict__ p) {
-  constexpr int NV = 5;  // prT u, prT row sums (3), prG q
-  __shared__ double red[NV][4];
+                                                                 const double *__restrict__ q,
+                                                                 double *__restrict__ part) {
+  __shared__ double red[2][4];
   const int r = blockIdx.x;
   const double s[3] = {g.cen[3 * r], g.cen[3 * r + 1], g.cen[3 * r + 2]};
-  double a[NV] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int e = threadIdx.x; e < g.ne; e += blockDim.x) {
+  double uc[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    uc[c] = (u[3 * g.con[3 * r] + c] + u[3 * g.con[3 * r + 1] + c] + u[3 * g.con[3 * r + 2] + c]) / 3.0;
+  double pu = 0.0, pq = 0.0;
+  const int e1 = min(g.ne, (int)(blockIdx.y + 1) * chunk);
+  for (int e = blockIdx.y * chunk + threadIdx.x; e < e1; e += blockDim.x) {
     if (e == r) continue;
-    const int vv[3] = {g.con[3 * e], g.con[3 * e + 1], g.con[3 * e + 2]};
-    const double m = g.mul[e];
-    double Gs[6], pG[3], Tv[6][3], pT[3][3];
-    stokes_tri_full(s, g.xyz + 3 * vv[0], g.xyz + 3 * vv[1], g.xyz + 3 * vv[2], m * g.nrm[3 * e],
-                    m * g.nrm[3 * e + 1], m * g.nrm[3 * e + 2], g.area[e], qoff, nq, Gs, pG, Tv, pT);
+    const int v1 = 3 * g.con[3 * e], v2 = 3 * g.con[3 * e + 1], v3 = 3 * g.con[3 * e + 2];
+    const double m = g.mul[e], A = g.area[e];
+    double d[3], xa[3], xb[3], u0[3], ua[3], ub[3];
+    double rn = 0.0, un0 = 0.0, una = 0.0, unb = 0.0, rq0 = 0.0, rqa = 0.0, rqb = 0.0;
 #pragma unroll
-    for (int v = 0; v < 3; ++v) {
-      const double *uv = u + 3 * vv[v];
-      a[0] += pT[0][v] * uv[0] + pT[1][v] * uv[1] + pT[2][v] * uv[2];
-      a[1] += pT[0][v];
-      a[2] += pT[1][v];
-      a[3] += pT[2][v];
+    for (int c = 0; c < 3; ++c) {
+      const double x3 = g.xyz[v3 + c], w3 = u[v3 + c], n = m * g.nrm[3 * e + c], qe = q[3 * e + c];
+      d[c] = x3 - s[c];
+      xa[c] = g.xyz[v1 + c] - x3;
+      xb[c] = g.xyz[v2 + c] - x3;
+      u0[c] = w3 - uc[c];
+      ua[c] = u[v1 + c] - w3;
+      ub[c] = u[v2 + c] - w3;
+      rn += d[c] * n;
+      un0 += n * u0[c];
+      una += n * ua[c];
+      unb += n * ub[c];
+      rq0 += d[c] * qe;
+      rqa += xa[c] * qe;
+      rqb += xb[c] * qe;
     }
-    a[4] += pG[0] * q[3 * e] + pG[1] * q[3 * e + 1] + pG[2] * q[3 * e + 2];
+    double sun = 0.0, sru = 0.0, srq = 0.0;
+    for (int p = 0; p < nq; ++p) {
+      const double l1 = c_qd[qoff + p][0], l2 = c_qd[qoff + p][1], w = c_qd[qoff + p][3];
+      const double rx = d[0] + l1 * xa[0] + l2 * xb[0], ry = d[1] + l1 * xa[1] + l2 * xb[1],
+                   rz = d[2] + l1 * xa[2] + l2 * xb[2];
+      const double ux = u0[0] + l1 * ua[0] + l2 * ub[0], uy = u0[1] + l1 * ua[1] + l2 * ub[1],
+                   uz = u0[2] + l1 * ua[2] + l2 * ub[2];
+      const double ir = rsqrt64(rx * rx + ry * ry + rz * rz);
+      const double ir2 = ir * ir, w3 = w * ir * ir2, w5 = w3 * ir2;
+      srq += w3 * (rq0 + l1 * rqa + l2 * rqb);
+      sun += w3 * (un0 + l1 * una + l2 * unb);
+      sru += w5 * (rx * ux + ry * uy + rz * uz);
+    }
+    pu += A * 4.0 * (3.0 * rn * sru - sun);
+    pq += A * 2.0 * srq;
   }
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    double v = a[i];
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (lane == 0) red[i][wid] = v;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  for (int off = 32; off >= 1; off >>= 1) {
+    pu += __shfl_xor(pu, off, 64);
+    pq += __shfl_xor(pq, off, 64);
+  }
+  if (lane == 0) {
+    red[0][wid] = pu;
+    red[1][wid] = pq;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double t[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) t[i] = (red[i][0] + red[i][1]) + (red[i][2] + red[i][3]);
-    const int c0 = g.con[3 * r], c1 = g.con[3 * r + 1], c2 = g.con[3 * r + 2];
-    double pu = t[0];
-    for (int k = 0; k < 3; ++k) pu -= t[1 + k] * ((u[3 * c0 + k] + u[3 * c1 + k] + u[3 * c2 + k]) / 3.0);
-    p[r] = -(diff * pu - t[4]) / osem * 2.0;
+  if (threadIdx.x < 2) {
+    double t = 0.0;
+    for (int w = 0; w < nw; ++w) t += red[threadIdx.x][w];
+    part[((size_t)blockIdx.y * g.ne + r) * 2 + threadIdx.x] = t;
   }
+}
+
+__global__ void k_stokes_surface_fin(int ne, int nchunk, const double *__restrict__ part, double diff, double osem,
+                                     double *__restrict__ p) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= ne) return;
+  double pu = 0.0, pq = 0.0;
+  for (int c = 0; c < nchunk; ++c) {
+    pu += part[((size_t)c * ne + r) * 2];
+    pq += part[((size_t)c * ne + r) * 2 + 1];
+  }
+  p[r] = -(diff * pu - pq) / osem * 2.0;
+}
+
+// How the elements of a sum over the body are dealt to workgroups: chunks of elements (so that a few
+// points still fill the chip: 2048 waves, down to one wave a chunk), and threads per workgroup such that
+// the last turn over a chunk is as full as the others.
+struct ElemSplit {
+  int chunk, nchunk, threads;
+};
+static ElemSplit elem_split(int ne, int points) {
+  ElemSplit s;
+  s.nchunk = 1;
+  if (points * 4 < 2048) s.nchunk = std::min((ne + 63) / 64, (2048 + 4 * points - 1) / (4 * points));
+  s.chunk = (ne + s.nchunk - 1) / s.nchunk;
+  s.chunk = (s.chunk + 63) / 64 * 64;
+  s.nchunk = (ne + s.chunk - 1) / s.chunk;
+  const int len = std::min(s.chunk, ne), turns = (len + 255) / 256;
+  s.threads = ((len + turns - 1) / turns + 63) / 64 * 64;
+  return s;
 }
 
 int andr_launch_stokes_surface_pressure(andr_ctx *ctx, DevBody &b, const double *u, const double *q, double diff,
@@ -907,10 +1020,16 @@ int andr_launch_stokes_surface_pressure(andr_ctx *ctx, DevBody &b, const double 
   const QuadRule qr = andr_rule(b.itri);
   const double osem = (double)atanf(1.0f) * 4.0 * 8.0;  // REAL(4) ATAN(1.0) (src/lib_Stokes.f90:17)
   const double evals = (double)b.g.ne * (b.g.ne - 1.0) * qr.npts;
-  const int tok = andr_prof_begin(ctx, "stokes_surface_pressure", 8.0 * (3.0 * b.g.nn + 4.0 * b.g.ne), evals * 175.0);
-  hipLaunchKernelGGL(k_stokes_surface_pressure, dim3(b.g.ne), dim3(256), 0, ctx->stream, b.g, qr.offset, qr.npts, u,
-                     q, diff, osem, p);
+  const ElemSplit sp = elem_split(b.g.ne, b.g.ne);
+  DevBuf<double> part;
+  if (part.alloc((size_t)sp.nchunk * b.g.ne * 2, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "surface pressure sums");
+  const int tok = andr_prof_begin(ctx, "stokes_surface_pressure", 8.0 * (3.0 * b.g.nn + 4.0 * b.g.ne),
+                                  evals * ANDR_FLOPS_PER_SURFACE_EVAL);
+  hipLaunchKernelGGL(k_stokes_surface_pressure, dim3(b.g.ne, sp.nchunk), dim3(sp.threads), 0, ctx->stream, b.g,
+                     qr.offset, qr.npts, sp.chunk, u, q, part.p);
   andr_prof_end(ctx, tok);
+  hipLaunchKernelGGL(k_stokes_surface_fin, dim3((b.g.ne + 255) / 256), dim3(256), 0, ctx->stream, b.g.ne, sp.nchunk,
+                     part.p, diff, osem, p);
   ANDR_HIP(ctx, hipGetLastError());
   return ANDR_OK;
 }
@@ -921,10 +1040,15 @@ int andr_launch_stokes_domain(andr_ctx *ctx, DevBody &b, int npts, const double 
   const QuadRule qr = andr_rule(b.itri);
   const double osem = (double)atanf(1.0f) * 4.0 * 8.0;  // REAL(4) ATAN(1.0) (src/lib_Stokes.f90:3089)
   const double evals = (double)npts * b.g.ne * qr.npts;
-  const int tok = andr_prof_begin(ctx, "stokes_domain", 8.0 * (3.0 * npts + 5.0 * npts), evals * 175.0);
-  hipLaunchKernelGGL(k_stokes_domain, dim3(npts), dim3(256), 0, ctx->stream, b.g, qr.offset, qr.npts, pts, u, q, diff,
-                     osem, out);
+  const ElemSplit sp = elem_split(b.g.ne, npts);
+  DevBuf<double> part;
+  if (part.alloc((size_t)sp.nchunk * npts * NDV, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "domain point sums");
+  const int tok = andr_prof_begin(ctx, "stokes_domain", 8.0 * (3.0 * npts + 5.0 * npts), evals * ANDR_FLOPS_PER_DOMAIN_EVAL);
+  hipLaunchKernelGGL(k_stokes_domain, dim3(npts, sp.nchunk), dim3(sp.threads), 0, ctx->stream, b.g, qr.offset, qr.npts,
+                     pts, npts, sp.chunk, u, q, diff, part.p);
   andr_prof_end(ctx, tok);
+  hipLaunchKernelGGL(k_stokes_domain_fin, dim3((npts + 255) / 256), dim3(256), 0, ctx->stream, npts, sp.nchunk, part.p,
+                     diff, osem, out);
   ANDR_HIP(ctx, hipGetLastError());
   return ANDR_OK;
 }

@@ -14,6 +14,15 @@ static inline int andr_upload_rules_here(andr_ctx *ctx, const double *tab, const
 }
 
 
+// 1 / sqrt(x) in FP64 for x > 0: the hardware estimate (v_rsq_f64, error e below 2^-20) and one step of
+// third order (Householder), which leaves e^3: five operations against the some twenty of a division and
+// a square root in their general forms.
+__device__ inline double rsqrt64(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
 // The regular integrals of one triangle seen from s, in FP64 with pressure (Triangle_3DStokesInt,
 // src/lib_Stokes.f90:2341-2446, with StokesKernel :2450-2544): Stokeslet Gs, pressure vector pG,
 // stresslet moments Tv and pressure moments pT per vertex, for the normal (nx, ny, nz) and area A.
