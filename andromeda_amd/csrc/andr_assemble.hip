@@ -2,11 +2,13 @@
 // direct emission of the Stokes resistance system (matrix in its final solver layout plus the
 // right-hand sides of the rigid-body problems), FP64 or FP32 regular quadrature.
 //
-// Work decomposition: one 256-thread workgroup per collocation row. The quadrature rule sits in
-// constant memory (every lane of a wave reads the same point, a scalar load). Node-indexed rows
-// (H, T, prT) are accumulated element colour by element colour: no two elements of a colour share
-// a node, so the scatter needs neither atomics nor a fixed thread-to-element map, and the sums are
-// reproducible run to run. The row buffer lives in LDS when it fits, else in the output row.
+// Work decomposition: one workgroup of up to 256 threads per collocation row. The quadrature rule sits
+// in constant memory (every lane of a wave reads the same point, a scalar load). Node-indexed rows
+// (H, T, prT) are summed turn by turn of the workgroup over the elements: a thread integrates one element
+// into registers, then the turn's elements are added colour by colour (no two elements of a colour share a
+// node), so that the integration fills the workgroup whatever the colours' sizes (a colour of 720 elements
+// holds some 90), the scatter needs no atomics and the sums are reproducible run to run. The row buffer
+// lives in LDS when it fits, else in the output row.
 #include "andr_internal.h"
 #include "andr_singular.h"
 #include "andr_wx_rules.h"
@@ -183,11 +185,13 @@ __global__ void k_geometry(int ne, int nv, const double *__restrict__ xyz, const
   }
 }
 
-// Greedy colouring of elements so that no two elements of a colour share a node.
-static int color_elements(int nn, int ne, int nv, const int *con, std::vector<int> &order, std::vector<int> &off) {
+// Greedy colouring of elements so that no two elements of a colour share a node: the elements in the
+// order the row kernels take them (quadrilaterals first, so that a wave integrates one kind) and their
+// colours in that order. Returns the number of colours, -1 when there are too many.
+static int color_elements(int nn, int ne, int nv, const int *con, std::vector<int> &order, std::vector<uint8_t> &color) {
   constexpr int MAXC = 256;  // an element sees at most sum over its nodes of (valence - 1) colours
   std::vector<std::bitset<MAXC>> used(nn);
-  std::vector<int> col(ne);
+  std::vector<uint8_t> col(ne);
   int ncol = 0;
   for (int e = 0; e < ne; ++e) {
     const int *cn = con + (size_t)nv * e;
@@ -197,17 +201,17 @@ static int color_elements(int nn, int ne, int nv, const int *con, std::vector<in
     int c = 0;
     while (c < MAXC && m[c]) ++c;
     if (c >= MAXC) return -1;
-    col[e] = c;
+    col[e] = (uint8_t)c;
     ncol = std::max(ncol, c + 1);
     for (int v = 0; v < nno; ++v) used[cn[v]].set(c);
   }
-  off.assign(ncol + 1, 0);
-  for (int e = 0; e < ne; ++e) off[col[e] + 1]++;
-  for (int c = 0; c < ncol; ++c) off[c + 1] += off[c];
-  order.resize(ne);
-  std::vector<int> pos(off.begin(), off.end() - 1);
-  for (int e = 0; e < ne; ++e) order[pos[col[e]]++] = e;
-  return 0;
+  order.clear();
+  for (int quad = 1; quad >= 0; --quad)
+    for (int e = 0; e < ne; ++e)
+      if ((nv == 4 && con[(size_t)nv * e + 3] >= 0) == (quad == 1)) order.push_back(e);
+  color.resize(ne);
+  for (int i = 0; i < ne; ++i) color[i] = col[order[i]];
+  return ncol;
 }
 
 // the mesh checks with the message in msg (host only: no context, no device)
@@ -291,13 +295,13 @@ int andr_body_upload(andr_ctx *ctx, const andr_mesh *m, DevBody &b, bool with_co
   ANDR_HIP(ctx, hipGetLastError());
   if (with_colors) {
     std::vector<int> order;
-    if (color_elements(nn, ne, nv, con.data(), order, b.color_off))
-      return andr_fail(ctx, ANDR_ERR_ARG, "mesh node valence too high for the element colouring");
-    if (b.color_elems.alloc(ne) || b.d_color_off.alloc(b.color_off.size()))
+    std::vector<uint8_t> color;
+    b.ncolors = color_elements(nn, ne, nv, con.data(), order, color);
+    if (b.ncolors < 0) return andr_fail(ctx, ANDR_ERR_ARG, "mesh node valence too high for the element colouring");
+    if (b.order.alloc(ne, ctx) || b.color.alloc(ne, ctx))
       return andr_fail(ctx, ANDR_ERR_ALLOC, "device allocation for colours");
-    ANDR_HIP(ctx, hipMemcpyAsync(b.color_elems.p, order.data(), sizeof(int) * ne, hipMemcpyHostToDevice, ctx->stream));
-    ANDR_HIP(ctx, hipMemcpyAsync(b.d_color_off.p, b.color_off.data(), sizeof(int) * b.color_off.size(),
-                                 hipMemcpyHostToDevice, ctx->stream));
+    ANDR_HIP(ctx, hipMemcpyAsync(b.order.p, order.data(), sizeof(int) * ne, hipMemcpyHostToDevice, ctx->stream));
+    ANDR_HIP(ctx, hipMemcpyAsync(b.color.p, color.data(), ne, hipMemcpyHostToDevice, ctx->stream));
   }
   // No synchronisation here: d_wm returns to the context's cache, and any later use of that block
   // is ordered after k_geometry on the same stream; the host vectors were staged by the copies.
@@ -380,23 +384,75 @@ __device__ inline double dist3(const double *a, const double *b) {
   return sqrt(dx * dx + dy * dy + dz * dz);
 }
 
-// Laplace pair of a quadrilateral: out = {G, H at nodes 1..4}; isrc 1..4 vertex, 5 centre source
-__device__ __noinline__ void quad_laplace_pair(const double *x1, const double *x2, const double *x3,
-                                               const double *x4, const double *s, double mul, int iq, int isrc,
-                                               double *out) {
+// Laplace pair of a quadrilateral: out = {G, H at nodes 1..4}; isrc 1..4 vertex, 5 centre source.
+// With f = c0 + gi c1 + gj c2 + gi gj c3 the point and the unnormalised normal x_ksi x x_eta are linear
+// in gj for a fixed gi (x_eta = c2 + gi c3 does not depend on gj), and so is r.n |J|, since the normal is
+// at right angles to x_eta: some 36 FP64 operations a point, where shape functions, both tangents and a
+// normalised normal at every point took over 200 with four divisions. Bound by FP64 issue (1402 rows of
+// 400 quadrilaterals at 256 points and 400 triangles at 126: 6910 -> 402 us).
+__device__ __forceinline__ void quad_laplace_pair(const double *x1, const double *x2, const double *x3, const double *x4,
+                                                  const double *s, double mul, int iq, int isrc, double out[5]) {
+#pragma unroll
   for (int k = 0; k < 5; ++k) out[k] = 0.0;
   if (isrc == 0) {
     const double d13 = fmax(dist3(x1, x2), dist3(x3, x4)), d24 = fmax(dist3(x2, x3), dist3(x4, x1));
     const int ndx = max(2, (int)(d13 + 0.5)), ndy = max(2, (int)(d24 + 0.5));  // minedge = 1
-    const double k4pi = 0.25 / ANDR_PI;
-    quad_cells(x1, x2, x3, x4, mul, iq, ndx, ndy, [&](const double *fig4, const double *f, const double *n, double w) {
-      const double rx = s[0] - f[0], ry = s[1] - f[1], rz = s[2] - f[2];  // r = s - f
-      const double ira = rsqrt(rx * rx + ry * ry + rz * rz);
-      const double fg = k4pi * ira;
-      const double fh = (rx * n[0] + ry * n[1] + rz * n[2]) * ira * ira * fg;
-      out[0] += w * fg;
-      for (int k = 0; k < 4; ++k) out[1 + k] += w * fh * fig4[k];
-    });
+    double sc0[3], c1[3], c2[3], c3[3];  // s - c0, c1, c2, c3
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      sc0[k] = s[k] - 0.25 * ((x1[k] + x2[k]) + (x3[k] + x4[k]));
+      c1[k] = 0.25 * ((x2[k] - x1[k]) + (x3[k] - x4[k]));
+      c2[k] = 0.25 * ((x4[k] - x1[k]) + (x3[k] - x2[k]));
+      c3[k] = 0.25 * ((x1[k] - x2[k]) + (x3[k] - x4[k]));
+    }
+    const int off = c_gl_off[iq], N = c_gl_n[iq];
+    const double hx = 1.0 / ndx, hy = 1.0 / ndy;  // half cell widths
+    for (int ix = 0; ix < ndx; ++ix)
+      for (int i = 0; i < N; ++i) {
+        const double gi = -1.0 + (2 * ix + 1) * hx + c_gl[off + i][0] * hx;
+        double r0[3], et[3], n0[3], n1[3];  // r = r0 - gj et, normal n0 + gj n1
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          r0[k] = sc0[k] - gi * c1[k];
+          et[k] = c2[k] + gi * c3[k];
+        }
+        n0[0] = c1[1] * et[2] - c1[2] * et[1];
+        n0[1] = c1[2] * et[0] - c1[0] * et[2];
+        n0[2] = c1[0] * et[1] - c1[1] * et[0];
+        n1[0] = c3[1] * et[2] - c3[2] * et[1];
+        n1[1] = c3[2] * et[0] - c3[0] * et[2];
+        n1[2] = c3[0] * et[1] - c3[1] * et[0];
+        const double ra = r0[0] * n0[0] + r0[1] * n0[1] + r0[2] * n0[2];
+        const double rb = r0[0] * n1[0] + r0[1] * n1[1] + r0[2] * n1[2];
+        double sg = 0.0, h0 = 0.0, h1 = 0.0;
+        for (int iy = 0; iy < ndy; ++iy) {
+          const double gc = -1.0 + (2 * iy + 1) * hy;
+          for (int j = 0; j < N; ++j) {
+            const double gj = gc + c_gl[off + j][0] * hy, w = c_gl[off + j][1];
+            const double rx = r0[0] - gj * et[0], ry = r0[1] - gj * et[1], rz = r0[2] - gj * et[2];
+            const double ax = n0[0] + gj * n1[0], ay = n0[1] + gj * n1[1], az = n0[2] + gj * n1[2];
+            const double l2 = ax * ax + ay * ay + az * az;
+            const double len = l2 > 0.0 ? l2 * rsqrt64(l2) : 0.0;
+            const double ir = rsqrt64(rx * rx + ry * ry + rz * rz);
+            const double wi = w * ir;
+            sg += wi * len;
+            const double wh = wi * (ir * ir) * (ra + gj * rb);
+            h0 += wh;
+            h1 += wh * gj;
+          }
+        }
+        const double wi = c_gl[off + i][1];
+        out[0] += wi * sg;
+        const double hm = wi * (h0 - h1), hp = wi * (h0 + h1);
+        out[1] += (1.0 - gi) * hm;
+        out[2] += (1.0 + gi) * hm;
+        out[3] += (1.0 + gi) * hp;
+        out[4] += (1.0 - gi) * hp;
+      }
+    const double sc = (0.25 / ANDR_PI) * hx * hy;
+    out[0] *= sc;
+#pragma unroll
+    for (int k = 1; k < 5; ++k) out[k] *= 0.25 * mul * sc;
     return;
   }
   const double *v[4] = {x1, x2, x3, x4};
@@ -465,10 +521,12 @@ __device__ __noinline__ void quad_stokes_pair(const double *x1, const double *x2
 // Triangle_3DLapInt (:859-905) with BemKernel (:911-936), singular by the analytic formula.
 // ------------------------------------------------------------------------------------------------
 // F32Q: the regular integrals in FP32 (relative geometry formed in FP64, quadrature and sums in FP32,
-// scaled by the area in FP64), the singular ones in FP64 (the mixed-precision Laplace form)
-template <bool ROW_IN_LDS, bool F32Q>
-__global__ __launch_bounds__(256) void k_laplace_rows(BodyGeom g, int qoff, int nq, const int *__restrict__ celems,
-                                                      const int *__restrict__ coff, int ncolors,
+// scaled by the area in FP64), the singular ones in FP64 (the mixed-precision Laplace form). QUADS: the mesh
+// may hold quadrilaterals. FP64 triangles: r.n is one number per flat element, 1 / r from rsqrt64, 27
+// FP64 operations a point (2164 rows of 1440 triangles 684 -> 312 us, bound by FP64 issue).
+template <bool ROW_IN_LDS, bool F32Q, bool QUADS>
+__global__ __launch_bounds__(256) void k_laplace_rows(BodyGeom g, int qoff, int nq, const int *__restrict__ order,
+                                                      const uint8_t *__restrict__ color, int ncolors,
                                                       double *__restrict__ H, double *__restrict__ G,
                                                       double *__restrict__ err_rows, int r0) {
   extern __shared__ double lds[];
@@ -488,90 +546,102 @@ __global__ __launch_bounds__(256) void k_laplace_rows(BodyGeom g, int qoff, int 
   for (int i = threadIdx.x; i < nn; i += blockDim.x) hrow[i] = 0.0;
   __syncthreads();
   const double k4pi = 0.25 / ANDR_PI;
-  for (int c = 0; c < ncolors; ++c) {
-    for (int idx = coff[c] + threadIdx.x; idx < coff[c + 1]; idx += blockDim.x) {
-      const int e = celems[idx];
+  for (int i0 = 0; i0 < ne; i0 += blockDim.x) {
+    const int idx = i0 + threadIdx.x;
+    int col = -1, v0 = 0, v1 = 0, v2 = 0, v3 = -1;
+    double h[4] = {0.0, 0.0, 0.0, 0.0};
+    if (idx < ne) {
+      const int e = order[idx];
+      col = color[idx];
       const int *cn = g.con + (size_t)g.nv * e;
-      const int v0 = cn[0], v1 = cn[1], v2 = cn[2];
+      v0 = cn[0];
+      v1 = cn[1];
+      v2 = cn[2];
+      if (QUADS) v3 = cn[3];
       const double *x1 = g.xyz + 3 * v0, *x2 = g.xyz + 3 * v1, *x3 = g.xyz + 3 * v2;
-      if (g.nv == 4 && cn[3] >= 0) {  // quadrilateral (Quad_BEMIntNumAna, src/lib_intAna.f90:153-176)
-        const int v3 = cn[3];
+      if (QUADS && v3 >= 0) {  // quadrilateral (Quad_BEMIntNumAna, src/lib_intAna.f90:153-176)
         int qs = 0;
         if (!qrow) qs = (v0 == r) ? 1 : (v1 == r) ? 2 : (v2 == r) ? 3 : (v3 == r) ? 4 : 0;
         else if (e == erow) qs = 5;
         double out[5];
         quad_laplace_pair(x1, x2, x3, g.xyz + 3 * v3, s, g.mul[e], g.iquad, qs, out);
         grow[e] = out[0];
-        hrow[v0] += out[1];
-        hrow[v1] += out[2];
-        hrow[v2] += out[3];
-        hrow[v3] += out[4];
-        continue;
-      }
-      int isrc = 0;
-      if (!qrow) isrc = (v0 == r) ? 1 : (v1 == r) ? 2 : (v2 == r) ? 3 : 0;
-      else if (e == erow) isrc = 4;
-      double gv, h1 = 0.0, h2 = 0.0, h3 = 0.0;
-      if (isrc == 0 && F32Q) {
-        const double m = g.mul[e];
-        const float nx = (float)(m * g.nrm[3 * e]), ny = (float)(m * g.nrm[3 * e + 1]), nz = (float)(m * g.nrm[3 * e + 2]);
-        // r = s - f = d - l1 a - l2 b with d = s - x3, a = x1 - x3, b = x2 - x3 (l3 = 1 - l1 - l2)
-        const float d0 = (float)(s[0] - x3[0]), d1 = (float)(s[1] - x3[1]), d2 = (float)(s[2] - x3[2]);
-        const float a0 = (float)(x1[0] - x3[0]), a1 = (float)(x1[1] - x3[1]), a2 = (float)(x1[2] - x3[2]);
-        const float b0 = (float)(x2[0] - x3[0]), b1 = (float)(x2[1] - x3[1]), b2 = (float)(x2[2] - x3[2]);
-        const float k4 = (float)k4pi;
-        float gs = 0.f, f1 = 0.f, f2 = 0.f, f3 = 0.f;
-        for (int q = 0; q < nq; ++q) {
-          const float l1 = c_qf[qoff + q][0], l2 = c_qf[qoff + q][1], l3 = c_qf[qoff + q][2], w = c_qf[qoff + q][3];
-          const float rx = d0 - l1 * a0 - l2 * b0;
-          const float ry = d1 - l1 * a1 - l2 * b1;
-          const float rz = d2 - l1 * a2 - l2 * b2;
-          const float ira = __frsqrt_rn(rx * rx + ry * ry + rz * rz);
-          const float fg = k4 * ira;
-          const float wh = w * (rx * nx + ry * ny + rz * nz) * ira * ira * fg;
-          gs += w * fg;
-          f1 += wh * l1;
-          f2 += wh * l2;
-          f3 += wh * l3;
-        }
-        const double A = g.area[e];
-        gv = (double)gs * A;
-        h1 = (double)f1 * A;
-        h2 = (double)f2 * A;
-        h3 = (double)f3 * A;
-      } else if (isrc == 0) {
-        const double m = g.mul[e];
-        const double nx = m * g.nrm[3 * e], ny = m * g.nrm[3 * e + 1], nz = m * g.nrm[3 * e + 2];
-        // r = s - f with f = l1 x1 + l2 x2 + l3 x3
-        double gs = 0.0;
-        for (int q = 0; q < nq; ++q) {
-          const double l1 = c_qd[qoff + q][0], l2 = c_qd[qoff + q][1], l3 = c_qd[qoff + q][2], w = c_qd[qoff + q][3];
-          const double rx = s[0] - (l1 * x1[0] + l2 * x2[0] + l3 * x3[0]);
-          const double ry = s[1] - (l1 * x1[1] + l2 * x2[1] + l3 * x3[1]);
-          const double rz = s[2] - (l1 * x1[2] + l2 * x2[2] + l3 * x3[2]);
-          const double ira = rsqrt(rx * rx + ry * ry + rz * rz);
-          const double fg = k4pi * ira;
-          const double fh = (rx * nx + ry * ny + rz * nz) * ira * ira * fg;
-          gs += w * fg;
-          const double wh = w * fh;
-          h1 += wh * l1;
-          h2 += wh * l2;
-          h3 += wh * l3;
-        }
-        const double A = g.area[e];
-        gv = gs * A;
-        h1 *= A;
-        h2 *= A;
-        h3 *= A;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) h[v] = out[1 + v];
       } else {
-        gv = andr_sing_lap(x1, x2, x3, s, isrc);
+        int isrc = 0;
+        if (!qrow) isrc = (v0 == r) ? 1 : (v1 == r) ? 2 : (v2 == r) ? 3 : 0;
+        else if (e == erow) isrc = 4;
+        double gv;
+        if (isrc == 0 && F32Q) {
+          const double m = g.mul[e];
+          const float nx = (float)(m * g.nrm[3 * e]), ny = (float)(m * g.nrm[3 * e + 1]), nz = (float)(m * g.nrm[3 * e + 2]);
+          // r = s - f = d - l1 a - l2 b with d = s - x3, a = x1 - x3, b = x2 - x3 (l3 = 1 - l1 - l2)
+          const float d0 = (float)(s[0] - x3[0]), d1 = (float)(s[1] - x3[1]), d2 = (float)(s[2] - x3[2]);
+          const float a0 = (float)(x1[0] - x3[0]), a1 = (float)(x1[1] - x3[1]), a2 = (float)(x1[2] - x3[2]);
+          const float b0 = (float)(x2[0] - x3[0]), b1 = (float)(x2[1] - x3[1]), b2 = (float)(x2[2] - x3[2]);
+          const float k4 = (float)k4pi;
+          float gs = 0.f, f1 = 0.f, f2 = 0.f, f3 = 0.f;
+          for (int q = 0; q < nq; ++q) {
+            const float l1 = c_qf[qoff + q][0], l2 = c_qf[qoff + q][1], l3 = c_qf[qoff + q][2], w = c_qf[qoff + q][3];
+            const float rx = d0 - l1 * a0 - l2 * b0;
+            const float ry = d1 - l1 * a1 - l2 * b1;
+            const float rz = d2 - l1 * a2 - l2 * b2;
+            const float ira = __frsqrt_rn(rx * rx + ry * ry + rz * rz);
+            const float fg = k4 * ira;
+            const float wh = w * (rx * nx + ry * ny + rz * nz) * ira * ira * fg;
+            gs += w * fg;
+            f1 += wh * l1;
+            f2 += wh * l2;
+            f3 += wh * l3;
+          }
+          const double A = g.area[e];
+          gv = (double)gs * A;
+          h[0] = (double)f1 * A;
+          h[1] = (double)f2 * A;
+          h[2] = (double)f3 * A;
+        } else if (isrc == 0) {
+          double d[3], xa[3], xb[3], rn = 0.0;  // r = s - f = d - l1 xa - l2 xb
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            d[c] = s[c] - x3[c];
+            xa[c] = x1[c] - x3[c];
+            xb[c] = x2[c] - x3[c];
+            rn += d[c] * g.nrm[3 * e + c];
+          }
+          double gs = 0.0, f1 = 0.0, f2 = 0.0, f3 = 0.0;
+          for (int q = 0; q < nq; ++q) {
+            const double l1 = c_qd[qoff + q][0], l2 = c_qd[qoff + q][1], l3 = c_qd[qoff + q][2], w = c_qd[qoff + q][3];
+            const double rx = d[0] - l1 * xa[0] - l2 * xb[0];
+            const double ry = d[1] - l1 * xa[1] - l2 * xb[1];
+            const double rz = d[2] - l1 * xa[2] - l2 * xb[2];
+            const double ir = rsqrt64(rx * rx + ry * ry + rz * rz);
+            const double w1 = w * ir, w3 = w1 * (ir * ir);
+            gs += w1;
+            f1 += w3 * l1;
+            f2 += w3 * l2;
+            f3 += w3 * l3;
+          }
+          gv = k4pi * g.area[e] * gs;
+          const double ch = k4pi * g.area[e] * (g.mul[e] * rn);
+          h[0] = ch * f1;
+          h[1] = ch * f2;
+          h[2] = ch * f3;
+        } else {
+          gv = andr_sing_lap(x1, x2, x3, s, isrc);
+        }
+        grow[e] = gv;
       }
-      grow[e] = gv;
-      hrow[v0] += h1;
-      hrow[v1] += h2;
-      hrow[v2] += h3;
     }
-    __syncthreads();
+    for (int c = 0; c < ncolors; ++c) {
+      if (col == c) {
+        hrow[v0] += h[0];
+        hrow[v1] += h[1];
+        hrow[v2] += h[2];
+        if (QUADS && v3 >= 0) hrow[v3] += h[3];
+      }
+      __syncthreads();
+    }
   }
   // free term c = -sum_row H (rigid-body trick, src/lib_sdBem.f90:552-562, 714-731)
   double acc[1] = {0.0};
@@ -608,21 +678,30 @@ __global__ __launch_bounds__(256) void k_laplace_rows(BodyGeom g, int qoff, int 
   if (threadIdx.x == 0) err_rows[ro] = err;
 }
 
+// threads of a row's workgroup: 256, fewer where that makes its turns over the elements equally full
+static int row_threads(int ne) {
+  const int turns = (ne + 255) / 256;
+  return ((ne + turns - 1) / turns + 63) / 64 * 64;
+}
+
 int andr_launch_laplace_rows(andr_ctx *ctx, DevBody &b, double *H, double *G, double *err_rows, int r0, int nrows,
                              bool fp32_quad) {
   QuadRule qr = andr_rule(b.itri);
   const int nsp = nrows < 0 ? b.g.nn + b.g.ne - r0 : nrows;  // rows r0 .. r0 + nsp - 1
-  const int ncol = (int)b.color_off.size() - 1;
   const size_t lds = sizeof(double) * b.g.nn;
   const double evals = (double)nsp * b.g.ne * qr.npts;
   const int tok = andr_prof_begin(ctx, fp32_quad ? "laplace_rows_fp32" : "laplace_rows",
                                   8.0 * nsp * ((double)b.g.nn + b.g.ne), evals * ANDR_FLOPS_PER_LAPLACE_EVAL);
-  const bool in_lds = lds <= 128 * 1024;
-  auto kern = in_lds ? (fp32_quad ? k_laplace_rows<true, true> : k_laplace_rows<true, false>)
-                     : (fp32_quad ? k_laplace_rows<false, true> : k_laplace_rows<false, false>);
+  const bool in_lds = lds <= 128 * 1024, quads = b.g.nv == 4;
+  using Kern = void (*)(BodyGeom, int, int, const int *, const uint8_t *, int, double *, double *, double *, int);
+  const Kern kerns[8] = {k_laplace_rows<false, false, false>, k_laplace_rows<false, false, true>,
+                         k_laplace_rows<false, true, false>,  k_laplace_rows<false, true, true>,
+                         k_laplace_rows<true, false, false>,  k_laplace_rows<true, false, true>,
+                         k_laplace_rows<true, true, false>,   k_laplace_rows<true, true, true>};
+  const Kern kern = kerns[(in_lds ? 4 : 0) + (fp32_quad ? 2 : 0) + (quads ? 1 : 0)];
   if (in_lds) ANDR_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(kern, dim3(nsp), dim3(256), in_lds ? lds : 0, ctx->stream, b.g, qr.offset, qr.npts,
-                     b.color_elems.p, b.d_color_off.p, ncol, H, G, err_rows, r0);
+  hipLaunchKernelGGL(kern, dim3(nsp), dim3(row_threads(b.g.ne)), in_lds ? lds : 0, ctx->stream, b.g, qr.offset, qr.npts,
+                     b.order.p, b.color.p, b.ncolors, H, G, err_rows, r0);
   andr_prof_end(ctx, tok);
   ANDR_HIP(ctx, hipGetLastError());
   return ANDR_OK;
@@ -633,9 +712,9 @@ int andr_launch_laplace_rows(andr_ctx *ctx, DevBody &b, double *H, double *G, do
 // by Triangle_3DStokesInt (:2341-2446) with StokesKernel (:2450-2544).
 // Outputs: T[6][nsp][nn], G[6][nsp][ne], prT[3][nsp][nn], prG[3][nsp][ne].
 // ------------------------------------------------------------------------------------------------
-template <bool ROW_IN_LDS>
-__global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int nq, const int *__restrict__ celems,
-                                                     const int *__restrict__ coff, int ncolors, double extra,
+template <bool ROW_IN_LDS, bool QUADS>
+__global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int nq, const int *__restrict__ order,
+                                                     const uint8_t *__restrict__ color, int ncolors, double extra,
                                                      double *__restrict__ T, double *__restrict__ G,
                                                      double *__restrict__ prT, double *__restrict__ prG,
                                                      double *__restrict__ err_rows, int r0, int nrows) {
@@ -662,59 +741,79 @@ __global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int n
     for (int i = threadIdx.x; i < nn; i += blockDim.x) p[i] = 0.0;
   }
   __syncthreads();
-  for (int c = 0; c < ncolors; ++c) {
-    for (int idx = coff[c] + threadIdx.x; idx < coff[c + 1]; idx += blockDim.x) {
-      const int e = celems[idx];
+  constexpr int NV = QUADS ? 4 : 3;
+  for (int i0 = 0; i0 < ne; i0 += blockDim.x) {
+    const int idx = i0 + threadIdx.x;
+    int col = -1, nno = 3, vv[NV] = {0};
+    double t[9][NV];  // T (6) and prT (3) at the element's nodes
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) t[k][v] = 0.0;
+    if (idx < ne) {
+      const int e = order[idx];
+      col = color[idx];
       const int *cn = g.con + (size_t)g.nv * e;
-      const int vv[3] = {cn[0], cn[1], cn[2]};
+#pragma unroll
+      for (int v = 0; v < NV; ++v) vv[v] = cn[v];
       const double *x1 = g.xyz + 3 * vv[0], *x2 = g.xyz + 3 * vv[1], *x3 = g.xyz + 3 * vv[2];
-      if (g.nv == 4 && cn[3] >= 0) {  // quadrilateral (Quad_StokesIntNumAna, src/lib_intAna.f90:5-37)
-        const int v4[4] = {cn[0], cn[1], cn[2], cn[3]};
-        int qs = 0;
-        if (!qrow) {
-          for (int j = 0; j < 4; ++j)
-            if (v4[j] == r) qs = j + 1;
-        } else if (e == erow) {
-          qs = 5;
-        }
-        double acc[45];
-        quad_stokes_pair(x1, x2, x3, g.xyz + 3 * v4[3], s, g.mul[e], g.iquad, qs, acc);
-        for (int k = 0; k < 6; ++k) G[k * mstrG + (size_t)ro * ne + e] = acc[k];
-        for (int k = 0; k < 3; ++k) prG[k * mstrG + (size_t)ro * ne + e] = acc[6 + k];
-        for (int k = 0; k < 6; ++k) {
-          double *p = trow(k);
-          for (int v = 0; v < 4; ++v) p[v4[v]] += acc[9 + 4 * k + v];
-        }
-        for (int k = 0; k < 3; ++k) {
-          double *p = trow(6 + k);
-          for (int v = 0; v < 4; ++v) p[v4[v]] += acc[33 + 4 * k + v];
-        }
-        continue;
-      }
-      int isrc = 0;
-      if (!qrow) isrc = (vv[0] == r) ? 1 : (vv[1] == r) ? 2 : (vv[2] == r) ? 3 : 0;
-      else if (e == erow) isrc = 4;
       double Gs[6] = {0, 0, 0, 0, 0, 0}, pG[3] = {0, 0, 0};
-      double Tv[6][3] = {{0}}, pT[3][3] = {{0}};
-      if (isrc == 0) {
-        const double m = g.mul[e];
-        stokes_tri_full(s, x1, x2, x3, m * g.nrm[3 * e], m * g.nrm[3 * e + 1], m * g.nrm[3 * e + 2], g.area[e], qoff,
-                        nq, Gs, pG, Tv, pT);
+      bool quad = false;
+      if constexpr (QUADS) quad = vv[3] >= 0;
+      if (QUADS && quad) {  // quadrilateral (Quad_StokesIntNumAna, src/lib_intAna.f90:5-37)
+        if constexpr (QUADS) {
+          nno = 4;
+          int qs = 0;
+          if (!qrow) {
+            for (int j = 0; j < 4; ++j)
+              if (vv[j] == r) qs = j + 1;
+          } else if (e == erow) {
+            qs = 5;
+          }
+          double acc[45];
+          quad_stokes_pair(x1, x2, x3, g.xyz + 3 * vv[3], s, g.mul[e], g.iquad, qs, acc);
+          for (int k = 0; k < 6; ++k) Gs[k] = acc[k];
+          for (int k = 0; k < 3; ++k) pG[k] = acc[6 + k];
+          for (int k = 0; k < 9; ++k)
+            for (int v = 0; v < 4; ++v) t[k][v] = acc[9 + 4 * k + v];
+        }
       } else {
-        andr_sing_stk(x1, x2, x3, s, isrc, Gs);  // T, prT, prG of a singular pair are zero
+        int isrc = 0;
+        if (!qrow) isrc = (vv[0] == r) ? 1 : (vv[1] == r) ? 2 : (vv[2] == r) ? 3 : 0;
+        else if (e == erow) isrc = 4;
+        if (isrc == 0) {
+          const double m = g.mul[e];
+          double Tv[6][3], pT[3][3];
+          stokes_tri_full(s, x1, x2, x3, m * g.nrm[3 * e], m * g.nrm[3 * e + 1], m * g.nrm[3 * e + 2], g.area[e],
+                          qoff, nq, Gs, pG, Tv, pT);
+#pragma unroll
+          for (int v = 0; v < 3; ++v) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) t[k][v] = Tv[k][v];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) t[6 + k][v] = pT[k][v];
+          }
+        } else {
+          andr_sing_stk(x1, x2, x3, s, isrc, Gs);  // T, prT, prG of a singular pair are zero
+        }
       }
+#pragma unroll
       for (int k = 0; k < 6; ++k) G[k * mstrG + (size_t)ro * ne + e] = Gs[k];
+#pragma unroll
       for (int k = 0; k < 3; ++k) prG[k * mstrG + (size_t)ro * ne + e] = pG[k];
-      for (int k = 0; k < 6; ++k) {
-        double *p = trow(k);
-        for (int v = 0; v < 3; ++v) p[vv[v]] += Tv[k][v];
-      }
-      for (int k = 0; k < 3; ++k) {
-        double *p = trow(6 + k);
-        for (int v = 0; v < 3; ++v) p[vv[v]] += pT[k][v];
-      }
     }
-    __syncthreads();
+    for (int c = 0; c < ncolors; ++c) {
+      if (col == c) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+          double *p = trow(k);
+#pragma unroll
+          for (int v = 0; v < NV; ++v)
+            if (v < nno) p[vv[v]] += t[k][v];
+        }
+      }
+      __syncthreads();
+    }
   }
   // row sums of the six T components and of the three prT components
   double sums[6] = {0, 0, 0, 0, 0, 0};
@@ -1057,20 +1156,19 @@ int andr_launch_stokes_rows(andr_ctx *ctx, DevBody &b, double extra, double *T, 
                             double *err_rows, int r0, int nrows) {
   QuadRule qr = andr_rule(b.itri);
   const int nsp = nrows < 0 ? b.g.nn + b.g.ne - r0 : nrows;  // rows r0 .. r0 + nsp - 1
-  const int ncol = (int)b.color_off.size() - 1;
   const size_t lds = sizeof(double) * 9 * (size_t)b.g.nn;
   const double evals = (double)nsp * b.g.ne * qr.npts;
   const int tok = andr_prof_begin(ctx, "stokes_rows", 8.0 * 9 * nsp * ((double)b.g.nn + b.g.ne),
                                   evals * ANDR_FLOPS_PER_STOKES_EVAL);
-  if (lds <= 144 * 1024) {
-    ANDR_HIP(ctx, hipFuncSetAttribute((const void *)k_stokes_rows<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)lds));
-    hipLaunchKernelGGL(k_stokes_rows<true>, dim3(nsp), dim3(256), lds, ctx->stream, b.g, qr.offset, qr.npts,
-                       b.color_elems.p, b.d_color_off.p, ncol, extra, T, G, prT, prG, err_rows, r0, nsp);
-  } else {
-    hipLaunchKernelGGL(k_stokes_rows<false>, dim3(nsp), dim3(256), 0, ctx->stream, b.g, qr.offset, qr.npts,
-                       b.color_elems.p, b.d_color_off.p, ncol, extra, T, G, prT, prG, err_rows, r0, nsp);
-  }
+  const bool in_lds = lds <= 144 * 1024, quads = b.g.nv == 4;
+  using Kern = void (*)(BodyGeom, int, int, const int *, const uint8_t *, int, double, double *, double *, double *,
+                        double *, double *, int, int);
+  const Kern kerns[4] = {k_stokes_rows<false, false>, k_stokes_rows<false, true>, k_stokes_rows<true, false>,
+                         k_stokes_rows<true, true>};
+  const Kern kern = kerns[(in_lds ? 2 : 0) + (quads ? 1 : 0)];
+  if (in_lds) ANDR_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(kern, dim3(nsp), dim3(row_threads(b.g.ne)), in_lds ? lds : 0, ctx->stream, b.g, qr.offset, qr.npts,
+                     b.order.p, b.color.p, b.ncolors, extra, T, G, prT, prG, err_rows, r0, nsp);
   andr_prof_end(ctx, tok);
   ANDR_HIP(ctx, hipGetLastError());
   return ANDR_OK;

@@ -145,9 +145,10 @@ struct BodyGeom {
 struct DevBody {
   DevBuf<double> xyz, nrm, area, cen, mul;
   DevBuf<float4> cenl;
-  DevBuf<int> con, bcid, color_elems;
-  std::vector<int> color_off;  // host copy of color offsets (size ncolors+1)
-  DevBuf<int> d_color_off;
+  DevBuf<int> con, bcid;
+  DevBuf<int> order;      // elements in the order the row kernels take them, and
+  DevBuf<uint8_t> color;  // the colour of each (with_colors)
+  int ncolors = 0;
   BodyGeom g;
   int itri = 5;
   int iquad = 4;
