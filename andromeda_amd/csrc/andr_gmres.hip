@@ -29,7 +29,7 @@ constexpr int NB = ANDR_NB;
 static_assert(NB == 8, "the matrix-core product packs two 8-column halves into the 16 B columns");
 constexpr int TILE = 64;   // rows per vector tile (256 threads: 32 rows x 8 right-hand sides per pass)
 constexpr int ICH = 8;   // basis vectors per block of the projection kernel
-constexpr int BT = 256;  // rows per tile of the block Gram-Schmidt sweeps
+constexpr int BT = 256;  // rows per tile of the block Gram-Schmidt dot sweeps
 // A cycle stops when the least-squares estimate of every column's residual is below EST_MARGIN tol |b|:
 // the other half of the tolerance covers the difference between the estimate and the true FP64
 // residual that the FP32 Krylov products leave (the restart test checks the true residual).
@@ -65,7 +65,7 @@ struct GSys {  // device view of one system
   // block GMRES (one Krylov space for all right-hand sides of the system; see kb_bsmall)
   int t40, nt4;  // tiles of BT rows of the system in the current map
   double *Rp;    // packed upper triangle of the rotated block Hessenberg: column q at q (q + 1) / 2
-  double *hv;    // Householder reflector of column q: tau, v_1 .. v_L at 8 q
+  double *hv;    // round b's reflectors as one 2 L x 2 L orthogonal matrix, row-major at 4 L^2 b
   double *gB;    // rotated right-hand sides: L (m + 1) rows x NB
   double *C1;    // first-sweep coefficients: 8 x 8 per basis block ([l][k]); the solution blocks Y at the end
   double *C2;    // second-sweep coefficients, then (block j + 1) the Gram matrix of the swept vector
@@ -160,7 +160,13 @@ __global__ __launch_bounds__(256) void kb_sred(const GSys *__restrict__ sys, con
   if (!all && !sys_iterating(S)) return;  // as kb_prep (uniform over the block)
   const int r = threadIdx.x & 31, p = threadIdx.x >> 5;
   double a = 0.0;
-  for (int i = p; i < S.net; i += 8) a += part_s[(size_t)(S.et0 + i) * MAXW * NB + r];
+  for (int i = p; i < S.net; i += 64) {  // eight loads in flight
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = i + 8 * u < S.net ? part_s[(size_t)(S.et0 + i + 8 * u) * MAXW * NB + r] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a += v[u];
+  }
   red[p][r] = a;
   __syncthreads();
   if (threadIdx.x < 32) {
@@ -371,8 +377,37 @@ __global__ __launch_bounds__(256, 2) void kb_gemv_sym(const GSys *__restrict__ s
     for (int t = 0; t < 4; ++t) step(a, z, t);
     flush();
   }
+  // A whole row: the null-space term (defl_term, the same products) is added here, its factors read for all
+  // of the lane's rows at once (row by row, each behind a branch, they were a chain of some twenty round
+  // trips, half of the kernel's 20 us on a body of 500 elements). Segments: kb_seg_sum adds it.
   const bool direct = S.nseg <= 1;
   double *Y = direct ? S.W : S.P + (size_t)wm.seg * S.n * NB;
+  double df[8], ds[8], dn[8][3];  // d_w area, sum of the wall, normal
+  if (direct && O.defl) {
+    int w8[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = min(row0 + 16 * (i >> 2) + (F32 ? 4 * g + (i & 3) : g + 4 * (i & 3)), ne - 1);
+      w8[i] = O.bcid[r];
+      df[i] = O.area[r];
+#pragma unroll
+      for (int co = 0; co < 3; ++co) dn[i][co] = O.nrm[3 * r + co];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const bool in = w8[i] >= 1 && w8[i] <= MAXW;
+      const double d = in ? O.defl[w8[i]] : 0.0;
+      ds[i] = in ? S.sdef[(w8[i] - 1) * NB + (c & (NB - 1))] : 0.0;
+      df[i] = d != 0.0 ? d * df[i] : 0.0;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      df[i] = ds[i] = 0.0;
+#pragma unroll
+      for (int co = 0; co < 3; ++co) dn[i][co] = 0.0;
+    }
+  }
 #pragma unroll
   for (int T = 0; T < 2; ++T)
 #pragma unroll
@@ -383,8 +418,11 @@ __global__ __launch_bounds__(256, 2) void kb_gemv_sym(const GSys *__restrict__ s
       if (hi || r >= ne) continue;
       const double y[3] = {p + qh, rr + ph, q + rh};
 #pragma unroll
-      for (int co = 0; co < 3; ++co)
-        Y[(size_t)(co * ne + r) * NB + c] = y[co] + (wm.seg == 0 ? defl_term(O, S.sdef, r, co, c) : 0.0);
+      for (int co = 0; co < 3; ++co) {
+#pragma clang fp contract(off)
+        const double t = df[4 * T + v] != 0.0 ? (df[4 * T + v] * dn[4 * T + v][co]) * ds[4 * T + v] : 0.0;
+        Y[(size_t)(co * ne + r) * NB + c] = y[co] + t;
+      }
     }
 }
 
@@ -459,22 +497,36 @@ __global__ __launch_bounds__(256) void kb_resid_zero(const GSys *__restrict__ sy
   }
 }
 
-// per tile of a system with nseg > 1: W = sx .* sum over segments of the partial products
+// per tile of a system with nseg > 1: W = sum over segments of the partial products, the first of them with
+// the null-space term; eight segments' loads in flight
 __global__ __launch_bounds__(256) void kb_seg_sum(const GSys *__restrict__ sys, const TileMap *__restrict__ tmap,
-                                                  const double *__restrict__ sxy) {
+                                                  int all) {
   const TileMap tm = tmap[blockIdx.x];
   const GSys &S = sys[tm.sys];
-  if (S.nseg <= 1) return;
-  const int n = S.n;
+  if (S.nseg <= 1 || (!all && !sys_iterating(S))) return;  // uniform over the block
+  const int n = S.n, nseg = S.nseg, ne = S.op.ne;
   const int k = threadIdx.x & 7, rr = threadIdx.x >> 3;
-  const double sx = sxy[(size_t)tm.sys * 2 * NB + k];
+  double y[TILE / 32], d[TILE / 32];
+#pragma unroll
+  for (int t = 0; t < TILE / 32; ++t) {
+    const int row = min(tm.row0 + rr + 32 * t, n - 1), co = row / ne;
+    d[t] = defl_term(S.op, S.sdef, row - co * ne, co, k);
+    const double *P = S.P + (size_t)row * NB + k;
+    double a = 0.0;
+    for (int sg = 0; sg < nseg; sg += 8) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = sg + u < nseg ? P[(size_t)(sg + u) * n * NB] : 0.0;
+      if (sg == 0) v[0] += d[t];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) a += v[u];
+    }
+    y[t] = a;
+  }
 #pragma unroll
   for (int t = 0; t < TILE / 32; ++t) {
     const int row = tm.row0 + rr + 32 * t;
-    if (row >= n) continue;
-    double y = 0.0;
-    for (int sg = 0; sg < S.nseg; ++sg) y += S.P[((size_t)sg * n + row) * NB + k];
-    S.W[(size_t)row * NB + k] = sx * y;
+    if (row < n) S.W[(size_t)row * NB + k] = y[t];
   }
 }
 
@@ -814,17 +866,32 @@ __global__ __launch_bounds__(256) void kb_copy_b(const GSys *__restrict__ sys, c
   }
 }
 
-// thread per (system, k): true residual norm from the gemv partials; restart set-up
-__global__ void kb_restart(const GSys *__restrict__ sys, int nsys, const double *__restrict__ part,
-                           const int *__restrict__ wave0, const int *__restrict__ nwv, double tol, int first,
-                           int nrhs, int *__restrict__ done) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nsys * NB) return;
-  const int s = t / NB, k = t % NB;
+// block per system: true residual norms from the band partials (thread (part, k): every 32nd partial,
+// eight loads in flight); then thread k < NB sets up the restart of column k
+__global__ __launch_bounds__(256) void kb_restart(const GSys *__restrict__ sys, const double *__restrict__ part,
+                                                  const int *__restrict__ wave0, const int *__restrict__ nwv,
+                                                  double tol, int first, int nrhs, int *__restrict__ done) {
+  __shared__ double red[4][NB];
+  const int s = blockIdx.x, k = threadIdx.x & 7;
   const GSys &S = sys[s];
-  double *sm = S.small + k * 8;
   double r2 = 0.0;
-  for (int w = 0; w < nwv[s]; ++w) r2 += part[(size_t)(wave0[s] + w) * NB + k];
+  const int nw = nwv[s];
+  const double *p = part + (size_t)wave0[s] * NB + k;
+  for (int w = threadIdx.x >> 3; w < nw; w += 256) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = w + 32 * u < nw ? p[(size_t)(w + 32 * u) * NB] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) r2 += v[u];
+  }
+  r2 += __shfl_xor(r2, 8, 64);
+  r2 += __shfl_xor(r2, 16, 64);
+  r2 += __shfl_xor(r2, 32, 64);
+  if ((threadIdx.x & 63) < NB) red[threadIdx.x >> 6][k] = r2;
+  __syncthreads();
+  if (threadIdx.x >= NB) return;
+  r2 = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
+  double *sm = S.small + k * 8;
   const double rn = sqrt(r2);
   const double prev = sm[1];
   if (first) {
@@ -893,7 +960,10 @@ __global__ __launch_bounds__(256) void kb_q0(const GSys *__restrict__ sys, const
 // takes blocks 16 y + 4 w .. + 3 as two FP64 matrix-core A operands of two blocks each (lane (g, i):
 // A[i][g] = Q_(b(i))[row + g][i & 7], B[g][i] = V[row + g][i & 7]); register v of lane (g, i < 8)
 // ends as C_b[l][i] with b, l from row g + 4 v of the product. Rows past the end meet zeros in V,
-// so the A operands load a valid row unconditionally.
+// so the A operands load a valid row unconditionally. H = 1: one A operand per wave, blocks
+// 8 y + 2 w, + 1: half the chain of matrix-core products and loads per wave where the tiles are too few to
+// fill the chip (the sums are the same ones).
+template <int H>
 __global__ __launch_bounds__(256) void kb_bdots(const GSys *__restrict__ sys, const TileMap *__restrict__ tmap,
                                                 int which, int nb, int gram, double *__restrict__ part, int pstride,
                                                 int all) {
@@ -914,39 +984,41 @@ __global__ __launch_bounds__(256) void kb_bdots(const GSys *__restrict__ sys, co
   __syncthreads();
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int g = lane >> 4, i = lane & 15, l = i & 7;
-  const int bw = blockIdx.y * 16 + 4 * wid;  // the wave's first block
+  const int bw = blockIdx.y * 8 * H + 2 * H * wid;  // the wave's first block
   if (bw >= nbt) return;                      // after the only barrier
-  const double *Ap[2];
+  const double *Ap[H];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
+  for (int h = 0; h < H; ++h) {
     const int b = bw + 2 * h + (i >> 3);
     const double *Ab = b < nb ? S.Q + (size_t)b * n * NB : (b == nb && gram ? V : nullptr);
     Ap[h] = Ab ? Ab : V;  // lanes without a block compute partials that are not written
   }
   const int rlast = n - 1;
-  d4v acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+  d4v acc[H];
+#pragma unroll
+  for (int h = 0; h < H; ++h) acc[h] = d4v{0.0, 0.0, 0.0, 0.0};
   for (int r = 0; r < BT; r += 64) {
-    double a[2][16], bv[16];
+    double a[H][16], bv[16];
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
       const size_t rr = (size_t)min(tm.row0 + r + 4 * t + g, rlast) * NB + l;
-      a[0][t] = Ap[0][rr];
-      a[1][t] = Ap[1][rr];
+#pragma unroll
+      for (int h = 0; h < H; ++h) a[h][t] = Ap[h][rr];
       bv[t] = vs[(r + 4 * t + g) * NB + l];
     }
-    // all 48 loads of the iteration go out before its products (left to itself the scheduler
+    // all loads of the iteration go out before its products (left to itself the scheduler
     // moves each load next to its use and a wave keeps few loads in flight)
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
-      acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[0][t], bv[t], acc[0], 0, 0, 0);
-      acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[1][t], bv[t], acc[1], 0, 0, 0);
+#pragma unroll
+      for (int h = 0; h < H; ++h) acc[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[h][t], bv[t], acc[h], 0, 0, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
   }
   if (i < 8) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < H; ++h)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int mrow = g + 4 * v, blk = bw + 2 * h + (mrow >> 3);
@@ -956,7 +1028,8 @@ __global__ __launch_bounds__(256) void kb_bdots(const GSys *__restrict__ sys, co
 }
 
 // block per (system, basis block b < nbt): C (dst 0: C1, 1: C2) block b = sum of the system's tile
-// partials (the four waves take every fourth tile). Systems outside the map have no tiles.
+// partials (the four waves take every fourth tile, eight loads in flight). Systems outside the map have no
+// tiles.
 __global__ __launch_bounds__(256) void kb_bdots_final(const GSys *__restrict__ sys, const double *__restrict__ part,
                                                       int pstride, int dst, int all) {
   __shared__ double red[4][64];
@@ -964,26 +1037,48 @@ __global__ __launch_bounds__(256) void kb_bdots_final(const GSys *__restrict__ s
   if (S.nt4 == 0 || (!all && !sys_iterating(S))) return;  // uniform over the block
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, b = blockIdx.y;
   double c = 0.0;
-  for (int tl = wv; tl < S.nt4; tl += 4) c += part[((size_t)(S.t40 + tl) * pstride + b) * 64 + lane];
+  const double *p = part + ((size_t)S.t40 * pstride + b) * 64 + lane;
+  for (int tl = wv; tl < S.nt4; tl += 32) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = tl + 4 * u < S.nt4 ? p[(size_t)(tl + 4 * u) * pstride * 64] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) c += v[u];
+  }
   red[wv][lane] = c;
   __syncthreads();
   if (wv == 0) (dst ? S.C2 : S.C1)[(size_t)b * 64 + lane] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
 }
 
-// thread per row, all NB columns (16-byte loads; the coefficients are uniform over the block):
 //   mode 0: W -= sum_(b < nb) Q_b C1_b
 //   mode 1: Q_nb = (W - sum_(b < nb) Q_b C2_b) Ri          (the next basis block)
 //   mode 2: X += sum_(b < kk) Q_b Y_b, Y in C1, kk the rounds the system used (at most nb)
 //   mode 3: Q_0 = R Ri                                      (start of a cycle)
+// A block takes a tile of 64 rows, four lanes a row, a lane two of its columns: one 16-byte load per basis
+// block, the row's other values from its neighbours (quad permutes), the coefficients staged in LDS UCH
+// blocks at a time with the next chunk's loads of both under way. With a whole row per lane, a body of 7000
+// rows was 109 waves, each with a round trip to memory every four blocks (73 rounds of it: 39.7 -> 10.8 us a
+// sweep; 40 bodies of 500 to 7220 elements 50.7 -> 33.7). Every sum runs over the blocks and columns in order, whatever the split: the Krylov vectors meet
+// FP32 products, where a last bit that differs can turn a rounding. HBM bound (the basis stream) on a
+// full batch.
+constexpr int UCH = 16;
+template <int U>
+__device__ inline double quad_lane(double x) {  // the value of lane U of the quad
+  constexpr int ctrl = U * 0x55;                 // quad_perm [U, U, U, U]
+  const long long v = __double_as_longlong(x);
+  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)v, ctrl, 0xf, 0xf, true);
+  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(v >> 32), ctrl, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | lo);
+}
 __global__ __launch_bounds__(256) void kb_bupdate(const GSys *__restrict__ sys, const TileMap *__restrict__ tmap, int nb,
                                                   int mode, int all) {
   typedef double d2 __attribute__((ext_vector_type(2)));
+  __shared__ __attribute__((aligned(16))) double sC[2][UCH * 64];
+  static_assert(TILE == 64, "four lanes per row");
   const TileMap tm = tmap[blockIdx.x];
   const GSys &S = sys[tm.sys];
-  if (mode < 2 && !all && !sys_iterating(S)) return;  // the sweeps of a round; no barriers here
-  const int n = S.n;
-  const int row = tm.row0 + threadIdx.x;
-  if (row >= n) return;  // no barriers in this kernel
+  if (mode < 2 && !all && !sys_iterating(S)) return;  // the sweeps of a round; uniform over the block
+  const int n = S.n, tid = threadIdx.x, p = tid & 3;
   int nbb = mode == 3 ? 0 : nb;
   if (mode == 2) {  // the rounds used: the live columns freeze together (none live: no update)
     int kk = -1;
@@ -994,337 +1089,489 @@ __global__ __launch_bounds__(256) void kb_bupdate(const GSys *__restrict__ sys, 
     }
     nbb = max(kk, 0);
   }
-  // the coefficients are uniform over the block and read-only here: loads through the constant
-  // address space go to the scalar cache and feed the FMAs as scalar operands
-  typedef const __attribute__((address_space(4))) double cdouble;
-  cdouble *Cf = (cdouble *)(uintptr_t)(mode == 1 ? S.C2 : S.C1);
-  cdouble *Ric = (cdouble *)(uintptr_t)S.Ri;
-  const double *src = mode == 3 ? S.R : (mode == 2 ? S.X : S.W);
-  d2 x[4], s[4];
+  const int row = tm.row0 + (tid >> 2);
+  const bool in = row < n;  // rows past the end repeat the last and are not stored
+  const size_t o = (size_t)(in ? row : n - 1) * NB + 2 * p, vstride = (size_t)n * NB;
+  const double *Cf = mode == 1 ? S.C2 : S.C1;
+  const double *Qr = S.Q + o;
+  const d2 x = *(const d2 *)((mode == 3 ? S.R : (mode == 2 ? S.X : S.W)) + o);
+  d2 s = {0.0, 0.0};
+  // chunk of UCH blocks from b0: this lane's values of its row, and its share of the coefficients (past the
+  // last block both repeat it and are not used)
+  static_assert(UCH * 64 == 2 * 2 * 256, "two 16-byte loads of the coefficients per thread");
+  d2 cq[UCH], cc[2];
+  auto load = [&](int b0) {
 #pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    x[p] = ((const d2 *)(src + (size_t)row * NB))[p];
-    s[p] = d2{0.0, 0.0};
-  }
-  // blocks in groups of four: the group's 16 row loads go out before its products (past the last
-  // block the loads repeat it and are not used)
-  const size_t vstride = (size_t)n * NB;
-  for (int b0 = 0; b0 < nbb; b0 += 4) {
-    d2 qv[4][4];
+    for (int u = 0; u < UCH; ++u) cq[u] = *(const d2 *)(Qr + (size_t)min(b0 + u, nbb - 1) * vstride);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const d2 *q = (const d2 *)(S.Q + (size_t)min(b0 + u, nbb - 1) * vstride + (size_t)row * NB);
-#pragma unroll
-      for (int p = 0; p < 4; ++p) qv[u][p] = q[p];
+    for (int h = 0; h < 2; ++h) {
+      const int e = 2 * (tid + 256 * h);  // block b0 + e / 64
+      cc[h] = *(const d2 *)(Cf + (size_t)min(b0 + (e >> 6), nbb - 1) * 64 + (e & 63));
     }
-    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (nbb > 0) {
+    load(0);
+#pragma unroll 1
+    for (int b0 = 0, w = 0; b0 < nbb; b0 += UCH, w ^= 1) {
+      double *sc = sC[w];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if (b0 + u >= nbb) break;  // uniform
-      cdouble *C = Cf + (size_t)(b0 + u) * 64;
+      for (int h = 0; h < 2; ++h) *(d2 *)&sc[2 * (tid + 256 * h)] = cc[h];
+      d2 q[UCH];
 #pragma unroll
-      for (int l = 0; l < 8; ++l) {
-        const double ql = (l & 1) ? qv[u][l >> 1].y : qv[u][l >> 1].x;
+      for (int u = 0; u < UCH; ++u) q[u] = cq[u];
+      __syncthreads();  // this buffer is written; the other one is read (before the last barrier)
+      load(min(b0 + UCH, nbb - 1));
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int p = 0; p < 4; ++p) s[p] += ql * d2{C[l * 8 + 2 * p], C[l * 8 + 2 * p + 1]};
+      for (int u = 0; u < UCH; ++u) {
+        if (b0 + u >= nbb) continue;  // uniform
+        const double *C = &sc[u * 64 + 2 * p];
+        const double ql[8] = {quad_lane<0>(q[u].x), quad_lane<0>(q[u].y), quad_lane<1>(q[u].x), quad_lane<1>(q[u].y),
+                              quad_lane<2>(q[u].x), quad_lane<2>(q[u].y), quad_lane<3>(q[u].x), quad_lane<3>(q[u].y)};
+#pragma unroll
+        for (int l = 0; l < 8; ++l) s += ql[l] * *(const d2 *)(C + 8 * l);
       }
     }
-    __builtin_amdgcn_sched_barrier(0);
   }
   if (mode == 0 || mode == 2) {
-    d2 *dst = (d2 *)((mode == 0 ? S.W : S.X) + (size_t)row * NB);
-#pragma unroll
-    for (int p = 0; p < 4; ++p) dst[p] = mode == 0 ? x[p] - s[p] : x[p] + s[p];
+    if (in) *(d2 *)((mode == 0 ? S.W : S.X) + o) = mode == 0 ? x - s : x + s;
     return;
   }
-  double w[8];
+  // the row's new vector times Ri
+  const d2 v = x - s;
+  const double w[8] = {quad_lane<0>(v.x), quad_lane<0>(v.y), quad_lane<1>(v.x), quad_lane<1>(v.y),
+                       quad_lane<2>(v.x), quad_lane<2>(v.y), quad_lane<3>(v.x), quad_lane<3>(v.y)};
+  d2 out = {0.0, 0.0};
 #pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    const d2 v = x[p] - s[p];
-    w[2 * p] = v.x;
-    w[2 * p + 1] = v.y;
-  }
+  for (int c = 0; c < 8; ++c) out += w[c] * *(const d2 *)(S.Ri + c * 8 + 2 * p);
   const size_t blk = mode == 1 ? (size_t)nb : 0;  // mode 3 writes Q_0
-  d2 *dst = (d2 *)(S.Q + (blk * n + row) * NB);
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    d2 o = {0.0, 0.0};
-#pragma unroll
-    for (int c = 0; c < 8; ++c) o += w[c] * d2{Ric[c * 8 + 2 * p], Ric[c * 8 + 2 * p + 1]};
-    dst[p] = o;
-  }
+  if (in) *(d2 *)(S.Q + blk * vstride + o) = out;
 }
 
-// Cholesky factor of an L x L Gram matrix G (row-major, stride 8) with dropped columns: column c is
-// dropped (zero row, zero diagonal) when it is dead or its pivot is at most drop * nrm2[c]; rows of
-// R are written to R (stride 8), the inverse over the kept columns to Ri (full 8 x 8, zero
-// elsewhere). Returns 1 when a live column with nrm2 > 0 was dropped. One thread.
-__device__ inline int chol_drop(const double *G, const double *nrm2, const bool *live, int L, double drop, double *R,
-                                double *Ri) {
+__device__ inline double lane_bcast(double x, int l) {  // the value of lane l (uniform)
+  const long long v = __double_as_longlong(x);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)v, l), hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l);
+  return __longlong_as_double(((long long)hi << 32) | lo);
+}
+__device__ inline void wave_sync_lds() {  // LDS traffic between the lanes of one wave
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Cholesky factor of an L x L Gram matrix with dropped columns, by one wave: lane 8 c + i holds G[c][i] and
+// returns R[c][i]. Column c is dropped (zero row of R) when it is dead or its pivot is at most
+// drop * nrm2[c] (n2 in the lanes of row c). Returns 1 when a live column with nrm2 > 0 was dropped: it
+// lost its new direction (breakdown); a zero product (the column has no basis vector, e.g. a right-hand side
+// that repeats another) is not one.
+template <int L>
+__device__ inline int wave_chol(double g, double n2, unsigned live, double drop, double &R) {
+  const int lane = threadIdx.x & 63, c = lane >> 3, i = lane & 7;
   int brk = 0;
-  for (int a = 0; a < 64; ++a) {
-    R[a] = 0.0;
-    Ri[a] = 0.0;
-  }
-  for (int c = 0; c < L; ++c) {
-    double d = G[c * 8 + c];
-    for (int t = 0; t < c; ++t) d -= R[t * 8 + c] * R[t * 8 + c];
-    if (!live[c] || !(d > drop * nrm2[c])) {
-      // a live column whose product still had a norm lost its new direction: breakdown; a zero
-      // product (the column has no basis vector, e.g. a right-hand side that repeats another) is not
-      if (live[c] && nrm2[c] > 0.0) brk = 1;
-      continue;  // row c stays zero
+  R = 0.0;
+#pragma unroll
+  for (int t = 0; t < L; ++t) {
+    const double d = lane_bcast(g, 9 * t), nt = lane_bcast(n2, 8 * t);
+    const bool lv = (live >> t) & 1;
+    if (!lv || !(d > drop * nt)) {  // uniform
+      if (lv && nt > 0.0) brk = 1;
+      continue;
     }
     const double r = sqrt(d);
-    R[c * 8 + c] = r;
-    for (int c2 = c + 1; c2 < L; ++c2) {
-      double v = G[c * 8 + c2];
-      for (int t = 0; t < c; ++t) v -= R[t * 8 + c] * R[t * 8 + c2];
-      R[c * 8 + c2] = v / r;
-    }
+    const double rti = __shfl(g, 8 * t + i, 64) / r, rtc = __shfl(g, 8 * t + c, 64) / r;
+    if (c == t) R = i < t ? 0.0 : (i == t ? r : rti);
+    else if (c > t) g = fma(-rtc, rti, g);
   }
-  // Ri = R^-1 over the kept columns (upper triangular), column by column
-  for (int k = 0; k < L; ++k) {
-    if (R[k * 8 + k] == 0.0) continue;
-    Ri[k * 8 + k] = 1.0 / R[k * 8 + k];
-    for (int a = k - 1; a >= 0; --a) {
-      if (R[a * 8 + a] == 0.0) continue;
-      double v = 0.0;
-      for (int t = a + 1; t <= k; ++t) v += R[a * 8 + t] * Ri[t * 8 + k];
-      Ri[a * 8 + k] = -v / R[a * 8 + a];
-    }
-  }
+  if (c >= L || i >= L) R = 0.0;
   return brk;
 }
-
-// wave per system of the cycle: Q_0 = R R0^-1 from the Gram matrix of the residual block (C2 block 0),
-// g = (R0; 0). Dead columns (converged or beyond nrhs) take no part.
-__global__ __launch_bounds__(64) void kb_binit(const GSys *__restrict__ sys, int m, int L) {
-  __shared__ double sR[64], sRi[64];
-  const GSys &S = sys[blockIdx.x];
-  if (!S.incyc) return;  // uniform over the block
-  const int lane = threadIdx.x;
-  if (lane == 0) {
-    bool live[NB], any = false;
-    double nrm2[NB];
-    for (int c = 0; c < NB; ++c) {
-      live[c] = c < L && S.small[8 * c + 4] > 0.0;
-      any = any || live[c];
-      nrm2[c] = S.C2[c * 9];
+// The inverse of wave_chol's factor over the kept columns (upper triangular, zero elsewhere), full 8 x 8, by
+// the same wave: lane k forms column k.
+template <int L>
+__device__ inline void wave_tri_inverse(double R, double *Ri) {
+  const int k = threadIdx.x & 63;
+  double ri[L];
+  const double rkk = __shfl(R, 9 * min(k, L - 1), 64);  // by every lane: the source has to take part
+#pragma unroll
+  for (int a = L - 1; a >= 0; --a) {
+    const double raa = lane_bcast(R, 9 * a);
+    double v = 0.0;
+#pragma unroll
+    for (int t = a + 1; t < L; ++t) {
+      const double rat = lane_bcast(R, 8 * a + t);
+      if (t <= k) v = fma(rat, ri[t], v);
     }
-    (void)chol_drop(S.C2, nrm2, live, L, 1e-24, sR, sRi);
-    S.small[6] = any ? 1.0 : 0.0;  // iterating in this cycle
+    double x = 0.0;
+    if (raa != 0.0 && rkk != 0.0) x = a == k ? 1.0 / raa : (a < k ? -v / raa : 0.0);
+    ri[a] = x;
   }
-  __syncthreads();
-  S.Ri[lane] = sRi[lane];
-  // rows 0 .. L - 1 of g hold R0 (column k of the live k), the rest zero
-  for (int idx = lane; idx < L * (m + 1) * NB; idx += 64) {
-    const int r = idx / NB, k = idx % NB;
-    S.gB[idx] = (r < L && k < L) ? sR[r * 8 + k] : 0.0;
-  }
+  if (k < 8)
+#pragma unroll
+    for (int a = 0; a < 8; ++a) Ri[8 * a + k] = a < L && k < L ? ri[a < L ? a : 0] : 0.0;
 }
 
-// wave per system of the current map: the small dense part of round j. Lane (c, i) = 8 c + i:
-// group c handles new Hessenberg column L j + c (and later right-hand side c), sub-lane i the row
-// q + i of the reflector window at step q.
-__global__ __launch_bounds__(64) void kb_bsmall(const GSys *__restrict__ sys, int j, int L, double tol, int all) {
-  __shared__ double sG[64], sR[64], sRi[64], sN[NB];
-  __shared__ double sv[NB][NB];  // reflectors of the round's new columns: tau, v_1 .. v_L
-  __shared__ double shv[NB][NB], sen[NB][NB];  // a chunk of 8 earlier reflectors, entering rows
-  __shared__ double sC1[8][64], sC2[8][64];       // a chunk of 8 coefficient blocks
-  __shared__ int sbrk, sok[NB];
+// block per system of the cycle: Q_0 = R R0^-1 from the Gram matrix of the residual block (C2 block 0),
+// g = (R0; 0). Dead columns (converged or beyond nrhs) take no part.
+__global__ __launch_bounds__(256) void kb_binit(const GSys *__restrict__ sys, int m, int L) {
+  const GSys &S = sys[blockIdx.x];
+  if (!S.incyc) return;  // uniform over the block
+  for (int idx = 64 + threadIdx.x; idx < L * (m + 1) * NB; idx += 256) S.gB[idx] = 0.0;
+  if (threadIdx.x >= 64) return;
+  const int lane = threadIdx.x, c = lane >> 3, i = lane & 7;
+  unsigned live = 0;
+  for (int k = 0; k < L; ++k) live |= S.small[8 * k + 4] > 0.0 ? 1u << k : 0u;
+  double R;  // the columns past L are zero and dead: factorised as eight
+  (void)wave_chol<8>(S.C2[lane], S.C2[9 * c], live, 1e-24, R);
+  if (lane == 0) S.small[6] = live ? 1.0 : 0.0;  // iterating in this cycle
+  wave_tri_inverse<8>(R, S.Ri);
+  // rows 0 .. L - 1 of g hold R0 (column k of the live k), the rest zero
+  if (lane < L * (m + 1) * NB) S.gB[lane] = (c < L && i < L) ? R : 0.0;
+}
+
+// block per system of the current map: the small dense part of round j, three waves that meet once.
+//   waves 0, 1  the earlier rounds' reflectors on the L new Hessenberg columns: round b's are one 2 L x 2 L
+//             orthogonal matrix (hv), so the chain is a product of a window of 2 L rows per round (L rows
+//             carried, L entering) instead of L reflectors of L + 1 rows; 16 lanes per column, a row each; the
+//             matrices and entering rows pass through the wave's own LDS, BCH rounds at a time, the next
+//             ones in registers meanwhile;
+//   wave 2    G2 = G1 - sum_b C2_b^T C2_b and its Cholesky factor R_(j+1), later its inverse;
+//   wave 0    then the round's own reflectors, a column per lane: the L new columns, 2 L unit columns (the
+//             round's matrix) and the L right-hand sides, all in registers.
+// Latency of one chain per body: 42.2 -> 12.3 us a round over rounds 1 .. 73 of three columns, 78.0 -> 19.2
+// over 71 of six (one wave, one reflector at a time, the factorisation on one lane).
+constexpr int BCH = 8;  // rounds per LDS chunk
+template <int L>
+__global__ __launch_bounds__(192) void kb_bsmall(const GSys *__restrict__ sys, int j, double tol, int all) {
+  constexpr int M2 = 2 * L, QP = M2 + 2;  // rows of the window; padded row of a matrix in LDS
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  __shared__ __attribute__((aligned(16))) double sQ[2][BCH][M2 * QP];
+  __shared__ double sC[3][BCH][64];  // waves 0, 1: entering rows (block b + 1 of C1 + C2); wave 2: C2
+  __shared__ __attribute__((aligned(16))) double sW[NB][16];
+  __shared__ double sR[64];
+  __shared__ int sbrk;
   const GSys &S = sys[blockIdx.x];
   if (S.nt4 == 0 || (!all && !sys_iterating(S))) return;  // uniform over the block
-  const int lane = threadIdx.x, c = lane >> 3, i = lane & 7;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const double *C1 = S.C1, *C2 = S.C2;
-  // G2 = G1 - sum_b C2_b^T C2_b; squared norms of the product's columns before the sweeps. The
-  // coefficient blocks pass through LDS 8 at a time (coalesced loads, all in flight together).
-  {
-    double gs = C2[(size_t)(j + 1) * 64 + c * 8 + i];
-    double w = C2[(size_t)(j + 1) * 64 + c * 9];
-    for (int b0 = 0; b0 <= j; b0 += 8) {
-      const int nb8 = min(8, j + 1 - b0);
-      double v1[8], v2[8];
+  const int LJ = L * j;
+  double R = 0.0;  // wave 2: the factor
+  if (wid == 2) {
+    // lane 8 c + i: the Gram matrix of the swept block, its part along the basis taken out block by block
+    const int c = lane >> 3, i = lane & 7;
+    double gs = C2[(size_t)(j + 1) * 64 + lane], n2 = 0.0;
+    const double n0 = C2[(size_t)(j + 1) * 64 + 9 * c];
+    double v[BCH], w[BCH];
+    auto fetch = [&](int b0) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        v1[u] = u < nb8 ? C1[(size_t)(b0 + u) * 64 + lane] : 0.0;
-        v2[u] = u < nb8 ? C2[(size_t)(b0 + u) * 64 + lane] : 0.0;
+      for (int u = 0; u < BCH; ++u) {
+        const size_t o = (size_t)min(b0 + u, j) * 64 + lane;
+        v[u] = C2[o];
+        w[u] = C1[o];
       }
-      __syncthreads();  // the previous chunk's reads are done
+    };
+    fetch(0);
+    for (int b0 = 0; b0 <= j; b0 += BCH) {
+      const int nr = min(BCH, j + 1 - b0);
+      wave_sync_lds();  // the last chunk is read
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        sC1[u][lane] = v1[u];
-        sC2[u][lane] = v2[u];
+      for (int u = 0; u < BCH; ++u) {
+        sC[2][u][lane] = v[u];
+        if (u < nr) n2 += w[u] * w[u];  // lane 8 l + c of a block is its entry [l][c]
       }
-      __syncthreads();
-      for (int u = 0; u < nb8; ++u)
-        for (int l = 0; l < L; ++l) {
-          gs -= sC2[u][l * 8 + c] * sC2[u][l * 8 + i];
-          w += sC1[u][l * 8 + c] * sC1[u][l * 8 + c];
+      wave_sync_lds();
+      fetch(b0 + BCH);
+      for (int u = 0; u < nr; ++u)
+#pragma unroll
+        for (int l = 0; l < L; ++l) gs = fma(-sC[2][u][l * 8 + c], sC[2][u][l * 8 + i], gs);
+    }
+    n2 += __shfl_xor(n2, 8, 64);
+    n2 += __shfl_xor(n2, 16, 64);
+    n2 += __shfl_xor(n2, 32, 64);  // lane 8 l + c: the sum of column c
+    n2 = n0 + __shfl(n2, c, 64);
+    unsigned live = 0;
+    for (int k = 0; k < L; ++k) live |= S.small[8 * k + 4] > 0.0 ? 1u << k : 0u;
+    const int brk = wave_chol<L>(gs, n2, live, 1e-20, R);
+    sR[lane] = R;
+    if (lane == 0) sbrk = brk;
+  } else {
+    const int col = tid >> 4, i = tid & 15;  // window row i of new column col
+    const bool mine = col < L && i < M2;
+    const int qc = LJ + col;
+    double *Rcol = S.Rp + (size_t)qc * (qc + 1) / 2;
+    constexpr int PER = (BCH * M2 * M2 + 63) / 64;
+    double v[PER], c1[BCH], c2[BCH];
+    auto fetch = [&](int b0) {  // the matrices and entering rows of rounds b0 .. b0 + BCH - 1, as far as b < j
+      const int nr = min(BCH, j - b0);
+      if (nr <= 0) return;
+      const double *src = S.hv + (size_t)b0 * M2 * M2;
+#pragma unroll
+      for (int u = 0; u < PER; ++u) v[u] = src[min(lane + 64 * u, nr * M2 * M2 - 1)];
+#pragma unroll
+      for (int u = 0; u < BCH; ++u) {
+        const size_t o = (size_t)(min(b0 + u, j - 1) + 1) * 64 + lane;
+        c1[u] = C1[o];
+        c2[u] = C2[o];
+      }
+    };
+    fetch(0);
+    if (mine && i < L) sW[col][i] = C1[i * 8 + col] + C2[i * 8 + col];  // block 0: the first carried rows
+    for (int b0 = 0; b0 < j; b0 += BCH) {
+      const int nr = min(BCH, j - b0);
+      wave_sync_lds();  // the last chunk is read
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        const int e = lane + 64 * u;
+        if (e < nr * M2 * M2) sQ[wid][e / (M2 * M2)][(e % (M2 * M2) / M2) * QP + e % M2] = v[u];
+      }
+#pragma unroll
+      for (int u = 0; u < BCH; ++u) sC[wid][u][lane] = c1[u] + c2[u];
+      wave_sync_lds();
+      fetch(b0 + BCH);
+      if (mine && i >= L) sW[col][i] = sC[wid][0][(i - L) * 8 + col];
+      for (int u = 0; u < nr; ++u) {
+        wave_sync_lds();  // the window is written (each wave holds whole columns)
+        double acc0 = 0.0, acc1 = 0.0;
+        if (mine) {
+          const double *qr = &sQ[wid][u][i * QP];
+#pragma unroll
+          for (int k = 0; k < M2; k += 2) {
+            const d2 a = *(const d2 *)(qr + k), w = *(const d2 *)&sW[col][k];
+            acc0 += a.x * w.x;
+            acc1 += a.y * w.y;
+          }
         }
-    }
-    sG[lane] = gs;
-    if (c == i) sN[c] = w;
-  }
-  __syncthreads();
-  if (lane == 0) {
-    bool live[NB];
-    for (int k = 0; k < NB; ++k) live[k] = k < L && S.small[8 * k + 4] > 0.0;
-    sbrk = chol_drop(sG, sN, live, L, 1e-20, sR, sRi);
-  }
-  __syncthreads();
-  S.Ri[lane] = sRi[lane];
-  const int LJ = L * j, rows = L * (j + 2);
-  const bool mine = c < L;  // a new column of this round
-  // H[r][LJ + c] as built: C1 + C2 rows of the blocks b <= j, then the subdiagonal block R_(j+1)
-  auto hval = [&](int r) -> double {
-    if (!mine || r >= rows) return 0.0;
-    if (r < L * (j + 1)) {
-      const int b = r / L, l = r - b * L;
-      return C1[(size_t)b * 64 + l * 8 + c] + C2[(size_t)b * 64 + l * 8 + c];
-    }
-    const int cc = r - L * (j + 1);
-    return cc <= c ? sR[cc * 8 + c] : 0.0;
-  };
-  auto gsum = [&](double x) {  // over the 8 sub-lanes of a group
-    x += __shfl_xor(x, 1, 64);
-    x += __shfl_xor(x, 2, 64);
-    x += __shfl_xor(x, 4, 64);
-    return x;
-  };
-  double w = i <= L ? hval(i) : 0.0;  // window: sub-lane i holds row q + i
-  const int qc = LJ + c;
-  double *Rcol = S.Rp + (size_t)qc * (qc + 1) / 2;
-  // the reflectors of earlier rounds, 8 steps at a time: lane (c, i) fetches entry i of reflector
-  // q0 + c and the row that enters group c's window at step q0 + i, so that the chain of steps
-  // reads LDS only
-  for (int q0 = 0; q0 < LJ; q0 += 8) {
-    const int qn = min(8, LJ - q0);
-    const double hvv = c < qn ? S.hv[(size_t)(q0 + c) * 8 + i] : 0.0;
-    const double env = i < qn ? hval(q0 + i + 1 + L) : 0.0;
-    __syncthreads();
-    shv[c][i] = hvv;
-    sen[c][i] = env;
-    __syncthreads();
-    for (int t = 0; t < qn; ++t) {
-      const double tau = shv[t][0], vi = i == 0 ? 1.0 : (i <= L ? shv[t][i] : 0.0);
-      const double sd = gsum(mine ? vi * w : 0.0);
-      if (mine) {
-        w -= tau * sd * vi;
-        if (i == 0) Rcol[q0 + t] = w;  // row q0 + t of column qc is final
+        wave_sync_lds();  // and read, before it is written again
+        if (mine) {
+          const double x = acc0 + acc1;
+          if (i < L) {
+            Rcol[L * (b0 + u) + i] = x;  // these rows are final
+          } else {
+            sW[col][i - L] = x;
+            if (u + 1 < nr) sW[col][i] = sC[wid][u + 1][(i - L) * 8 + col];
+          }
+        }
       }
-      const double up = __shfl_down(w, 1, 8);
-      if (mine) w = i < L ? up : (i == L ? sen[c][t] : 0.0);
-    }
-  }
-  // the round's own columns: column LJ + cq forms its reflector at step LJ + cq, the later ones apply it
-  for (int q = LJ; q < LJ + L; ++q) {
-    const int cq = q - LJ;  // the new column whose reflector this step forms
-    const double x0 = __shfl(w, 8 * c, 64);
-    const double s2 = gsum(i >= 1 && i <= L ? w * w : 0.0);
-    if (c == cq) {
-      double alpha = x0, t = 0.0, sc = 0.0;
-      if (s2 > 0.0) {
-        const double nx = sqrt(x0 * x0 + s2);
-        alpha = x0 > 0.0 ? -nx : nx;
-        t = (alpha - x0) / alpha;
-        sc = 1.0 / (x0 - alpha);
-      }
-      if (i == 0) {
-        sv[cq][0] = t;
-        Rcol[q] = alpha;
-      } else if (i <= L) {
-        sv[cq][i] = w * sc;
-      }
-      if (i <= L) S.hv[(size_t)q * 8 + i] = i == 0 ? t : w * sc;
-    }
-    __syncthreads();
-    const double tau = sv[cq][0], vi = i == 0 ? 1.0 : (i <= L ? sv[cq][i] : 0.0);
-    const bool act = mine && q < qc;  // group c applies the reflectors of the columns before its own
-    const double sd = gsum(act ? vi * w : 0.0);
-    if (act) {
-      w -= tau * sd * vi;
-      if (i == 0) Rcol[q] = w;  // row q of column qc is final
-    }
-    const double up = __shfl_down(w, 1, 8);
-    const double enter = (act && i == L) ? hval(q + 1 + L) : 0.0;
-    if (act) w = i < L ? up : enter;
-  }
-  __syncthreads();
-  // the round's reflectors on the right-hand sides: group k, window rows LJ + t + i
-  const int k = c;
-  const bool klive = k < L && S.small[8 * k + 4] > 0.0;
-  double gw = (klive && i <= L) ? S.gB[(size_t)(LJ + i) * NB + k] : 0.0;
-  for (int t = 0; t < L; ++t) {
-    const double tau = sv[t][0], vi = i == 0 ? 1.0 : (i <= L ? sv[t][i] : 0.0);
-    const double s = gsum(vi * gw);
-    gw -= tau * s * vi;
-    if (klive && i == 0) S.gB[(size_t)(LJ + t) * NB + k] = gw;
-    const double up = __shfl_down(gw, 1, 8);
-    const int r = LJ + t + 1 + L;
-    const double enter = (klive && i == L && r < rows) ? S.gB[(size_t)r * NB + k] : 0.0;
-    gw = i < L ? up : (i == L ? enter : 0.0);
-  }
-  // rows L (j + 1) .. L (j + 2) - 1: the residual of right-hand side k
-  if (klive && i < L) S.gB[(size_t)(L * (j + 1) + i) * NB + k] = gw;
-  const double est = sqrt(gsum(i < L ? gw * gw : 0.0));
-  double *sm = S.small + 8 * k;
-  if (i == 0) {
-    sok[k] = 1;
-    if (klive) {
-      sm[2] = est;
-      sok[k] = est <= EST_MARGIN * tol * sm[0] ? 1 : 0;
     }
   }
   __syncthreads();
-  if (i == 0 && klive && sm[5] < 0.0) {
-    bool all = sbrk != 0;
-    if (!all) {
-      all = true;
-      for (int kk = 0; kk < NB; ++kk) all = all && sok[kk];
+  if (wid == 2) wave_tri_inverse<L>(R, S.Ri);
+  if (wid != 0) return;
+  // lane: 0 .. L - 1 new column, then 2 L unit columns, then right-hand side k = lane - 3 L
+  const int k = lane - 3 * L;
+  const bool rhs = k >= 0 && k < L;
+  double w[M2];
+  bool klive = false;
+  if (rhs) klive = S.small[8 * k + 4] > 0.0;
+#pragma unroll
+  for (int r = 0; r < M2; ++r) {
+    double v = 0.0;
+    if (lane < L) v = r < L ? sW[lane][r] : (r - L <= lane ? sR[(r - L) * 8 + lane] : 0.0);
+    else if (lane < 3 * L) v = r == lane - L ? 1.0 : 0.0;
+    else if (klive) v = S.gB[(size_t)(LJ + r) * NB + k];
+    w[r] = v;
+  }
+#pragma unroll
+  for (int q = 0; q < L; ++q) {  // column q forms its reflector (rows q .. q + L), the others apply it
+    double s2 = 0.0;
+#pragma unroll
+    for (int r = 1; r <= L; ++r) s2 += w[q + r] * w[q + r];
+    const double x0 = lane_bcast(w[q], q);
+    s2 = lane_bcast(s2, q);
+    double alpha = x0, tau = 0.0, sc = 0.0;
+    if (s2 > 0.0) {
+      const double nx = sqrt(x0 * x0 + s2);
+      alpha = x0 > 0.0 ? -nx : nx;
+      tau = (alpha - x0) / alpha;
+      sc = 1.0 / (x0 - alpha);
     }
-    if (all) {
-      sm[5] = (double)(j + 1);  // rounds to use; the product skips the system from now on
-      S.small[6] = 0.0;         // and the sweeps (every live column writes the same value)
+    double v[L + 1];
+    v[0] = 1.0;
+#pragma unroll
+    for (int r = 1; r <= L; ++r) v[r] = lane_bcast(w[q + r], q) * sc;
+    double dot = w[q];
+#pragma unroll
+    for (int r = 1; r <= L; ++r) dot += v[r] * w[q + r];
+    dot *= tau;
+    if (lane == q) {
+      w[q] = alpha;
+#pragma unroll
+      for (int r = 1; r <= L; ++r) w[q + r] = 0.0;
+    } else if (lane > q) {
+#pragma unroll
+      for (int r = 0; r <= L; ++r) w[q + r] -= dot * v[r];
     }
+  }
+  if (lane < L) {
+    const int qn = LJ + lane;
+    double *Rn = S.Rp + (size_t)qn * (qn + 1) / 2 + LJ;
+#pragma unroll
+    for (int r = 0; r < L; ++r)
+      if (r <= lane) Rn[r] = w[r];
+  } else if (lane < 3 * L) {
+    double *Q = S.hv + (size_t)j * M2 * M2 + (lane - L);
+#pragma unroll
+    for (int r = 0; r < M2; ++r) Q[r * M2] = w[r];
+  } else if (klive) {
+#pragma unroll
+    for (int r = 0; r < M2; ++r) S.gB[(size_t)(LJ + r) * NB + k] = w[r];
+  }
+  // rows L (j + 1) .. L (j + 2) - 1 of the right-hand sides: their residuals
+  bool ok = true;
+  if (klive) {
+    double e2 = 0.0;
+#pragma unroll
+    for (int r = L; r < M2; ++r) e2 += w[r] * w[r];
+    const double est = sqrt(e2);
+    double *sm = S.small + 8 * k;
+    sm[2] = est;
+    ok = est <= EST_MARGIN * tol * sm[0];
+  }
+  const bool fin = sbrk != 0 || __ballot(!ok) == 0;
+  if (klive && fin && S.small[8 * k + 5] < 0.0) {
+    S.small[8 * k + 5] = (double)(j + 1);  // rounds to use; the product skips the system from now on
+    S.small[6] = 0.0;                      // and the sweeps (every live column writes the same value)
   }
 }
 
-// wave per system of the cycle: Y = R^-1 g over the rounds used (in place in g), then the solution
-// blocks Y_b[l][k] into C1. Lane 8 p + k owns the entries (r, k) with r = p (mod 8) of g, so that
-// each element of g is only ever read back by the lane that wrote it.
-__global__ __launch_bounds__(64) void kb_bsolve(const GSys *__restrict__ sys, int steps, int L) {
-  __shared__ double sy[NB];
+// two A operands per wave while that leaves a block per CU: 28 tiles over 73 rounds 10.1 -> 7.2 us a sweep
+void launch_bdots(hipStream_t st, int ntiles, const GSys *sys, const TileMap *tmap, int which, int nb, int gram,
+                  double *part, int pstride, int all) {
+  const int nbt = nb + (gram ? 1 : 0);
+  if ((long)ntiles * ((nbt + 15) / 16) >= 512)
+    hipLaunchKernelGGL(kb_bdots<2>, dim3(ntiles, (nbt + 15) / 16), dim3(256), 0, st, sys, tmap, which, nb, gram, part,
+                       pstride, all);
+  else
+    hipLaunchKernelGGL(kb_bdots<1>, dim3(ntiles, (nbt + 7) / 8), dim3(256), 0, st, sys, tmap, which, nb, gram, part,
+                       pstride, all);
+}
+
+void launch_bsmall(hipStream_t st, int nsys, int L, const GSys *sys, int j, double tol, int all) {
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(nsys), dim3(192), 0, st, sys, j, tol, all); };
+  switch (L) {
+    case 1: go(kb_bsmall<1>); break;
+    case 2: go(kb_bsmall<2>); break;
+    case 3: go(kb_bsmall<3>); break;
+    case 4: go(kb_bsmall<4>); break;
+    case 5: go(kb_bsmall<5>); break;
+    case 6: go(kb_bsmall<6>); break;
+    default: go(kb_bsmall<7>); break;
+  }
+}
+
+// block per system of the cycle: Y = R^-1 g over the rounds used, the solution blocks Y_b[l][k] into C1, from
+// the last block of L rows up: eight lanes solve the block's triangle for their right-hand side, then every
+// thread takes the block's columns out of its rows of g, r = tid + BS u. A thread's first row of the next
+// blocks' columns is requested two blocks ahead (R does not depend on the chain). g lives in LDS while it
+// fits (GL; 341 rounds of six), else in place. Latency: 108 us at 73 rounds of three (577 with a
+// column at a time through global memory), 183 at 65 of six (1766).
+constexpr int BSV = 512;
+template <int L, bool GL>
+__global__ __launch_bounds__(BSV) void kb_bsolve(const GSys *__restrict__ sys, int steps) {
+  extern __shared__ __attribute__((aligned(16))) double lg[];
+  __shared__ double sD[L][L + 1], sY[L][NB];
   const GSys &S = sys[blockIdx.x];
   if (!S.incyc) return;  // uniform over the block
-  const int lane = threadIdx.x, p = lane >> 3, k = lane & 7;
   int kk = -1;
   for (int c = 0; c < L; ++c) {
     const double *sm = S.small + 8 * c;
     if (sm[4] > 0.0) kk = max(kk, sm[5] > 0.0 ? min((int)sm[5], steps) : steps);
   }
   kk = max(kk, 0);
-  const int N = L * kk;
-  for (int q = N - 1; q >= 0; --q) {
-    const double *Rc = S.Rp + (size_t)q * (q + 1) / 2;
-    if (p == (q & 7)) {
-      double *gq = S.gB + (size_t)q * NB + k;
-      const double d = Rc[q];
-      const double y = d != 0.0 ? *gq / d : 0.0;
-      *gq = y;
-      sy[k] = y;
+  const int tid = threadIdx.x, N = L * kk;
+  double *g = GL ? lg : S.gB;
+  if (GL)
+    for (int e = tid; e < N * NB; e += BSV) lg[e] = S.gB[e];
+  // row r of block column b of R (columns q = L b + m, rows r <= q)
+  auto load = [&](int r, int b, double (&v)[L]) {
+#pragma unroll
+    for (int m = 0; m < L; ++m) {
+      const int q = L * b + m;
+      v[m] = b >= 0 && r <= q && r < N ? S.Rp[(size_t)q * (q + 1) / 2 + r] : 0.0;
+    }
+  };
+  double cur[L], nxt[L];
+  load(tid, kk - 1, cur);
+  load(tid, kk - 2, nxt);
+  for (int b = kk - 1; b >= 0; --b) {
+    double far[L];
+    load(tid, b - 2, far);
+    __syncthreads();  // g is up to date; the last block's triangle and solution are read
+    for (int r = tid; r < L * (b + 1); r += BSV)
+      if (r >= L * b) {  // the block's own rows: its triangle, reciprocals on the diagonal
+        double v[L];
+        if (r == tid) {
+#pragma unroll
+          for (int m = 0; m < L; ++m) v[m] = cur[m];
+        } else {
+          load(r, b, v);
+        }
+        const int l = r - L * b;
+#pragma unroll
+        for (int m = 0; m < L; ++m)
+          if (m >= l) sD[l][m] = m > l ? v[m] : (v[m] != 0.0 ? 1.0 / v[m] : 0.0);
+      }
+    __syncthreads();
+    if (tid < NB) {
+      double y[L];
+#pragma unroll
+      for (int l = L - 1; l >= 0; --l) {
+        double a = g[(size_t)(L * b + l) * NB + tid];
+#pragma unroll
+        for (int m = l + 1; m < L; ++m) a -= sD[l][m] * y[m];
+        y[l] = a * sD[l][l];
+        sY[l][tid] = y[l];
+        S.C1[(size_t)b * 64 + l * 8 + tid] = y[l];
+      }
+#pragma unroll
+      for (int l = L; l < 8; ++l) S.C1[(size_t)b * 64 + l * 8 + tid] = 0.0;
     }
     __syncthreads();
-    const double yk = sy[k];
-    for (int r = p; r < q; r += 8) S.gB[(size_t)r * NB + k] -= Rc[r] * yk;
-    __syncthreads();
+    for (int r = tid; r < L * b; r += BSV) {
+      double v[L];
+      if (r == tid) {
+#pragma unroll
+        for (int m = 0; m < L; ++m) v[m] = cur[m];
+      } else {
+        load(r, b, v);
+      }
+      double *gr = g + (size_t)r * NB;
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        double a = gr[k];
+#pragma unroll
+        for (int m = 0; m < L; ++m) a -= v[m] * sY[m][k];
+        gr[k] = a;
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < L; ++m) {
+      cur[m] = nxt[m];
+      nxt[m] = far[m];
+    }
   }
-  for (int r = p; r < N; r += 8) {
-    const int b = r / L, l = r - b * L;
-    S.C1[(size_t)b * 64 + l * 8 + k] = S.gB[(size_t)r * NB + k];
+}
+
+template <int L>
+int launch_bsolve_l(andr_ctx *ctx, int nsys, const GSys *sys, int steps) {
+  const size_t lds = sizeof(double) * (size_t)L * steps * NB;
+  if (lds <= 128 * 1024) {
+    ANDR_HIP(ctx, hipFuncSetAttribute((const void *)kb_bsolve<L, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)lds));
+    hipLaunchKernelGGL((kb_bsolve<L, true>), dim3(nsys), dim3(BSV), lds, ctx->stream, sys, steps);
+  } else {
+    hipLaunchKernelGGL((kb_bsolve<L, false>), dim3(nsys), dim3(BSV), 0, ctx->stream, sys, steps);
   }
-  for (int idx = lane; idx < kk * 64; idx += 64)
-    if (((idx >> 3) & 7) >= L) S.C1[idx] = 0.0;
+  return ANDR_OK;
+}
+int launch_bsolve(andr_ctx *ctx, int nsys, int L, const GSys *sys, int steps) {
+  switch (L) {
+    case 1: return launch_bsolve_l<1>(ctx, nsys, sys, steps);
+    case 2: return launch_bsolve_l<2>(ctx, nsys, sys, steps);
+    case 3: return launch_bsolve_l<3>(ctx, nsys, sys, steps);
+    case 4: return launch_bsolve_l<4>(ctx, nsys, sys, steps);
+    case 5: return launch_bsolve_l<5>(ctx, nsys, sys, steps);
+    case 6: return launch_bsolve_l<6>(ctx, nsys, sys, steps);
+    default: return launch_bsolve_l<7>(ctx, nsys, sys, steps);
+  }
 }
 
 }  // namespace
@@ -1361,8 +1608,8 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
   const int L = nrhs;
   auto small_of = [&](int mc) {
     if (blk)  // Rp, hv, gB, C1, C2, Ri
-      return (size_t)L * mc * ((size_t)L * mc + 1) / 2 + (size_t)8 * L * mc + (size_t)L * (mc + 1) * NB +
-             (size_t)(mc + 1) * 64 + (size_t)(mc + 2) * 64 + 64;
+      return (size_t)L * mc * ((size_t)L * mc + 1) / 2 + (size_t)4 * L * L * mc + (size_t)L * (mc + 1) * NB +
+             (size_t)(mc + 1) * 64 + (size_t)(mc + 2) * 64 + 64 ;
     // H, Hu, cs, sn, g, cw per rhs
     return (size_t)NB * (2 * (size_t)(mc + 1) * mc + 2 * mc + (mc + 1) + cw_stride(mc));
   };
@@ -1534,7 +1781,7 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
         g.Rp = sp;
         sp += (size_t)L * mc * ((size_t)L * mc + 1) / 2;
         g.hv = sp;
-        sp += (size_t)8 * L * mc;
+        sp += (size_t)4 * L * L * mc;
         g.gB = sp;
         sp += (size_t)L * (mc + 1) * NB;
         g.C1 = sp;
@@ -1580,23 +1827,12 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
   ANDR_HIP(ctx, hipMemsetAsync(SM.p, 0, sizeof(double) * small_per * nsys, st));
   ANDR_HIP(ctx, hipMemsetAsync(ST8.p, 0, sizeof(double) * state_per * nsys, st));
   for (int s = 0; s < nsys; ++s) ANDR_HIP(ctx, hipMemsetAsync(in[s].X, 0, sizeof(double) * in[s].n * NB, st));
-  // scale factors of the segment sums (sx = 1, sy = 0): W = A z for the Krylov and residual products
-  std::vector<double> h_arn(2 * NB * (size_t)nsys);
-  for (int s = 0; s < nsys; ++s)
-    for (int k = 0; k < NB; ++k) {
-      h_arn[s * 2 * NB + k] = 1.0;
-      h_arn[s * 2 * NB + NB + k] = 0.0;
-    }
-  DevBuf<double> d_arn;
-  if (d_arn.alloc(h_arn.size(), ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "GMRES scales");
-  ANDR_HIP(ctx, hipMemcpyAsync(d_arn.p, h_arn.data(), sizeof(double) * h_arn.size(), hipMemcpyHostToDevice, st));
-
   const int gs = (nsys * NB + 63) / 64;
   // ANDR_GMRES_NO_SKIP=1: converged systems keep their products (and block sweeps) until the next map
   // rebuild (the rounds after convergence are never used, so the results are the same bit for bit)
   const int noskip = getenv("ANDR_GMRES_NO_SKIP") ? 1 : 0;
   // which_x 0: residual R = B - A M^-1 X (R holds B); 1: Krylov product W = A M^-1 Q_j
-  auto gemv = [&](const MapSet &ms, int which_x, int jq, const double *scales, bool prof = true) {
+  auto gemv = [&](const MapSet &ms, int which_x, int jq, bool prof = true) {
     if (ms.n_w == 0) return;
     double n2 = 0.0, n1 = 0.0;
     for (int s = 0; s < nsys; ++s)
@@ -1621,7 +1857,7 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     else
       hipLaunchKernelGGL(kb_gemv_sym<false>, dim3((ms.n_mw + 3) / 4), dim3(256), 0, st, dsys.p, ms.mw.p, ms.n_mw,
                          krylov ? noskip : 1);
-    if (ms.max_seg > 1) hipLaunchKernelGGL(kb_seg_sum, dim3(ms.n_t), dim3(256), 0, st, dsys.p, ms.t.p, scales);
+    if (ms.max_seg > 1) hipLaunchKernelGGL(kb_seg_sum, dim3(ms.n_t), dim3(256), 0, st, dsys.p, ms.t.p, all);
     if (!krylov) hipLaunchKernelGGL(kb_resid_fin, dim3(ms.n_w), dim3(256), 0, st, dsys.p, ms.w.p, partW.p);
     andr_prof_end(ctx, tok);
   };
@@ -1645,11 +1881,11 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     float best_ms = 1e30f;
     for (int target : {1024, 2048, 4096, 8192}) {
       if (build(list, live, target) || use_tiles(live)) break;
-      gemv(live, 1, jq, d_arn.p, false);  // warm-up
+      gemv(live, 1, jq, false);  // warm-up
       float ms = 1e30f;
       for (int rep = 0; rep < 2; ++rep) {
         (void)hipEventRecord(e0, st);
-        gemv(live, 1, jq, d_arn.p, false);
+        gemv(live, 1, jq, false);
         (void)hipEventRecord(e1, st);
         (void)hipEventSynchronize(e1);
         float t = 0.f;
@@ -1719,10 +1955,10 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     if (first) {
       if (cyc.n_w) hipLaunchKernelGGL(kb_resid_zero, dim3(cyc.n_w), dim3(256), 0, st, dsys.p, cyc.w.p, partW.p);
     } else {
-      gemv(cyc, 0, 0, d_arn.p);
+      gemv(cyc, 0, 0);
     }
     ANDR_HIP(ctx, hipMemsetAsync(ddone.p, 0, sizeof(int), st));
-    hipLaunchKernelGGL(kb_restart, dim3(gs), dim3(64), 0, st, dsys.p, nsys, partW.p, cyc.w0.p, cyc.nw.p, tol,
+    hipLaunchKernelGGL(kb_restart, dim3(nsys), dim3(256), 0, st, dsys.p, partW.p, cyc.w0.p, cyc.nw.p, tol,
                        first ? 1 : 0, nrhs, ddone.p);
     ANDR_HIP(ctx, hipGetLastError());
     if ((rc = read_small())) return rc;
@@ -1753,10 +1989,10 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     if ((rc = use_tiles(live))) return rc;
     std::fill(skip_counted.begin(), skip_counted.end(), 0);
     if (blk) {  // Q_0 R0 = R (Cholesky QR of the residual block), g = (R0; 0)
-      hipLaunchKernelGGL(kb_bdots, dim3(live.n_t4, 1), dim3(256), 0, st, dsys.p, live.t4.p, 1, 0, 1, partB.p, mc + 2, 1);
+      launch_bdots(st, live.n_t4, dsys.p, live.t4.p, 1, 0, 1, partB.p, mc + 2, 1);
       hipLaunchKernelGGL(kb_bdots_final, dim3(nsys, 1), dim3(256), 0, st, dsys.p, partB.p, mc + 2, 1, 1);
-      hipLaunchKernelGGL(kb_binit, dim3(nsys), dim3(64), 0, st, dsys.p, mc, L);
-      hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t4), dim3(256), 0, st, dsys.p, live.t4.p, 0, 3, 1);
+      hipLaunchKernelGGL(kb_binit, dim3(nsys), dim3(256), 0, st, dsys.p, mc, L);
+      hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t.p, 0, 3, 1);
     } else {
       hipLaunchKernelGGL(kb_ginit, dim3(gs), dim3(64), 0, st, dsys.p, nsys, mc);
       hipLaunchKernelGGL(kb_q0, dim3(cyc.n_t), dim3(256), 0, st, dsys.p, cyc.t.p);
@@ -1772,7 +2008,7 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     const int steps_max = std::min(mc, maxit - total);
     int steps = 0;
     for (int j = 0; j < steps_max; ++j) {
-      gemv(live, 1, j, d_arn.p);  // W = A Q_j
+      gemv(live, 1, j);  // W = A Q_j
       // one sweep of dot products and one of updates over the basis (delayed reorthogonalisation)
       double nlive = 0.0;
       for (int s = 0; s < nsys; ++s)
@@ -1783,15 +2019,13 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
         // twice); the second update also normalises the new block
         const int tok_o = andr_prof_begin(ctx, "gmres_orthogonalise", (4.0 * j + 10.0) * vbytes,
                                           2.0 * 64.0 * (4.0 * j + 5.0) * nlive);
-        hipLaunchKernelGGL(kb_bdots, dim3(live.n_t4, (j + 16) / 16), dim3(256), 0, st, dsys.p, live.t4.p, 0, j + 1,
-                           0, partB.p, mc + 2, noskip);
+        launch_bdots(st, live.n_t4, dsys.p, live.t4.p, 0, j + 1, 0, partB.p, mc + 2, noskip);
         hipLaunchKernelGGL(kb_bdots_final, dim3(nsys, j + 1), dim3(256), 0, st, dsys.p, partB.p, mc + 2, 0, noskip);
-        hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t4), dim3(256), 0, st, dsys.p, live.t4.p, j + 1, 0, noskip);
-        hipLaunchKernelGGL(kb_bdots, dim3(live.n_t4, (j + 17) / 16), dim3(256), 0, st, dsys.p, live.t4.p, 0, j + 1,
-                           1, partB.p, mc + 2, noskip);
+        hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t.p, j + 1, 0, noskip);
+        launch_bdots(st, live.n_t4, dsys.p, live.t4.p, 0, j + 1, 1, partB.p, mc + 2, noskip);
         hipLaunchKernelGGL(kb_bdots_final, dim3(nsys, j + 2), dim3(256), 0, st, dsys.p, partB.p, mc + 2, 1, noskip);
-        hipLaunchKernelGGL(kb_bsmall, dim3(nsys), dim3(64), 0, st, dsys.p, j, L, tol, noskip);
-        hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t4), dim3(256), 0, st, dsys.p, live.t4.p, j + 1, 1, noskip);
+        launch_bsmall(st, nsys, L, dsys.p, j, tol, noskip);
+        hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t.p, j + 1, 1, noskip);
         andr_prof_end(ctx, tok_o);
       } else {
         const int tok_o = andr_prof_begin(ctx, "gmres_orthogonalise", (2.0 * j + 6.0) * vbytes,
@@ -1839,8 +2073,8 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     }
     total += steps;
     if (blk) {
-      hipLaunchKernelGGL(kb_bsolve, dim3(nsys), dim3(64), 0, st, dsys.p, steps, L);
-      hipLaunchKernelGGL(kb_bupdate, dim3(cyc.n_t4), dim3(256), 0, st, dsys.p, cyc.t4.p, steps, 2, 1);
+      if ((rc = launch_bsolve(ctx, nsys, L, dsys.p, steps))) return rc;
+      hipLaunchKernelGGL(kb_bupdate, dim3(cyc.n_t), dim3(256), 0, st, dsys.p, cyc.t.p, steps, 2, 1);
     } else {
       hipLaunchKernelGGL(kb_solve_y, dim3(nsys * NB), dim3(64), sizeof(double) * (mc + 1), st, dsys.p, steps, mc);
       hipLaunchKernelGGL(kb_xupdate, dim3(cyc.n_t), dim3(256), 0, st, dsys.p, cyc.t.p, steps, mc);
