@@ -1633,49 +1633,60 @@ int andr_launch_stokes_system(andr_ctx *ctx, const SysJob *d_jobs, const int2 *d
 // block per body: force and torque of the six problems on wall 1, F = sum_e A_e q_e and
 // T = sum_e A_e (c_e - centre) x q_e (the reductions of src/lib_particle.f90:1751-1831), and the
 // largest row self-check error. out[37 b + 6 k + (0..5)] = (F, T) of problem k, out[37 b + 36] = error.
-__global__ __launch_bounds__(256) void k_force_torque(const SysJob *__restrict__ jobs, double *__restrict__ out) {
-  __shared__ double red[36 * 4];
-  __shared__ double emax[4];
+// Latency of one block: a lane takes one problem of every 128th element, eight lanes a row of X (all 36 sums in
+// one lane were a reduction of 432 lane exchanges in a row: 40 -> 8 us for 80 elements, 46 -> 21 for about 2300; forty
+// bodies of up to 7220 are bound by the largest one's turns over memory, 76 -> 79).
+constexpr int FT_THREADS = 1024, FT_WAVES = FT_THREADS / 64;
+__global__ __launch_bounds__(FT_THREADS) void k_force_torque(const SysJob *__restrict__ jobs, double *__restrict__ out) {
+  __shared__ double red[FT_WAVES][ANDR_NRHS][7];
   const SysJob &J = jobs[blockIdx.x];
-  const BodyGeom &g = J.g;
-  const int ne = g.ne;
-  double v[36];
-#pragma unroll
-  for (int i = 0; i < 36; ++i) v[i] = 0.0;
-  double err = 0.0;
-  for (int e = threadIdx.x; e < ne; e += blockDim.x) {
-    if (J.err_rows) err = fmax(err, J.err_rows[e]);
-    if (g.bcid[e] != 1) continue;
-    const double a = g.area[e];
-    const double r0 = g.cen[3 * e] - J.center[0], r1 = g.cen[3 * e + 1] - J.center[1],
-                 r2 = g.cen[3 * e + 2] - J.center[2];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      const double q0 = J.X[(size_t)e * ANDR_NRHS + k], q1 = J.X[(size_t)(ne + e) * ANDR_NRHS + k],
-                   q2 = J.X[(size_t)(2 * ne + e) * ANDR_NRHS + k];
-      v[6 * k] += a * q0;
-      v[6 * k + 1] += a * q1;
-      v[6 * k + 2] += a * q2;
-      v[6 * k + 3] += a * (r1 * q2 - r2 * q1);
-      v[6 * k + 4] += a * (r2 * q0 - r0 * q2);
-      v[6 * k + 5] += a * (r0 * q1 - r1 * q0);
-    }
+  const int ne = J.g.ne, t = threadIdx.x, k = t % ANDR_NRHS;
+  const double *__restrict__ X = J.X + k, *__restrict__ cen = J.g.cen, *__restrict__ area = J.g.area;
+  const double *__restrict__ rows = k == 0 ? J.err_rows : nullptr;
+  const int *__restrict__ bcid = J.g.bcid;
+  const double c0 = J.center[0], c1 = J.center[1], c2 = J.center[2];
+  double v[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};  // F, T, largest error
+#pragma unroll 8
+  for (int e = t / ANDR_NRHS; e < ne; e += FT_THREADS / ANDR_NRHS) {
+    if (rows) v[6] = fmax(v[6], rows[e]);
+    const bool on = bcid[e] == 1;
+    const double a = area[e];
+    const double r0 = cen[3 * e] - c0, r1 = cen[3 * e + 1] - c1, r2 = cen[3 * e + 2] - c2;
+    double q0 = X[(size_t)e * ANDR_NRHS], q1 = X[(size_t)(ne + e) * ANDR_NRHS], q2 = X[(size_t)(2 * ne + e) * ANDR_NRHS];
+    if (!on) q0 = q1 = q2 = 0.0;  // an element of another wall adds nothing
+    v[0] += a * q0;
+    v[1] += a * q1;
+    v[2] += a * q2;
+    v[3] += a * (r1 * q2 - r2 * q1);
+    v[4] += a * (r2 * q0 - r0 * q2);
+    v[5] += a * (r0 * q1 - r1 * q0);
   }
-  for (int o = 32; o > 0; o >>= 1) err = fmax(err, __shfl_xor(err, o, 64));
-  if ((threadIdx.x & 63) == 0) emax[threadIdx.x >> 6] = err;
-  block_sum<36>(v, red);
-  if (threadIdx.x == 0) {
+  for (int o = ANDR_NRHS; o < 64; o <<= 1) {
 #pragma unroll
-    for (int i = 0; i < 36; ++i) out[(size_t)blockIdx.x * 37 + i] = v[i];
+    for (int c = 0; c < 6; ++c) v[c] += __shfl_xor(v[c], o, 64);
+    v[6] = fmax(v[6], __shfl_xor(v[6], o, 64));
+  }
+  if ((t & 63) < ANDR_NRHS)
+#pragma unroll
+    for (int c = 0; c < 7; ++c) red[t >> 6][k][c] = v[c];
+  __syncthreads();
+  if (t < 36) {
+    double s = 0.0;
+#pragma unroll
+    for (int h = 0; h < FT_WAVES; ++h) s += red[h][t / 6][t % 6];
+    out[(size_t)blockIdx.x * 37 + t] = s;
+  } else if (t == 36) {
     double m = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) m = fmax(m, emax[w]);
+#pragma unroll
+    for (int h = 0; h < FT_WAVES; ++h) m = fmax(m, red[h][0][6]);
     out[(size_t)blockIdx.x * 37 + 36] = m;
   }
 }
+static_assert(ANDR_NRHS == 8, "k_force_torque: eight lanes per element");
 
 int andr_launch_force_torque(andr_ctx *ctx, const SysJob *d_jobs, int njobs, double *d_out) {
   if (njobs <= 0) return ANDR_OK;
-  hipLaunchKernelGGL(k_force_torque, dim3(njobs), dim3(256), 0, ctx->stream, d_jobs, d_out);
+  hipLaunchKernelGGL(k_force_torque, dim3(njobs), dim3(FT_THREADS), 0, ctx->stream, d_jobs, d_out);
   ANDR_HIP(ctx, hipGetLastError());
   return ANDR_OK;
 }
@@ -1779,7 +1790,7 @@ int andr_copy_out(andr_ctx *ctx, const double *d, int64_t m, int64_t n, int32_t 
     return ANDR_OK;
   }
   DevBuf<double> t;
-  if (t.alloc((size_t)m * n)) return andr_fail(ctx, ANDR_ERR_ALLOC, "transpose buffer");
+  if (t.alloc((size_t)m * n, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "transpose buffer");
   dim3 grid((unsigned)((n + 31) / 32), (unsigned)((m + 31) / 32));
   hipLaunchKernelGGL(k_transpose, grid, dim3(32, 8), 0, ctx->stream, d, t.p, m, n);
   ANDR_HIP(ctx, hipGetLastError());
