@@ -711,22 +711,22 @@ __global__ __launch_bounds__(256) void k_lsqr_v(int n, int nsplit, const double 
     if (!any) return;  // uniform over the grid; state A holds the stopped columns already
     const double uu = block_sum<WD, 256>(uut, red);
     if (tid < WD) {
-      LsqrState S = sb[tid];
+      const LsqrState &S = sb[tid];
+      const int active = S.active;
+      const double beta = sqrt(uu), alpha = S.alpha;
       st[tid] = S.t1;
       st[WD + tid] = S.t2;
       st[2 * WD + tid] = S.inv_alpha;
       su[tid] = S.upd;
-      double sx = 0.0, sy = 0.0;
-      if (S.active) {
-        const double beta = sqrt(uu);
-        sx = beta > 0.0 ? 1.0 / beta : 0.0;
-        sy = beta > 0.0 ? -beta / S.alpha : 1.0;  // beta = 0: V unchanged
-        S.itn += 1;
-        S.beta = beta;
+      sc[tid] = active && beta > 0.0 ? 1.0 / beta : 0.0;
+      sc[WD + tid] = active ? (beta > 0.0 ? -beta / alpha : 1.0) : 0.0;  // beta = 0: V unchanged
+      if (blockIdx.x == gridDim.x - 1) {
+        sa[tid] = S;
+        if (active) {
+          sa[tid].itn += 1;
+          sa[tid].beta = beta;
+        }
       }
-      sc[tid] = sx;
-      sc[WD + tid] = sy;
-      if (blockIdx.x == gridDim.x - 1) sa[tid] = S;
     }
   } else {
     load(blockIdx.x * NV + val, cur);
