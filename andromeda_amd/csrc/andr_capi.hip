@@ -463,7 +463,7 @@ int upload_csr(andr_ctx *ctx, int m, int n, int64_t nnz, const int64_t *ia, cons
   DevBuf<int32_t> dja;
   DevBuf<double> da;
   const int64_t ld = dense_ld(n);
-  if (c.D.alloc((size_t)m * ld) || dia.alloc(m + 1) || dja.alloc(nnz) || da.alloc(nnz))
+  if (c.D.alloc((size_t)m * ld) || dia.alloc(m + 1, ctx) || dja.alloc(nnz, ctx) || da.alloc(nnz, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "LSQR matrix %d x %d", m, n);
   ANDR_HIP(ctx, hipMemsetAsync(c.D.p, 0, sizeof(double) * (size_t)m * ld, st));
   ANDR_HIP(ctx, hipMemcpyAsync(dia.p, ia, sizeof(int64_t) * (m + 1), hipMemcpyHostToDevice, st));
@@ -544,7 +544,8 @@ extern "C" void lsqr_solve_(const int32_t *m, const int32_t *n, const int64_t *n
   if (*maxit == 0) *maxit = 10 * (*m + *n + 50);
   const int M = *m, N = *n;
   DevBuf<double> dq, dB, dX, tmp;
-  if (dq.alloc(N) || dB.alloc((size_t)M * ANDR_NB) || dX.alloc((size_t)N * ANDR_NB) || tmp.alloc(std::max(M, N))) {
+  if (dq.alloc(N, ctx) || dB.alloc((size_t)M * ANDR_NB, ctx) || dX.alloc((size_t)N * ANDR_NB, ctx) ||
+      tmp.alloc(std::max(M, N), ctx)) {
     *ierr = -3;
     return;
   }
@@ -619,7 +620,8 @@ extern "C" int andr_lsqr_dense(andr_ctx *ctx, int64_t m, int64_t n, const double
   andr_lsqr_opts o = opts ? *opts : andr_lsqr_opts{0, 1e-15, 1};
   DevBuf<double> dA, dq, dB, dX;
   const int64_t lda = (n + 15) / 16 * 16;  // rows start on 128-byte lines
-  if (dA.alloc((size_t)m * lda) || dq.alloc(n) || dB.alloc((size_t)m * ANDR_NB) || dX.alloc((size_t)n * ANDR_NB))
+  if (dA.alloc((size_t)m * lda, ctx) || dq.alloc(n, ctx) || dB.alloc((size_t)m * ANDR_NB, ctx) ||
+      dX.alloc((size_t)n * ANDR_NB, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "andr_lsqr_dense workspace");
   ANDR_HIP(ctx, hipMemcpy2DAsync(dA.p, sizeof(double) * lda, A, sizeof(double) * n, sizeof(double) * n, m,
                                  hipMemcpyHostToDevice, ctx->stream));

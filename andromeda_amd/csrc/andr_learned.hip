@@ -326,12 +326,13 @@ __global__ void k_gather(int M, const int *__restrict__ idx, const float *__rest
 struct MlpWork {
   DevBuf<float> Z1, H1, Z2, H2, Z3, H3, Z4, P, dZ4, dH, dZb, loss;
   int B = 0;
-  int alloc(int b) {
+  int alloc(andr_ctx *ctx, int b) {
     B = b;
-    if (Z1.alloc((size_t)b * NH) || H1.alloc((size_t)b * NH) || Z2.alloc((size_t)b * NH) || H2.alloc((size_t)b * NH) ||
-        Z3.alloc((size_t)b * NH) || H3.alloc((size_t)b * NH) || Z4.alloc((size_t)b * NOUT) || P.alloc((size_t)b * NOUT) ||
-        dZ4.alloc((size_t)b * NOUT) || dH.alloc((size_t)b * NH) || dZb.alloc((size_t)b * NH) || loss.alloc(b))
-      return 1;
+    for (DevBuf<float> *h : {&Z1, &H1, &Z2, &H2, &Z3, &H3, &dH, &dZb})
+      if (h->alloc((size_t)b * NH, ctx)) return 1;
+    for (DevBuf<float> *o : {&Z4, &P, &dZ4})
+      if (o->alloc((size_t)b * NOUT, ctx)) return 1;
+    if (loss.alloc(b, ctx)) return 1;
     return 0;
   }
 };
@@ -667,7 +668,12 @@ static int labels_common(andr_ctx *ctx, const andr_mesh *mesh, double near_ratio
   DevBuf<int> dl, dfar;
   DevBuf<unsigned long long> cnt;
   const int64_t mp = mode == 0 ? std::max<int64_t>(max_pairs, 1) : 1;
-  if (df.alloc((size_t)mp * 6) || dl.alloc(mp) || dfar.alloc(ANDR_FAR_BINS) || cnt.alloc(1))
+  // the label kernel needs scratch memory of the runtime's own, which a cache that fills the device leaves
+  // no room for
+  size_t free_b = 0, total_b = 0;
+  ANDR_HIP(ctx, hipMemGetInfo(&free_b, &total_b));
+  if (free_b < ((size_t)2 << 30)) andr_pool_trim(ctx);
+  if (df.alloc((size_t)mp * 6, ctx) || dl.alloc(mp, ctx) || dfar.alloc(ANDR_FAR_BINS, ctx) || cnt.alloc(1, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "training pair buffers");
   uint32_t keep = 0xFFFFFFFFu;
   unsigned long long n = 0;
@@ -724,7 +730,8 @@ extern "C" int andr_mlp_loss_grad(andr_ctx *ctx, int64_t npairs, const float *fe
   MlpWork w;
   DevBuf<float> X, p, gr;
   DevBuf<int> L;
-  if (w.alloc(M) || X.alloc((size_t)M * NIN) || p.alloc(NPARAM) || gr.alloc(NPARAM) || L.alloc(M))
+  if (w.alloc(ctx, M) || X.alloc((size_t)M * NIN, ctx) || p.alloc(NPARAM, ctx) || gr.alloc(NPARAM, ctx) ||
+      L.alloc(M, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "MLP buffers");
   hipStream_t st = ctx->stream;
   ANDR_HIP(ctx, hipMemcpyAsync(X.p, features, sizeof(float) * M * NIN, hipMemcpyHostToDevice, st));
@@ -750,7 +757,8 @@ extern "C" int andr_mlp_infer(andr_ctx *ctx, int64_t npairs, const float *featur
   const int chunk = 1 << 16;
   MlpWork w;
   DevBuf<float> X, p;
-  if (w.alloc(chunk) || X.alloc((size_t)chunk * NIN) || p.alloc(NPARAM)) return andr_fail(ctx, ANDR_ERR_ALLOC, "MLP buffers");
+  if (w.alloc(ctx, chunk) || X.alloc((size_t)chunk * NIN, ctx) || p.alloc(NPARAM, ctx))
+    return andr_fail(ctx, ANDR_ERR_ALLOC, "MLP buffers");
   hipStream_t st = ctx->stream;
   ANDR_HIP(ctx, hipMemcpyAsync(p.p, params, sizeof(float) * NPARAM, hipMemcpyHostToDevice, st));
   for (int64_t i0 = 0; i0 < npairs; i0 += chunk) {
@@ -777,8 +785,9 @@ extern "C" int andr_mlp_train(andr_ctx *ctx, int64_t npairs, const float *featur
   MlpWork w;
   DevBuf<float> X, Xb, p, gr, m, v, lossacc;
   DevBuf<int> L, Lb, idx;
-  if (w.alloc(B) || X.alloc((size_t)N * NIN) || Xb.alloc((size_t)B * NIN) || p.alloc(NPARAM) || gr.alloc(NPARAM) ||
-      m.alloc(NPARAM) || v.alloc(NPARAM) || L.alloc(N) || Lb.alloc(B) || idx.alloc(N))
+  if (w.alloc(ctx, B) || X.alloc((size_t)N * NIN, ctx) || Xb.alloc((size_t)B * NIN, ctx) ||
+      p.alloc(NPARAM, ctx) || gr.alloc(NPARAM, ctx) || m.alloc(NPARAM, ctx) || v.alloc(NPARAM, ctx) ||
+      L.alloc(N, ctx) || Lb.alloc(B, ctx) || idx.alloc(N, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "MLP training buffers");
   hipStream_t st = ctx->stream;
   ANDR_HIP(ctx, hipMemcpyAsync(X.p, features, sizeof(float) * (size_t)N * NIN, hipMemcpyHostToDevice, st));
@@ -881,7 +890,7 @@ int andr_launch_stokes_system_learned(andr_ctx *ctx, SysJob *h_jobs, const SysJo
   const size_t tiles_off = model_tiles_off();
   const bf16x4 *tiles = (const bf16x4 *)(base + tiles_off);
   DevBuf<unsigned long long> st;
-  if (st.alloc(3 * (size_t)njobs)) return andr_fail(ctx, ANDR_ERR_ALLOC, "stats");
+  if (st.alloc(3 * (size_t)njobs, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "stats");
   ANDR_HIP(ctx, hipMemsetAsync(st.p, 0, 3 * sizeof(unsigned long long) * njobs, ctx->stream));
   const int tok = andr_prof_begin(ctx, "classify_pairs", 0.0, 0.0);
   hipLaunchKernelGGL(k_classify, dim3(nrows), dim3(CLS_THREADS), 0, ctx->stream, d_jobs, d_rowmap, tiles, fp, far,
