@@ -178,200 +178,286 @@ __global__ __launch_bounds__(256) void k_pair_labels(BodyGeom g, int qoff_ref, i
   }
 }
 
-// ---- small FP32 GEMMs on the matrix cores (v_mfma_f32_16x16x4f32), row-major -------------------
+// ---- the network in FP32 on the matrix cores (v_mfma_f32_16x16x4f32), row-major ------------------
 // Lane layout of one 16x16x4 step: lane 16 g + i supplies A[i][g] and B[g][i] and, after the K
 // loop, holds C[4 g + v][i], v = 0..3. Inside a 16-deep K block, step t gives lane group g the index
 // k0 + 4 g + t on both operands (one permutation of K, so every k is summed once); the four steps
 // go to four accumulators, added at the end. Out-of-range rows, columns and k read as 0.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// Z = op(A) op(B) (+ bias[col]); H = relu(Z) if H; Z = 0 where mask <= 0 if mask (ReLU backward,
-// mask = the forward pre-activation of the same shape). One wave per 16x16 tile of Z.
-__global__ __launch_bounds__(256) void k_sgemm(int M, int N, int K, const float *__restrict__ A, int lda, int ta,
-                                               const float *__restrict__ B, int ldb, int tb, float *__restrict__ Z,
-                                               int ldz, const float *__restrict__ bias, float *__restrict__ H,
-                                               const float *__restrict__ mask) {
-  const int lane = threadIdx.x & 63;
-  const int tiles_n = (N + 15) >> 4;
-  const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (tile >= tiles_n * ((M + 15) >> 4)) return;
-  const int tm = tile / tiles_n, tn = tile - tm * tiles_n;
-  const int g = lane >> 4, i = lane & 15;
-  const int row = 16 * tm + i, col = 16 * tn + i;
-  const bool rok = row < M, cok = col < N;
-  f32x4 acc[4];
+// A 64-thread wave owns 16 of the 64 columns of every layer. wf: B operand of a forward layer,
+// W[16 kb + 4 g + t][col]; wt: of a backward one, W[col][16 kb + 4 g + t] (ldw a multiple of four and the
+// parameters of each layer on 16 bytes, so four k of a row are one load).
+template <int K>
+__device__ inline void wf(const float *__restrict__ W, int ldw, int col, bool cok, int g, f32x4 b[(K + 15) / 16]) {
 #pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < K; k0 += 16) {
+  for (int kb = 0; kb < (K + 15) / 16; ++kb)
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const int k = k0 + 4 * g + t;
-      const bool kok = k < K;
-      const float a = (rok && kok) ? (ta ? A[(size_t)k * lda + row] : A[(size_t)row * lda + k]) : 0.f;
-      const float b = (cok && kok) ? (tb ? B[(size_t)col * ldb + k] : B[(size_t)k * ldb + col]) : 0.f;
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc[t], 0, 0, 0);
+      const int k = 16 * kb + 4 * g + t;
+      const float x = W[(size_t)(k < K ? k : 0) * ldw + (cok ? col : 0)];
+      b[kb][t] = (k < K && cok) ? x : 0.f;
     }
-  }
-  if (!cok) return;
-  const float bc = bias ? bias[col] : 0.f;
+}
+template <int K>
+__device__ inline void wt(const float *__restrict__ W, int ldw, int col, int g, f32x4 b[(K + 15) / 16]) {
 #pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int r = 16 * tm + 4 * g + v;
-    if (r >= M) break;
-    const size_t o = (size_t)r * ldz + col;
-    float z = (acc[0][v] + acc[1][v]) + (acc[2][v] + acc[3][v]) + bc;
-    if (mask && !(mask[o] > 0.f)) z = 0.f;
-    Z[o] = z;
-    if (H) H[o] = fmaxf(z, 0.f);
+  for (int kb = 0; kb < (K + 15) / 16; ++kb) {
+    const int k = 16 * kb + 4 * g;
+    const f32x4 x = *(const f32x4 *)(W + (size_t)col * ldw + (k < K ? k : 0));
+    b[kb] = k < K ? x : f32x4{0.f, 0.f, 0.f, 0.f};
   }
 }
 
-// Weight and bias gradients of one layer: G = A^T D (A: M x NI, D: M x NO, row-major with leading
-// dimensions NI and NO; G: NI x NO) and gb = the column sums of D. One 1024-thread block per 16x16
-// tile of G: its 16 waves take the samples 16 at a time in turn and their partial tiles are added
-// in a fixed order through LDS. The blocks of the first row of tiles (tm = 0) also write gb.
-constexpr int WG_WAVES = 16;
-__global__ __launch_bounds__(1024) void k_wgrad(int M, int NI, int NO, const float *__restrict__ A,
-                                                const float *__restrict__ D, float *__restrict__ G,
-                                                float *__restrict__ gb) {
+// C tile of 16 samples: A from LDS (rows of MT_LD floats), B in registers; returns (+ bias)
+constexpr int MT_LD = NH + 4;
+template <int KB>
+__device__ inline f32x4 mlp_tile(const float *__restrict__ A, const f32x4 b[KB], int g, int i, float bias) {
+  f32x4 acc[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    const f32x4 a = *(const f32x4 *)(A + i * MT_LD + 16 * kb + 4 * g);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], b[kb][t], acc[t], 0, 0, 0);
+  }
+  f32x4 z;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) z[v] = (acc[0][v] + acc[1][v]) + (acc[2][v] + acc[3][v]) + bias;
+  return z;
+}
+
+// What a minibatch leaves for the weight gradients: inputs and outputs' gradients of the four layers (M rows each).
+struct MlpAct {
+  float *X, *H1, *H2, *H3, *D1, *D2, *D3, *D4;
+};
+
+// Forward pass of M samples (rows idx[m] of X and lab, or m itself): Z_l = H_(l-1) W_l + b_l, H_l = relu(Z_l),
+// then the softmax of the logits into P; with GRAD the mean cross-entropy's gradient goes back through the
+// layers instead: loss (per sample) and everything that the weight gradients read into `act`.
+// Latency bound on a minibatch (a chain of seven layers for each 16 samples), so one launch keeps the tile in
+// LDS with all weights of the wave's columns loaded ahead into registers: 8.4 us for 1024 samples, where a launch
+// per layer (gather, four forward, softmax, three backward, each through memory) cost 6 to 9 us nine times.
+template <bool GRAD>
+__global__ __launch_bounds__(256) void k_mlp(int M, const int *__restrict__ idx, const float *__restrict__ X,
+                                             const int *__restrict__ lab, const float *__restrict__ p,
+                                             float *__restrict__ P, float *__restrict__ loss, MlpAct act, float scale) {
+  __shared__ __align__(16) float T[2][16 * MT_LD];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, i = lane & 15;
+  const int col = 16 * w + i;
+  f32x4 w1[1], w2[4], w3[4], w4[4], t4[1], t3[4], t2[4];
+  wf<NIN>(p + P_W1, NH, col, true, g, w1);
+  wf<NH>(p + P_W2, NH, col, true, g, w2);
+  wf<NH>(p + P_W3, NH, col, true, g, w3);
+  wf<NH>(p + P_W4, NOUT, i, i < NOUT, g, w4);  // every wave holds the one tile of the output layer
+  if (GRAD) {
+    wt<NOUT>(p + P_W4, NOUT, col, g, t4);
+    wt<NH>(p + P_W3, NH, col, g, t3);
+    wt<NH>(p + P_W2, NH, col, g, t2);
+  }
+  const float b1 = p[P_B1 + col], b2 = p[P_B2 + col], b3 = p[P_B3 + col], b4 = p[P_B4 + (i & (NOUT - 1))];
+  const int ntiles = (M + 15) >> 4;
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const int m0 = 16 * tile;
+    // lane (s, k) of the first two waves: input k and, later, logit k of sample s
+    const int s = tid >> 3, k = tid & 7, ms = m0 + s;
+    const bool sok = tid < 128 && ms < M;
+    const int src = sok ? (idx ? idx[ms] : ms) : 0;
+    int ls = -1;
+    if (tid < 128) {
+      const float x = sok && k < NIN ? X[(size_t)src * NIN + k] : 0.f;
+      if (sok && lab) ls = lab[src];
+      T[0][s * MT_LD + k] = x;
+      T[0][s * MT_LD + 8 + k] = 0.f;
+      if (GRAD && act.X && sok && k < NIN) act.X[(size_t)ms * NIN + k] = x;
+    }
+    __syncthreads();
+    // H of a layer into the other tile and, for the weight gradients, to memory
+    auto put = [&](float *dst, float *glob, f32x4 h) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        dst[(4 * g + v) * MT_LD + col] = h[v];
+        if (GRAD && m0 + 4 * g + v < M) glob[(size_t)(m0 + 4 * g + v) * NH + col] = h[v];
+      }
+      __syncthreads();
+    };
+    auto relu = [](f32x4 z) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) z[v] = fmaxf(z[v], 0.f);
+      return z;
+    };
+    auto where = [](f32x4 z, f32x4 h) {  // the ReLU's backward: h > 0 where its input was
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (!(h[v] > 0.f)) z[v] = 0.f;
+      return z;
+    };
+    const f32x4 h1 = relu(mlp_tile<1>(T[0], w1, g, i, b1));
+    put(T[1], act.H1, h1);
+    const f32x4 h2 = relu(mlp_tile<4>(T[1], w2, g, i, b2));
+    put(T[0], act.H2, h2);
+    const f32x4 h3 = relu(mlp_tile<4>(T[0], w3, g, i, b3));
+    put(T[1], act.H3, h3);
+    if (w == 0) {
+      const f32x4 z = mlp_tile<4>(T[1], w4, g, i, b4);
+      if (i < NOUT)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) T[0][(4 * g + v) * MT_LD + i] = z[v];
+    }
+    __syncthreads();
+    if (w < 2) {  // softmax cross-entropy, a lane per logit; the sum runs over the logits in order
+      const float *z = &T[0][s * MT_LD];
+      const float zk = z[k];
+      float mx = z[0];
+#pragma unroll
+      for (int j = 1; j < NOUT; ++j) mx = fmaxf(mx, z[j]);
+      const float ek = expf(zk - mx);
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < NOUT; ++j) sum += __shfl(ek, (lane & ~7) + j, 64);
+      const float pk = ek / sum;
+      if (P && sok) P[(size_t)ms * NOUT + k] = pk;
+      if (GRAD) {
+        const float d = (pk - (ls == k ? 1.f : 0.f)) * scale;
+        if (sok && ls == k) loss[ms] = -(zk - mx - logf(sum));
+        T[1][s * MT_LD + k] = sok ? d : 0.f;
+        T[1][s * MT_LD + 8 + k] = 0.f;
+        if (sok) act.D4[(size_t)ms * NOUT + k] = d;
+      }
+    }
+    __syncthreads();
+    if (GRAD) {
+      const f32x4 d3 = where(mlp_tile<1>(T[1], t4, g, i, 0.f), h3);
+      put(T[0], act.D3, d3);
+      const f32x4 d2 = where(mlp_tile<4>(T[0], t3, g, i, 0.f), h2);
+      put(T[1], act.D2, d2);
+      const f32x4 d1 = where(mlp_tile<4>(T[1], t2, g, i, 0.f), h1);
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (m0 + 4 * g + v < M) act.D1[(size_t)(m0 + 4 * g + v) * NH + col] = d1[v];
+    }
+  }
+}
+
+struct AdamStep {
+  float *m, *v;  // moments; the parameters move when m is set, else the gradient is written
+  float lr, b1, b2, eps, c1, c2;
+};
+
+// Weight and bias gradients of all layers, G = A^T D (A: M x NI, D: M x NO, row-major) and the column sums of
+// D, and the Adam step with them. One 1024-thread block per 16x16 tile of a G: its 16 waves take the samples
+// 16 at a time in turn, four turns' loads together, and their partial tiles are added in a fixed order through
+// LDS, a wave per row of the lanes' results. The blocks of the first row of tiles (tm = 0) also take the bias.
+// Latency bound on a minibatch: 6.5 us for 1024 samples, where the four layers and Adam's step were five launches of
+// 6 to 9 us in a row. A minibatch with its host share went from 98 to 19 us.
+constexpr int WG_WAVES = 16, WG_TURNS = 4;
+constexpr int WG_BLOCKS = 4 + 16 + 16 + 4;
+__global__ __launch_bounds__(1024) void k_mlp_update(int M, MlpAct act, float *__restrict__ p, float *__restrict__ grad,
+                                                     AdamStep ad) {
   __shared__ float part[WG_WAVES][5][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int bid = blockIdx.x;
+  const int layer = bid < 4 ? 0 : bid < 20 ? 1 : bid < 36 ? 2 : 3;
+  const int tile = bid - (layer == 0 ? 0 : layer == 1 ? 4 : layer == 2 ? 20 : 36);
+  const int NI = layer == 0 ? NIN : NH, NO = layer == 3 ? NOUT : NH;
+  const float *__restrict__ A = layer == 0 ? act.X : layer == 1 ? act.H1 : layer == 2 ? act.H2 : act.H3;
+  const float *__restrict__ D = layer == 0 ? act.D1 : layer == 1 ? act.D2 : layer == 2 ? act.D3 : act.D4;
+  const int pw = layer == 0 ? P_W1 : layer == 1 ? P_W2 : layer == 2 ? P_W3 : P_W4;
+  const int pb = layer == 0 ? P_B1 : layer == 1 ? P_B2 : layer == 2 ? P_B3 : P_B4;
   const int tiles_n = (NO + 15) >> 4;
-  const int tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
+  const int tm = tile / tiles_n, tn = tile - tm * tiles_n;
   const int g = lane >> 4, i = lane & 15;
   const int row = 16 * tm + i, col = 16 * tn + i;
   const bool rok = row < NI, cok = col < NO;
+  const float *__restrict__ Ar = A + (rok ? row : 0), *__restrict__ Dc = D + (cok ? col : 0);
   f32x4 acc[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   float cs = 0.f;  // this lane's share of the column sum of D
-  for (int m0 = 16 * w; m0 < M; m0 += 16 * WG_WAVES) {
+  for (int m0 = 16 * w; m0 < M; m0 += 16 * WG_WAVES * WG_TURNS) {
+    f32x4 a[WG_TURNS], d[WG_TURNS];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int m = m0 + 4 * g + t;
-      const bool mok = m < M;
-      const float a = (rok && mok) ? A[(size_t)m * NI + row] : 0.f;
-      const float d = (cok && mok) ? D[(size_t)m * NO + col] : 0.f;
-      cs += d;
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, d, acc[t], 0, 0, 0);
+    for (int u = 0; u < WG_TURNS; ++u)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int m = m0 + 16 * WG_WAVES * u + 4 * g + t;
+        const size_t mm = m < M ? m : 0;
+        a[u][t] = Ar[mm * NI];
+        d[u][t] = Dc[mm * NO];
+      }
+#pragma unroll
+    for (int u = 0; u < WG_TURNS; ++u) {
+      if (m0 + 16 * WG_WAVES * u >= M) break;  // uniform over the wave
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const bool mok = m0 + 16 * WG_WAVES * u + 4 * g + t < M;
+        const float av = rok && mok ? a[u][t] : 0.f, dv = cok && mok ? d[u][t] : 0.f;
+        cs += dv;
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, dv, acc[t], 0, 0, 0);
+      }
     }
   }
 #pragma unroll
   for (int v = 0; v < 4; ++v) part[w][v][lane] = (acc[0][v] + acc[1][v]) + (acc[2][v] + acc[3][v]);
   part[w][4][lane] = cs;
   __syncthreads();
-  if (w != 0) return;
-  float s[5];
+  if (w > 4) return;
+  float gg = 0.f;
 #pragma unroll
-  for (int v = 0; v < 5; ++v) {
-    s[v] = 0.f;
-    for (int u = 0; u < WG_WAVES; ++u) s[v] += part[u][v][lane];
+  for (int u = 0; u < WG_WAVES; ++u) gg += part[u][w][lane];
+  int t;
+  bool ok;
+  if (w < 4) {
+    const int r = 16 * tm + 4 * g + w;
+    ok = cok && r < NI;
+    t = pw + r * NO + col;
+  } else {
+    // the column sum: the four lane groups hold sums over disjoint samples (all lanes take part)
+    gg += __shfl_xor(gg, 16, 64);
+    gg += __shfl_xor(gg, 32, 64);
+    ok = cok && tm == 0 && g == 0;
+    t = pb + col;
   }
-  // the column sum: the four lane groups hold sums over disjoint samples (all lanes take part)
-  float c = s[4];
-  c += __shfl_xor(c, 16, 64);
-  c += __shfl_xor(c, 32, 64);
-  if (!cok) return;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int r = 16 * tm + 4 * g + v;
-    if (r < NI) G[(size_t)r * NO + col] = s[v];
+  if (!ok) return;
+  if (!ad.m) {
+    grad[t] = gg;
+    return;
   }
-  if (gb && tm == 0 && g == 0) gb[col] = c;
+  const float mm = ad.b1 * ad.m[t] + (1.f - ad.b1) * gg;
+  const float vv = ad.b2 * ad.v[t] + (1.f - ad.b2) * gg * gg;
+  ad.m[t] = mm;
+  ad.v[t] = vv;
+  p[t] -= ad.lr * (mm / ad.c1) / (sqrtf(vv / ad.c2) + ad.eps);
 }
 
-// softmax cross-entropy over NOUT logits: P, per-sample loss, dZ = (P - onehot) * scale
-__global__ void k_softmax_xent(int M, const float *__restrict__ Z, const int *__restrict__ lab, float *__restrict__ P,
-                               float *__restrict__ loss, float *__restrict__ dZ, float scale) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= M) return;
-  const float *z = Z + (size_t)i * NOUT;
-  float mx = z[0];
-  for (int k = 1; k < NOUT; ++k) mx = fmaxf(mx, z[k]);
-  float e[NOUT], s = 0.f;
-  for (int k = 0; k < NOUT; ++k) {
-    e[k] = expf(z[k] - mx);
-    s += e[k];
-  }
-  for (int k = 0; k < NOUT; ++k) {
-    const float p = e[k] / s;
-    if (P) P[(size_t)i * NOUT + k] = p;
-    if (dZ) dZ[(size_t)i * NOUT + k] = (p - (lab && lab[i] == k ? 1.f : 0.f)) * scale;
-  }
-  if (loss && lab) loss[i] = -(z[lab[i]] - mx - logf(s));
-}
-
-__global__ void k_adam(int n, float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
-                       float *__restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const float gg = g[t];
-  const float mm = b1 * m[t] + (1.f - b1) * gg;
-  const float vv = b2 * v[t] + (1.f - b2) * gg * gg;
-  m[t] = mm;
-  v[t] = vv;
-  p[t] -= lr * (mm / c1) / (sqrtf(vv / c2) + eps);
-}
-
-__global__ void k_gather(int M, const int *__restrict__ idx, const float *__restrict__ F, const int *__restrict__ L,
-                         float *__restrict__ Fo, int *__restrict__ Lo) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= M) return;
-  const int j = idx[i];
-  for (int k = 0; k < NIN; ++k) Fo[(size_t)i * NIN + k] = F[(size_t)j * NIN + k];
-  Lo[i] = L[j];
-}
-
-// Buffers of one forward/backward pass on a minibatch of at most B samples.
+// Buffers of one forward/backward pass on a minibatch of at most b samples.
 struct MlpWork {
-  DevBuf<float> Z1, H1, Z2, H2, Z3, H3, Z4, P, dZ4, dH, dZb, loss;
-  int B = 0;
+  DevBuf<float> buf;
+  MlpAct act{};
   int alloc(andr_ctx *ctx, int b) {
-    B = b;
-    for (DevBuf<float> *h : {&Z1, &H1, &Z2, &H2, &Z3, &H3, &dH, &dZb})
-      if (h->alloc((size_t)b * NH, ctx)) return 1;
-    for (DevBuf<float> *o : {&Z4, &P, &dZ4})
-      if (o->alloc((size_t)b * NOUT, ctx)) return 1;
-    if (loss.alloc(b, ctx)) return 1;
+    const size_t B = ((size_t)b + 3) / 4 * 4;
+    if (buf.alloc(B * (NIN + 6 * NH + NOUT), ctx)) return 1;
+    float *q = buf.p;
+    for (float **h : {&act.H1, &act.H2, &act.H3, &act.D1, &act.D2, &act.D3}) {
+      *h = q;
+      q += B * NH;
+    }
+    act.D4 = q;
+    act.X = q + B * NOUT;
     return 0;
   }
 };
 
-void sgemm(hipStream_t st, int M, int N, int K, const float *A, int lda, int ta, const float *B, int ldb, int tb,
-           float *Z, int ldz, const float *bias = nullptr, float *H = nullptr, const float *mask = nullptr) {
-  const int tiles = ((M + 15) / 16) * ((N + 15) / 16);
-  hipLaunchKernelGGL(k_sgemm, dim3((tiles + 3) / 4), dim3(256), 0, st, M, N, K, A, lda, ta, B, ldb, tb, Z, ldz, bias, H,
-                     mask);
-}
+// blocks of k_mlp: more tiles than four blocks per CU share the weights in a block's registers
+int mlp_blocks(int M) { return std::min((M + 15) / 16, 1024); }
 
-void wgrad(hipStream_t st, int M, int NI, int NO, const float *A, const float *D, float *G, float *gb) {
-  const int tiles = ((NI + 15) / 16) * ((NO + 15) / 16);
-  hipLaunchKernelGGL(k_wgrad, dim3(tiles), dim3(64 * WG_WAVES), 0, st, M, NI, NO, A, D, G, gb);
-}
-
-// forward pass of M samples (X: M x NIN) with parameters p: Z_l = H_(l-1) W_l + b_l, H_l = relu(Z_l)
-void mlp_forward(hipStream_t st, int M, const float *X, const float *p, MlpWork &w) {
-  sgemm(st, M, NH, NIN, X, NIN, 0, p + P_W1, NH, 0, w.Z1.p, NH, p + P_B1, w.H1.p);
-  sgemm(st, M, NH, NH, w.H1.p, NH, 0, p + P_W2, NH, 0, w.Z2.p, NH, p + P_B2, w.H2.p);
-  sgemm(st, M, NH, NH, w.H2.p, NH, 0, p + P_W3, NH, 0, w.Z3.p, NH, p + P_B3, w.H3.p);
-  sgemm(st, M, NOUT, NH, w.H3.p, NH, 0, p + P_W4, NOUT, 0, w.Z4.p, NOUT, p + P_B4);
-}
-
-// backward of the mean cross-entropy: grad (NPARAM) from a forward pass already in w
-void mlp_backward(hipStream_t st, int M, const float *X, const int *lab, const float *p, MlpWork &w, float *grad) {
-  hipLaunchKernelGGL(k_softmax_xent, dim3((M + 255) / 256), dim3(256), 0, st, M, w.Z4.p, lab, w.P.p, w.loss.p,
-                     w.dZ4.p, 1.f / (float)M);
-  // layer 4, then the gradient through W4 and the ReLU of layer 3
-  wgrad(st, M, NH, NOUT, w.H3.p, w.dZ4.p, grad + P_W4, grad + P_B4);
-  sgemm(st, M, NH, NOUT, w.dZ4.p, NOUT, 0, p + P_W4, NOUT, 1, w.dH.p, NH, nullptr, nullptr, w.Z3.p);
-  // layer 3
-  wgrad(st, M, NH, NH, w.H2.p, w.dH.p, grad + P_W3, grad + P_B3);
-  sgemm(st, M, NH, NH, w.dH.p, NH, 0, p + P_W3, NH, 1, w.dZb.p, NH, nullptr, nullptr, w.Z2.p);
-  // layer 2
-  wgrad(st, M, NH, NH, w.H1.p, w.dZb.p, grad + P_W2, grad + P_B2);
-  sgemm(st, M, NH, NH, w.dZb.p, NH, 0, p + P_W2, NH, 1, w.dH.p, NH, nullptr, nullptr, w.Z1.p);
-  // layer 1
-  wgrad(st, M, NIN, NH, X, w.dH.p, grad + P_W1, grad + P_B1);
+// loss and gradients of the mean cross-entropy over M samples, then the step of `ad` (or the gradient out)
+void mlp_step(hipStream_t st, int M, const int *idx, const float *X, const int *lab, float *p, MlpWork &w,
+              float *loss, float *grad, const AdamStep &ad) {
+  hipLaunchKernelGGL(k_mlp<true>, dim3(mlp_blocks(M)), dim3(256), 0, st, M, idx, X, lab, p, (float *)nullptr, loss,
+                     w.act, 1.f / (float)M);
+  hipLaunchKernelGGL(k_mlp_update, dim3(WG_BLOCKS), dim3(64 * WG_WAVES), 0, st, M, w.act, p, grad, ad);
 }
 
 // ---- inference inside the assembly: BF16 matrix cores, FP32 accumulation --------------------------
@@ -728,20 +814,19 @@ extern "C" int andr_mlp_loss_grad(andr_ctx *ctx, int64_t npairs, const float *fe
   for (int64_t i = 0; i < npairs; ++i)
     if (labels[i] < 0 || labels[i] >= NOUT) return andr_fail(ctx, ANDR_ERR_ARG, "label out of range");
   MlpWork w;
-  DevBuf<float> X, p, gr;
+  DevBuf<float> X, p, gr, dloss;
   DevBuf<int> L;
   if (w.alloc(ctx, M) || X.alloc((size_t)M * NIN, ctx) || p.alloc(NPARAM, ctx) || gr.alloc(NPARAM, ctx) ||
-      L.alloc(M, ctx))
+      dloss.alloc(M, ctx) || L.alloc(M, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "MLP buffers");
   hipStream_t st = ctx->stream;
   ANDR_HIP(ctx, hipMemcpyAsync(X.p, features, sizeof(float) * M * NIN, hipMemcpyHostToDevice, st));
   ANDR_HIP(ctx, hipMemcpyAsync(L.p, labels, sizeof(int) * M, hipMemcpyHostToDevice, st));
   ANDR_HIP(ctx, hipMemcpyAsync(p.p, params, sizeof(float) * NPARAM, hipMemcpyHostToDevice, st));
-  mlp_forward(st, M, X.p, p.p, w);
-  mlp_backward(st, M, X.p, L.p, p.p, w, gr.p);
+  mlp_step(st, M, nullptr, X.p, L.p, p.p, w, dloss.p, gr.p, AdamStep{});
   ANDR_HIP(ctx, hipGetLastError());
   std::vector<float> hl(M);
-  ANDR_HIP(ctx, hipMemcpyAsync(hl.data(), w.loss.p, sizeof(float) * M, hipMemcpyDeviceToHost, st));
+  ANDR_HIP(ctx, hipMemcpyAsync(hl.data(), dloss.p, sizeof(float) * M, hipMemcpyDeviceToHost, st));
   ANDR_HIP(ctx, hipMemcpyAsync(grad, gr.p, sizeof(float) * NPARAM, hipMemcpyDeviceToHost, st));
   ANDR_HIP(ctx, hipStreamSynchronize(st));
   double s = 0.0;
@@ -755,20 +840,18 @@ extern "C" int andr_mlp_infer(andr_ctx *ctx, int64_t npairs, const float *featur
     return ctx ? andr_fail(ctx, ANDR_ERR_ARG, "andr_mlp_infer arguments") : ANDR_ERR_ARG;
   ANDR_HIP(ctx, hipSetDevice(ctx->device));
   const int chunk = 1 << 16;
-  MlpWork w;
-  DevBuf<float> X, p;
-  if (w.alloc(ctx, chunk) || X.alloc((size_t)chunk * NIN, ctx) || p.alloc(NPARAM, ctx))
+  DevBuf<float> X, p, P;
+  if (P.alloc((size_t)chunk * NOUT, ctx) || X.alloc((size_t)chunk * NIN, ctx) || p.alloc(NPARAM, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "MLP buffers");
   hipStream_t st = ctx->stream;
   ANDR_HIP(ctx, hipMemcpyAsync(p.p, params, sizeof(float) * NPARAM, hipMemcpyHostToDevice, st));
   for (int64_t i0 = 0; i0 < npairs; i0 += chunk) {
     const int M = (int)std::min<int64_t>(chunk, npairs - i0);
     ANDR_HIP(ctx, hipMemcpyAsync(X.p, features + i0 * NIN, sizeof(float) * M * NIN, hipMemcpyHostToDevice, st));
-    mlp_forward(st, M, X.p, p.p, w);
-    hipLaunchKernelGGL(k_softmax_xent, dim3((M + 255) / 256), dim3(256), 0, st, M, w.Z4.p, (const int *)nullptr, w.P.p,
-                       (float *)nullptr, (float *)nullptr, 1.f);
+    hipLaunchKernelGGL(k_mlp<false>, dim3(mlp_blocks(M)), dim3(256), 0, st, M, (const int *)nullptr, X.p,
+                       (const int *)nullptr, p.p, P.p, (float *)nullptr, MlpAct{}, 1.f);
     ANDR_HIP(ctx, hipGetLastError());
-    ANDR_HIP(ctx, hipMemcpyAsync(probs + i0 * NOUT, w.P.p, sizeof(float) * M * NOUT, hipMemcpyDeviceToHost, st));
+    ANDR_HIP(ctx, hipMemcpyAsync(probs + i0 * NOUT, P.p, sizeof(float) * M * NOUT, hipMemcpyDeviceToHost, st));
     ANDR_HIP(ctx, hipStreamSynchronize(st));
   }
   return ANDR_OK;
@@ -782,12 +865,12 @@ extern "C" int andr_mlp_train(andr_ctx *ctx, int64_t npairs, const float *featur
   for (int64_t i = 0; i < npairs; ++i)
     if (labels[i] < 0 || labels[i] >= NOUT) return andr_fail(ctx, ANDR_ERR_ARG, "label out of range");
   const int N = (int)npairs, B = std::min<int>(batch, N);
+  const int steps = N / B, samples = (steps + 15) / 16;  // the loss of every 16th minibatch of an epoch is kept
   MlpWork w;
-  DevBuf<float> X, Xb, p, gr, m, v, lossacc;
-  DevBuf<int> L, Lb, idx;
-  if (w.alloc(ctx, B) || X.alloc((size_t)N * NIN, ctx) || Xb.alloc((size_t)B * NIN, ctx) ||
-      p.alloc(NPARAM, ctx) || gr.alloc(NPARAM, ctx) || m.alloc(NPARAM, ctx) || v.alloc(NPARAM, ctx) ||
-      L.alloc(N, ctx) || Lb.alloc(B, ctx) || idx.alloc(N, ctx))
+  DevBuf<float> X, p, m, v, loss;
+  DevBuf<int> L, idx;
+  if (w.alloc(ctx, B) || X.alloc((size_t)N * NIN, ctx) || p.alloc(NPARAM, ctx) || m.alloc(NPARAM, ctx) ||
+      v.alloc(NPARAM, ctx) || loss.alloc((size_t)(samples + 1) * B, ctx) || L.alloc(N, ctx) || idx.alloc(N, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "MLP training buffers");
   hipStream_t st = ctx->stream;
   ANDR_HIP(ctx, hipMemcpyAsync(X.p, features, sizeof(float) * (size_t)N * NIN, hipMemcpyHostToDevice, st));
@@ -797,34 +880,30 @@ extern "C" int andr_mlp_train(andr_ctx *ctx, int64_t npairs, const float *featur
   ANDR_HIP(ctx, hipMemsetAsync(v.p, 0, sizeof(float) * NPARAM, st));
   std::mt19937_64 rng(seed);
   std::vector<int> perm(N);
-  std::vector<float> hl(B);
+  std::vector<float> hl((size_t)samples * B);
   int64_t t = 0;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   for (int ep = 0; ep < epochs; ++ep) {
     std::iota(perm.begin(), perm.end(), 0);
     std::shuffle(perm.begin(), perm.end(), rng);
     ANDR_HIP(ctx, hipMemcpyAsync(idx.p, perm.data(), sizeof(int) * N, hipMemcpyHostToDevice, st));
-    double lsum = 0.0;
-    int nb = 0;
-    for (int i0 = 0; i0 + B <= N; i0 += B) {
-      hipLaunchKernelGGL(k_gather, dim3((B + 255) / 256), dim3(256), 0, st, B, idx.p + i0, X.p, L.p, Xb.p, Lb.p);
-      mlp_forward(st, B, Xb.p, p.p, w);
-      mlp_backward(st, B, Xb.p, Lb.p, p.p, w, gr.p);
+    for (int b = 0; b < steps; ++b) {
       ++t;
       const float c1 = 1.f - powf(b1, (float)t), c2 = 1.f - powf(b2, (float)t);
-      hipLaunchKernelGGL(k_adam, dim3((NPARAM + 255) / 256), dim3(256), 0, st, NPARAM, p.p, gr.p, m.p, v.p, lr, b1, b2,
-                         eps, c1, c2);
-      if ((nb & 15) == 0) {  // sample the loss every 16 minibatches
-        ANDR_HIP(ctx, hipMemcpyAsync(hl.data(), w.loss.p, sizeof(float) * B, hipMemcpyDeviceToHost, st));
-        ANDR_HIP(ctx, hipStreamSynchronize(st));
-        double s = 0.0;
-        for (float x : hl) s += x;
-        lsum += s / B;
-      }
-      ++nb;
+      float *bl = loss.p + (size_t)((b & 15) == 0 ? b / 16 : samples) * B;
+      mlp_step(st, B, idx.p + (size_t)b * B, X.p, L.p, p.p, w, bl, nullptr,
+               AdamStep{m.p, v.p, lr, b1, b2, eps, c1, c2});
     }
     ANDR_HIP(ctx, hipGetLastError());
-    if (loss_out) loss_out[ep] = (float)(lsum / std::max(1, (nb + 15) / 16));
+    ANDR_HIP(ctx, hipMemcpyAsync(hl.data(), loss.p, sizeof(float) * hl.size(), hipMemcpyDeviceToHost, st));
+    ANDR_HIP(ctx, hipStreamSynchronize(st));
+    double lsum = 0.0;
+    for (int b = 0; b < samples; ++b) {
+      double s = 0.0;
+      for (int i = 0; i < B; ++i) s += hl[(size_t)b * B + i];
+      lsum += s / B;
+    }
+    if (loss_out) loss_out[ep] = (float)(lsum / std::max(1, samples));
   }
   ANDR_HIP(ctx, hipMemcpyAsync(params, p.p, sizeof(float) * NPARAM, hipMemcpyDeviceToHost, st));
   ANDR_HIP(ctx, hipStreamSynchronize(st));
