@@ -36,6 +36,7 @@
 #include <cmath>
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -178,8 +179,14 @@ __device__ inline void lsqr_u_scales(const LsqrState &S, double sv, double &sx, 
   }
 }
 
-template <int WD>
-__device__ inline bool any_active(const LsqrState *st) {
+// BiCGSTAB's column state
+struct BicgState {
+  double rho, alpha, omega, bnorm2, tol2, a;  // a: alpha of this iteration (0 for a column that stopped)
+  int active, itn, status;  // status: 0 converged, 1 iteration limit, 2 breakdown
+};
+
+template <int WD, class State>
+__device__ inline bool any_active(const State *st) {
   int a = 0;
 #pragma unroll
   for (int k = 0; k < WD; ++k) a |= st[k].active;
@@ -236,9 +243,12 @@ __device__ inline void lsqr_end_block(const LsqrVecs &L, double *red, LsqrState 
 // upper half c >= NB is zero). The result D[g + 4 v][c] sits in register v of lane (g, c).
 // The tiles are read in whole 128-byte row segments and redistributed to the matrix-core layout
 // through LDS (rows padded to 18 doubles): the matrix-core lane pattern itself covers 16 half lines a
-// load, measured 4.6-5.3 against 6.9 TB/s on a 30 GB matrix. VEC: 16-byte loads (lane = row rr =
-// lane / 8 of an 8-row half tile, columns 2 p, 2 p + 1); otherwise (odd row length or an 8-byte base)
-// 8-byte loads, four rows of 16 columns each (3841^2: 46.8 -> 32.7 us).
+// load, measured 4.6-5.3 against 6.9 TB/s on a 30 GB matrix. Lane = row rr = lane / 8 of an 8-row half
+// tile, columns 2 p, 2 p + 1. LINES: every row starts on a 128-byte line. Otherwise a segment that
+// starts at a row's own column 16 kb lies across two lines, and every line is asked for twice (3841^2: 31.8 us
+// against 22.4 for 3840^2, with 8- and with 16-byte loads); so the lines themselves are read and put
+// side by side in LDS, where row c's block kb starts sh(c) columns into line kb: 26 us. The first and last full
+// blocks of a wave's columns, whose lines may reach past the matrix, are then read in the lane pattern.
 // The column split depends on the matrix shape only, and every row's sum runs over its columns in the
 // same order for every T, so the tile count (chosen by size or by the autotuner) never changes a bit.
 constexpr int AV_WAVES = 8;
@@ -246,78 +256,80 @@ constexpr int AV_MAXCOLS = 1024;  // columns per wave at most
 
 // SEP: the waves' sums stay apart, P[segment * AV_WAVES + wave] (BiCGSTAB, whose iterates part from
 // each other by far more than rounding when the sums of a product are formed in another order).
-template <int T, bool VEC, bool SEP>
+template <int T, bool LINES, bool SEP>
 __global__ __launch_bounds__(64 * AV_WAVES) void k_lsqr_av(const double *__restrict__ A, int64_t lda, int m, int n,
                                                            const double *__restrict__ X, int wcols,
-                                                           double *__restrict__ P, const LsqrState *__restrict__ st) {
+                                                           double *__restrict__ P,
+                                                           const std::conditional_t<SEP, BicgState, LsqrState> *__restrict__ st) {
   const bool act = !st || any_active<NB>(st);
+  if (!LINES && !act) return;  // uniform over the grid
   typedef const double __attribute__((address_space(1))) *gdp;
-  constexpr int LR = 18;
+  constexpr int LR = LINES ? 18 : 34;
   __shared__ __attribute__((aligned(16))) double lt[AV_WAVES][T][16 * LR];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int row0 = blockIdx.x * 16 * T;
   const int g = lane >> 4, c = lane & 15;
   const bool hi = c >= NB;
   const int k0 = (blockIdx.y * AV_WAVES + wid) * wcols, kend = min(n, k0 + wcols);
-  gdp lrow[T][VEC ? 2 : 4];
+  gdp lrow[T][2];
+  int sh[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) {
-    if (VEC) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-        lrow[t][h] = (gdp)(A + (size_t)min(row0 + 16 * t + 8 * h + (lane >> 3), m - 1) * lda + 2 * (lane & 7));
-    } else {
-#pragma unroll
-      for (int h = 0; h < 4; ++h) lrow[t][h] = (gdp)(A + (size_t)min(row0 + 16 * t + 4 * h + g, m - 1) * lda + c);
+    for (int h = 0; h < 2; ++h) {
+      const uintptr_t r = (uintptr_t)(A + (size_t)min(row0 + 16 * t + 8 * h + (lane >> 3), m - 1) * lda);
+      lrow[t][h] = (gdp)(LINES ? r : r & ~(uintptr_t)127) + 2 * (lane & 7);
     }
+    sh[t] = LINES ? 0 : (int)((uintptr_t)(A + (size_t)min(row0 + 16 * t + c, m - 1) * lda) >> 3 & 15);
   }
   const gdp xb = (gdp)(X + (size_t)(4 * g) * NB + (c & (NB - 1)));
   d4v acc[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) acc[t] = d4v{0.0, 0.0, 0.0, 0.0};
-  // raw operands of one 16-column block; the matrix is streamed: non-temporal, so that X keeps its place in L2
+  // the matrix is streamed: non-temporal, so that X keeps its place in L2
+  auto lines = [&](int j, double (&a)[T][4]) {
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const d2n u = __builtin_nontemporal_load((const d2n __attribute__((address_space(1))) *)(lrow[t][h] + 16 * j));
+        a[t][2 * h] = u.x;
+        a[t][2 * h + 1] = u.y;
+      }
+  };
+  // raw operands of one 16-column block (its second line, if it has two)
   auto load = [&](int kb, double (&a)[T][4], double (&x)[4]) {
+    lines(LINES ? kb : kb + 1, a);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x[s] = xb[(size_t)(16 * kb + s) * NB];
+  };
+  auto put = [&](int j, const double (&a)[T][4]) {
+    const int rr = lane >> 3, p = (LINES ? 0 : 16 * (j & 1)) + 2 * (lane & 7);
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-      if constexpr (VEC) {
-        const d2n u = __builtin_nontemporal_load((const d2n __attribute__((address_space(1))) *)(lrow[t][0] + 16 * kb));
-        const d2n w = __builtin_nontemporal_load((const d2n __attribute__((address_space(1))) *)(lrow[t][1] + 16 * kb));
+      double *l = lt[wid][t];
+      *(d2n *)&l[rr * LR + p] = d2n{a[t][0], a[t][1]};
+      *(d2n *)&l[(8 + rr) * LR + p] = d2n{a[t][2], a[t][3]};
+    }
+  };
+  // row segments -> LDS -> matrix-core values (in place); the tiles are per wave
+  auto stage = [&](int kb, double (&a)[T][4]) {
+    put(LINES ? kb : kb + 1, a);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const double *l = &lt[wid][t][c * LR];
+      if constexpr (LINES) {
+        const d2n u = *(const d2n *)&l[4 * g], w = *(const d2n *)&l[4 * g + 2];
         a[t][0] = u.x;
         a[t][1] = u.y;
         a[t][2] = w.x;
         a[t][3] = w.y;
       } else {
 #pragma unroll
-        for (int h = 0; h < 4; ++h) a[t][h] = __builtin_nontemporal_load(lrow[t][h] + 16 * kb);
+        for (int s = 0; s < 4; ++s) a[t][s] = l[(16 * (kb & 1) + sh[t] + 4 * g + s) & 31];
       }
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s) x[s] = xb[(size_t)(16 * kb + s) * NB];
-  };
-  // row segments -> LDS -> matrix-core values (in place); the tiles are per wave
-  auto stage = [&](double (&a)[T][4]) {
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      double *l = lt[wid][t];
-      if constexpr (VEC) {
-        const int rr = lane >> 3, p = lane & 7;
-        *(d2n *)&l[rr * LR + 2 * p] = d2n{a[t][0], a[t][1]};
-        *(d2n *)&l[(8 + rr) * LR + 2 * p] = d2n{a[t][2], a[t][3]};
-      } else {
-#pragma unroll
-        for (int h = 0; h < 4; ++h) l[(4 * h + g) * LR + c] = a[t][h];
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      const d2n u = *(const d2n *)&lt[wid][t][c * LR + 4 * g];
-      const d2n w = *(const d2n *)&lt[wid][t][c * LR + 4 * g + 2];
-      a[t][0] = u.x;
-      a[t][1] = u.y;
-      a[t][2] = w.x;
-      a[t][3] = w.y;
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -330,34 +342,8 @@ __global__ __launch_bounds__(64 * AV_WAVES) void k_lsqr_av(const double *__restr
       for (int t = 0; t < T; ++t) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t][s], b, acc[t], 0, 0, 0);
     }
   };
-  // full 16-column blocks, two register sets in turn: the operands of the next block are requested
-  // before the products of the current one (the last prefetch re-reads the final block)
-  int kb = k0 >> 4;
-  const int kb_end = kend >> 4;
-  if (kb < kb_end) {
-    double a0[T][4], a1[T][4], x0[4], x1[4];
-    load(kb, a0, x0);
-    if (!act) return;  // uniform over the grid; the first loads are under way while the state arrives
-    for (; kb + 1 < kb_end; kb += 2) {
-      load(kb + 1, a1, x1);
-      __builtin_amdgcn_sched_barrier(0);
-      stage(a0);
-      step(a0, x0);
-      __builtin_amdgcn_sched_barrier(0);
-      load(min(kb + 2, kb_end - 1), a0, x0);
-      __builtin_amdgcn_sched_barrier(0);
-      stage(a1);
-      step(a1, x1);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (kb < kb_end) {  // odd count: a0 holds block kb
-      stage(a0);
-      step(a0, x0);
-      ++kb;
-    }
-  }
-  if (!act) return;
-  if (16 * kb < kend) {  // last, partial column block of the matrix: masked
+  // one block in the lane pattern of the products, masked at the matrix's last column
+  auto direct = [&](int kb) {
     double a[T][4], x[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -368,7 +354,43 @@ __global__ __launch_bounds__(64 * AV_WAVES) void k_lsqr_av(const double *__restr
       for (int t = 0; t < T; ++t) a[t][s] = in ? A[(size_t)min(row0 + 16 * t + c, m - 1) * lda + col] : 0.0;
     }
     step(a, x);
+  };
+  int kb = k0 >> 4, kb_end = kend >> 4;
+  const int kb_all = (kend + 15) >> 4;
+  if (!LINES && kb < kb_end) {
+    direct(kb++);
+    --kb_end;
   }
+  // full 16-column blocks, two register sets in turn: the operands of the next block are requested
+  // before the products of the current one (the last prefetch re-reads the final block)
+  if (kb < kb_end) {
+    double a0[T][4], a1[T][4], x0[4], x1[4];
+    if (!LINES) {
+      lines(kb, a1);
+      put(kb, a1);
+    }
+    load(kb, a0, x0);
+    if (!act) return;  // uniform over the grid; the first loads are under way while the state arrives
+    for (; kb + 1 < kb_end; kb += 2) {
+      load(kb + 1, a1, x1);
+      __builtin_amdgcn_sched_barrier(0);
+      stage(kb, a0);
+      step(a0, x0);
+      __builtin_amdgcn_sched_barrier(0);
+      load(min(kb + 2, kb_end - 1), a0, x0);
+      __builtin_amdgcn_sched_barrier(0);
+      stage(kb + 1, a1);
+      step(a1, x1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (kb < kb_end) {  // odd count: a0 holds block kb
+      stage(kb, a0);
+      step(a0, x0);
+      ++kb;
+    }
+  }
+  if (!act) return;
+  for (; kb < kb_all; ++kb) direct(kb);
   if (SEP) {
     if (k0 < n) {
       double *p = P + (size_t)(blockIdx.y * AV_WAVES + wid) * m * NB;
@@ -862,16 +884,6 @@ __global__ void k_lsqr_finish(int n, const double *__restrict__ q, const double 
   *px = (q ? q[j] * x : x) + *px;
 }
 
-// Y = sum_s P[s]: a product on its own (BiCGSTAB)
-__global__ __launch_bounds__(256) void k_combine_n(int m, int nseg, const double *__restrict__ P,
-                                                   double *__restrict__ Y) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;  // one (row, k) pair per thread
-  if (t >= m * NB) return;
-  double s = 0.0;
-  for (int sg = 0; sg < nseg; ++sg) s += P[(size_t)sg * m * NB + t];
-  Y[t] = s;
-}
-
 // ---- sparse products (CSR) -----------------------------------------------------------------------
 // y = A x, 0-based row pointers and columns: eight lanes per row take its entries in turn, their sums
 // meet in a fixed order. For one right-hand side (the Fortran seam has one).
@@ -980,23 +992,21 @@ int av_tiles(int m, int nseg) { return (m + 63) / 64 * nseg < 512 ? 2 : 4; }
 // A X into the segment partials P (FP64, NB interleaved columns)
 template <int T, bool SEP>
 void launch_av_t(hipStream_t st, const double *A, int64_t lda, int m, int n, const double *X, AvShape sh, double *P,
-                 const LsqrState *s) {
-  const dim3 blk(64 * AV_WAVES);
-  if (lda % 2 == 0 && ((uintptr_t)A % 16) == 0) {
-    hipLaunchKernelGGL((k_lsqr_av<T, true, SEP>), dim3((m + 16 * T - 1) / (16 * T), sh.nseg), blk, 0, st, A, lda, m, n, X,
-                       sh.wcols, P, s);
-  } else {
-    constexpr int U = T < 4 ? T : 4;  // eight tiles of 8-byte loads do not fit the registers
-    hipLaunchKernelGGL((k_lsqr_av<U, false, SEP>), dim3((m + 16 * U - 1) / (16 * U), sh.nseg), blk, 0, st, A, lda, m, n, X,
-                       sh.wcols, P, s);
-  }
+                 const std::conditional_t<SEP, BicgState, LsqrState> *s) {
+  const dim3 grid((m + 16 * T - 1) / (16 * T), sh.nseg), blk(64 * AV_WAVES);
+  if (lda % 16 == 0 && (uintptr_t)A % 128 == 0)
+    hipLaunchKernelGGL((k_lsqr_av<T, true, SEP>), grid, blk, 0, st, A, lda, m, n, X, sh.wcols, P, s);
+  else if constexpr (T <= 4)
+    hipLaunchKernelGGL((k_lsqr_av<T, false, SEP>), grid, blk, 0, st, A, lda, m, n, X, sh.wcols, P, s);
+  else  // two lines of eight tiles do not fit the LDS
+    launch_av_t<4, SEP>(st, A, lda, m, n, X, sh, P, s);
 }
 template <bool SEP>
 void launch_av(hipStream_t st, int tiles, const double *A, int64_t lda, int m, int n, const double *X, AvShape sh,
-               double *P, const LsqrState *s) {
+               double *P, const std::conditional_t<SEP, BicgState, LsqrState> *s) {
   if (tiles == 2) launch_av_t<2, SEP>(st, A, lda, m, n, X, sh, P, s);
   else if (SEP || tiles == 4) launch_av_t<4, SEP>(st, A, lda, m, n, X, sh, P, s);
-  else launch_av_t<8, false>(st, A, lda, m, n, X, sh, P, s);
+  else if constexpr (!SEP) launch_av_t<8, false>(st, A, lda, m, n, X, sh, P, s);
 }
 
 // One LSQR solve, advanced in blocks of iterations on a stream of its own (several solves of a batch
@@ -1368,28 +1378,22 @@ int andr_lsqr_device_batch(andr_ctx *ctx, int count, const LsqrJob *jobs) {
 // scalars; the products are the matrix-core A X above.
 namespace {
 
-struct BicgState {
-  double rho, alpha, omega, bnorm2, tol2;
-  int active, itn, status;  // status: 0 converged, 1 iteration limit, 2 breakdown
-};
-
-// per-block partial sums of X.Y (and of Z.W when Z is given) over n x NB column-interleaved arrays
-__global__ __launch_bounds__(256) void k_bicg_dots(int n, const double *__restrict__ X, const double *__restrict__ Y,
-                                                   const double *__restrict__ Z, const double *__restrict__ W,
-                                                   double *__restrict__ p1, double *__restrict__ p2) {
-  __shared__ double red[2][4 * NB];
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  double a = 0.0, b = 0.0;
-  if (t < n * NB) {
-    a = X[t] * Y[t];
-    if (Z) b = Z[t] * W[t];
-  }
+// An iteration is seven launches (the products two of them): vector kernels over n x NB elements, a thread
+// each, that leave the dot products' partial sums p1 and p2, a pair of rows per block, and begin with the scalar
+// step from the sums of the one before, done by every block alike; one block writes the new states to another
+// array, as the others may still read the old one: S0 -> k_bicg_p -> S1 -> k_bicg_s -> S2 -> k_bicg_x -> S0.
+// Latency of 121 blocks at n = 3841: 13 launches of 2.3 to 4.9 us beside the two products are now five of 4.3 to
+// 4.6; the iterations enqueued past the end return at once. The sums keep the order of separate dot products:
+// the iterates part from each other by far more than rounding where it changes.
+__device__ inline void bicg_parts(double a, double b, double *__restrict__ p1, double *__restrict__ p2,
+                                  double (*red)[4 * NB]) {
 #pragma unroll
   for (int off = 8; off < 64; off <<= 1) {
     a += __shfl_xor(a, off, 64);
     b += __shfl_xor(b, off, 64);
   }
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  __syncthreads();  // red may still be read
   if (lane < NB) {
     red[0][wid * NB + lane] = a;
     red[1][wid * NB + lane] = b;
@@ -1398,8 +1402,22 @@ __global__ __launch_bounds__(256) void k_bicg_dots(int n, const double *__restri
   if (threadIdx.x < NB) {
     const int k = threadIdx.x;
     p1[(size_t)blockIdx.x * NB + k] = (red[0][k] + red[0][NB + k]) + (red[0][2 * NB + k] + red[0][3 * NB + k]);
-    if (Z) p2[(size_t)blockIdx.x * NB + k] = (red[1][k] + red[1][NB + k]) + (red[1][2 * NB + k] + red[1][3 * NB + k]);
+    if (p2) p2[(size_t)blockIdx.x * NB + k] = (red[1][k] + red[1][NB + k]) + (red[1][2 * NB + k] + red[1][3 * NB + k]);
   }
+}
+
+// element t of A X from its segments' partial sums
+__device__ inline double bicg_seg_sum(int64_t nb, int nseg, const double *__restrict__ P, int64_t t) {
+  double s = 0.0;
+  for (int s0 = 0; s0 < nseg; s0 += 8) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = P[(size_t)min(s0 + u, nseg - 1) * nb + t];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (s0 + u < nseg) s += v[u];
+  }
+  return s;
 }
 
 // Jacobi: dinv[j] = 1 / A[j][j] (1 where the diagonal is zero, as a Jacobi preconditioner leaves it)
@@ -1410,145 +1428,51 @@ __global__ void k_bicg_diag(const double *__restrict__ A, int64_t lda, int n, do
   dinv[j] = d != 0.0 ? 1.0 / d : 1.0;
 }
 
-// r = b - A x from Y = A x; r_hat = r; p = v = 0
-__global__ void k_bicg_init(int n, const double *__restrict__ B, const double *__restrict__ AX, double *__restrict__ R,
-                            double *__restrict__ Rh, double *__restrict__ P, double *__restrict__ V) {
+// r = b - A x from the segments of A x; r_hat = r; p = v = 0; partials of b . b and r . r
+__global__ __launch_bounds__(256) void k_bicg_init(int n, const double *__restrict__ B, int nseg,
+                                                   const double *__restrict__ AX, double *__restrict__ R,
+                                                   double *__restrict__ Rh, double *__restrict__ P,
+                                                   double *__restrict__ V, double *__restrict__ pb,
+                                                   double *__restrict__ pr) {
+  __shared__ double red[2][4 * NB];
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * NB) return;
-  const double r = B[t] - AX[t];
-  R[t] = r;
-  Rh[t] = r;
-  P[t] = 0.0;
-  V[t] = 0.0;
+  double bb = 0.0, rr = 0.0;
+  if (t < n * NB) {
+    const double b = B[t], r = b - bicg_seg_sum((int64_t)n * NB, nseg, AX, t);
+    R[t] = r;
+    Rh[t] = r;
+    P[t] = 0.0;
+    V[t] = 0.0;
+    bb = b * b;
+    rr = r * r;
+  }
+  bicg_parts(bb, rr, pb, pr, red);
 }
 
-// start: ||b||^2 and ||r0||^2; columns with r0 already small are done
+// start: ||b||^2 and ||r0||^2; columns with r0 already small are done. rr, rho: r . r and r_hat . r (the same as
+// r_hat = r) for the first iteration
 __global__ void k_bicg_start(BicgState *st, const double *pb, const double *pr, int np, double tol, int nrhs,
-                             double *sc) {
+                             double *rr, double *rho) {
   __shared__ double red[4 * NB];
   const double b2 = block_sum_parts<NB, 256>(pb, np, red);
   const double r2 = block_sum_parts<NB, 256>(pr, np, red);
+  for (int i = threadIdx.x; i < np * NB; i += blockDim.x) rr[i] = rho[i] = pr[i];
   const int k = threadIdx.x;
   if (k >= NB) return;
-  BicgState &S = st[k];
+  BicgState S;
   S.rho = S.alpha = S.omega = 1.0;
+  S.a = 0.0;
   S.bnorm2 = b2;
   S.tol2 = tol * tol * b2;
   S.itn = 0;
   S.status = 0;
   S.active = k < nrhs && r2 > S.tol2 ? 1 : 0;
-  for (int i = 0; i < 6; ++i) sc[i * NB + k] = 0.0;
+  st[k] = S;
 }
 
-// scalar slots sc[i * NB + k]: 0 beta, 1 omega (for p), 2 alpha, 3 omega (for x, r)
-// rho_new = r_hat . r; beta = (rho_new / rho) (alpha / omega)
-__global__ void k_bicg_beta(BicgState *st, const double *part, int np, double *sc) {
-  __shared__ double red[4 * NB];
-  const double rho = block_sum_parts<NB, 256>(part, np, red);
-  const int k = threadIdx.x;
-  if (k >= NB) return;
-  BicgState &S = st[k];
-  if (!S.active) {
-    sc[k] = 0.0;
-    sc[NB + k] = 0.0;
-    return;
-  }
-  if (rho == 0.0) {  // breakdown: r_hat orthogonal to r
-    S.active = 0;
-    S.status = 2;
-    sc[k] = sc[NB + k] = 0.0;
-    return;
-  }
-  S.itn += 1;
-  const double beta = S.itn == 1 ? 0.0 : (rho / S.rho) * (S.alpha / S.omega);
-  S.rho = rho;
-  sc[k] = beta;
-  sc[NB + k] = S.omega;
-}
-
-// p = r + beta (p - omega v); y = dinv .* p
-__global__ void k_bicg_p(int n, const double *__restrict__ R, const double *__restrict__ V, double *__restrict__ P,
-                         double *__restrict__ Yv, const double *__restrict__ dinv, const double *__restrict__ sc,
-                         const BicgState *__restrict__ st) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * NB) return;
-  const int k = t & 7;
-  if (!st[k].active) {
-    Yv[t] = 0.0;
-    return;
-  }
-  const double p = R[t] + sc[k] * (P[t] - sc[NB + k] * V[t]);
-  P[t] = p;
-  Yv[t] = dinv[t >> 3] * p;
-}
-
-// alpha = rho / (r_hat . v)
-__global__ void k_bicg_alpha(BicgState *st, const double *part, int np, double *sc) {
-  __shared__ double red[4 * NB];
-  const double rv = block_sum_parts<NB, 256>(part, np, red);
-  const int k = threadIdx.x;
-  if (k >= NB) return;
-  BicgState &S = st[k];
-  if (!S.active || rv == 0.0) {
-    if (S.active) {
-      S.active = 0;
-      S.status = 2;
-    }
-    sc[2 * NB + k] = 0.0;
-    return;
-  }
-  S.alpha = S.rho / rv;
-  sc[2 * NB + k] = S.alpha;
-}
-
-// x += alpha y; s = r - alpha v (into R); z = dinv .* s
-__global__ void k_bicg_s(int n, double *__restrict__ X, const double *__restrict__ Yv, double *__restrict__ R,
-                         const double *__restrict__ V, double *__restrict__ Z, const double *__restrict__ dinv,
-                         const double *__restrict__ sc) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * NB) return;
-  const int k = t & 7;
-  const double a = sc[2 * NB + k];
-  X[t] += a * Yv[t];
-  const double s = R[t] - a * V[t];
-  R[t] = s;
-  Z[t] = dinv[t >> 3] * s;
-}
-
-// omega = (t . s) / (t . t)
-__global__ void k_bicg_omega(BicgState *st, const double *pts, const double *ptt, int np, double *sc) {
-  __shared__ double red[4 * NB];
-  const double ts = block_sum_parts<NB, 256>(pts, np, red);
-  const double tt = block_sum_parts<NB, 256>(ptt, np, red);
-  const int k = threadIdx.x;
-  if (k >= NB) return;
-  BicgState &S = st[k];
-  if (!S.active || tt == 0.0) {
-    sc[3 * NB + k] = 0.0;
-    return;
-  }
-  S.omega = ts / tt;
-  sc[3 * NB + k] = S.omega;
-}
-
-// x += omega z; r = s - omega t
-__global__ void k_bicg_x(int n, double *__restrict__ X, const double *__restrict__ Z, double *__restrict__ R,
-                         const double *__restrict__ Tv, const double *__restrict__ sc) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * NB) return;
-  const int k = t & 7;
-  const double w = sc[3 * NB + k];
-  X[t] += w * Z[t];
-  R[t] -= w * Tv[t];
-}
-
-// convergence: ||r||^2 <= tol^2 ||b||^2; omega = 0 (with r not small) is a breakdown
-__global__ void k_bicg_check(BicgState *st, const double *part, int np, int itnlim) {
-  __shared__ double red[4 * NB];
-  const double r2 = block_sum_parts<NB, 256>(part, np, red);
-  const int k = threadIdx.x;
-  if (k >= NB) return;
-  BicgState &S = st[k];
+// convergence: ||r||^2 <= tol^2 ||b||^2; omega = 0 (with r not small) is a breakdown. Done again with the same
+// sum it changes nothing: the poll's kernel and the next iteration both begin with it.
+__device__ inline void bicg_check(BicgState &S, double r2, int itnlim) {
   if (!S.active) return;
   if (r2 <= S.tol2) {
     S.active = 0;
@@ -1560,6 +1484,162 @@ __global__ void k_bicg_check(BicgState *st, const double *part, int np, int itnl
     S.active = 0;
     S.status = 1;
   }
+}
+__global__ void k_bicg_check(BicgState *st, const double *rr, int np, int itnlim) {
+  __shared__ double red[4 * NB];
+  const double r2 = block_sum_parts<NB, 256>(rr, np, red);
+  if (threadIdx.x < NB) bicg_check(st[threadIdx.x], r2, itnlim);
+}
+
+// rho_new = r_hat . r; beta = (rho_new / rho) (alpha / omega); p = r + beta (p - omega v); y = dinv .* p
+__global__ __launch_bounds__(256) void k_bicg_p(int n, int np, const double *__restrict__ rr,
+                                                const double *__restrict__ rhop, const double *__restrict__ R,
+                                                const double *__restrict__ V, double *__restrict__ P,
+                                                double *__restrict__ Yv, const double *__restrict__ dinv,
+                                                const BicgState *__restrict__ s0, BicgState *__restrict__ s1,
+                                                int itnlim) {
+  __shared__ double red[4 * NB], sc[2][NB];
+  __shared__ int act[NB];
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, tt = min(t, n * NB - 1);
+  const double r = R[tt], p0 = P[tt], v = V[tt], d = dinv[tt >> 3];
+  const double ps = thread_parts<NB, 256>(rr, np), qs = thread_parts<NB, 256>(rhop, np);
+  const double r2 = block_sum<NB, 256>(ps, red);
+  const double rho = block_sum<NB, 256>(qs, red);
+  if (threadIdx.x < NB) {
+    const int k = threadIdx.x;
+    BicgState S = s0[k];
+    bicg_check(S, r2, itnlim);
+    double beta = 0.0;
+    if (S.active && rho == 0.0) {  // breakdown: r_hat orthogonal to r
+      S.active = 0;
+      S.status = 2;
+    } else if (S.active) {
+      S.itn += 1;
+      beta = S.itn == 1 ? 0.0 : (rho / S.rho) * (S.alpha / S.omega);
+      S.rho = rho;
+    }
+    sc[0][k] = beta;
+    sc[1][k] = S.omega;
+    act[k] = S.active;
+    if (blockIdx.x == gridDim.x - 1) s1[k] = S;
+  }
+  __syncthreads();
+  if (t >= n * NB) return;
+  const int k = t & 7;
+  if (!act[k]) {
+    Yv[t] = 0.0;
+    return;
+  }
+  const double p = r + sc[0][k] * (p0 - sc[1][k] * v);
+  P[t] = p;
+  Yv[t] = d * p;
+}
+
+// v = A y from its segments; partials of r_hat . v
+__global__ __launch_bounds__(256) void k_bicg_v(int n, int nseg, const double *__restrict__ AY,
+                                                const double *__restrict__ Rh, double *__restrict__ V,
+                                                double *__restrict__ p1, const BicgState *__restrict__ st) {
+  __shared__ double red[2][4 * NB];
+  if (!any_active<NB>(st)) return;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  double a = 0.0;
+  if (t < n * NB) {
+    const double v = bicg_seg_sum((int64_t)n * NB, nseg, AY, t);
+    V[t] = v;
+    a = Rh[t] * v;
+  }
+  bicg_parts(a, 0.0, p1, nullptr, red);
+}
+
+// alpha = rho / (r_hat . v); s = r - alpha v (into R); z = dinv .* s
+__global__ __launch_bounds__(256) void k_bicg_s(int n, int np, const double *__restrict__ p1, double *__restrict__ R,
+                                                const double *__restrict__ V, double *__restrict__ Z,
+                                                const double *__restrict__ dinv, const BicgState *__restrict__ s1,
+                                                BicgState *__restrict__ s2) {
+  __shared__ double red[4 * NB], sc[NB];
+  const bool any = any_active<NB>(s1);
+  if (!any && blockIdx.x != gridDim.x - 1) return;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, tt = min(t, n * NB - 1);
+  const double r = R[tt], v = V[tt], d = dinv[tt >> 3];
+  const double rv = block_sum_parts<NB, 256>(p1, np, red);
+  if (threadIdx.x < NB) {
+    const int k = threadIdx.x;
+    BicgState S = s1[k];
+    S.a = 0.0;
+    if (S.active && rv == 0.0) {
+      S.active = 0;
+      S.status = 2;
+    } else if (S.active) {
+      S.alpha = S.a = S.rho / rv;
+    }
+    sc[k] = S.a;
+    if (blockIdx.x == gridDim.x - 1) s2[k] = S;
+  }
+  __syncthreads();
+  if (!any || t >= n * NB) return;
+  const double s = r - sc[t & 7] * v;
+  R[t] = s;
+  Z[t] = d * s;
+}
+
+// t = A z from its segments; partials of t . s and t . t
+__global__ __launch_bounds__(256) void k_bicg_t(int n, int nseg, const double *__restrict__ AZ,
+                                                const double *__restrict__ R, double *__restrict__ Tv,
+                                                double *__restrict__ p1, double *__restrict__ p2,
+                                                const BicgState *__restrict__ st) {
+  __shared__ double red[2][4 * NB];
+  if (!any_active<NB>(st)) return;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  double a = 0.0, b = 0.0;
+  if (t < n * NB) {
+    const double v = bicg_seg_sum((int64_t)n * NB, nseg, AZ, t);
+    Tv[t] = v;
+    a = v * R[t];
+    b = v * v;
+  }
+  bicg_parts(a, b, p1, p2, red);
+}
+
+// omega = (t . s) / (t . t); x += alpha y; x += omega z; r = s - omega t; partials of r . r and r_hat . r
+__global__ __launch_bounds__(256) void k_bicg_x(int n, int np, const double *__restrict__ p1,
+                                                const double *__restrict__ p2, double *__restrict__ X,
+                                                const double *__restrict__ Yv, const double *__restrict__ Z,
+                                                double *__restrict__ R, const double *__restrict__ Tv,
+                                                const double *__restrict__ Rh, double *__restrict__ rr,
+                                                double *__restrict__ rho, const BicgState *__restrict__ s2,
+                                                BicgState *__restrict__ s0) {
+  __shared__ double red[2][4 * NB], sc[2][NB];
+  const bool any = any_active<NB>(s2);
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, tt = min(t, n * NB - 1);
+  const double x0 = X[tt], y = Yv[tt], z = Z[tt], s = R[tt], v = Tv[tt], h = Rh[tt];
+  const double as = thread_parts<NB, 256>(p1, np), bs = thread_parts<NB, 256>(p2, np);
+  const double ts = block_sum<NB, 256>(as, red[0]);
+  const double tp = block_sum<NB, 256>(bs, red[0]);
+  if (threadIdx.x < NB) {
+    const int k = threadIdx.x;
+    BicgState S = s2[k];
+    double om = 0.0;
+    if (S.active && tp != 0.0) S.omega = om = ts / tp;
+    sc[0][k] = S.a;
+    sc[1][k] = om;
+    if (blockIdx.x == gridDim.x - 1) s0[k] = S;
+  }
+  __syncthreads();
+  double a = 0.0, b = 0.0;
+  if (t < n * NB) {
+    const double al = sc[0][t & 7], w = sc[1][t & 7];
+    double x = x0;
+    x += al * y;
+    x += w * z;
+    const double r = s - w * v;
+    if (any) {
+      X[t] = x;
+      R[t] = r;
+    }
+    a = r * r;
+    b = h * r;
+  }
+  if (any) bicg_parts(a, b, rr, rho, red);
 }
 
 }  // namespace
@@ -1580,26 +1660,20 @@ BicgLayout bicg_layout(int n) {
   return L;
 }
 // doubles of each workspace array, in the order they are carved from a caller's region
-void bicg_sizes(int n, size_t sz[15]) {
+void bicg_sizes(int n, size_t sz[12]) {
   const BicgLayout L = bicg_layout(n);
   for (int i = 0; i < 7; ++i) sz[i] = (size_t)n * NB;  // r, r_hat, p, v, y, z, t
   sz[7] = n;                                           // dinv
   sz[8] = (size_t)L.blocksM * NB;                      // p1
   sz[9] = (size_t)L.blocksM * NB;                      // p2
-  sz[10] = NB;                                         // one
-  sz[11] = NB;                                         // zero
-  sz[12] = 6 * NB;                                     // scalars
-  sz[13] = (sizeof(BicgState) * NB + 7) / 8;           // per-column states
-  sz[14] = (size_t)L.nseg * n * NB;                 // A X segment partials
-}
-__global__ void k_fill(size_t n, double v, double *__restrict__ p) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) p[t] = v;
+  sz[10] = 3 * ((sizeof(BicgState) * NB + 7) / 8);     // per-column states S0, S1, S2
+  // A X segment partials; from the end of an iteration to its next product, those of r . r and r_hat . r
+  sz[11] = std::max((size_t)L.nseg * n, 2 * (size_t)L.blocksM) * NB;
 }
 }  // namespace
 
 size_t andr_bicgstab_ws_bytes(int n) {
-  size_t sz[15], tot = 0;
+  size_t sz[12], tot = 0;
   bicg_sizes(n, sz);
   for (size_t v : sz) tot += (v + 31) / 32 * 32;  // every array on a 256-byte boundary
   return tot * sizeof(double);
@@ -1614,68 +1688,53 @@ int andr_bicgstab_device(andr_ctx *ctx, const double *A, int64_t lda, int n, con
   const int tiles = av_tiles(n, (L.nseg + AV_WAVES - 1) / AV_WAVES);
   const int nb = L.blocksM;
   // workspace: the context's memory cache, or carved from the caller's region (no allocation)
-  DevBuf<double> own[15];
-  double *w[15];
-  size_t sz[15];
+  constexpr int NW = 12;
+  DevBuf<double> own[NW];
+  double *w[NW];
+  size_t sz[NW];
   bicg_sizes(n, sz);
   if (ws) {
     if (ws_bytes < andr_bicgstab_ws_bytes(n))
       return andr_fail(ctx, ANDR_ERR_ARG, "BiCGSTAB workspace of %zu bytes, %zu needed (n=%d)", ws_bytes,
                        andr_bicgstab_ws_bytes(n), n);
     double *cur = ws;
-    for (int i = 0; i < 15; ++i) {
-      w[i] = sz[i] ? cur : nullptr;
+    for (int i = 0; i < NW; ++i) {
+      w[i] = cur;
       cur += (sz[i] + 31) / 32 * 32;
     }
   } else {
-    for (int i = 0; i < 15; ++i) {
+    for (int i = 0; i < NW; ++i) {
       if (own[i].alloc(sz[i], ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "BiCGSTAB workspace (n=%d)", n);
       w[i] = own[i].p;
     }
   }
   double *Rr = w[0], *Rh = w[1], *P = w[2], *V = w[3], *Yv = w[4], *Z = w[5], *Tt = w[6], *dinv = w[7], *p1 = w[8],
-         *p2 = w[9], *one = w[10], *zero = w[11], *sc = w[12];
-  BicgState *S = (BicgState *)w[13];
-  double *pn = w[14];
-  // constants and cleared outputs by fill kernels (no host copies, no memset nodes): the products
-  // write out = 1 * (A in) + 0 * out, so their outputs start finite
-  hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, (size_t)NB, 1.0, one);
-  hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, (size_t)NB, 0.0, zero);
-  hipLaunchKernelGGL(k_fill, dim3((n * NB + 255) / 256), dim3(256), 0, st, (size_t)n * NB, 0.0, V);
-  hipLaunchKernelGGL(k_fill, dim3((n * NB + 255) / 256), dim3(256), 0, st, (size_t)n * NB, 0.0, Tt);
-  const int gb = (n * NB + 255) / 256;
-  auto product = [&](const double *in, double *out) {  // out = A in; no profiling records with a caller's workspace
+         *p2 = w[9], *pn = w[11];
+  BicgState *S = (BicgState *)w[10], *S1 = S + NB, *S2 = S + 2 * NB;
+  double *rr = pn, *rho = pn + (size_t)nb * NB;
+  const int gb = nb;
+  auto product = [&](const double *in, const BicgState *s) {  // no profiling records with a caller's workspace
     const int t = ws ? -1 : andr_prof_begin(ctx, "lsqr_gemv_n", (double)n * n * 8.0 + (2.0 + L.nseg) * n * NB * 8.0, 2.0 * n * n * nrhs);
-    launch_av<true>(st, tiles, A, lda, n, n, in, {(L.nseg + AV_WAVES - 1) / AV_WAVES, L.seglen}, pn, nullptr);
-    hipLaunchKernelGGL(k_combine_n, dim3(gb), dim3(256), 0, st, n, L.nseg, pn, out);
+    launch_av<true>(st, tiles, A, lda, n, n, in, {(L.nseg + AV_WAVES - 1) / AV_WAVES, L.seglen}, pn, s);
     andr_prof_end(ctx, t);
   };
   hipLaunchKernelGGL(k_bicg_diag, dim3((n + 255) / 256), dim3(256), 0, st, A, lda, n, dinv);
-  product(X, V);  // A x0
-  hipLaunchKernelGGL(k_bicg_init, dim3(gb), dim3(256), 0, st, n, B, V, Rr, Rh, P, V);
-  hipLaunchKernelGGL(k_bicg_dots, dim3(gb), dim3(256), 0, st, n, B, B, Rr, Rr, p1, p2);
-  hipLaunchKernelGGL(k_bicg_start, dim3(1), dim3(256), 0, st, S, p1, p2, nb, tol, nrhs, sc);
+  product(X, nullptr);  // A x0
+  hipLaunchKernelGGL(k_bicg_init, dim3(gb), dim3(256), 0, st, n, B, L.nseg, pn, Rr, Rh, P, V, p1, p2);
+  hipLaunchKernelGGL(k_bicg_start, dim3(1), dim3(256), 0, st, S, p1, p2, nb, tol, nrhs, rr, rho);
   const int itnlim = maxit > 0 ? maxit : 1000;
   BicgState hs[NB];
   for (int it = 0; it < itnlim;) {
     for (int inner = 0; inner < 8 && it < itnlim; ++inner, ++it) {
-      hipLaunchKernelGGL(k_bicg_dots, dim3(gb), dim3(256), 0, st, n, Rh, Rr, (const double *)nullptr,
-                         (const double *)nullptr, p1, p2);
-      hipLaunchKernelGGL(k_bicg_beta, dim3(1), dim3(256), 0, st, S, p1, nb, sc);
-      hipLaunchKernelGGL(k_bicg_p, dim3(gb), dim3(256), 0, st, n, Rr, V, P, Yv, dinv, sc, S);
-      product(Yv, V);
-      hipLaunchKernelGGL(k_bicg_dots, dim3(gb), dim3(256), 0, st, n, Rh, V, (const double *)nullptr,
-                         (const double *)nullptr, p1, p2);
-      hipLaunchKernelGGL(k_bicg_alpha, dim3(1), dim3(256), 0, st, S, p1, nb, sc);
-      hipLaunchKernelGGL(k_bicg_s, dim3(gb), dim3(256), 0, st, n, X, Yv, Rr, V, Z, dinv, sc);
-      product(Z, Tt);
-      hipLaunchKernelGGL(k_bicg_dots, dim3(gb), dim3(256), 0, st, n, Tt, Rr, Tt, Tt, p1, p2);
-      hipLaunchKernelGGL(k_bicg_omega, dim3(1), dim3(256), 0, st, S, p1, p2, nb, sc);
-      hipLaunchKernelGGL(k_bicg_x, dim3(gb), dim3(256), 0, st, n, X, Z, Rr, Tt, sc);
-      hipLaunchKernelGGL(k_bicg_dots, dim3(gb), dim3(256), 0, st, n, Rr, Rr, (const double *)nullptr,
-                         (const double *)nullptr, p1, p2);
-      hipLaunchKernelGGL(k_bicg_check, dim3(1), dim3(256), 0, st, S, p1, nb, itnlim);
+      hipLaunchKernelGGL(k_bicg_p, dim3(gb), dim3(256), 0, st, n, nb, rr, rho, Rr, V, P, Yv, dinv, S, S1, itnlim);
+      product(Yv, S1);
+      hipLaunchKernelGGL(k_bicg_v, dim3(gb), dim3(256), 0, st, n, L.nseg, pn, Rh, V, p1, S1);
+      hipLaunchKernelGGL(k_bicg_s, dim3(gb), dim3(256), 0, st, n, nb, p1, Rr, V, Z, dinv, S1, S2);
+      product(Z, S2);
+      hipLaunchKernelGGL(k_bicg_t, dim3(gb), dim3(256), 0, st, n, L.nseg, pn, Rr, Tt, p1, p2, S2);
+      hipLaunchKernelGGL(k_bicg_x, dim3(gb), dim3(256), 0, st, n, nb, p1, p2, X, Yv, Z, Rr, Tt, Rh, rr, rho, S2, S);
     }
+    hipLaunchKernelGGL(k_bicg_check, dim3(1), dim3(256), 0, st, S, rr, nb, itnlim);
     ANDR_HIP(ctx, hipGetLastError());
     ANDR_HIP(ctx, hipMemcpyAsync(hs, S, sizeof(hs), hipMemcpyDeviceToHost, st));
     ANDR_HIP(ctx, hipStreamSynchronize(st));
