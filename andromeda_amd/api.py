@@ -390,8 +390,8 @@ class Context:
         nsp = nn + ne
         shapeH = (nsp, nn) if layout == ROW_MAJOR else (nn, nsp)
         shapeG = (nsp, ne) if layout == ROW_MAJOR else (ne, nsp)
-        H = np.zeros(shapeH)
-        G = np.zeros(shapeG)
+        H = np.empty(shapeH)
+        G = np.empty(shapeG)
         err = np.zeros(2)
         self._check(self.lib.andr_assemble_laplace(self.h, C.byref(mv.s), layout, _p(H), _p(G), _p(err)),
                     "andr_assemble_laplace")
@@ -404,8 +404,8 @@ class Context:
         """Rows row_begin .. row_end - 1 of H and G (andr_assemble_laplace_rows)."""
         mv = _MeshView(mesh, normmul, itri, iquad)
         nn, ne, nr = mv.m.nnodes, mv.m.nelem, row_end - row_begin
-        H = np.zeros((nr, nn) if layout == ROW_MAJOR else (nn, nr))
-        G = np.zeros((nr, ne) if layout == ROW_MAJOR else (ne, nr))
+        H = np.empty((nr, nn) if layout == ROW_MAJOR else (nn, nr))
+        G = np.empty((nr, ne) if layout == ROW_MAJOR else (ne, nr))
         err = np.zeros(2)
         self._check(self.lib.andr_assemble_laplace_rows(self.h, C.byref(mv.s), row_begin, row_end, layout, _p(H),
                                                         _p(G), _p(err)), "andr_assemble_laplace_rows")
@@ -418,10 +418,10 @@ class Context:
         """Rows row_begin .. row_end - 1 of the 18 Stokes matrices (andr_assemble_stokes_rows)."""
         mv = _MeshView(mesh, normmul, itri, iquad)
         nn, ne, nr = mv.m.nnodes, mv.m.nelem, row_end - row_begin
-        T = [np.zeros((nr, nn)) for _ in range(6)]
-        G = [np.zeros((nr, ne)) for _ in range(6)]
-        prT = [np.zeros((nr, nn)) for _ in range(3)]
-        prG = [np.zeros((nr, ne)) for _ in range(3)]
+        T = [np.empty((nr, nn)) for _ in range(6)]
+        G = [np.empty((nr, ne)) for _ in range(6)]
+        prT = [np.empty((nr, nn)) for _ in range(3)]
+        prG = [np.empty((nr, ne)) for _ in range(3)]
         err = np.zeros(2)
         self._check(self.lib.andr_assemble_stokes_rows(
             self.h, C.byref(mv.s), row_begin, row_end, ROW_MAJOR, extra, (_D * 6)(*[_p(x) for x in T]),
@@ -480,10 +480,10 @@ class Context:
         mv = _MeshView(mesh, normmul, itri, iquad)
         nn, ne = mv.m.nnodes, mv.m.nelem
         nsp = nn + ne
-        T = [np.zeros((nsp, nn)) for _ in range(6)]
-        G = [np.zeros((nsp, ne)) for _ in range(6)]
-        prT = [np.zeros((nsp, nn)) for _ in range(3)] if pressure else None
-        prG = [np.zeros((nsp, ne)) for _ in range(3)] if pressure else None
+        T = [np.empty((nsp, nn)) for _ in range(6)]
+        G = [np.empty((nsp, ne)) for _ in range(6)]
+        prT = [np.empty((nsp, nn)) for _ in range(3)] if pressure else None
+        prG = [np.empty((nsp, ne)) for _ in range(3)] if pressure else None
         err = np.zeros(2)
         Tp = (_D * 6)(*[_p(x) for x in T])
         Gp = (_D * 6)(*[_p(x) for x in G])

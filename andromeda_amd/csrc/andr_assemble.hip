@@ -1782,19 +1782,22 @@ __global__ void k_transpose(const double *__restrict__ in, double *__restrict__ 
   }
 }
 
-int andr_copy_out(andr_ctx *ctx, const double *d, int64_t m, int64_t n, int32_t layout, double *h) {
-  if (!h) return ANDR_OK;
-  if (layout == ANDR_ROW_MAJOR) {
-    ANDR_HIP(ctx, hipMemcpyAsync(h, d, sizeof(double) * m * n, hipMemcpyDeviceToHost, ctx->stream));
-    ANDR_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return ANDR_OK;
+int andr_copy_out(andr_ctx *ctx, int32_t layout, const std::vector<andr_matrix_out> &out) {
+  std::vector<andr_copy> copies;
+  for (const andr_matrix_out &o : out) {
+    if (!o.h) continue;
+    const size_t bytes = sizeof(double) * (size_t)o.m * o.n;
+    if (layout == ANDR_ROW_MAJOR) {
+      copies.push_back({o.h, o.d, bytes});
+      continue;
+    }
+    DevBuf<double> t;  // one transposed matrix at a time
+    if (t.alloc((size_t)o.m * o.n, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "transpose buffer");
+    dim3 grid((unsigned)((o.n + 31) / 32), (unsigned)((o.m + 31) / 32));
+    hipLaunchKernelGGL(k_transpose, grid, dim3(32, 8), 0, ctx->stream, o.d, t.p, o.m, o.n);
+    ANDR_HIP(ctx, hipGetLastError());
+    int rc = andr_copy_to_host(ctx, {{o.h, t.p, bytes}});
+    if (rc) return rc;
   }
-  DevBuf<double> t;
-  if (t.alloc((size_t)m * n, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "transpose buffer");
-  dim3 grid((unsigned)((n + 31) / 32), (unsigned)((m + 31) / 32));
-  hipLaunchKernelGGL(k_transpose, grid, dim3(32, 8), 0, ctx->stream, d, t.p, m, n);
-  ANDR_HIP(ctx, hipGetLastError());
-  ANDR_HIP(ctx, hipMemcpyAsync(h, t.p, sizeof(double) * m * n, hipMemcpyDeviceToHost, ctx->stream));
-  ANDR_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return ANDR_OK;
+  return copies.empty() ? ANDR_OK : andr_copy_to_host(ctx, copies);
 }

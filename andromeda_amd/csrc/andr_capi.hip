@@ -5,6 +5,7 @@
 #include "andr_solve.h"
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdarg>
@@ -72,6 +73,7 @@ extern "C" int andr_destroy(andr_ctx *ctx) {
   for (auto &kv : ctx->pool.size_of) (void)hipFree(kv.first);  // blocks still held by nobody's buffers
   ctx->pool.size_of.clear();
   for (void *c : ctx->pinned.chunks) (void)hipHostFree(c);
+  if (ctx->copy_stage) (void)hipHostFree(ctx->copy_stage);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return ANDR_OK;
@@ -147,6 +149,59 @@ void *andr_pinned_alloc(andr_ctx *ctx) {
 
 void andr_pinned_release(andr_ctx *ctx, void *slot) { ctx->pinned.free_slots.push_back(slot); }
 
+int andr_copy_to_host(andr_ctx *ctx, const std::vector<andr_copy> &copies) {
+  size_t total = 0;
+  for (const andr_copy &c : copies) total += c.bytes;
+  std::vector<andr_copy> rest = copies;
+  if (total >= ANDR_COPY_MIN) {
+    if (!ctx->copy_stage &&
+        hipHostMalloc(&ctx->copy_stage, ANDR_COPY_THREADS * ANDR_COPY_PIECE, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      ctx->copy_stage = nullptr;
+    }
+    if (ctx->copy_stage) {
+      rest.clear();
+      for (const andr_copy &c : copies)
+        for (size_t o = 0; o < c.bytes; o += ANDR_COPY_PIECE)
+          rest.push_back({(char *)c.dst + o, (const char *)c.src + o, std::min(ANDR_COPY_PIECE, c.bytes - o)});
+      std::atomic<size_t> next{0};
+      std::atomic<int> failed{(int)hipSuccess};
+      auto work = [&](int w) {
+        void *stage = (char *)ctx->copy_stage + w * ANDR_COPY_PIECE;
+        hipEvent_t ev = nullptr;
+        hipError_t e = hipSetDevice(ctx->device);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        while (e == hipSuccess && failed == (int)hipSuccess) {
+          const size_t i = next++;
+          if (i >= rest.size()) break;
+          e = hipMemcpyAsync(stage, rest[i].src, rest[i].bytes, hipMemcpyDeviceToHost, ctx->stream);
+          if (e == hipSuccess) e = hipEventRecord(ev, ctx->stream);
+          if (e == hipSuccess) e = hipEventSynchronize(ev);
+          if (e == hipSuccess) std::memcpy(rest[i].dst, stage, rest[i].bytes);
+        }
+        if (ev) (void)hipEventDestroy(ev);
+        if (e != hipSuccess) failed = (int)e;
+      };
+      std::vector<std::thread> threads;
+      try {
+        threads.reserve(ANDR_COPY_THREADS);
+        for (int w = 1; w < ANDR_COPY_THREADS; ++w) threads.emplace_back(work, w);
+      } catch (const std::exception &) {  // no more threads: those that started and this one do the work
+      }
+      work(0);
+      for (std::thread &t : threads) t.join();
+      ANDR_HIP(ctx, hipStreamSynchronize(ctx->stream));  // a failed thread's copy no longer writes its piece
+      if (failed != (int)hipSuccess)
+        return andr_fail(ctx, ANDR_ERR_HIP, "copy to the host: %s", hipGetErrorString((hipError_t)(int)failed));
+      return ANDR_OK;
+    }
+  }
+  for (const andr_copy &c : rest)
+    if (c.bytes) ANDR_HIP(ctx, hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyDeviceToHost, ctx->stream));
+  ANDR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  return ANDR_OK;
+}
+
 extern "C" const char *andr_last_error(const andr_ctx *ctx) { return ctx ? ctx->err.c_str() : "no context"; }
 
 // ---- seam 1 ----------------------------------------------------------------------------------
@@ -191,8 +246,7 @@ extern "C" int andr_assemble_laplace_rows(andr_ctx *ctx, const andr_mesh *mesh, 
   if (dH.alloc((size_t)nr * nn, ctx) || dG.alloc((size_t)nr * ne, ctx) || dE.alloc(nr, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "integral matrices (%d x %d)", nr, nn + ne);
   if ((rc = andr_launch_laplace_rows(ctx, b, dH.p, dG.p, dE.p, row_begin, nr))) return rc;
-  if (H && (rc = andr_copy_out(ctx, dH.p, nr, nn, layout, H))) return rc;
-  if (G && (rc = andr_copy_out(ctx, dG.p, nr, ne, layout, G))) return rc;
+  if ((rc = andr_copy_out(ctx, layout, {{dH.p, nr, nn, H}, {dG.p, nr, ne, G}}))) return rc;
   return max_err(ctx, dE.p, row_begin, nr, nn, err);
 }
 
@@ -219,14 +273,16 @@ extern "C" int andr_assemble_stokes_rows(andr_ctx *ctx, const andr_mesh *mesh, i
       dE.alloc(nr, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "Stokes integral matrices (%zu doubles)", 9 * (sT + sG));
   if ((rc = andr_launch_stokes_rows(ctx, b, extra_free_term, dT.p, dG.p, dpT.p, dpG.p, dE.p, row_begin, nr))) return rc;
+  std::vector<andr_matrix_out> out;
   for (int k = 0; k < 6; ++k) {
-    if (T && T[k] && (rc = andr_copy_out(ctx, dT.p + k * sT, nr, nn, layout, T[k]))) return rc;
-    if (G && G[k] && (rc = andr_copy_out(ctx, dG.p + k * sG, nr, ne, layout, G[k]))) return rc;
+    out.push_back({dT.p + k * sT, nr, nn, T ? T[k] : nullptr});
+    out.push_back({dG.p + k * sG, nr, ne, G ? G[k] : nullptr});
   }
   for (int k = 0; k < 3; ++k) {
-    if (prT && prT[k] && (rc = andr_copy_out(ctx, dpT.p + k * sT, nr, nn, layout, prT[k]))) return rc;
-    if (prG && prG[k] && (rc = andr_copy_out(ctx, dpG.p + k * sG, nr, ne, layout, prG[k]))) return rc;
+    out.push_back({dpT.p + k * sT, nr, nn, prT ? prT[k] : nullptr});
+    out.push_back({dpG.p + k * sG, nr, ne, prG ? prG[k] : nullptr});
   }
+  if ((rc = andr_copy_out(ctx, layout, out))) return rc;
   return max_err(ctx, dE.p, row_begin, nr, nn, err);
 }
 

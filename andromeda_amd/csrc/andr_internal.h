@@ -40,12 +40,28 @@ struct andr_pinned {
   std::vector<void *> chunks, free_slots;
 };
 
+// Large results to pageable host memory (andr_copy_out): the runtime's own copy is one thread's, which also takes
+// the page faults of memory that was never touched (84 MB in 18 arrays: 10 of the call's 12 ms). Here each of
+// ANDR_COPY_THREADS threads takes pieces of ANDR_COPY_PIECE bytes through a piece of pinned memory of its own, which
+// the context keeps from the first such copy to andr_destroy: the call takes 4 ms (5.4 with pieces of half that
+// size, 4.2 with twelve threads on sixteen cores). Less than ANDR_COPY_MIN bytes are left to the runtime: the
+// threads' start costs about 0.2 ms.
+#define ANDR_COPY_THREADS 8
+#define ANDR_COPY_PIECE ((size_t)2 << 20)
+#define ANDR_COPY_MIN ((size_t)4 << 20)
+struct andr_copy {
+  void *dst;
+  const void *src;
+  size_t bytes;
+};
+
 struct andr_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   std::string err;
   andr_pool pool;
   andr_pinned pinned;
+  void *copy_stage = nullptr;  // ANDR_COPY_THREADS pieces of pinned memory
   // learned quadrature model (BF16 copy lives in the device buffer below)
   bool has_model = false;
   float model_conf = 0.9f;
@@ -76,6 +92,8 @@ void andr_dev_release(andr_ctx *ctx, void *p);       // back to the context's ca
 void andr_pool_trim(andr_ctx *ctx);                  // return every cached block to the driver
 void *andr_pinned_alloc(andr_ctx *ctx);              // one slot; null on failure
 void andr_pinned_release(andr_ctx *ctx, void *slot);
+// device to host behind the work on the context's stream; the copies are done when it returns
+int andr_copy_to_host(andr_ctx *ctx, const std::vector<andr_copy> &copies);
 
 // RAII device buffer; with a context it draws on the context's memory cache
 template <class T>
@@ -166,8 +184,13 @@ int andr_launch_laplace_rows(andr_ctx *ctx, DevBody &b, double *H, double *G, do
                              int nrows = -1, bool fp32_quad = false);
 int andr_launch_stokes_rows(andr_ctx *ctx, DevBody &b, double extra, double *T, double *G, double *prT,
                             double *prG, double *err_rows, int r0 = 0, int nrows = -1);
-// transposes an m x n row-major device matrix into a column-major host buffer
-int andr_copy_out(andr_ctx *ctx, const double *d, int64_t m, int64_t n, int32_t layout, double *h);
+// device matrices to the host, row- or column-major
+struct andr_matrix_out {
+  const double *d;  // m x n, row-major on the device
+  int64_t m, n;
+  double *h;  // on the host; null: not wanted
+};
+int andr_copy_out(andr_ctx *ctx, int32_t layout, const std::vector<andr_matrix_out> &out);
 
 // Device address of the no-allocation work space on the context's device, looked up once per
 // device (andr_noalloc.hip); called by andr_create with the device current.
