@@ -281,38 +281,42 @@ int andr_body_upload(andr_ctx *ctx, const andr_mesh *m, DevBody &b, bool with_co
   if (m->normmul)
     for (int w = 0; w < nw; ++w) wm[w] = m->normmul[w];
   b.itri = m->itri == 0 ? 5 : m->itri;
-  DevBuf<double> d_wm;
-  if (b.xyz.alloc(3 * (size_t)nn, ctx) || b.con.alloc((size_t)nv * ne, ctx) || b.bcid.alloc(ne, ctx) ||
-      b.nrm.alloc(3 * (size_t)ne, ctx) || b.area.alloc(ne, ctx) || b.cen.alloc(3 * (size_t)ne, ctx) ||
-      b.mul.alloc(ne, ctx) || b.cenl.alloc(ne, ctx) || d_wm.alloc(nw, ctx))
-    return andr_fail(ctx, ANDR_ERR_ALLOC, "device allocation for mesh");
-  ANDR_HIP(ctx, hipMemcpyAsync(b.xyz.p, m->xyz, sizeof(double) * 3 * nn, hipMemcpyHostToDevice, ctx->stream));
-  ANDR_HIP(ctx, hipMemcpyAsync(b.con.p, con.data(), sizeof(int) * nv * ne, hipMemcpyHostToDevice, ctx->stream));
-  ANDR_HIP(ctx, hipMemcpyAsync(b.bcid.p, bcid.data(), sizeof(int) * ne, hipMemcpyHostToDevice, ctx->stream));
-  ANDR_HIP(ctx, hipMemcpyAsync(d_wm.p, wm.data(), sizeof(double) * nw, hipMemcpyHostToDevice, ctx->stream));
-  hipLaunchKernelGGL(k_geometry, dim3((ne + 255) / 256), dim3(256), 0, ctx->stream, ne, nv, b.xyz.p, b.con.p,
-                     b.bcid.p, d_wm.p, b.nrm.p, b.area.p, b.cen.p, b.mul.p, b.cenl.p);
-  ANDR_HIP(ctx, hipGetLastError());
+  std::vector<int> order;
+  std::vector<uint8_t> color;
   if (with_colors) {
-    std::vector<int> order;
-    std::vector<uint8_t> color;
     b.ncolors = color_elements(nn, ne, nv, con.data(), order, color);
     if (b.ncolors < 0) return andr_fail(ctx, ANDR_ERR_ARG, "mesh node valence too high for the element colouring");
-    if (b.order.alloc(ne, ctx) || b.color.alloc(ne, ctx))
-      return andr_fail(ctx, ANDR_ERR_ALLOC, "device allocation for colours");
-    ANDR_HIP(ctx, hipMemcpyAsync(b.order.p, order.data(), sizeof(int) * ne, hipMemcpyHostToDevice, ctx->stream));
-    ANDR_HIP(ctx, hipMemcpyAsync(b.color.p, color.data(), ne, hipMemcpyHostToDevice, ctx->stream));
   }
-  // No synchronisation here: d_wm returns to the context's cache, and any later use of that block
-  // is ordered after k_geometry on the same stream; the host vectors were staged by the copies.
+  std::vector<char> host;
+  auto put = [&](const void *src, size_t bytes) {
+    const size_t at = host.size();
+    host.resize(at + (bytes + 15) / 16 * 16);
+    if (bytes) std::memcpy(host.data() + at, src, bytes);
+    return at;
+  };
+  const size_t o_xyz = put(m->xyz, sizeof(double) * 3 * nn), o_wm = put(wm.data(), sizeof(double) * nw),
+               o_con = put(con.data(), sizeof(int) * nv * ne), o_bcid = put(bcid.data(), sizeof(int) * ne),
+               o_order = put(order.data(), sizeof(int) * order.size()), o_color = put(color.data(), color.size());
+  if (b.mesh.alloc(host.size(), ctx) || b.nrm.alloc(3 * (size_t)ne, ctx) || b.area.alloc(ne, ctx) ||
+      b.cen.alloc(3 * (size_t)ne, ctx) || b.mul.alloc(ne, ctx) || b.cenl.alloc(ne, ctx))
+    return andr_fail(ctx, ANDR_ERR_ALLOC, "device allocation for mesh");
+  ANDR_HIP(ctx, hipMemcpyAsync(b.mesh.p, host.data(), host.size(), hipMemcpyHostToDevice, ctx->stream));
+  const double *d_xyz = (double *)(b.mesh.p + o_xyz), *d_wm = (double *)(b.mesh.p + o_wm);
+  const int *d_con = (int *)(b.mesh.p + o_con), *d_bcid = (int *)(b.mesh.p + o_bcid);
+  b.order = with_colors ? (int *)(b.mesh.p + o_order) : nullptr;
+  b.color = with_colors ? (uint8_t *)(b.mesh.p + o_color) : nullptr;
+  hipLaunchKernelGGL(k_geometry, dim3((ne + 255) / 256), dim3(256), 0, ctx->stream, ne, nv, d_xyz, d_con, d_bcid, d_wm,
+                     b.nrm.p, b.area.p, b.cen.p, b.mul.p, b.cenl.p);
+  ANDR_HIP(ctx, hipGetLastError());
+  // No synchronisation here: the host vector was staged by the copy.
   b.g.nn = nn;
   b.g.ne = ne;
   b.g.nwalls = nw;
   b.g.nv = nv;
   b.g.iquad = b.iquad;
-  b.g.xyz = b.xyz.p;
-  b.g.con = b.con.p;
-  b.g.bcid = b.bcid.p;
+  b.g.xyz = d_xyz;
+  b.g.con = d_con;
+  b.g.bcid = d_bcid;
   b.g.nrm = b.nrm.p;
   b.g.area = b.area.p;
   b.g.cen = b.cen.p;
@@ -701,7 +705,7 @@ int andr_launch_laplace_rows(andr_ctx *ctx, DevBody &b, double *H, double *G, do
   const Kern kern = kerns[(in_lds ? 4 : 0) + (fp32_quad ? 2 : 0) + (quads ? 1 : 0)];
   if (in_lds) ANDR_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   hipLaunchKernelGGL(kern, dim3(nsp), dim3(row_threads(b.g.ne)), in_lds ? lds : 0, ctx->stream, b.g, qr.offset, qr.npts,
-                     b.order.p, b.color.p, b.ncolors, H, G, err_rows, r0);
+                     b.order, b.color, b.ncolors, H, G, err_rows, r0);
   andr_prof_end(ctx, tok);
   ANDR_HIP(ctx, hipGetLastError());
   return ANDR_OK;
@@ -1168,7 +1172,7 @@ int andr_launch_stokes_rows(andr_ctx *ctx, DevBody &b, double extra, double *T, 
   const Kern kern = kerns[(in_lds ? 2 : 0) + (quads ? 1 : 0)];
   if (in_lds) ANDR_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   hipLaunchKernelGGL(kern, dim3(nsp), dim3(row_threads(b.g.ne)), in_lds ? lds : 0, ctx->stream, b.g, qr.offset, qr.npts,
-                     b.order.p, b.color.p, b.ncolors, extra, T, G, prT, prG, err_rows, r0, nsp);
+                     b.order, b.color, b.ncolors, extra, T, G, prT, prG, err_rows, r0, nsp);
   andr_prof_end(ctx, tok);
   ANDR_HIP(ctx, hipGetLastError());
   return ANDR_OK;

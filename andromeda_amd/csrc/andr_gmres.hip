@@ -20,6 +20,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <list>
 #include <type_traits>
 #include <vector>
 
@@ -855,14 +856,17 @@ __global__ __launch_bounds__(256) void kb_xupdate(const GSys *__restrict__ sys, 
 }
 
 // per tile: R = B (start of the residual product)
-__global__ __launch_bounds__(256) void kb_copy_b(const GSys *__restrict__ sys, const TileMap *__restrict__ tmap) {
+__global__ __launch_bounds__(256) void kb_copy_b(const GSys *__restrict__ sys, const TileMap *__restrict__ tmap,
+                                                 int first) {
   const TileMap tm = tmap[blockIdx.x];
   const GSys &S = sys[tm.sys];
   const int k = threadIdx.x & 7, rr = threadIdx.x >> 3;
 #pragma unroll
   for (int t = 0; t < TILE / 32; ++t) {
     const int row = tm.row0 + rr + 32 * t;
-    if (row < S.n) S.R[(size_t)row * NB + k] = S.B[(size_t)row * NB + k];
+    if (row >= S.n) continue;
+    S.R[(size_t)row * NB + k] = S.B[(size_t)row * NB + k];
+    if (first) S.X[(size_t)row * NB + k] = 0.0;
   }
 }
 
@@ -870,7 +874,7 @@ __global__ __launch_bounds__(256) void kb_copy_b(const GSys *__restrict__ sys, c
 // eight loads in flight); then thread k < NB sets up the restart of column k
 __global__ __launch_bounds__(256) void kb_restart(const GSys *__restrict__ sys, const double *__restrict__ part,
                                                   const int *__restrict__ wave0, const int *__restrict__ nwv,
-                                                  double tol, int first, int nrhs, int *__restrict__ done) {
+                                                  double tol, int first, int nrhs) {
   __shared__ double red[4][NB];
   const int s = blockIdx.x, k = threadIdx.x & 7;
   const GSys &S = sys[s];
@@ -911,7 +915,6 @@ __global__ __launch_bounds__(256) void kb_restart(const GSys *__restrict__ sys, 
   }
   sm[5] = -1.0;
   sm[3] = (sm[4] > 0.0 && rn > 0.0) ? 1.0 / rn : 0.0;
-  if (sm[4] > 0.0) atomicAdd(done, 1);
 }
 
 // thread per (system, k) of the cycle: g = (||r||, 0, ..., 0) in the cycle's layout
@@ -1615,17 +1618,17 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
   };
   const size_t small_per = small_of(m);
   const size_t state_per = (size_t)NB * 8;
-  DevBuf<double> R, W, Q, SM, ST8, partW, partT, SDEF, partS, partB;
+  DevBuf<double> R, W, Q, SM, partW, partT, SDEF, partS, partB;  // SM: the small arrays, then the states
   DevBuf<double> ZT;
   DevBuf<float> ZT32;
   DevBuf<GSys> dsys;
-  DevBuf<int> ddone;
   if (R.alloc(vec_elems, ctx) || W.alloc(vec_elems, ctx) || Q.alloc(basis_elems, ctx) ||
-      SM.alloc(small_per * nsys, ctx) || ST8.alloc(state_per * nsys, ctx) || partW.alloc((size_t)nw_full * NB, ctx) ||
+      SM.alloc((small_per + state_per) * nsys, ctx) || partW.alloc((size_t)nw_full * NB, ctx) ||
       (!blk && partT.alloc((size_t)nt_full * part_stride(m) * NB, ctx)) ||
       (blk && partB.alloc((size_t)nt4_full * (m + 2) * 64, ctx)) ||
-      dsys.alloc(nsys, ctx) || ddone.alloc(1, ctx))
+      dsys.alloc(nsys, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "GMRES workspace (%zu basis doubles)", basis_elems);
+  double *const states = SM.p + small_per * nsys;
   // Krylov products on the FP32 matrix cores at relative residuals of 1e-6 and above (their ~1e-7
   // relative error stays below the tolerance); FP64 products for tighter tolerances.
   // ANDR_GMRES_FP64_PRODUCTS=1 keeps FP64 products at every tolerance.
@@ -1640,22 +1643,29 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
   constexpr int MF_TARGET_WAVES = 2048, MF_MAX_SEG = 16;
   // structured operator: w = residual blocks of 64 element rows (4 partial entries each), mw =
   // matrix-core waves of 32 element rows, et = element tiles of 32 (z = M^-1 v and wall sums)
+  // The maps of a set go up in one copy (each copy is some 8 us of a small body's solve), from host memory
+  // that lives until the end: the host needs not wait for it.
   struct MapSet {
-    DevBuf<WaveMap> w;
-    DevBuf<TileMap> t, et, t4;
-    DevBuf<MWave> mw;
-    DevBuf<int> w0, nw;
+    DevBuf<char> buf;
+    WaveMap *w = nullptr;
+    TileMap *t = nullptr, *et = nullptr, *t4 = nullptr;
+    MWave *mw = nullptr;
+    int *w0 = nullptr, *nw = nullptr;
     int n_w = 0, n_t = 0, n_et = 0, n_mw = 0, n_t4 = 0, max_seg = 1;
-    size_t mw_cap = 0;
     std::vector<int> tile0, ntiles, et0, net, nseg, t40, nt4;
     std::vector<size_t> poff;
     size_t p_elems = 0;
   };
   MapSet cyc, live;
-  for (MapSet *ms : {&cyc, &live})
-    if (ms->w.alloc(nw_full, ctx) || ms->t.alloc(nt_full, ctx) || ms->w0.alloc(nsys, ctx) || ms->nw.alloc(nsys, ctx) ||
-        ms->et.alloc(net_full, ctx) || (blk && ms->t4.alloc(nt4_full, ctx)))
-      return andr_fail(ctx, ANDR_ERR_ALLOC, "GMRES work maps");
+  struct Staging {
+    hipStream_t st;
+    std::list<std::vector<char>> host;
+    ~Staging() { (void)hipStreamSynchronize(st); }
+  } staging{st, {}};
+  auto stage = [&](size_t bytes) {
+    staging.host.emplace_back(bytes);
+    return staging.host.back().data();
+  };
   std::vector<GSys> hs(nsys);
   DevBuf<double> Pseg;
   size_t pseg_cap = 0;
@@ -1709,18 +1719,36 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     ms.n_et = (int)em.size();
     ms.n_mw = (int)mw.size();
     ms.n_t4 = (int)t4.size();
-    if (ms.n_t4) ANDR_HIP(ctx, hipMemcpyAsync(ms.t4.p, t4.data(), sizeof(TileMap) * t4.size(), hipMemcpyHostToDevice, st));
-    if (ms.n_et) ANDR_HIP(ctx, hipMemcpyAsync(ms.et.p, em.data(), sizeof(TileMap) * em.size(), hipMemcpyHostToDevice, st));
-    if (mw.size() > ms.mw_cap) {
-      if (ms.mw.alloc(mw.size(), ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "GMRES matrix-core map");
-      ms.mw_cap = mw.size();
-    }
-    if (ms.n_w) ANDR_HIP(ctx, hipMemcpyAsync(ms.w.p, wm.data(), sizeof(WaveMap) * wm.size(), hipMemcpyHostToDevice, st));
-    if (ms.n_t) ANDR_HIP(ctx, hipMemcpyAsync(ms.t.p, tm.data(), sizeof(TileMap) * tm.size(), hipMemcpyHostToDevice, st));
-    if (ms.n_mw) ANDR_HIP(ctx, hipMemcpyAsync(ms.mw.p, mw.data(), sizeof(MWave) * mw.size(), hipMemcpyHostToDevice, st));
-    ANDR_HIP(ctx, hipMemcpyAsync(ms.w0.p, w0.data(), sizeof(int) * nsys, hipMemcpyHostToDevice, st));
-    ANDR_HIP(ctx, hipMemcpyAsync(ms.nw.p, nw.data(), sizeof(int) * nsys, hipMemcpyHostToDevice, st));
-    ANDR_HIP(ctx, hipStreamSynchronize(st));  // host vectors go out of scope
+    size_t bytes = 0;
+    auto room = [&](size_t n) {
+      const size_t at = bytes;
+      bytes += (n + 255) / 256 * 256;
+      return at;
+    };
+    const size_t o[7] = {room(sizeof(WaveMap) * wm.size()), room(sizeof(TileMap) * tm.size()),
+                         room(sizeof(TileMap) * em.size()), room(sizeof(TileMap) * t4.size()),
+                         room(sizeof(MWave) * mw.size()),   room(sizeof(int) * nsys),
+                         room(sizeof(int) * nsys)};
+    if (bytes > ms.buf.n && ms.buf.alloc(bytes, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "GMRES work maps");
+    char *h = stage(bytes), *d = ms.buf.p;
+    auto put = [&](size_t at, const void *src, size_t n) {
+      if (n) std::memcpy(h + at, src, n);
+    };
+    put(o[0], wm.data(), sizeof(WaveMap) * wm.size());
+    put(o[1], tm.data(), sizeof(TileMap) * tm.size());
+    put(o[2], em.data(), sizeof(TileMap) * em.size());
+    put(o[3], t4.data(), sizeof(TileMap) * t4.size());
+    put(o[4], mw.data(), sizeof(MWave) * mw.size());
+    put(o[5], w0.data(), sizeof(int) * nsys);
+    put(o[6], nw.data(), sizeof(int) * nsys);
+    ms.w = (WaveMap *)(d + o[0]);
+    ms.t = (TileMap *)(d + o[1]);
+    ms.et = (TileMap *)(d + o[2]);
+    ms.t4 = (TileMap *)(d + o[3]);
+    ms.mw = (MWave *)(d + o[4]);
+    ms.w0 = (int *)(d + o[5]);
+    ms.nw = (int *)(d + o[6]);
+    ANDR_HIP(ctx, hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, st));
     return ANDR_OK;
   };
   // the reductions index partials through S.tile0/ntiles; the product reads S.nseg/P
@@ -1739,7 +1767,9 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
       hs[s].nseg = ms.nseg[s];
       hs[s].P = ms.nseg[s] > 1 ? Pseg.p + ms.poff[s] : nullptr;
     }
-    ANDR_HIP(ctx, hipMemcpyAsync(dsys.p, hs.data(), sizeof(GSys) * nsys, hipMemcpyHostToDevice, st));
+    char *h = stage(sizeof(GSys) * nsys);
+    std::memcpy(h, hs.data(), sizeof(GSys) * nsys);
+    ANDR_HIP(ctx, hipMemcpyAsync(dsys.p, h, sizeof(GSys) * nsys, hipMemcpyHostToDevice, st));
     return ANDR_OK;
   };
   size_t vo = 0, zo = 0;
@@ -1759,7 +1789,7 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     g.X = in[s].X;
     g.R = R.p + vo;
     g.W = W.p + vo;
-    g.small = ST8.p + state_per * s;
+    g.small = states + state_per * s;
     vo += (size_t)n * NB;
   }
   // Basis and Hessenberg storage of the systems of a cycle, for restart length mc. The first cycle
@@ -1824,9 +1854,7 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     for (int s = 0; s < nsys; ++s) all[s] = s;
     layout(all, m);
   }
-  ANDR_HIP(ctx, hipMemsetAsync(SM.p, 0, sizeof(double) * small_per * nsys, st));
-  ANDR_HIP(ctx, hipMemsetAsync(ST8.p, 0, sizeof(double) * state_per * nsys, st));
-  for (int s = 0; s < nsys; ++s) ANDR_HIP(ctx, hipMemsetAsync(in[s].X, 0, sizeof(double) * in[s].n * NB, st));
+  ANDR_HIP(ctx, hipMemsetAsync(SM.p, 0, sizeof(double) * (small_per + state_per) * nsys, st));
   const int gs = (nsys * NB + 63) / 64;
   // ANDR_GMRES_NO_SKIP=1: converged systems keep their products (and block sweeps) until the next map
   // rebuild (the rounds after convergence are never used, so the results are the same bit for bit)
@@ -1849,16 +1877,16 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     // the block solver's Krylov products skip converged systems' operands too (the flag read by
     // sys_iterating is kept by the block kernels only)
     const int all = (krylov && blk) ? noskip : 1;
-    hipLaunchKernelGGL(kb_prep, dim3(ms.n_et), dim3(256), 0, st, dsys.p, ms.et.p, krylov ? 0 : 1, jq, partS.p, all);
+    hipLaunchKernelGGL(kb_prep, dim3(ms.n_et), dim3(256), 0, st, dsys.p, ms.et, krylov ? 0 : 1, jq, partS.p, all);
     hipLaunchKernelGGL(kb_sred, dim3(nsys), dim3(256), 0, st, dsys.p, partS.p, all);
     if (krylov && f32prod)
-      hipLaunchKernelGGL(kb_gemv_sym<true>, dim3((ms.n_mw + 3) / 4), dim3(256), 0, st, dsys.p, ms.mw.p, ms.n_mw,
+      hipLaunchKernelGGL(kb_gemv_sym<true>, dim3((ms.n_mw + 3) / 4), dim3(256), 0, st, dsys.p, ms.mw, ms.n_mw,
                          noskip);
     else
-      hipLaunchKernelGGL(kb_gemv_sym<false>, dim3((ms.n_mw + 3) / 4), dim3(256), 0, st, dsys.p, ms.mw.p, ms.n_mw,
+      hipLaunchKernelGGL(kb_gemv_sym<false>, dim3((ms.n_mw + 3) / 4), dim3(256), 0, st, dsys.p, ms.mw, ms.n_mw,
                          krylov ? noskip : 1);
-    if (ms.max_seg > 1) hipLaunchKernelGGL(kb_seg_sum, dim3(ms.n_t), dim3(256), 0, st, dsys.p, ms.t.p, all);
-    if (!krylov) hipLaunchKernelGGL(kb_resid_fin, dim3(ms.n_w), dim3(256), 0, st, dsys.p, ms.w.p, partW.p);
+    if (ms.max_seg > 1) hipLaunchKernelGGL(kb_seg_sum, dim3(ms.n_t), dim3(256), 0, st, dsys.p, ms.t, all);
+    if (!krylov) hipLaunchKernelGGL(kb_resid_fin, dim3(ms.n_w), dim3(256), 0, st, dsys.p, ms.w, partW.p);
     andr_prof_end(ctx, tok);
   };
   // Autotuner of the product's column segments: when few rows are live (the slowest bodies of a
@@ -1866,14 +1894,22 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
   // number of waves. The first time a size bucket (ceil log2 of the live 32-row waves) occurs, the
   // candidates are timed on the live systems' current Krylov vector and the fastest is kept in the
   // context. The split changes the summation order of the product (segments are summed apart).
-  auto krylov_target = [&](const std::vector<int> &list, int jq) -> int {
-    int row_waves = 0;
+  auto krylov_key = [&](const std::vector<int> &list) {
+    int row_waves = 0, key = 0;
     for (int s : list) row_waves += (in[s].op.ne + 31) / 32;
-    if (!ctx->autotune || row_waves <= 0 || row_waves >= 4096) return MF_TARGET_WAVES;
-    int key = 0;
+    if (!ctx->autotune || row_waves <= 0 || row_waves >= 4096) return -1;
     while ((1 << key) < row_waves) ++key;
+    return key;
+  };
+  auto krylov_tuned = [&](const std::vector<int> &list) {  // 0: to be timed
+    const int key = krylov_key(list);
+    if (key < 0) return MF_TARGET_WAVES;
     auto it = ctx->tune_krylov.find(key);
-    if (it != ctx->tune_krylov.end()) return it->second.first;
+    return it != ctx->tune_krylov.end() ? it->second.first : 0;
+  };
+  auto krylov_target = [&](const std::vector<int> &list, int jq) -> int {
+    const int tuned = krylov_tuned(list), key = krylov_key(list);
+    if (tuned > 0) return tuned;
     hipEvent_t e0, e1;
     ANDR_HIP(ctx, hipEventCreate(&e0));
     ANDR_HIP(ctx, hipEventCreate(&e1));
@@ -1906,7 +1942,7 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
   std::vector<int> it_count((size_t)nsys * NB, 0);
   std::vector<double> hsmall(state_per * nsys);
   auto read_small = [&]() -> int {
-    ANDR_HIP(ctx, hipMemcpyAsync(hsmall.data(), ST8.p, sizeof(double) * state_per * nsys, hipMemcpyDeviceToHost, st));
+    ANDR_HIP(ctx, hipMemcpyAsync(hsmall.data(), states, sizeof(double) * state_per * nsys, hipMemcpyDeviceToHost, st));
     ANDR_HIP(ctx, hipStreamSynchronize(st));
     return ANDR_OK;
   };
@@ -1943,6 +1979,7 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
   };
   std::vector<int> cyc_list(nsys);
   for (int s = 0; s < nsys; ++s) cyc_list[s] = s;
+  std::vector<int> cyc_built = cyc_list;
   int rc = build(cyc_list, cyc);
   if (rc) return rc;
   if ((rc = use_tiles(cyc))) return rc;
@@ -1951,15 +1988,14 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
   const bool debug = getenv("ANDR_DEBUG_GMRES") != nullptr;
   while (true) {
     // residual r = b - A x of every system of the last cycle (x = 0 on the first), FP64 accumulation
-    if (cyc.n_t) hipLaunchKernelGGL(kb_copy_b, dim3(cyc.n_t), dim3(256), 0, st, dsys.p, cyc.t.p);
+    if (cyc.n_t) hipLaunchKernelGGL(kb_copy_b, dim3(cyc.n_t), dim3(256), 0, st, dsys.p, cyc.t, first ? 1 : 0);
     if (first) {
-      if (cyc.n_w) hipLaunchKernelGGL(kb_resid_zero, dim3(cyc.n_w), dim3(256), 0, st, dsys.p, cyc.w.p, partW.p);
+      if (cyc.n_w) hipLaunchKernelGGL(kb_resid_zero, dim3(cyc.n_w), dim3(256), 0, st, dsys.p, cyc.w, partW.p);
     } else {
       gemv(cyc, 0, 0);
     }
-    ANDR_HIP(ctx, hipMemsetAsync(ddone.p, 0, sizeof(int), st));
-    hipLaunchKernelGGL(kb_restart, dim3(nsys), dim3(256), 0, st, dsys.p, partW.p, cyc.w0.p, cyc.nw.p, tol,
-                       first ? 1 : 0, nrhs, ddone.p);
+    hipLaunchKernelGGL(kb_restart, dim3(nsys), dim3(256), 0, st, dsys.p, partW.p, cyc.w0, cyc.nw, tol,
+                       first ? 1 : 0, nrhs);
     ANDR_HIP(ctx, hipGetLastError());
     if ((rc = read_small())) return rc;
     first = false;
@@ -1981,29 +2017,32 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
           break;
         }
     if (cyc_list.empty() || total >= maxit) break;
-    if ((rc = build(cyc_list, cyc))) return rc;
-    if ((rc = build(cyc_list, live))) return rc;
+    if (cyc_list != cyc_built) {
+      if ((rc = build(cyc_list, cyc))) return rc;
+      cyc_built = cyc_list;
+    }
+    // a cycle that starts with few rows (a small batch) takes the tuned column split at once
+    const int tuned = krylov_tuned(cyc_list);
+    if ((rc = build(cyc_list, live, tuned > 0 ? tuned : MF_TARGET_WAVES))) return rc;
     mc = first_cycle ? m : restart_for(cyc_list);
     layout(cyc_list, mc);
     first_cycle = false;
     if ((rc = use_tiles(live))) return rc;
     std::fill(skip_counted.begin(), skip_counted.end(), 0);
     if (blk) {  // Q_0 R0 = R (Cholesky QR of the residual block), g = (R0; 0)
-      launch_bdots(st, live.n_t4, dsys.p, live.t4.p, 1, 0, 1, partB.p, mc + 2, 1);
+      launch_bdots(st, live.n_t4, dsys.p, live.t4, 1, 0, 1, partB.p, mc + 2, 1);
       hipLaunchKernelGGL(kb_bdots_final, dim3(nsys, 1), dim3(256), 0, st, dsys.p, partB.p, mc + 2, 1, 1);
       hipLaunchKernelGGL(kb_binit, dim3(nsys), dim3(256), 0, st, dsys.p, mc, L);
-      hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t.p, 0, 3, 1);
+      hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t, 0, 3, 1);
     } else {
       hipLaunchKernelGGL(kb_ginit, dim3(gs), dim3(64), 0, st, dsys.p, nsys, mc);
-      hipLaunchKernelGGL(kb_q0, dim3(cyc.n_t), dim3(256), 0, st, dsys.p, cyc.t.p);
+      hipLaunchKernelGGL(kb_q0, dim3(cyc.n_t), dim3(256), 0, st, dsys.p, cyc.t);
     }
-    {  // a cycle that starts with few rows (a small batch) takes the tuned column split at once
+    if (tuned <= 0) {
       const int target = krylov_target(cyc_list, 0);
       if (target < 0) return target;  // a failed timing run
-      if (target != MF_TARGET_WAVES) {
-        if ((rc = build(cyc_list, live, target))) return rc;
-        if ((rc = use_tiles(live))) return rc;
-      }
+      if ((rc = build(cyc_list, live, target))) return rc;
+      if ((rc = use_tiles(live))) return rc;
     }
     const int steps_max = std::min(mc, maxit - total);
     int steps = 0;
@@ -2019,23 +2058,23 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
         // twice); the second update also normalises the new block
         const int tok_o = andr_prof_begin(ctx, "gmres_orthogonalise", (4.0 * j + 10.0) * vbytes,
                                           2.0 * 64.0 * (4.0 * j + 5.0) * nlive);
-        launch_bdots(st, live.n_t4, dsys.p, live.t4.p, 0, j + 1, 0, partB.p, mc + 2, noskip);
+        launch_bdots(st, live.n_t4, dsys.p, live.t4, 0, j + 1, 0, partB.p, mc + 2, noskip);
         hipLaunchKernelGGL(kb_bdots_final, dim3(nsys, j + 1), dim3(256), 0, st, dsys.p, partB.p, mc + 2, 0, noskip);
-        hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t.p, j + 1, 0, noskip);
-        launch_bdots(st, live.n_t4, dsys.p, live.t4.p, 0, j + 1, 1, partB.p, mc + 2, noskip);
+        hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t, j + 1, 0, noskip);
+        launch_bdots(st, live.n_t4, dsys.p, live.t4, 0, j + 1, 1, partB.p, mc + 2, noskip);
         hipLaunchKernelGGL(kb_bdots_final, dim3(nsys, j + 2), dim3(256), 0, st, dsys.p, partB.p, mc + 2, 1, noskip);
         launch_bsmall(st, nsys, L, dsys.p, j, tol, noskip);
-        hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t.p, j + 1, 1, noskip);
+        hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t, j + 1, 1, noskip);
         andr_prof_end(ctx, tok_o);
       } else {
         const int tok_o = andr_prof_begin(ctx, "gmres_orthogonalise", (2.0 * j + 6.0) * vbytes,
                                           2.0 * 4.0 * j * nlive * NB);
         hipLaunchKernelGGL(kb_adots, dim3(live.n_t, std::max(1, (j + ICH - 1) / ICH)), dim3(256), 0, st, dsys.p,
-                           live.t.p, j, mc, partT.p, 0);
+                           live.t, j, mc, partT.p, 0);
         hipLaunchKernelGGL(kb_adots_final, dim3(nsys, (2 * j + 3 + 7) / 8), dim3(256), 0, st, dsys.p, j, mc, partT.p);
         hipLaunchKernelGGL(kb_arnoldi, dim3(nsys * NB), dim3(64), sizeof(double) * (5 * mc + 2), st, dsys.p, j, mc,
                            tol, 0);
-        hipLaunchKernelGGL(kb_aupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t.p, j, mc);
+        hipLaunchKernelGGL(kb_aupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t, j, mc);
         andr_prof_end(ctx, tok_o);
       }
       steps = j + 1;
@@ -2065,7 +2104,7 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     if (!blk && steps == steps_max && live.n_t > 0) {
       // close the cycle: the last column is final once its candidate is reorthogonalised
       hipLaunchKernelGGL(kb_adots, dim3(live.n_t, std::max(1, (steps + ICH - 1) / ICH)), dim3(256), 0, st, dsys.p,
-                         live.t.p, steps, mc, partT.p, 1);
+                         live.t, steps, mc, partT.p, 1);
       hipLaunchKernelGGL(kb_adots_final, dim3(nsys, (2 * steps + 3 + 7) / 8), dim3(256), 0, st, dsys.p, steps, mc,
                          partT.p);
       hipLaunchKernelGGL(kb_arnoldi, dim3(nsys * NB), dim3(64), sizeof(double) * (5 * mc + 2), st, dsys.p, steps, mc,
@@ -2074,10 +2113,10 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     total += steps;
     if (blk) {
       if ((rc = launch_bsolve(ctx, nsys, L, dsys.p, steps))) return rc;
-      hipLaunchKernelGGL(kb_bupdate, dim3(cyc.n_t), dim3(256), 0, st, dsys.p, cyc.t.p, steps, 2, 1);
+      hipLaunchKernelGGL(kb_bupdate, dim3(cyc.n_t), dim3(256), 0, st, dsys.p, cyc.t, steps, 2, 1);
     } else {
       hipLaunchKernelGGL(kb_solve_y, dim3(nsys * NB), dim3(64), sizeof(double) * (mc + 1), st, dsys.p, steps, mc);
-      hipLaunchKernelGGL(kb_xupdate, dim3(cyc.n_t), dim3(256), 0, st, dsys.p, cyc.t.p, steps, mc);
+      hipLaunchKernelGGL(kb_xupdate, dim3(cyc.n_t), dim3(256), 0, st, dsys.p, cyc.t, steps, mc);
     }
     ANDR_HIP(ctx, hipGetLastError());
     if ((rc = read_small())) return rc;

@@ -161,11 +161,11 @@ struct BodyGeom {
 
 // Host-side owner of a body's device arrays.
 struct DevBody {
-  DevBuf<double> xyz, nrm, area, cen, mul;
+  DevBuf<char> mesh;      // what comes from the host, in one copy: g.xyz, the wall factors, g.con, g.bcid, and
+  int *order = nullptr;      // the elements in the order the row kernels take them with
+  uint8_t *color = nullptr;  // the colour of each (with_colors)
+  DevBuf<double> nrm, area, cen, mul;
   DevBuf<float4> cenl;
-  DevBuf<int> con, bcid;
-  DevBuf<int> order;      // elements in the order the row kernels take them, and
-  DevBuf<uint8_t> color;  // the colour of each (with_colors)
   int ncolors = 0;
   BodyGeom g;
   int itri = 5;

@@ -176,6 +176,14 @@ size_t body_bytes(int ne, int nn, bool plain, bool learned, int restart) {
 // restart that fits the same buffers.
 constexpr int RESTART = 128, RESTART_MAX = 192;
 
+struct Mark {  // a point of the stream
+  hipEvent_t ev = nullptr;
+  ~Mark() {
+    if (ev) (void)hipEventDestroy(ev);
+  }
+  bool record(hipStream_t st) { return hipEventCreate(&ev) != hipSuccess || hipEventRecord(ev, st) != hipSuccess; }
+};
+
 // The resistance tensors of one wave of prepared bodies: assembly, solve, force and torque.
 // FT and reports point at the wave's first body; t_up is the wave's upload time (reported).
 int run_wave(andr_ctx *ctx, Prepared *const *P, int nb, const andr_resistance_opts *opts, int restart, bool timing,
@@ -193,11 +201,23 @@ int run_wave(andr_ctx *ctx, Prepared *const *P, int nb, const andr_resistance_op
   const double extra = exterior ? 8.0 * ANDR_PI : 0.0;
   const double ta0 = andr_now();
   std::vector<DevBuf<char>> Abuf(nb);
-  std::vector<DevBuf<double>> Bbuf(nb), Xbuf(nb), Ebuf(nb), Dbuf(nb), Pbuf(nb);
-  std::vector<DevBuf<uint8_t>> Mbuf(nb);
+  std::vector<DevBuf<double>> Bbuf(nb), Xbuf(nb), Ebuf(nb), Pbuf(nb);
   std::vector<DevBuf<uint8_t>> Cbuf(nb);
   std::vector<SysJob> jobs(nb);
-  std::vector<int2> rowmap;
+  // the wave's tables go up in one copy: null-space scales, jobs, row map, moving-node flags
+  size_t ndefl = 0, nrows = 0, nflags = 0;
+  for (int i = 0; i < nb; ++i) {
+    if (!plain) ndefl += P[i]->defl.size();
+    nrows += P[i]->ne;
+    if (!exterior) nflags += P[i]->nn;
+  }
+  const size_t o_jobs = sizeof(double) * ndefl, o_rows = o_jobs + sizeof(SysJob) * nb,
+               o_flags = o_rows + sizeof(int2) * nrows, tbytes = o_flags + nflags;
+  static_assert(alignof(SysJob) == 8 && sizeof(SysJob) % 8 == 0 && alignof(int2) == 8, "tables side by side");
+  std::vector<char> tables(tbytes);
+  DevBuf<char> dtab;
+  if (dtab.alloc(tbytes, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "job tables");
+  size_t at_defl = 0, at_row = 0, at_flag = 0;
   for (int i = 0; i < nb; ++i) {
     Prepared &p = *P[i];
     const int n = 3 * p.ne;
@@ -206,20 +226,16 @@ int run_wave(andr_ctx *ctx, Prepared *const *P, int nb, const andr_resistance_op
         Bbuf[i].alloc((size_t)n * ANDR_NRHS, ctx) || Xbuf[i].alloc((size_t)n * ANDR_NRHS, ctx) ||
         Ebuf[i].alloc(p.ne, ctx))
       return andr_fail(ctx, ANDR_ERR_ALLOC, "resistance system of body %d (n = %d)", i, n);
-    if (!exterior) {  // bounded form: only the nodes of wall 2 move (src/lib_particle.f90:220-256, 386-409)
-      std::vector<uint8_t> mv(p.nn);
-      for (int k = 0; k < p.nn; ++k) mv[k] = p.node_wall[k] == 2 ? 1 : 0;
-      if (Mbuf[i].alloc(p.nn, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "moving-node flags");
-      ANDR_HIP(ctx, hipMemcpyAsync(Mbuf[i].p, mv.data(), p.nn, hipMemcpyHostToDevice, ctx->stream));
-      ANDR_HIP(ctx, hipStreamSynchronize(ctx->stream));  // mv goes out of scope
-    }
+    const size_t flag0 = o_flags + at_flag;
+    if (!exterior)  // bounded form: only the nodes of wall 2 move (src/lib_particle.f90:220-256, 386-409)
+      for (int k = 0; k < p.nn; ++k) tables[o_flags + at_flag++] = p.node_wall[k] == 2 ? 1 : 0;
     const QuadRule qr = andr_rule(p.body.itri);
     SysJob &J = jobs[i];
     J.g = p.body.g;
     J.A_ = Abuf[i].p;
     J.lda = lda;
     J.B = Bbuf[i].p;
-    J.moving = exterior ? nullptr : Mbuf[i].p;
+    J.moving = exterior ? nullptr : (uint8_t *)dtab.p + flag0;
     for (int d = 0; d < 3; ++d) J.center[d] = opts->center[d];
     J.strain = opts->problems == ANDR_PROBLEMS_STRAIN ? 1 : 0;
     J.mu = opts->mu;
@@ -234,23 +250,21 @@ int run_wave(andr_ctx *ctx, Prepared *const *P, int nb, const andr_resistance_op
     if (!plain) {
       if (Pbuf[i].alloc(9 * (size_t)p.ne, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "preconditioner blocks");
       J.minv = Pbuf[i].p;
-      const std::vector<double> &dh = p.defl;
-      if (Dbuf[i].alloc(dh.size(), ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "deflation scales");
-      ANDR_HIP(ctx, hipMemcpyAsync(Dbuf[i].p, dh.data(), sizeof(double) * dh.size(), hipMemcpyHostToDevice, ctx->stream));
-      J.defl = Dbuf[i].p;
+      J.defl = (double *)dtab.p + at_defl;
+      std::memcpy((double *)tables.data() + at_defl, p.defl.data(), sizeof(double) * p.defl.size());
+      at_defl += p.defl.size();
     }
     if (learned) {
       if (Cbuf[i].alloc((size_t)p.ne * p.ne, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "rule classes of body %d", i);
       J.cls = Cbuf[i].p;
     }
-    for (int r = 0; r < p.ne; ++r) rowmap.push_back(make_int2(i, r));
+    for (int r = 0; r < p.ne; ++r) ((int2 *)(tables.data() + o_rows))[at_row++] = make_int2(i, r);
   }
   const double tu1 = andr_now();  // job tables
-  DevBuf<SysJob> djobs;
-  DevBuf<int2> drow;
-  if (djobs.alloc(nb, ctx) || drow.alloc(rowmap.size(), ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "job tables");
-  ANDR_HIP(ctx, hipMemcpyAsync(djobs.p, jobs.data(), sizeof(SysJob) * nb, hipMemcpyHostToDevice, ctx->stream));
-  ANDR_HIP(ctx, hipMemcpyAsync(drow.p, rowmap.data(), sizeof(int2) * rowmap.size(), hipMemcpyHostToDevice, ctx->stream));
+  std::memcpy(tables.data() + o_jobs, jobs.data(), sizeof(SysJob) * nb);
+  ANDR_HIP(ctx, hipMemcpyAsync(dtab.p, tables.data(), tbytes, hipMemcpyHostToDevice, ctx->stream));
+  const SysJob *djobs = (const SysJob *)(dtab.p + o_jobs);
+  const int2 *drow = (const int2 *)(dtab.p + o_rows);
   std::vector<LearnedStats> ls(nb, LearnedStats{0, 0, 0});
   double alg_bytes = 0.0, alg_flops = 0.0;
   // fast forms: vertex-summed stresslet moments when every element moves rigidly as a whole
@@ -262,14 +276,14 @@ int run_wave(andr_ctx *ctx, Prepared *const *P, int nb, const andr_resistance_op
     alg_bytes += (plain ? 9.0 : 6.0) * ne * ne * esz + 3.0 * ne * ANDR_NRHS * 8.0;
     alg_flops += ne * (ne - 1.0) * jobs[i].nq * (summed ? ANDR_FLOPS_PER_STOKES_EVAL_SUM : ANDR_FLOPS_PER_STOKES_EVAL);
   }
-  if (!plain && (rc = andr_launch_self_blocks(ctx, djobs.p, drow.p, (int)rowmap.size()))) return rc;
+  if (!plain && (rc = andr_launch_self_blocks(ctx, djobs, drow, (int)nrows))) return rc;
   if (learned)
-    rc = andr_launch_stokes_system_learned(ctx, jobs.data(), djobs.p, drow.p, (int)rowmap.size(), nb, summed, ls.data());
+    rc = andr_launch_stokes_system_learned(ctx, jobs.data(), djobs, drow, (int)nrows, nb, summed, ls.data());
   else
-    rc = andr_launch_stokes_system(ctx, djobs.p, drow.p, (int)rowmap.size(), !plain, !plain, alg_bytes, alg_flops, summed);
+    rc = andr_launch_stokes_system(ctx, djobs, drow, (int)nrows, !plain, !plain, alg_bytes, alg_flops, summed);
   if (rc) return rc;
-  ANDR_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  const double ta1 = andr_now();
+  Mark assembled, finished;  // the reported times come from the device's clock: the host runs on
+  if (assembled.record(ctx->stream)) return andr_fail(ctx, ANDR_ERR_HIP, "event");
   // ---- solve ----------------------------------------------------------------------------------
   std::vector<int> iters((size_t)nb * 6, 0), stops((size_t)nb * 6, 0);
   const int nprob = opts->problems == ANDR_PROBLEMS_STRAIN ? 3 : 6;  // right-hand sides per body
@@ -303,21 +317,23 @@ int run_wave(andr_ctx *ctx, Prepared *const *P, int nb, const andr_resistance_op
         stops[(size_t)i * 6 + k] = st_g[(size_t)i * nprob + k];
       }
     if (rc) return rc;
-    if ((rc = andr_launch_unprecondition(ctx, djobs.p, drow.p, (int)rowmap.size()))) return rc;
+    if ((rc = andr_launch_unprecondition(ctx, djobs, drow, (int)nrows))) return rc;
   }
-  ANDR_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  const double ts1 = andr_now();
   // ---- force and torque on wall 1 (on the device, one copy back for the wave) ------------------
   std::vector<double> ftbuf;  // per body: 36 force/torque values and the self-check error
   {
     DevBuf<double> dft;
     if (dft.alloc((size_t)nb * 37, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "force/torque results");
-    if ((rc = andr_launch_force_torque(ctx, djobs.p, nb, dft.p))) return rc;
+    if ((rc = andr_launch_force_torque(ctx, djobs, nb, dft.p))) return rc;
     ftbuf.resize((size_t)nb * 37);
     ANDR_HIP(ctx, hipMemcpyAsync(ftbuf.data(), dft.p, sizeof(double) * ftbuf.size(), hipMemcpyDeviceToHost,
                                  ctx->stream));
+    if (finished.record(ctx->stream)) return andr_fail(ctx, ANDR_ERR_HIP, "event");
     ANDR_HIP(ctx, hipStreamSynchronize(ctx->stream));
   }
+  float solve_ms = 0.f;
+  ANDR_HIP(ctx, hipEventElapsedTime(&solve_ms, assembled.ev, finished.ev));
+  const double ts1 = andr_now(), t_solve = solve_ms * 1e-3, t_assemble = std::max(0.0, t_up + ts1 - ta0 - t_solve);
   for (int i = 0; i < nb; ++i) {
     Prepared &p = *P[i];
     const int ne = p.ne;
@@ -331,8 +347,8 @@ int run_wave(andr_ctx *ctx, Prepared *const *P, int nb, const andr_resistance_op
       }
       R.err[0] = 0.0;
       R.err[1] = ftbuf[(size_t)i * 37 + 36];
-      R.t_assemble = (t_up + ta1 - ta0) / nb;
-      R.t_solve = (ts1 - ta1) / nb;
+      R.t_assemble = t_assemble / nb;
+      R.t_solve = t_solve / nb;
       const QuadRule qr = andr_rule(p.body.itri);
       R.quad_points = learned ? ls[i].points : (int64_t)ne * (ne - 1) * qr.npts;
       R.pairs_learned = learned ? ls[i].learned : 0;
@@ -340,8 +356,8 @@ int run_wave(andr_ctx *ctx, Prepared *const *P, int nb, const andr_resistance_op
     }
   }
   if (timing)
-    fprintf(stderr, "[andr] wave of %d bodies: upload %.3f s, system set-up %.3f s, assembly %.3f s, solve %.3f s, "
-            "force/torque %.3f s\n", nb, t_up, tu1 - ta0, ta1 - tu1, ts1 - ta1, andr_now() - ts1);
+    fprintf(stderr, "[andr] wave of %d bodies: upload %.3f s, system set-up %.3f s, set-up and assembly %.3f s, "
+            "solve, force and torque %.3f s\n", nb, t_up, tu1 - ta0, t_assemble - t_up, t_solve);
   return ANDR_OK;
 }
 
