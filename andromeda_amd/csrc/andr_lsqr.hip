@@ -11,7 +11,9 @@
 // v = V / alpha); the products fold the normalisation into their scale factors, which removes the
 // separate scaling passes of the reference (dscal at :947, :974, :980).
 //
-// An iteration is three launches. A small system (an A of the order of the 256 MB cache) spends its
+// A single right-hand side of at most 8192 unknowns takes two launches an iteration and reads A once: k_lsqr_pass
+// does the work of 1. and 2. below on rows that stay in registers. Otherwise
+// an iteration is three launches. A small system (an A of the order of the 256 MB cache) spends its
 // time in the gaps and the latency of small kernels, not in the products, so the recurrences' scalar
 // work and the vector updates ride along in the products' own kernels:
 //   1. k_lsqr_av: the partial products of A V over column segments;
@@ -52,6 +54,18 @@ __device__ inline double d2norm(double a, double b) {  // lsqr_d2norm (src/lib_l
 
 typedef double d2n __attribute__((ext_vector_type(2)));
 typedef double d4v __attribute__((ext_vector_type(4)));
+
+// Loads of the system matrix. A matrix that the 256 MB cache holds is read with ordinary loads (KEEP): what of it
+// is left in an L2 from the product before, and the second half of a line that two rows share, are then hits.
+// A larger one is streamed past them. Measured: one pass over 106 MB 21.6 us streamed, 18.8 kept, 20 MB 9.9 and
+// 7.5, FP32 96 MB 25.8 and 20.5; A^T U of 78 MB 20.0 and 17.2, A V 15.5 and 13.5; but 512 MB 84 and 90, 1.15 GB 173
+// and 188.
+constexpr double KEEP_BYTES = 256e6;
+template <bool KEEP, class P>
+__device__ inline auto stream_load(P p) {
+  if constexpr (KEEP) return *p;
+  else return __builtin_nontemporal_load(p);
+}
 typedef float f4n __attribute__((ext_vector_type(4)));
 
 // ---- scalar state ----------------------------------------------------------------------------
@@ -203,6 +217,7 @@ struct LsqrVecs {
   double *partU;                // |U|^2 per block of the kernel that forms U
   const double *partV, *partW;  // |V|^2, |W|^2 per block of k_lsqr_v
   int npv;
+  LsqrState *host;              // a copy of state B for the host (pinned memory), or null
 };
 
 // The scales of U for the kernel that forms it, from a thread's share of the |V|^2 partials:
@@ -222,14 +237,14 @@ __device__ inline void lsqr_u_prologue(const LsqrVecs &L, double svt, double *re
 // some forty dependent operations would hold up a block that has a share of the product); host: a copy
 // for the host (pinned memory) or null.
 template <int WD, int BS>
-__device__ inline void lsqr_end_block(const LsqrVecs &L, double *red, LsqrState *host) {
+__device__ inline void lsqr_end_block(const LsqrVecs &L, double *red) {
   const double svt = thread_parts<WD, BS>(L.partV, L.npv), swt = thread_parts<WD, BS>(L.partW, L.npv);
   const double sv = block_sum<WD, BS>(svt, red), sw = block_sum<WD, BS>(swt, red);
   if (threadIdx.x < WD) {
     LsqrState S = L.sa[threadIdx.x];
     lsqr_end(S, sv, sw);
     L.sb[threadIdx.x] = S;
-    if (host) host[threadIdx.x] = S;
+    if (L.host) L.host[threadIdx.x] = S;
   }
 }
 
@@ -256,7 +271,7 @@ constexpr int AV_MAXCOLS = 1024;  // columns per wave at most
 
 // SEP: the waves' sums stay apart, P[segment * AV_WAVES + wave] (BiCGSTAB, whose iterates part from
 // each other by far more than rounding when the sums of a product are formed in another order).
-template <int T, bool LINES, bool SEP>
+template <int T, bool LINES, bool SEP, bool KEEP>
 __global__ __launch_bounds__(64 * AV_WAVES) void k_lsqr_av(const double *__restrict__ A, int64_t lda, int m, int n,
                                                            const double *__restrict__ X, int wcols,
                                                            double *__restrict__ P,
@@ -286,13 +301,12 @@ __global__ __launch_bounds__(64 * AV_WAVES) void k_lsqr_av(const double *__restr
   d4v acc[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) acc[t] = d4v{0.0, 0.0, 0.0, 0.0};
-  // the matrix is streamed: non-temporal, so that X keeps its place in L2
   auto lines = [&](int j, double (&a)[T][4]) {
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const d2n u = __builtin_nontemporal_load((const d2n __attribute__((address_space(1))) *)(lrow[t][h] + 16 * j));
+        const d2n u = stream_load<KEEP>((const d2n __attribute__((address_space(1))) *)(lrow[t][h] + 16 * j));
         a[t][2 * h] = u.x;
         a[t][2 * h + 1] = u.y;
       }
@@ -424,7 +438,7 @@ __global__ __launch_bounds__(64 * AV_WAVES) void k_lsqr_av(const double *__restr
 
 // P[segment][row] = A x for one right-hand side: a wave owns eight rows over a column segment, 16 bytes
 // per lane and row (1 KB of a row per load), two register sets in turn; bound by the matrix stream.
-template <class ST>
+template <class ST, bool KEEP>
 __global__ __launch_bounds__(256) void k_lsqr_av1(const ST *__restrict__ A, int64_t lda, int m, int n,
                                                   const double *__restrict__ x, int seglen, double *__restrict__ P,
                                                   const LsqrState *__restrict__ st) {
@@ -450,7 +464,7 @@ __global__ __launch_bounds__(256) void k_lsqr_av1(const ST *__restrict__ A, int6
   auto load = [&](int k, Set &s) {
     const int j = k + CPL * lane;
 #pragma unroll
-    for (int r = 0; r < 8; ++r) s.a[r] = __builtin_nontemporal_load((gvp)(row[r] + j));
+    for (int r = 0; r < 8; ++r) s.a[r] = stream_load<KEEP>((gvp)(row[r] + j));
 #pragma unroll
     for (int q = 0; q < CPL; ++q) s.x[q] = x[j + q];
   };
@@ -518,7 +532,7 @@ __global__ __launch_bounds__(256) void k_lsqr_av1(const ST *__restrict__ A, int6
 constexpr int AT_WAVES = 8, AT_MAXRW = 32;
 constexpr int at_cols(size_t elem) { return 64 * 16 / (int)elem; }  // a 16-byte load per lane
 
-template <class ST, int WD, bool FORM>
+template <class ST, int WD, bool FORM, bool KEEP>
 __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restrict__ A, int64_t lda, int m, int n, int rw,
                                                             LsqrVecs L, double *__restrict__ P) {
   constexpr int BS = 64 * AT_WAVES, CW = at_cols(sizeof(ST)), LV = CW / 64;  // columns per lane
@@ -530,7 +544,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restr
   __shared__ double sc[2 * WD];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   if (FORM && blockIdx.y == gridDim.y - 1) {  // one block more for the scalars
-    if (blockIdx.x == 0) lsqr_end_block<WD, BS>(L, red, nullptr);
+    if (blockIdx.x == 0) lsqr_end_block<WD, BS>(L, red);
     return;
   }
   const int i0 = blockIdx.y * AT_WAVES * rw, nr = min(AT_WAVES * rw, m - i0);  // nr >= 1
@@ -548,7 +562,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restr
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
       const ST *row = base + (size_t)min(r0 + min(r + u, max(rn - 1, 0)), nr - 1) * lda;
-      s.a[u] = __builtin_nontemporal_load((gvp)(row + jc));
+      s.a[u] = stream_load<KEEP>((gvp)(row + jc));
     }
   };
   Set s0, s1;
@@ -656,13 +670,191 @@ __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restr
     }
 }
 
+// ---- both products of an iteration in one pass over A (one right-hand side) ----------------------
+// A row gives u_i = sx (A_i v) + sy u_i and then takes u_i A_i into A^T u, whose normalisation comes later
+// anyway: with a block owning whole rows (rpb of them, n <= 1024 PASS_CHUNKS PASS_LV columns over its 1024 threads)
+// they stay in registers in between, and A is read once per iteration instead of twice. A thread holds CH
+// pairs of columns of R rows in each of two register sets, its part of v and of A^T u. The rows' sums
+// meet in LDS, one barrier per R rows: a wave adds across its halves and 16-lane rows with lane swaps, each wave
+// then sums the sixteen waves' shares for itself. One block per CU, each with its part of A^T u for
+// k_lsqr_v. A block's rows, and its XCD, are the same in every iteration. Bound by the matrix stream: 4881 x
+// 2717 18.8 us where the two products took 20.3 and 19.4, 1587^2 7.5 (6.2 + 8.2), 4897^2 in FP32 20.5 (17.5 + 16.2).
+constexpr int PASS_BS = 1024, PASS_BLOCKS = 255, PASS_CHUNKS = 4, PASS_LV = 2;
+// rows of a register set: 128 bytes a thread in both
+constexpr int pass_rows(size_t elem, int ch) { return (ch == 1 ? 8 : ch == 2 ? 4 : 2) * (elem == 4 && ch > 1 ? 2 : 1); }
+
+// a over lanes i and i + 32 in the lower half, b's in the upper half
+__device__ inline double swap_add32(double a, double b) {
+  const uint64_t ua = __builtin_bit_cast(uint64_t, a), ub = __builtin_bit_cast(uint64_t, b);
+  const auto l = __builtin_amdgcn_permlane32_swap((unsigned)ua, (unsigned)ub, false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+  return __builtin_bit_cast(double, (uint64_t)h[0] << 32 | l[0]) + __builtin_bit_cast(double, (uint64_t)h[1] << 32 | l[1]);
+}
+// the same for neighbouring rows of 16 lanes: a in the even ones, b in the odd ones
+__device__ inline double swap_add16(double a, double b) {
+  const uint64_t ua = __builtin_bit_cast(uint64_t, a), ub = __builtin_bit_cast(uint64_t, b);
+  const auto l = __builtin_amdgcn_permlane16_swap((unsigned)ua, (unsigned)ub, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+  return __builtin_bit_cast(double, (uint64_t)h[0] << 32 | l[0]) + __builtin_bit_cast(double, (uint64_t)h[1] << 32 | l[1]);
+}
+template <int CTRL>
+__device__ inline double dpp_add(double a) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, a);
+  const unsigned l = __builtin_amdgcn_mov_dpp((int)u, CTRL, 0xf, 0xf, true),
+                 h = __builtin_amdgcn_mov_dpp((int)(u >> 32), CTRL, 0xf, 0xf, true);
+  return a + __builtin_bit_cast(double, (uint64_t)h << 32 | l);
+}
+// the sum over each row of 16 lanes, in all of them (rotations by 8, 4, 2 and 1)
+__device__ inline double row_sum16(double a) {
+  return dpp_add<0x121>(dpp_add<0x122>(dpp_add<0x124>(dpp_add<0x128>(a))));
+}
+__device__ inline double read_lane(double a, int lane) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, a);
+  const unsigned l = __builtin_amdgcn_readlane((int)u, lane), h = __builtin_amdgcn_readlane((int)(u >> 32), lane);
+  return __builtin_bit_cast(double, (uint64_t)h << 32 | l);
+}
+
+template <class ST, int CH, bool KEEP>
+__global__ __launch_bounds__(PASS_BS) void k_lsqr_pass(const ST *__restrict__ A, int64_t lda, int m, int n, int rpb,
+                                                       const double *__restrict__ V, LsqrVecs L,
+                                                       double *__restrict__ P) {
+  constexpr int LV = PASS_LV, R = pass_rows(sizeof(ST), CH), RQ = (R + 3) / 4;
+  typedef ST vec __attribute__((ext_vector_type(LV)));
+  typedef const vec __attribute__((address_space(1))) *gvp;
+  __shared__ double red[2][R][16], pre[PASS_BS / 64], sc[2];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, g = lane >> 4, w = lane & 15;
+  if (blockIdx.x == gridDim.x - 1) {  // one block more for the scalars
+    lsqr_end_block<1, PASS_BS>(L, pre);
+    return;
+  }
+  const int i0 = blockIdx.x * rpb, nr = min(rpb, m - i0);  // nr >= 1
+  const ST *base = A + (size_t)i0 * lda;
+  // row of the R in this lane's row of 16 lanes (q = 0, 1): where the sums end up
+  auto rof = [&](int q) { return R == 2 ? g >> 1 : g + 4 * q; };
+  struct Set {
+    vec a[R][CH];
+    double u[RQ];  // the old U of the rows rof(q)
+  };
+  auto load = [&](int r, Set &s) {
+#pragma unroll
+    for (int rr = 0; rr < R; ++rr) {
+      const ST *row = base + (size_t)min(r + rr, nr - 1) * lda;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        const int j = LV * (tid + PASS_BS * c);
+        const gvp p = (gvp)(row + (c < CH - 1 || j < n ? j : 0));  // all pieces but the last are within the row
+        s.a[rr][c] = stream_load<KEEP>(p);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) s.u[q] = L.uin[i0 + min(r + rof(q), nr - 1)];
+  };
+  Set s0, s1;
+  load(0, s0);  // the first rows are under way while the scalars are formed
+  const bool act = any_active<1>(L.sa);
+  const double svt = thread_parts<1, PASS_BS>(L.partV, L.npv);
+  double x[CH][LV], acc[CH][LV];
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+#pragma unroll
+    for (int q = 0; q < LV; ++q) {
+      const int j = LV * (tid + PASS_BS * c) + q;
+      x[c][q] = j < n ? V[j] : 0.0;
+      acc[c][q] = 0.0;
+    }
+  __builtin_amdgcn_sched_barrier(0);
+  if (!act) return;  // uniform over the grid
+  lsqr_u_prologue<1, PASS_BS>(L, svt, pre, sc);
+  const double sx = sc[0], sy = sc[1];
+  double y2 = 0.0;
+  auto dots = [&](const Set &s, int b) {
+    double d[R];
+#pragma unroll
+    for (int rr = 0; rr < R; ++rr) {
+      d[rr] = 0.0;
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int q = 0; q < LV; ++q) {
+          double a = (double)s.a[rr][c][q];
+          if (c == CH - 1 && LV * (tid + PASS_BS * c) + q >= n) a = 0.0;  // row padding, whatever it holds
+          d[rr] += a * x[c][q];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) {
+      double t;
+      if constexpr (R == 2) {
+        const double h = swap_add32(d[0], d[1]);
+        t = swap_add16(h, h);
+      } else {
+        t = swap_add16(swap_add32(d[4 * q], d[4 * q + 2]), swap_add32(d[4 * q + 1], d[4 * q + 3]));
+      }
+      t = row_sum16(t);
+      if (w == 0) red[b][rof(q)][wid] = t;
+    }
+  };
+  auto update = [&](int r, const Set &s, int b) {
+    double y[RQ];
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) {
+      const double t = row_sum16(red[b][rof(q)][w]);
+      y[q] = r + rof(q) < nr ? sx * t + sy * s.u[q] : 0.0;
+      if (wid == 0 && w == 0 && (R > 2 || (g & 1) == 0) && r + rof(q) < nr) {
+        L.uout[i0 + r + rof(q)] = y[q];
+        y2 += y[q] * y[q];
+      }
+    }
+#pragma unroll
+    for (int rr = 0; rr < R; ++rr) {
+      const double yr = read_lane(y[rr / 4], R == 2 ? 32 * rr : 16 * (rr & 3));
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        vec a = s.a[rr][c];
+        if (sizeof(ST) == 4) asm("" : "+v"(a));  // converted again: the FP64 values kept from dots() would spill
+#pragma unroll
+        for (int q = 0; q < LV; ++q) acc[c][q] += (double)a[q] * yr;
+      }
+    }
+  };
+  // (asking for both sets before the scalars and for each again as soon as it is used up: 21.9 against 21.5 us)
+#pragma unroll 1
+  for (int r = 0; r < nr; r += 2 * R) {
+    load(r + R, s1);
+    __builtin_amdgcn_sched_barrier(0);
+    dots(s0, 0);
+    __syncthreads();
+    update(r, s0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (r + R >= nr) break;  // uniform over the block
+    load(r + 2 * R, s0);
+    __builtin_amdgcn_sched_barrier(0);
+    dots(s1, 1);
+    __syncthreads();
+    update(r + R, s1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+#pragma unroll
+    for (int q = 0; q < LV; ++q) {
+      const int j = LV * (tid + PASS_BS * c) + q;
+      if (j < n) P[(size_t)blockIdx.x * n + j] = acc[c][q];
+    }
+  if (wid == 0) {
+    y2 += __shfl_xor(y2, 16, 64);
+    y2 += __shfl_xor(y2, 32, 64);
+    if (tid == 0) L.partU[blockIdx.x] = y2;
+  }
+}
+
 // U formed on its own (many column segments, CSR): U = sx .* sum_s P[s] + sy .* U, |U|^2 per block.
 template <int WD>
 __global__ __launch_bounds__(256) void k_lsqr_u(int m, LsqrVecs L) {
   __shared__ double red[4 * WD];
   __shared__ double sc[2 * WD];
   if (blockIdx.x == gridDim.x - 1) {  // one block more for the scalars
-    lsqr_end_block<WD, 256>(L, red, nullptr);
+    lsqr_end_block<WD, 256>(L, red);
     return;
   }
   const bool act = any_active<WD>(L.sa);
@@ -687,18 +879,20 @@ __global__ __launch_bounds__(256) void k_lsqr_u(int m, LsqrVecs L) {
 // old V): X += t1 W, W = V / alpha + t2 W; |V|^2 and |W|^2 per block. beta = |U| first. INIT: V = sum_s P[s] / beta, W = 0 before the first iteration.
 // A block's 256 threads are 64 values (j, k) times four quarters of the splits; at most V_MAXBLOCKS
 // blocks, so that the norms are few partials for the kernels that sum them.
-constexpr int V_QUARTERS = 4, V_VALUES = 256 / V_QUARTERS, V_MAXBLOCKS = 512;
+// (After k_lsqr_pass, with its 255 splits: 16 values times sixteen shares.)
+constexpr int V_MAXBLOCKS = 512;
+constexpr int v_values(int shares) { return 256 / shares; }
 
-template <int WD, bool INIT>
+template <int WD, bool INIT, int SHARES>
 __global__ __launch_bounds__(256) void k_lsqr_v(int n, int nsplit, const double *__restrict__ P, LsqrState *sa,
                                                 LsqrState *sb, const double *__restrict__ partU, int npu,
                                                 double *__restrict__ V, double *__restrict__ X, double *__restrict__ W,
                                                 double *__restrict__ partV, double *__restrict__ partW) {
-  constexpr int NV = V_VALUES;
+  constexpr int NV = v_values(SHARES);
   __shared__ double red[4 * WD];
   __shared__ double sc[2 * WD], st[3 * WD];
   __shared__ int su[WD];
-  __shared__ double part[V_QUARTERS][NV];
+  __shared__ double part[SHARES][NV];
   const int tid = threadIdx.x;
   // k is the same in every turn of the loop below (NV % WD == 0, also times the grid)
   const int val = tid % NV, q = tid / NV, k = val % WD;
@@ -710,11 +904,12 @@ __global__ __launch_bounds__(256) void k_lsqr_v(int n, int nsplit, const double 
     if (t >= n * WD) return;
     const double *p = P + t;
     const size_t stride = (size_t)n * WD;
-    for (int sp = q; sp < nsplit; sp += 8 * V_QUARTERS) {
+    for (int sp = q; sp < nsplit; sp += 8 * SHARES) {
       double a[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) a[u] = sp + u * V_QUARTERS < nsplit ? p[(sp + u * V_QUARTERS) * stride] : 0.0;
-      c.s += ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+      for (int u = 0; u < 8; ++u) a[u] = sp + u * SHARES < nsplit ? p[(sp + u * SHARES) * stride] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) c.s += a[u];
     }
     if (!INIT && q == 0) {
       c.v = V[t];
@@ -762,8 +957,11 @@ __global__ __launch_bounds__(256) void k_lsqr_v(int n, int nsplit, const double 
     __syncthreads();
     const double vold = cur.v, wold = cur.w, xold = cur.x;
     if (t0 + gridDim.x * NV < n * WD) load(t + gridDim.x * NV, cur);
-    if (q == 0 && t < n * WD) {  // the first wave holds the turn's values
-      const double s = (part[0][val] + part[1][val]) + (part[2][val] + part[3][val]);
+    if (q == 0 && t < n * WD) {  // the first share's lanes hold the turn's values
+      double s = 0.0;
+#pragma unroll
+      for (int h = 0; h < SHARES; h += 4)
+        s += (part[h][val] + part[h + 1][val]) + (part[h + 2][val] + part[h + 3][val]);
       if (INIT) {
         const double v = sc[k] * s;
         V[t] = v;
@@ -784,7 +982,7 @@ __global__ __launch_bounds__(256) void k_lsqr_v(int n, int nsplit, const double 
       }
     }
   }
-  if (q != 0) return;
+  if (tid >= 64) return;  // the first wave's first NV lanes hold the sums, the others zeros
 #pragma unroll
   for (int o = WD; o < 64; o <<= 1) {
     v2 += __shfl_xor(v2, o, 64);
@@ -865,11 +1063,11 @@ __global__ __launch_bounds__(256) void k_lsqr_start(LsqrState *sa, LsqrState *sb
   sb[k] = S;
 }
 
-// the state at the end of the last enqueued iteration, for the host: what the next k_lsqr_atu writes
+// the state at the end of the last iteration of all (the limit): what the next one's end block would write
 template <int WD>
-__global__ __launch_bounds__(256) void k_lsqr_poll(LsqrVecs L, LsqrState *host) {
+__global__ __launch_bounds__(256) void k_lsqr_poll(LsqrVecs L) {
   __shared__ double red[4 * WD];
-  lsqr_end_block<WD, 256>(L, red, host);
+  lsqr_end_block<WD, 256>(L, red);
 }
 
 // x = q .* (x + the owed update) + x0, into the interleaved X
@@ -994,12 +1192,17 @@ template <int T, bool SEP>
 void launch_av_t(hipStream_t st, const double *A, int64_t lda, int m, int n, const double *X, AvShape sh, double *P,
                  const std::conditional_t<SEP, BicgState, LsqrState> *s) {
   const dim3 grid((m + 16 * T - 1) / (16 * T), sh.nseg), blk(64 * AV_WAVES);
-  if (lda % 16 == 0 && (uintptr_t)A % 128 == 0)
-    hipLaunchKernelGGL((k_lsqr_av<T, true, SEP>), grid, blk, 0, st, A, lda, m, n, X, sh.wcols, P, s);
-  else if constexpr (T <= 4)
-    hipLaunchKernelGGL((k_lsqr_av<T, false, SEP>), grid, blk, 0, st, A, lda, m, n, X, sh.wcols, P, s);
-  else  // two lines of eight tiles do not fit the LDS
-    launch_av_t<4, SEP>(st, A, lda, m, n, X, sh, P, s);
+  const bool lines = lda % 16 == 0 && (uintptr_t)A % 128 == 0;
+  if constexpr (T > 4)
+    if (!lines) return launch_av_t<4, SEP>(st, A, lda, m, n, X, sh, P, s);  // two lines of eight tiles do not fit the LDS
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, blk, 0, st, A, lda, m, n, X, sh.wcols, P, s); };
+  const bool keep = (double)m * lda * sizeof(double) <= KEEP_BYTES;
+  if (lines && keep) go(k_lsqr_av<T, true, SEP, true>);
+  else if (lines) go(k_lsqr_av<T, true, SEP, false>);
+  else if constexpr (T <= 4) {
+    if (keep) go(k_lsqr_av<T, false, SEP, true>);
+    else go(k_lsqr_av<T, false, SEP, false>);
+  }
 }
 template <bool SEP>
 void launch_av(hipStream_t st, int tiles, const double *A, int64_t lda, int m, int n, const double *X, AvShape sh,
@@ -1026,6 +1229,7 @@ struct LsqrRun {
   int rw = 8, splits = 1;  // A^T U: rows per wave, row splits
   int blocksV = 0, partsU = 0;
   bool fuse = false;  // U is formed in the A^T U kernel
+  int rpb = 0, blocksP = 0, chunks = 0;  // both products in one pass: rows per block and blocks (0: not so)
   int cur = 0;        // U of the last iteration is U[cur]
   // sparse mode: A and A^T in CSR (0-based, device); A is then unused
   const int64_t *cia = nullptr, *tia = nullptr;
@@ -1051,7 +1255,10 @@ struct LsqrRun {
     for (auto e : ev)
       if (e) (void)hipEventDestroy(e);
   }
-  int tok(const char *name, double bytes) { return st == ctx->stream ? andr_prof_begin(ctx, name, bytes, aflops) : -1; }
+  int tok(const char *name, double bytes) { return tok(name, bytes, aflops); }
+  int tok(const char *name, double bytes, double flops) {
+    return st == ctx->stream ? andr_prof_begin(ctx, name, bytes, flops) : -1;
+  }
   LsqrState *sa() const { return S.p; }
   LsqrState *sb() const { return S.p + NB; }
 
@@ -1103,7 +1310,7 @@ struct LsqrRun {
   }
 
   LsqrVecs vecs() {
-    return {sa(), sb(), PN.p, av.nseg, U[cur].p, U[cur ^ 1].p, partU.p, partV.p, partW.p, blocksV};
+    return {sa(), sb(), PN.p, av.nseg, U[cur].p, U[cur ^ 1].p, partU.p, partV.p, partW.p, blocksV, nullptr};
   }
   // A Xin into the segment partials
   void gemv_n(const double *Xin) {
@@ -1112,10 +1319,14 @@ struct LsqrRun {
       hipLaunchKernelGGL(k_csr_mv, dim3((m + 31) / 32), dim3(256), 0, st, m, cia, cja, cva, Xin, PN.p, sb());
     } else if (wd == 1) {
       const dim3 grid((m + 31) / 32, av.nseg);
-      if (fp32)
-        hipLaunchKernelGGL(k_lsqr_av1<float>, grid, dim3(256), 0, st, (const float *)A, lda, m, n, Xin, av.wcols, PN.p, sb());
-      else
-        hipLaunchKernelGGL(k_lsqr_av1<double>, grid, dim3(256), 0, st, (const double *)A, lda, m, n, Xin, av.wcols, PN.p, sb());
+      const bool keep = (double)m * lda * (fp32 ? 4 : 8) <= KEEP_BYTES;
+      auto go = [&](auto kernel, auto elem) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, (const decltype(elem) *)A, lda, m, n, Xin, av.wcols, PN.p, sb());
+      };
+      if (fp32 && keep) go(k_lsqr_av1<float, true>, 0.0f);
+      else if (fp32) go(k_lsqr_av1<float, false>, 0.0f);
+      else if (keep) go(k_lsqr_av1<double, true>, 0.0);
+      else go(k_lsqr_av1<double, false>, 0.0);
     } else {
       launch_av<false>(st, tilesN, (const double *)A, lda, m, n, Xin, av, PN.p, sb());
     }
@@ -1128,18 +1339,22 @@ struct LsqrRun {
     const dim3 grid((n + cols - 1) / cols, splits + (form ? 1 : 0)), blk(64 * AT_WAVES);
     if (cia) {
       hipLaunchKernelGGL(k_csr_mv, dim3((n + 31) / 32), dim3(256), 0, st, n, tia, tja, tva, L.uin, P.p, sb());
-    } else if (wd == 1) {
-      if (fp32) {
-        if (form) hipLaunchKernelGGL((k_lsqr_atu<float, 1, true>), grid, blk, 0, st, (const float *)A, lda, m, n, rw, L, P.p);
-        else hipLaunchKernelGGL((k_lsqr_atu<float, 1, false>), grid, blk, 0, st, (const float *)A, lda, m, n, rw, L, P.p);
-      } else {
-        if (form) hipLaunchKernelGGL((k_lsqr_atu<double, 1, true>), grid, blk, 0, st, (const double *)A, lda, m, n, rw, L, P.p);
-        else hipLaunchKernelGGL((k_lsqr_atu<double, 1, false>), grid, blk, 0, st, (const double *)A, lda, m, n, rw, L, P.p);
-      }
-    } else if (form) {
-      hipLaunchKernelGGL((k_lsqr_atu<double, NB, true>), grid, blk, 0, st, (const double *)A, lda, m, n, rw, L, P.p);
     } else {
-      hipLaunchKernelGGL((k_lsqr_atu<double, NB, false>), grid, blk, 0, st, (const double *)A, lda, m, n, rw, L, P.p);
+      const bool keep = (double)m * lda * (fp32 ? 4 : 8) <= KEEP_BYTES;
+      auto go = [&](auto kernel, auto elem) {
+        hipLaunchKernelGGL(kernel, grid, blk, 0, st, (const decltype(elem) *)A, lda, m, n, rw, L, P.p);
+      };
+      auto pick = [&](auto wdc, auto elem) {
+        typedef decltype(elem) E;
+        constexpr int W = decltype(wdc)::value;
+        if (form && keep) go(k_lsqr_atu<E, W, true, true>, elem);
+        else if (form) go(k_lsqr_atu<E, W, true, false>, elem);
+        else if (keep) go(k_lsqr_atu<E, W, false, true>, elem);
+        else go(k_lsqr_atu<E, W, false, false>, elem);
+      };
+      if (wd != 1) pick(std::integral_constant<int, NB>{}, 0.0);
+      else if (fp32) pick(std::integral_constant<int, 1>{}, 0.0f);
+      else pick(std::integral_constant<int, 1>{}, 0.0);
     }
     andr_prof_end(ctx, t);
   }
@@ -1182,12 +1397,21 @@ struct LsqrRun {
     rw = 16;
     while (rw < AT_MAXRW && panels * ((m + AT_WAVES * rw - 1) / (AT_WAVES * rw) + 1) > 512) rw += wd == 1 ? 16 : 8;
     splits = cia ? 1 : (m + AT_WAVES * rw - 1) / (AT_WAVES * rw);
-    blocksV = std::min((n * wd + V_VALUES - 1) / V_VALUES, V_MAXBLOCKS);
+    // one pass over A where a block's threads hold whole rows (4881 x 2717, with k_lsqr_v: 24 us an iteration, 44
+    // with a kernel for each product)
+    chunks = (n + PASS_BS * PASS_LV - 1) / (PASS_BS * PASS_LV);
+    if (wd == 1 && !cia && chunks <= PASS_CHUNKS) {
+      const int R = pass_rows(fp32 ? 4 : 8, chunks);  // whole register sets: a shorter last one loads as much
+      rpb = ((m + PASS_BLOCKS - 1) / PASS_BLOCKS + R - 1) / R * R;
+      blocksP = (m + rpb - 1) / rpb;
+    }
+    const int vv = v_values(blocksP ? 16 : 4);
+    blocksV = std::min((n * wd + vv - 1) / vv, V_MAXBLOCKS);
     const int blocksM = (m * wd + 255) / 256;
-    partsU = fuse ? splits : blocksM;
+    partsU = blocksP ? blocksP : (fuse ? splits : blocksM);
     if (U[0].alloc((size_t)m * wd, ctx) || U[1].alloc((size_t)m * wd, ctx) || V.alloc((size_t)n * wd, ctx) ||
         W.alloc((size_t)n * wd, ctx) || Xl.alloc((size_t)n * wd, ctx) || Xs.alloc((size_t)n * wd, ctx) ||
-        P.alloc((size_t)splits * n * wd, ctx) || PN.alloc((size_t)av.nseg * m * wd, ctx) ||
+        P.alloc((size_t)std::max(splits, blocksP) * n * wd, ctx) || PN.alloc((size_t)av.nseg * m * wd, ctx) ||
         partU.alloc((size_t)std::max(partsU, blocksM) * wd, ctx) || partB.alloc((size_t)blocksM * wd, ctx) ||
         partV.alloc((size_t)blocksV * wd, ctx) || partW.alloc((size_t)blocksV * wd, ctx) || S.alloc(2 * NB, ctx))
       return andr_fail(ctx, ANDR_ERR_ALLOC, "LSQR workspace (m=%d n=%d)", m, n);
@@ -1221,14 +1445,13 @@ struct LsqrRun {
                        itnlim);
     cur = 0;
     gemv_t(vecs(), false);
-    hipLaunchKernelGGL((k_lsqr_v<WD, true>), dim3(blocksV), dim3(256), 0, st, n, splits, P.p, sa(), sb(),
-                       (const double *)nullptr, 0, V.p, Xl.p, W.p, partV.p, partW.p);
+    launch_v<WD, true>(splits, nullptr, 0);
     ANDR_HIP(ctx, hipGetLastError());
     return ANDR_OK;
   }
 
-  // enqueues iterations up to the next multiple of LSQR_POLL (or the iteration limit), then a kernel that
-  // leaves the columns' states in pinned host memory; no host wait
+  // enqueues iterations up to the next multiple of LSQR_POLL (or the iteration limit); the last one leaves
+  // the columns' states in pinned host memory; no host wait
   int advance() {
     if (it >= itnlim) return ANDR_OK;
     if (wd == 1) iterate<1>();
@@ -1238,22 +1461,63 @@ struct LsqrRun {
     ++polls;
     return ANDR_OK;
   }
+  template <int WD, bool INIT>
+  void launch_v(int parts, const double *pu, int npu) {
+    if (WD == 1 && blocksP)
+      hipLaunchKernelGGL((k_lsqr_v<WD, INIT, WD == 1 ? 16 : 4>), dim3(blocksV), dim3(256), 0, st, n, parts, P.p, sa(),
+                         sb(), pu, npu, V.p, Xl.p, W.p, partV.p, partW.p);
+    else
+      hipLaunchKernelGGL((k_lsqr_v<WD, INIT, 4>), dim3(blocksV), dim3(256), 0, st, n, parts, P.p, sa(), sb(), pu, npu,
+                         V.p, Xl.p, W.p, partV.p, partW.p);
+  }
+  template <class ST, int CH>
+  void pass_ch(const LsqrVecs &L) {
+    const dim3 grid(blocksP + 1), blk(PASS_BS);
+    if ((double)m * lda * sizeof(ST) <= KEEP_BYTES)
+      hipLaunchKernelGGL((k_lsqr_pass<ST, CH, true>), grid, blk, 0, st, (const ST *)A, lda, m, n, rpb, V.p, L, P.p);
+    else
+      hipLaunchKernelGGL((k_lsqr_pass<ST, CH, false>), grid, blk, 0, st, (const ST *)A, lda, m, n, rpb, V.p, L, P.p);
+  }
+  template <class ST>
+  void pass_st(const LsqrVecs &L) {
+    if (chunks == 1) pass_ch<ST, 1>(L);
+    else if (chunks == 2) pass_ch<ST, 2>(L);
+    else if (chunks == 3) pass_ch<ST, 3>(L);
+    else pass_ch<ST, 4>(L);
+  }
+  void pass(const LsqrVecs &L) {
+    const int t = tok("lsqr_pass", abytes + 2.0 * vbytes + (double)blocksP * n * 8.0, 2.0 * aflops);
+    if (fp32) pass_st<float>(L);
+    else pass_st<double>(L);
+    andr_prof_end(ctx, t);
+  }
   template <int WD>
   void iterate() {
+    LsqrState *host = slot + (polls % 2) * NB;
+    bool last;
     do {
-      gemv_n(V.p);
       LsqrVecs L = vecs();
-      if (!fuse) {
-        hipLaunchKernelGGL(k_lsqr_u<WD>, dim3((m * WD + 255) / 256 + 1), dim3(256), 0, st, m, L);
-        L.uin = L.uout;
-      }
-      gemv_t(L, fuse);
-      hipLaunchKernelGGL((k_lsqr_v<WD, false>), dim3(blocksV), dim3(256), 0, st, n, splits, P.p, sa(), sb(), partU.p,
-                         partsU, V.p, Xl.p, W.p, partV.p, partW.p);
-      cur ^= 1;
       ++it;
-    } while (it % LSQR_POLL != 0 && it < itnlim);
-    hipLaunchKernelGGL(k_lsqr_poll<WD>, dim3(1), dim3(256), 0, st, vecs(), slot + (polls % 2) * NB);
+      last = it % LSQR_POLL == 0 || it >= itnlim;
+      if (last && it < itnlim) L.host = host;  // the state before this iteration, by the way
+      if (WD == 1 && blocksP) {
+        pass(L);
+      } else {
+        gemv_n(V.p);
+        if (!fuse) {
+          hipLaunchKernelGGL(k_lsqr_u<WD>, dim3((m * WD + 255) / 256 + 1), dim3(256), 0, st, m, L);
+          L.uin = L.uout;
+        }
+        gemv_t(L, fuse);
+      }
+      launch_v<WD, false>(blocksP ? blocksP : splits, partU.p, partsU);
+      cur ^= 1;
+    } while (!last);
+    if (it >= itnlim) {
+      LsqrVecs L = vecs();
+      L.host = host;
+      hipLaunchKernelGGL(k_lsqr_poll<WD>, dim3(1), dim3(256), 0, st, L);
+    }
   }
 
   // waits for the oldest poll that was not read yet; done when no column is active or the limit is
