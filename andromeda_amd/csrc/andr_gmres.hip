@@ -1055,104 +1055,6 @@ __global__ __launch_bounds__(256) void kb_bdots_final(const GSys *__restrict__ s
   if (wv == 0) (dst ? S.C2 : S.C1)[(size_t)b * 64 + lane] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
 }
 
-//   mode 0: W -= sum_(b < nb) Q_b C1_b
-//   mode 1: Q_nb = (W - sum_(b < nb) Q_b C2_b) Ri          (the next basis block)
-//   mode 2: X += sum_(b < kk) Q_b Y_b, Y in C1, kk the rounds the system used (at most nb)
-//   mode 3: Q_0 = R Ri                                      (start of a cycle)
-// A block takes a tile of 64 rows, four lanes a row, a lane two of its columns: one 16-byte load per basis
-// block, the row's other values from its neighbours (quad permutes), the coefficients staged in LDS UCH
-// blocks at a time with the next chunk's loads of both under way. With a whole row per lane, a body of 7000
-// rows was 109 waves, each with a round trip to memory every four blocks (73 rounds of it: 39.7 -> 10.8 us a
-// sweep; 40 bodies of 500 to 7220 elements 50.7 -> 33.7). Every sum runs over the blocks and columns in order, whatever the split: the Krylov vectors meet
-// FP32 products, where a last bit that differs can turn a rounding. HBM bound (the basis stream) on a
-// full batch.
-constexpr int UCH = 16;
-template <int U>
-__device__ inline double quad_lane(double x) {  // the value of lane U of the quad
-  constexpr int ctrl = U * 0x55;                 // quad_perm [U, U, U, U]
-  const long long v = __double_as_longlong(x);
-  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)v, ctrl, 0xf, 0xf, true);
-  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(v >> 32), ctrl, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)hi << 32) | lo);
-}
-__global__ __launch_bounds__(256) void kb_bupdate(const GSys *__restrict__ sys, const TileMap *__restrict__ tmap, int nb,
-                                                  int mode, int all) {
-  typedef double d2 __attribute__((ext_vector_type(2)));
-  __shared__ __attribute__((aligned(16))) double sC[2][UCH * 64];
-  static_assert(TILE == 64, "four lanes per row");
-  const TileMap tm = tmap[blockIdx.x];
-  const GSys &S = sys[tm.sys];
-  if (mode < 2 && !all && !sys_iterating(S)) return;  // the sweeps of a round; uniform over the block
-  const int n = S.n, tid = threadIdx.x, p = tid & 3;
-  int nbb = mode == 3 ? 0 : nb;
-  if (mode == 2) {  // the rounds used: the live columns freeze together (none live: no update)
-    int kk = -1;
-#pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      const double *sm = S.small + 8 * k;
-      if (sm[4] > 0.0) kk = max(kk, sm[5] > 0.0 ? min((int)sm[5], nb) : nb);
-    }
-    nbb = max(kk, 0);
-  }
-  const int row = tm.row0 + (tid >> 2);
-  const bool in = row < n;  // rows past the end repeat the last and are not stored
-  const size_t o = (size_t)(in ? row : n - 1) * NB + 2 * p, vstride = (size_t)n * NB;
-  const double *Cf = mode == 1 ? S.C2 : S.C1;
-  const double *Qr = S.Q + o;
-  const d2 x = *(const d2 *)((mode == 3 ? S.R : (mode == 2 ? S.X : S.W)) + o);
-  d2 s = {0.0, 0.0};
-  // chunk of UCH blocks from b0: this lane's values of its row, and its share of the coefficients (past the
-  // last block both repeat it and are not used)
-  static_assert(UCH * 64 == 2 * 2 * 256, "two 16-byte loads of the coefficients per thread");
-  d2 cq[UCH], cc[2];
-  auto load = [&](int b0) {
-#pragma unroll
-    for (int u = 0; u < UCH; ++u) cq[u] = *(const d2 *)(Qr + (size_t)min(b0 + u, nbb - 1) * vstride);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int e = 2 * (tid + 256 * h);  // block b0 + e / 64
-      cc[h] = *(const d2 *)(Cf + (size_t)min(b0 + (e >> 6), nbb - 1) * 64 + (e & 63));
-    }
-  };
-  if (nbb > 0) {
-    load(0);
-#pragma unroll 1
-    for (int b0 = 0, w = 0; b0 < nbb; b0 += UCH, w ^= 1) {
-      double *sc = sC[w];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) *(d2 *)&sc[2 * (tid + 256 * h)] = cc[h];
-      d2 q[UCH];
-#pragma unroll
-      for (int u = 0; u < UCH; ++u) q[u] = cq[u];
-      __syncthreads();  // this buffer is written; the other one is read (before the last barrier)
-      load(min(b0 + UCH, nbb - 1));
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int u = 0; u < UCH; ++u) {
-        if (b0 + u >= nbb) continue;  // uniform
-        const double *C = &sc[u * 64 + 2 * p];
-        const double ql[8] = {quad_lane<0>(q[u].x), quad_lane<0>(q[u].y), quad_lane<1>(q[u].x), quad_lane<1>(q[u].y),
-                              quad_lane<2>(q[u].x), quad_lane<2>(q[u].y), quad_lane<3>(q[u].x), quad_lane<3>(q[u].y)};
-#pragma unroll
-        for (int l = 0; l < 8; ++l) s += ql[l] * *(const d2 *)(C + 8 * l);
-      }
-    }
-  }
-  if (mode == 0 || mode == 2) {
-    if (in) *(d2 *)((mode == 0 ? S.W : S.X) + o) = mode == 0 ? x - s : x + s;
-    return;
-  }
-  // the row's new vector times Ri
-  const d2 v = x - s;
-  const double w[8] = {quad_lane<0>(v.x), quad_lane<0>(v.y), quad_lane<1>(v.x), quad_lane<1>(v.y),
-                       quad_lane<2>(v.x), quad_lane<2>(v.y), quad_lane<3>(v.x), quad_lane<3>(v.y)};
-  d2 out = {0.0, 0.0};
-#pragma unroll
-  for (int c = 0; c < 8; ++c) out += w[c] * *(const d2 *)(S.Ri + c * 8 + 2 * p);
-  const size_t blk = mode == 1 ? (size_t)nb : 0;  // mode 3 writes Q_0
-  if (in) *(d2 *)(S.Q + blk * vstride + o) = out;
-}
-
 __device__ inline double lane_bcast(double x, int l) {  // the value of lane l (uniform)
   const long long v = __double_as_longlong(x);
   const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)v, l), hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l);
@@ -1214,6 +1116,170 @@ __device__ inline void wave_tri_inverse(double R, double *Ri) {
     for (int a = 0; a < 8; ++a) Ri[8 * a + k] = a < L && k < L ? ri[a < L ? a : 0] : 0.0;
 }
 
+// The factor of a swept block from its Gram matrix without the part along the basis (gs, lane 8 c + i), the
+// square g0 of its column c before and the lane's share n2 of the squared coefficients
+template <int L>
+__device__ inline int gram_chol(const GSys &S, double gs, double g0, double n2, double &R) {
+  const int c = (threadIdx.x & 63) >> 3;
+  n2 += __shfl_xor(n2, 8, 64);
+  n2 += __shfl_xor(n2, 16, 64);
+  n2 += __shfl_xor(n2, 32, 64);  // lane 8 l + c: the sum of column c
+  n2 = g0 + __shfl(n2, c, 64);
+  unsigned live = 0;
+  for (int k = 0; k < L; ++k) live |= S.small[8 * k + 4] > 0.0 ? 1u << k : 0u;
+  return wave_chol<L>(gs, n2, live, 1e-20, R);
+}
+
+//   mode 0: W -= sum_(b < nb) Q_b C1_b
+//   mode 1: Q_nb = (W - sum_(b < nb) Q_b C2_b) Ri          (the next basis block)
+//   mode 2: X += sum_(b < kk) Q_b Y_b, Y in C1, kk the rounds the system used (at most nb)
+//   mode 3: Q_0 = R Ri                                      (start of a cycle)
+// A block takes a tile of 64 rows, four lanes a row, a lane two of its columns: one 16-byte load per basis
+// block, the row's other values from its neighbours (quad permutes), the coefficients staged in LDS UCH
+// blocks at a time with the next chunk's loads of both under way. With a whole row per lane, a body of 7000
+// rows was 109 waves, each with a round trip to memory every four blocks (73 rounds of it: 39.7 -> 10.8 us a
+// sweep; 40 bodies of 500 to 7220 elements 50.7 -> 33.7). Every sum runs over the blocks and columns in order,
+// whatever the split: the Krylov vectors meet FP32 products, where a last bit that differs can turn a rounding.
+// HBM bound (the basis stream) on a full batch.
+constexpr int UCH = 16;
+template <int U>
+__device__ inline double quad_lane(double x) {  // the value of lane U of the quad
+  constexpr int ctrl = U * 0x55;                 // quad_perm [U, U, U, U]
+  const long long v = __double_as_longlong(x);
+  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)v, ctrl, 0xf, 0xf, true);
+  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(v >> 32), ctrl, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | lo);
+}
+//   GL > 0 (mode 1 of kb_bround): a fifth wave forms Ri for its block from the same coefficients, GL columns
+struct UpdateLds {
+  double C[2][UCH * 64];
+  double Ri[64];
+  int on;
+};
+template <int GL>
+__device__ inline void bupdate_tile(const GSys &S, int row0, int nb, int mode, int all, UpdateLds &lds) {
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  static_assert(TILE == 64, "four lanes per row");
+  const int n = S.n, tid = threadIdx.x, p = tid & 3;
+  const bool sweeps = GL == 0 || tid < 256;
+  int nbb = mode == 3 ? 0 : nb;
+  if (mode == 2) {  // the rounds used: the live columns freeze together (none live: no update)
+    int kk = -1;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      const double *sm = S.small + 8 * k;
+      if (sm[4] > 0.0) kk = max(kk, sm[5] > 0.0 ? min((int)sm[5], nb) : nb);
+    }
+    nbb = max(kk, 0);
+  }
+  const int row = row0 + (tid >> 2);
+  const bool in = row < n;  // rows past the end repeat the last and are not stored
+  const size_t o = (size_t)(in ? row : n - 1) * NB + 2 * p, vstride = (size_t)n * NB;
+  const double *Cf = mode == 1 ? S.C2 : S.C1;
+  // the fifth wave (kb_bsmall's third): the Gram matrix of the swept block, lane 8 c + i
+  const int lane = tid & 63, gc = lane >> 3, gi = lane & 7;
+  double gs = 0.0, g0 = 0.0, n2 = 0.0, wc[UCH];
+  auto load1 = [&](int b0) {
+#pragma unroll
+    for (int u = 0; u < UCH; ++u) wc[u] = S.C1[(size_t)min(b0 + u, nbb - 1) * 64 + lane];
+  };
+  if (GL > 0 && !sweeps) {
+    gs = S.C2[(size_t)nb * 64 + lane];
+    g0 = S.C2[(size_t)nb * 64 + 9 * gc];
+    load1(0);
+    if (lane == 0) lds.on = all || sys_iterating(S);
+  }
+  const double *Qr = S.Q + o;
+  d2 x = {0.0, 0.0};
+  if (sweeps) x = *(const d2 *)((mode == 3 ? S.R : (mode == 2 ? S.X : S.W)) + o);
+  d2 s = {0.0, 0.0};
+  // chunk of UCH blocks from b0: this lane's values of its row, and its share of the coefficients (past the
+  // last block both repeat it and are not used)
+  static_assert(UCH * 64 == 2 * 2 * 256, "two 16-byte loads of the coefficients per thread");
+  d2 cq[UCH], cc[2];
+  auto load = [&](int b0) {
+#pragma unroll
+    for (int u = 0; u < UCH; ++u) cq[u] = *(const d2 *)(Qr + (size_t)min(b0 + u, nbb - 1) * vstride);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int e = 2 * (tid + 256 * h);  // block b0 + e / 64
+      cc[h] = *(const d2 *)(Cf + (size_t)min(b0 + (e >> 6), nbb - 1) * 64 + (e & 63));
+    }
+  };
+  if (nbb > 0) {
+    if (sweeps) load(0);
+#pragma unroll 1
+    for (int b0 = 0, w = 0; b0 < nbb; b0 += UCH, w ^= 1) {
+      double *sc = lds.C[w];
+      if (sweeps)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) *(d2 *)&sc[2 * (tid + 256 * h)] = cc[h];
+      d2 q[UCH];
+#pragma unroll
+      for (int u = 0; u < UCH; ++u) q[u] = cq[u];
+      __syncthreads();  // this buffer is written; the other one is read (before the last barrier)
+      if constexpr (GL > 0) {
+        if (b0 == 0 && !lds.on) return;  // read once for the block: kb_bsmall's part clears it in this launch
+        if (!sweeps) {
+          const int nr = min(UCH, nbb - b0);
+#pragma unroll
+          for (int u = 0; u < UCH; ++u)
+            if (u < nr) n2 += wc[u] * wc[u];  // lane 8 l + c of a block is its entry [l][c]
+          load1(min(b0 + UCH, nbb - 1));
+          for (int u = 0; u < nr; ++u)
+#pragma unroll
+            for (int l = 0; l < GL; ++l) gs = fma(-sc[u * 64 + l * 8 + gc], sc[u * 64 + l * 8 + gi], gs);
+          continue;
+        }
+      }
+      load(min(b0 + UCH, nbb - 1));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < UCH; ++u) {
+        if (b0 + u >= nbb) continue;  // uniform
+        const double *C = &sc[u * 64 + 2 * p];
+        const double ql[8] = {quad_lane<0>(q[u].x), quad_lane<0>(q[u].y), quad_lane<1>(q[u].x), quad_lane<1>(q[u].y),
+                              quad_lane<2>(q[u].x), quad_lane<2>(q[u].y), quad_lane<3>(q[u].x), quad_lane<3>(q[u].y)};
+#pragma unroll
+        for (int l = 0; l < 8; ++l) s += ql[l] * *(const d2 *)(C + 8 * l);
+      }
+    }
+  }
+  if (mode == 0 || mode == 2) {
+    if (in) *(d2 *)((mode == 0 ? S.W : S.X) + o) = mode == 0 ? x - s : x + s;
+    return;
+  }
+  const double *Ri = S.Ri;
+  if constexpr (GL > 0) {
+    if (!sweeps) {
+      double R;
+      (void)gram_chol<GL>(S, gs, g0, n2, R);
+      wave_tri_inverse<GL>(R, lds.Ri);
+    }
+    __syncthreads();
+    if (!sweeps) return;
+    Ri = lds.Ri;
+  }
+  // the row's new vector times Ri
+  const d2 v = x - s;
+  const double w[8] = {quad_lane<0>(v.x), quad_lane<0>(v.y), quad_lane<1>(v.x), quad_lane<1>(v.y),
+                       quad_lane<2>(v.x), quad_lane<2>(v.y), quad_lane<3>(v.x), quad_lane<3>(v.y)};
+  d2 out = {0.0, 0.0};
+#pragma unroll
+  for (int c = 0; c < 8; ++c) out += w[c] * *(const d2 *)(Ri + c * 8 + 2 * p);
+  const size_t blk = mode == 1 ? (size_t)nb : 0;  // mode 3 writes Q_0
+  if (in) *(d2 *)(S.Q + blk * vstride + o) = out;
+}
+
+__global__ __launch_bounds__(256) void kb_bupdate(const GSys *__restrict__ sys, const TileMap *__restrict__ tmap, int nb,
+                                                  int mode, int all) {
+  __shared__ __attribute__((aligned(16))) UpdateLds lds;
+  const TileMap tm = tmap[blockIdx.x];
+  const GSys &S = sys[tm.sys];
+  if (mode < 2 && !all && !sys_iterating(S)) return;  // the sweeps of a round; uniform over the block
+  bupdate_tile<0>(S, tm.row0, nb, mode, all, lds);
+}
+
 // block per system of the cycle: Q_0 = R R0^-1 from the Gram matrix of the residual block (C2 block 0),
 // g = (R0; 0). Dead columns (converged or beyond nrhs) take no part.
 __global__ __launch_bounds__(256) void kb_binit(const GSys *__restrict__ sys, int m, int L) {
@@ -1245,16 +1311,24 @@ __global__ __launch_bounds__(256) void kb_binit(const GSys *__restrict__ sys, in
 // over 71 of six (one wave, one reflector at a time, the factorisation on one lane).
 constexpr int BCH = 8;  // rounds per LDS chunk
 template <int L>
-__global__ __launch_bounds__(192) void kb_bsmall(const GSys *__restrict__ sys, int j, double tol, int all) {
-  constexpr int M2 = 2 * L, QP = M2 + 2;  // rows of the window; padded row of a matrix in LDS
+struct SmallLds {
+  static constexpr int M2 = 2 * L, QP = M2 + 2;  // rows of the window; padded row of a matrix
+  double Q[2][BCH][M2 * QP];
+  double W[NB][16];
+  double C[3][BCH][64];  // waves 0, 1: entering rows (block b + 1 of C1 + C2); wave 2: C2
+  double R[64];
+  int brk;
+};
+// (waves past the third only meet the others; ri: the inverse of the factor goes to memory)
+template <int L>
+__device__ inline void bsmall_round(const GSys &S, int j, double tol, bool ri, SmallLds<L> &lds) {
+  constexpr int M2 = 2 * L, QP = M2 + 2;
   typedef double d2 __attribute__((ext_vector_type(2)));
-  __shared__ __attribute__((aligned(16))) double sQ[2][BCH][M2 * QP];
-  __shared__ double sC[3][BCH][64];  // waves 0, 1: entering rows (block b + 1 of C1 + C2); wave 2: C2
-  __shared__ __attribute__((aligned(16))) double sW[NB][16];
-  __shared__ double sR[64];
-  __shared__ int sbrk;
-  const GSys &S = sys[blockIdx.x];
-  if (S.nt4 == 0 || (!all && !sys_iterating(S))) return;  // uniform over the block
+  auto &sQ = lds.Q;
+  auto &sC = lds.C;
+  auto &sW = lds.W;
+  auto &sR = lds.R;
+  int &sbrk = lds.brk;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const double *C1 = S.C1, *C2 = S.C2;
   const int LJ = L * j;
@@ -1288,16 +1362,10 @@ __global__ __launch_bounds__(192) void kb_bsmall(const GSys *__restrict__ sys, i
 #pragma unroll
         for (int l = 0; l < L; ++l) gs = fma(-sC[2][u][l * 8 + c], sC[2][u][l * 8 + i], gs);
     }
-    n2 += __shfl_xor(n2, 8, 64);
-    n2 += __shfl_xor(n2, 16, 64);
-    n2 += __shfl_xor(n2, 32, 64);  // lane 8 l + c: the sum of column c
-    n2 = n0 + __shfl(n2, c, 64);
-    unsigned live = 0;
-    for (int k = 0; k < L; ++k) live |= S.small[8 * k + 4] > 0.0 ? 1u << k : 0u;
-    const int brk = wave_chol<L>(gs, n2, live, 1e-20, R);
+    const int brk = gram_chol<L>(S, gs, n0, n2, R);
     sR[lane] = R;
     if (lane == 0) sbrk = brk;
-  } else {
+  } else if (wid < 2) {
     const int col = tid >> 4, i = tid & 15;  // window row i of new column col
     const bool mine = col < L && i < M2;
     const int qc = LJ + col;
@@ -1358,7 +1426,7 @@ __global__ __launch_bounds__(192) void kb_bsmall(const GSys *__restrict__ sys, i
     }
   }
   __syncthreads();
-  if (wid == 2) wave_tri_inverse<L>(R, S.Ri);
+  if (ri && wid == 2) wave_tri_inverse<L>(R, S.Ri);
   if (wid != 0) return;
   // lane: 0 .. L - 1 new column, then 2 L unit columns, then right-hand side k = lane - 3 L
   const int k = lane - 3 * L;
@@ -1437,6 +1505,40 @@ __global__ __launch_bounds__(192) void kb_bsmall(const GSys *__restrict__ sys, i
   }
 }
 
+template <int L>
+__global__ __launch_bounds__(192) void kb_bsmall(const GSys *__restrict__ sys, int j, double tol, int all) {
+  __shared__ __attribute__((aligned(16))) SmallLds<L> lds;
+  const GSys &S = sys[blockIdx.x];
+  if (S.nt4 == 0 || (!all && !sys_iterating(S))) return;  // uniform over the block
+  bsmall_round<L>(S, j, tol, true, lds);
+}
+
+// The end of round j for a small map in one launch: the first blocks are kb_bsmall's, the others the tiles of
+// kb_bupdate's mode 1, which needs nothing of them but the inverse factor: a fifth wave of every tile's block
+// forms it from the coefficients that pass through its LDS, while the other four sweep.
+// 73 rounds of three columns, 109 tiles: 12.8 + 11.2 -> 15.2 us; 17 of six, 24 tiles 11.0 + 5.7 -> 13.0.
+template <int L>
+__global__ __launch_bounds__(320) void kb_bround(const GSys *__restrict__ sys, int nsys, const TileMap *__restrict__ tmap,
+                                                 int j, double tol, int all) {
+  __shared__ __attribute__((aligned(16))) union Lds {
+    SmallLds<L> small;
+    UpdateLds upd;
+    __device__ Lds() {}
+  } lds;
+  if ((int)blockIdx.x < nsys) {
+    const GSys &S = sys[blockIdx.x];
+    if (S.nt4 == 0 || (!all && !sys_iterating(S))) return;  // uniform over the block
+    bsmall_round<L>(S, j, tol, false, lds.small);
+  } else {
+    const TileMap tm = tmap[blockIdx.x - nsys];
+    bupdate_tile<L>(sys[tm.sys], tm.row0, j + 1, 1, all, lds.upd);
+  }
+}
+
+// tiles up to which the two parts share a launch (its blocks take twice the registers of kb_bupdate's):
+// of six columns 94 tiles 33 us apart, 22 together; 446 tiles 39 and 32; 1805 tiles 39 and 48
+constexpr int BROUND_TILES = 512;
+
 // two A operands per wave while that leaves a block per CU: 28 tiles over 73 rounds 10.1 -> 7.2 us a sweep
 void launch_bdots(hipStream_t st, int ntiles, const GSys *sys, const TileMap *tmap, int which, int nb, int gram,
                   double *part, int pstride, int all) {
@@ -1449,16 +1551,26 @@ void launch_bdots(hipStream_t st, int ntiles, const GSys *sys, const TileMap *tm
                        pstride, all);
 }
 
-void launch_bsmall(hipStream_t st, int nsys, int L, const GSys *sys, int j, double tol, int all) {
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(nsys), dim3(192), 0, st, sys, j, tol, all); };
+// the end of round j: the small dense part and the next basis block
+void launch_bround(hipStream_t st, int nsys, int L, const GSys *sys, const TileMap *tmap, int ntiles, int j, double tol,
+                   int all) {
+  auto go = [&](auto l) {
+    constexpr int N = decltype(l)::value;
+    if (ntiles <= BROUND_TILES) {
+      hipLaunchKernelGGL(kb_bround<N>, dim3(nsys + ntiles), dim3(320), 0, st, sys, nsys, tmap, j, tol, all);
+    } else {
+      hipLaunchKernelGGL(kb_bsmall<N>, dim3(nsys), dim3(192), 0, st, sys, j, tol, all);
+      hipLaunchKernelGGL(kb_bupdate, dim3(ntiles), dim3(256), 0, st, sys, tmap, j + 1, 1, all);
+    }
+  };
   switch (L) {
-    case 1: go(kb_bsmall<1>); break;
-    case 2: go(kb_bsmall<2>); break;
-    case 3: go(kb_bsmall<3>); break;
-    case 4: go(kb_bsmall<4>); break;
-    case 5: go(kb_bsmall<5>); break;
-    case 6: go(kb_bsmall<6>); break;
-    default: go(kb_bsmall<7>); break;
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 3: go(std::integral_constant<int, 3>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 5: go(std::integral_constant<int, 5>{}); break;
+    case 6: go(std::integral_constant<int, 6>{}); break;
+    default: go(std::integral_constant<int, 7>{}); break;
   }
 }
 
@@ -2073,8 +2185,7 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
         hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t, j + 1, 0, noskip);
         launch_bdots(st, live.n_t4, dsys.p, live.t4, 0, j + 1, 1, partB.p, mc + 2, noskip);
         hipLaunchKernelGGL(kb_bdots_final, dim3(nsys, j + 2), dim3(256), 0, st, dsys.p, partB.p, mc + 2, 1, noskip);
-        launch_bsmall(st, nsys, L, dsys.p, j, tol, noskip);
-        hipLaunchKernelGGL(kb_bupdate, dim3(live.n_t), dim3(256), 0, st, dsys.p, live.t, j + 1, 1, noskip);
+        launch_bround(st, nsys, L, dsys.p, live.t, live.n_t, j, tol, noskip);
         andr_prof_end(ctx, tok_o);
       } else {
         const int tok_o = andr_prof_begin(ctx, "gmres_orthogonalise", (2.0 * j + 6.0) * vbytes,
