@@ -153,12 +153,8 @@ __global__ __launch_bounds__(256) void kb_prep(const GSys *__restrict__ sys, con
 
 // block per system, thread per (wall, rhs) and eighth of the element tiles: sdef = sum of the
 // system's tile partials
-__global__ __launch_bounds__(256) void kb_sred(const GSys *__restrict__ sys, const double *__restrict__ part_s,
-                                               int all) {
+__device__ inline double wall_sums(const GSys &S, const double *__restrict__ part_s, double (*red)[32]) {
   static_assert(MAXW * NB == 32, "eight partial sums per (wall, rhs)");
-  __shared__ double red[8][32];
-  const GSys &S = sys[blockIdx.x];
-  if (!all && !sys_iterating(S)) return;  // as kb_prep (uniform over the block)
   const int r = threadIdx.x & 31, p = threadIdx.x >> 5;
   double a = 0.0;
   for (int i = p; i < S.net; i += 64) {  // eight loads in flight
@@ -170,12 +166,19 @@ __global__ __launch_bounds__(256) void kb_sred(const GSys *__restrict__ sys, con
   }
   red[p][r] = a;
   __syncthreads();
-  if (threadIdx.x < 32) {
-    double v = 0.0;
+  double v = 0.0;  // in thread (wall, rhs) < 32
+  if (threadIdx.x < 32)
 #pragma unroll
     for (int q = 0; q < 8; ++q) v += red[q][threadIdx.x];
-    S.sdef[threadIdx.x] = v;
-  }
+  return v;
+}
+__global__ __launch_bounds__(256) void kb_sred(const GSys *__restrict__ sys, const double *__restrict__ part_s,
+                                               int all) {
+  __shared__ double red[8][32];
+  const GSys &S = sys[blockIdx.x];
+  if (!all && !sys_iterating(S)) return;  // as kb_prep (uniform over the block)
+  const double v = wall_sums(S, part_s, red);
+  if (threadIdx.x < 32) S.sdef[threadIdx.x] = v;
 }
 
 // null-space term of row (element r, component c) for rhs k
@@ -501,19 +504,28 @@ __global__ __launch_bounds__(256) void kb_resid_zero(const GSys *__restrict__ sy
 }
 
 // per tile of a system with nseg > 1: W = sum over segments of the partial products, the first of them with
-// the null-space term; eight segments' loads in flight
+// the null-space term; eight segments' loads in flight. part_s: the wall sums of that term are formed here, by
+// every block for itself, instead of in a launch of kb_sred
 __global__ __launch_bounds__(256) void kb_seg_sum(const GSys *__restrict__ sys, const TileMap *__restrict__ tmap,
-                                                  int all) {
+                                                  const double *__restrict__ part_s, int all) {
+  __shared__ double red[8][32], wall[32];
   const TileMap tm = tmap[blockIdx.x];
   const GSys &S = sys[tm.sys];
   if (S.nseg <= 1 || (!all && !sys_iterating(S))) return;  // uniform over the block
   const int n = S.n, nseg = S.nseg, ne = S.op.ne;
   const int k = threadIdx.x & 7, rr = threadIdx.x >> 3;
+  const double *sdef = S.sdef;
+  if (part_s) {
+    const double v = wall_sums(S, part_s, red);
+    if (threadIdx.x < 32) wall[threadIdx.x] = v;
+    __syncthreads();
+    sdef = wall;
+  }
   double y[TILE / 32], d[TILE / 32];
 #pragma unroll
   for (int t = 0; t < TILE / 32; ++t) {
     const int row = min(tm.row0 + rr + 32 * t, n - 1), co = row / ne;
-    d[t] = defl_term(S.op, S.sdef, row - co * ne, co, k);
+    d[t] = defl_term(S.op, sdef, row - co * ne, co, k);
     const double *P = S.P + (size_t)row * NB + k;
     double a = 0.0;
     for (int sg = 0; sg < nseg; sg += 8) {
@@ -1765,17 +1777,24 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     TileMap *t = nullptr, *et = nullptr, *t4 = nullptr;
     MWave *mw = nullptr;
     int *w0 = nullptr, *nw = nullptr;
-    int n_w = 0, n_t = 0, n_et = 0, n_mw = 0, n_t4 = 0, max_seg = 1;
+    int n_w = 0, n_t = 0, n_et = 0, n_mw = 0, n_t4 = 0, max_seg = 1, min_seg = 1;
     std::vector<int> tile0, ntiles, et0, net, nseg, t40, nt4;
     std::vector<size_t> poff;
     size_t p_elems = 0;
   };
   MapSet cyc, live;
   struct Staging {
-    hipStream_t st;
+    andr_ctx *ctx;
     std::list<std::vector<char>> host;
-    ~Staging() { (void)hipStreamSynchronize(st); }
-  } staging{st, {}};
+    double *slot[2] = {nullptr, nullptr};  // pinned: the states of a poll, and of a cycle's end
+    hipEvent_t polled = nullptr;
+    ~Staging() {
+      (void)hipStreamSynchronize(ctx->stream);
+      for (double *p : slot)
+        if (p) andr_pinned_release(ctx, p);
+      if (polled) (void)hipEventDestroy(polled);
+    }
+  } staging{ctx};
   auto stage = [&](size_t bytes) {
     staging.host.emplace_back(bytes);
     return staging.host.back().data();
@@ -1798,6 +1817,7 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     ms.poff.assign(nsys, 0);
     ms.p_elems = 0;
     ms.max_seg = 1;
+    ms.min_seg = MF_MAX_SEG;
     int row_waves = 0;
     for (int s : list) row_waves += (in[s].op.ne + 31) / 32;
     const int want = row_waves > 0 ? std::min(MF_MAX_SEG, (target_waves + row_waves - 1) / row_waves) : 1;
@@ -1821,6 +1841,7 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
       const int nseg = (ne + seglen - 1) / seglen;
       ms.nseg[s] = nseg;
       ms.max_seg = std::max(ms.max_seg, nseg);
+      ms.min_seg = std::min(ms.min_seg, nseg);
       if (nseg > 1) {
         ms.poff[s] = ms.p_elems;
         ms.p_elems += (size_t)nseg * n * NB;
@@ -1992,7 +2013,10 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     // sys_iterating is kept by the block kernels only)
     const int all = (krylov && blk) ? noskip : 1;
     hipLaunchKernelGGL(kb_prep, dim3(ms.n_et), dim3(256), 0, st, dsys.p, ms.et, krylov ? 0 : 1, jq, partS.p, all);
-    hipLaunchKernelGGL(kb_sred, dim3(nsys), dim3(256), 0, st, dsys.p, partS.p, all);
+    // the wall sums ahead of the product where a system's single segment takes the null-space term there; with
+    // few tiles kb_seg_sum forms them (2.4 to 3.1 us of a launch for 0.2 to 1.0 more in it)
+    const bool fold = ms.min_seg > 1 && ms.n_t <= 512;
+    if (!fold) hipLaunchKernelGGL(kb_sred, dim3(nsys), dim3(256), 0, st, dsys.p, partS.p, all);
     // Blocks of systems that the 256 MB cache holds together are read with ordinary loads: what an L2 still has of
     // them from the round before are hits. More are streamed past the caches, where the operand z keeps its place.
     // 129 MB a round: 37.2 -> 33.6 us kept; the matrices of a large batch (10 GB) are streamed.
@@ -2007,7 +2031,8 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
       if (keep) product(kb_gemv_sym<false, true>, krylov ? noskip : 1);
       else product(kb_gemv_sym<false, false>, krylov ? noskip : 1);
     }
-    if (ms.max_seg > 1) hipLaunchKernelGGL(kb_seg_sum, dim3(ms.n_t), dim3(256), 0, st, dsys.p, ms.t, all);
+    if (ms.max_seg > 1) 
+      hipLaunchKernelGGL(kb_seg_sum, dim3(ms.n_t), dim3(256), 0, st, dsys.p, ms.t, fold ? partS.p : nullptr, all);
     if (!krylov) hipLaunchKernelGGL(kb_resid_fin, dim3(ms.n_w), dim3(256), 0, st, dsys.p, ms.w, partW.p);
     andr_prof_end(ctx, tok);
   };
@@ -2069,6 +2094,20 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     return ANDR_OK;
   };
   auto sm_of = [&](int s, int k) { return hsmall.data() + state_per * s + k * 8; };
+  // With few systems the states come through pinned memory one round late (a poll), and with the next cycle's
+  // restart test (a cycle's end), so that the device does not wait for the host: some 30 us each.
+  const size_t state_bytes = sizeof(double) * state_per * nsys;
+  const bool late = blk && state_bytes <= ANDR_PINNED_SLOT;
+  if (late) {
+    for (double *&p : staging.slot)
+      if (!(p = (double *)andr_pinned_alloc(ctx))) return andr_fail(ctx, ANDR_ERR_ALLOC, "pinned memory for the states");
+    ANDR_HIP(ctx, hipEventCreateWithFlags(&staging.polled, hipEventDisableTiming));
+  }
+  auto send_states = [&](int i) -> int {
+    ANDR_HIP(ctx, hipMemcpyAsync(staging.slot[i], states, state_bytes, hipMemcpyDeviceToHost, st));
+    if (i == 0) ANDR_HIP(ctx, hipEventRecord(staging.polled, st));
+    return ANDR_OK;
+  };
   // The Krylov product skips a system once every column has converged in the cycle (kb_gemv_sym);
   // the host learns the step afterwards from the columns' step counts, and takes the skipped
   // matrix reads out of the profiled totals (a system once, when it leaves the live map).
@@ -2101,6 +2140,16 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
   };
   std::vector<int> cyc_list(nsys);
   for (int s = 0; s < nsys; ++s) cyc_list[s] = s;
+  int cyc_steps = 0;
+  auto count_cycle = [&]() {  // from the states at the cycle's end
+    for (int s : cyc_list)
+      if (live.ntiles[s]) account_skips(s, cyc_steps - 1);
+    for (int s : cyc_list)
+      for (int k = 0; k < NB; ++k) {
+        const double *sm = sm_of(s, k);
+        if (sm[4] > 0.0) it_count[(size_t)s * NB + k] += sm[5] > 0.0 ? (int)sm[5] : cyc_steps;
+      }
+  };
   std::vector<int> cyc_built = cyc_list;
   int rc = build(cyc_list, cyc);
   if (rc) return rc;
@@ -2119,7 +2168,17 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
     hipLaunchKernelGGL(kb_restart, dim3(nsys), dim3(256), 0, st, dsys.p, partW.p, cyc.w0, cyc.nw, tol,
                        first ? 1 : 0, nrhs);
     ANDR_HIP(ctx, hipGetLastError());
-    if ((rc = read_small())) return rc;
+    if (late) {
+      if ((rc = send_states(0))) return rc;
+      ANDR_HIP(ctx, hipStreamSynchronize(st));
+      if (!first) {  // the cycle's end states are there with these
+        std::memcpy(hsmall.data(), staging.slot[1], state_bytes);
+        count_cycle();
+      }
+      std::memcpy(hsmall.data(), staging.slot[0], state_bytes);
+    } else if ((rc = read_small())) {
+      return rc;
+    }
     first = false;
     if (debug) {  // per-cycle true residuals of the first systems (ANDR_DEBUG_GMRES=1)
       for (int s = 0; s < std::min(nsys, 4); ++s) {
@@ -2167,7 +2226,7 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
       if ((rc = use_tiles(live))) return rc;
     }
     const int steps_max = std::min(mc, maxit - total);
-    int steps = 0;
+    int steps = 0, polled = 0;  // polled: the step whose states are on their way
     for (int j = 0; j < steps_max; ++j) {
       gemv(live, 1, j);  // W = A Q_j
       // one sweep of dot products and one of updates over the basis (delayed reorthogonalisation)
@@ -2199,9 +2258,21 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
         andr_prof_end(ctx, tok_o);
       }
       steps = j + 1;
-      if (steps % 8 == 0 && steps < steps_max) {  // drop systems whose columns are all resolved
+      const bool poll = steps % 8 == 0 && steps < steps_max;
+      if (poll && late) {
         ANDR_HIP(ctx, hipGetLastError());
-        if ((rc = read_small())) return rc;
+        if ((rc = send_states(0))) return rc;
+        polled = steps;
+        continue;
+      }
+      if (poll || polled) {  // drop systems whose columns are all resolved
+        ANDR_HIP(ctx, hipGetLastError());
+        if (polled) {
+          ANDR_HIP(ctx, hipEventSynchronize(staging.polled));
+          std::memcpy(hsmall.data(), staging.slot[0], state_bytes);
+        } else if ((rc = read_small())) {
+          return rc;
+        }
         std::vector<int> still;
         for (int s : cyc_list) {
           if (!live.ntiles[s]) continue;
@@ -2211,7 +2282,11 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
           if (l) still.push_back(s);
           else account_skips(s, j);
         }
-        if (still.empty()) break;
+        if (still.empty()) {
+          if (polled) steps = polled;  // the round after it did nothing
+          break;
+        }
+        polled = 0;
         int nlive = 0;
         for (int s = 0; s < nsys; ++s) nlive += live.ntiles[s] ? 1 : 0;
         if ((int)still.size() < nlive) {
@@ -2240,14 +2315,13 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
       hipLaunchKernelGGL(kb_xupdate, dim3(cyc.n_t), dim3(256), 0, st, dsys.p, cyc.t, steps, mc);
     }
     ANDR_HIP(ctx, hipGetLastError());
-    if ((rc = read_small())) return rc;
-    for (int s : cyc_list)
-      if (live.ntiles[s]) account_skips(s, steps - 1);
-    for (int s : cyc_list)
-      for (int k = 0; k < NB; ++k) {
-        const double *sm = sm_of(s, k);
-        if (sm[4] > 0.0) it_count[(size_t)s * NB + k] += sm[5] > 0.0 ? (int)sm[5] : steps;
-      }
+    cyc_steps = steps;
+    if (late) {
+      if ((rc = send_states(1))) return rc;
+    } else {
+      if ((rc = read_small())) return rc;
+      count_cycle();
+    }
     if ((rc = use_tiles(cyc))) return rc;
   }
   if (iters)
