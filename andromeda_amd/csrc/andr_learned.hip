@@ -475,6 +475,9 @@ __device__ inline short f2bf(float x) {  // round to nearest even (v_cvt_pk_bf16
 }
 
 constexpr int CLS_THREADS = 256, CLS_WAVES = CLS_THREADS / 64, CLS_Q = 128;
+// rows from which k_classify gives each wave one: 1280 rows 91 us either way, 2000 rows 108 (139 with a block
+// a row), 3920 196 (248); but 500 rows 76 (46)
+constexpr int CLS_WAVE_ROWS = 1536;
 
 // lane (g, i): A[m = 16 mt + i][k = 16 kt + 4 g + t] = W[in = 16 kt + 4 g + t][out = 16 mt + i]
 // (0 outside the layer). The 40 tiles are packed on the host when the model is set, lane by lane in
@@ -578,9 +581,13 @@ __device__ inline void mlp_block(const bf16x4 *lt /* this lane's entry of tile 0
   *conf = found ? 1.f : 0.f;
 }
 
-// one block per (job, row): rule class of every pair of the row
+// Rule class of every pair of a row: a wave per (job, row) (WROW), or the block's four waves a row in turn where
+// the rows are too few to fill the chip. Latency of the batches: near pairs are few (of the order of a hundred a
+// row), so four waves of a row end with a quarter-full batch each, and every row pays for the network's tiles
+// in LDS. 40 bodies, 102752 rows: 4.9 -> 3.0 ms with a wave per row.
+template <bool WROW>
 __global__ __launch_bounds__(CLS_THREADS, 3) void k_classify(const SysJob *__restrict__ jobs,
-                                                          const int2 *__restrict__ rowmap,
+                                                          const int2 *__restrict__ rowmap, int nrows,
                                                           const bf16x4 *__restrict__ tiles, const float *__restrict__ wf,
                                                           const int *__restrict__ far_table,
                                                           double near_ratio,
@@ -590,7 +597,6 @@ __global__ __launch_bounds__(CLS_THREADS, 3) void k_classify(const SysJob *__res
   __shared__ int qe[CLS_WAVES][CLS_Q];                // queued near pairs: element
   __shared__ float qf[CLS_WAVES][64][3];              // three geometric features of a batch
   __shared__ int qres[CLS_WAVES][64][2];              // class per kernel of a processed batch
-  __shared__ unsigned long long red[3];
   __shared__ bf16x4 s_tiles[CLS_NTILES * 64];  // the network's operand tiles, shared by the block's waves
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
@@ -601,13 +607,14 @@ __global__ __launch_bounds__(CLS_THREADS, 3) void k_classify(const SysJob *__res
   }
   if (threadIdx.x < NOUT) sb[3 * NH + threadIdx.x] = wf[P_B4 + threadIdx.x];
   if (threadIdx.x < ANDR_FAR_BINS) sfar[threadIdx.x] = far_table[threadIdx.x];
-  if (threadIdx.x < 3) red[threadIdx.x] = 0ull;
   // the operand tiles (packed lane by lane when the model was set) into LDS: the four waves use the
   // same tiles, and registers stay free for occupancy
   for (int i = threadIdx.x; i < CLS_NTILES * 64; i += blockDim.x) s_tiles[i] = tiles[i];
   const bf16x4 *lt = s_tiles + lane;
   __syncthreads();
-  const int2 jr = rowmap[blockIdx.x];
+  const int row = WROW ? blockIdx.x * CLS_WAVES + __builtin_amdgcn_readfirstlane(wid) : blockIdx.x;
+  if (row >= nrows) return;  // no barriers of the block below
+  const int2 jr = rowmap[row];
   const SysJob &J = jobs[jr.x];
   const BodyGeom &g_ = J.g;
   const int r = jr.y, ne = g_.ne;
@@ -671,9 +678,9 @@ __global__ __launch_bounds__(CLS_THREADS, 3) void k_classify(const SysJob *__res
     }
     __builtin_amdgcn_wave_barrier();
   };
-  // scan the row (the wave takes every fourth group of 64 elements); near pairs are queued and
+  // scan the row (or every fourth group of 64 elements of it); near pairs are queued and
   // classified 64 at a time, the rest of the queue once the scan is done (one batch call site)
-  int base = wid * 64;
+  int base = WROW ? 0 : wid * 64;
   for (;;) {
     if (base < ne) {
       const int e = base + lane;
@@ -699,7 +706,7 @@ __global__ __launch_bounds__(CLS_THREADS, 3) void k_classify(const SysJob *__res
       const int pos = qn + __popcll(m & ((1ull << lane) - 1ull));
       if (near) qe[wid][pos] = e;
       qn += __popcll(m);
-      base += CLS_THREADS;
+      base += WROW ? 64 : CLS_THREADS;
       __builtin_amdgcn_wave_barrier();
     }
     const bool scanned = base >= ne;  // uniform over the wave
@@ -716,11 +723,13 @@ __global__ __launch_bounds__(CLS_THREADS, 3) void k_classify(const SysJob *__res
       break;
     }
   }
-  atomicAdd(&red[0], (unsigned long long)pts);
-  atomicAdd(&red[1], (unsigned long long)nl);
-  atomicAdd(&red[2], (unsigned long long)nf);
-  __syncthreads();
-  if (threadIdx.x < 3) atomicAdd(stats + 3 * (size_t)jr.x + threadIdx.x, red[threadIdx.x]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    pts += __shfl_xor(pts, o, 64);
+    nl += __shfl_xor(nl, o, 64);
+    nf += __shfl_xor(nf, o, 64);
+  }
+  if (lane < 3) atomicAdd(stats + 3 * (size_t)jr.x + lane, (unsigned long long)(lane == 0 ? pts : lane == 1 ? nl : nf));
 }
 
 RuleTab dunavant_tab(int qoff_fixed, int nq_fixed) {
@@ -972,8 +981,12 @@ int andr_launch_stokes_system_learned(andr_ctx *ctx, SysJob *h_jobs, const SysJo
   if (st.alloc(3 * (size_t)njobs, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "stats");
   ANDR_HIP(ctx, hipMemsetAsync(st.p, 0, 3 * sizeof(unsigned long long) * njobs, ctx->stream));
   const int tok = andr_prof_begin(ctx, "classify_pairs", 0.0, 0.0);
-  hipLaunchKernelGGL(k_classify, dim3(nrows), dim3(CLS_THREADS), 0, ctx->stream, d_jobs, d_rowmap, tiles, fp, far,
-                     ctx->model_near, ctx->model_conf, st.p);
+  auto classify = [&](auto kernel, int blocks) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(CLS_THREADS), 0, ctx->stream, d_jobs, d_rowmap, nrows, tiles, fp, far,
+                       ctx->model_near, ctx->model_conf, st.p);
+  };
+  if (nrows >= CLS_WAVE_ROWS) classify(k_classify<true>, (nrows + CLS_WAVES - 1) / CLS_WAVES);
+  else classify(k_classify<false>, nrows);
   andr_prof_end(ctx, tok);
   ANDR_HIP(ctx, hipGetLastError());
   std::vector<unsigned long long> hs(3 * (size_t)njobs);
