@@ -1149,11 +1149,11 @@ __device__ inline int gram_chol(const GSys &S, double gs, double g0, double n2, 
 // A block takes a tile of 64 rows, four lanes a row, a lane two of its columns: one 16-byte load per basis
 // block, the row's other values from its neighbours (quad permutes), the coefficients staged in LDS UCH
 // blocks at a time with the next chunk's loads of both under way. With a whole row per lane, a body of 7000
-// rows was 109 waves, each with a round trip to memory every four blocks (73 rounds of it: 39.7 -> 10.8 us a
-// sweep; 40 bodies of 500 to 7220 elements 50.7 -> 33.7). Every sum runs over the blocks and columns in order,
+// rows was 109 waves, each with a round trip to memory every four blocks (73 rounds of it: 39.7 -> 10.0 us a
+// sweep; 40 bodies of 500 to 7220 elements, the first rounds: 40 us). Every sum runs over the blocks and columns in order,
 // whatever the split: the Krylov vectors meet FP32 products, where a last bit that differs can turn a rounding.
 // HBM bound (the basis stream) on a full batch.
-constexpr int UCH = 16;
+constexpr int UCH = 8;  // (16: twice the registers, half the waves: 40 -> 59 us at 4826 tiles, 10.0 -> 10.9 at 109)
 template <int U>
 __device__ inline double quad_lane(double x) {  // the value of lane U of the quad
   constexpr int ctrl = U * 0x55;                 // quad_perm [U, U, U, U]
@@ -1207,25 +1207,19 @@ __device__ inline void bupdate_tile(const GSys &S, int row0, int nb, int mode, i
   d2 s = {0.0, 0.0};
   // chunk of UCH blocks from b0: this lane's values of its row, and its share of the coefficients (past the
   // last block both repeat it and are not used)
-  static_assert(UCH * 64 == 2 * 2 * 256, "two 16-byte loads of the coefficients per thread");
-  d2 cq[UCH], cc[2];
+  static_assert(UCH * 64 == 2 * 256, "a 16-byte load of the coefficients per thread");
+  d2 cq[UCH], cc;
   auto load = [&](int b0) {
 #pragma unroll
     for (int u = 0; u < UCH; ++u) cq[u] = *(const d2 *)(Qr + (size_t)min(b0 + u, nbb - 1) * vstride);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int e = 2 * (tid + 256 * h);  // block b0 + e / 64
-      cc[h] = *(const d2 *)(Cf + (size_t)min(b0 + (e >> 6), nbb - 1) * 64 + (e & 63));
-    }
+    cc = *(const d2 *)(Cf + (size_t)min(b0 + (tid >> 5), nbb - 1) * 64 + 2 * (tid & 31));
   };
   if (nbb > 0) {
     if (sweeps) load(0);
 #pragma unroll 1
     for (int b0 = 0, w = 0; b0 < nbb; b0 += UCH, w ^= 1) {
       double *sc = lds.C[w];
-      if (sweeps)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) *(d2 *)&sc[2 * (tid + 256 * h)] = cc[h];
+      if (sweeps) *(d2 *)&sc[2 * tid] = cc;
       d2 q[UCH];
 #pragma unroll
       for (int u = 0; u < UCH; ++u) q[u] = cq[u];
