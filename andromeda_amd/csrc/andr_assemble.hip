@@ -1638,7 +1638,7 @@ int andr_launch_stokes_system(andr_ctx *ctx, const SysJob *d_jobs, const int2 *d
 // T = sum_e A_e (c_e - centre) x q_e (the reductions of src/lib_particle.f90:1751-1831), and the
 // largest row self-check error. out[37 b + 6 k + (0..5)] = (F, T) of problem k, out[37 b + 36] = error.
 // Latency of one block: a lane takes one problem of every 128th element, eight lanes a row of X (all 36 sums in
-// one lane were a reduction of 432 lane exchanges in a row: 40 -> 8 us for 80 elements, 46 -> 21 for about 2300; forty
+// one lane were a reduction of 432 lane exchanges in a row: 40 -> 8 us for 500 elements, 46 -> 21 for about 2300; forty
 // bodies of up to 7220 are bound by the largest one's turns over memory, 76 -> 79).
 constexpr int FT_THREADS = 1024, FT_WAVES = FT_THREADS / 64;
 __global__ __launch_bounds__(FT_THREADS) void k_force_torque(const SysJob *__restrict__ jobs, double *__restrict__ out) {
