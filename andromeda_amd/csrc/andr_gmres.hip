@@ -2091,10 +2091,10 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
   // With few systems the states come through pinned memory one round late (a poll), and with the next cycle's
   // restart test (a cycle's end), so that the device does not wait for the host: some 30 us each.
   const size_t state_bytes = sizeof(double) * state_per * nsys;
-  const bool late = blk && state_bytes <= ANDR_PINNED_SLOT;
+  bool late = blk && state_bytes <= ANDR_PINNED_SLOT;
   if (late) {
-    for (double *&p : staging.slot)
-      if (!(p = (double *)andr_pinned_alloc(ctx))) return andr_fail(ctx, ANDR_ERR_ALLOC, "pinned memory for the states");
+    for (double *&p : staging.slot) p = (double *)andr_pinned_alloc(ctx);
+    late = staging.slot[0] && staging.slot[1];  // no pinned memory: with waits
     ANDR_HIP(ctx, hipEventCreateWithFlags(&staging.polled, hipEventDisableTiming));
   }
   auto send_states = [&](int i) -> int {
