@@ -714,9 +714,10 @@ int andr_launch_laplace_rows(andr_ctx *ctx, DevBody &b, double *H, double *G, do
 // ------------------------------------------------------------------------------------------------
 // Stokes rows: sdIntRowUStokes / sdIntRowQStokes (src/lib_Stokes.f90:1562-2245), regular integrals
 // by Triangle_3DStokesInt (:2341-2446) with StokesKernel (:2450-2544).
-// Outputs: T[6][nsp][nn], G[6][nsp][ne], prT[3][nsp][nn], prG[3][nsp][ne].
+// Outputs: T[6][nsp][nn], G[6][nsp][ne], prT[3][nsp][nn], prG[3][nsp][ne]. PRES: with the pressure integrals prT
+// and prG, which a boundary-value solve does not read (1082 rows of 720 triangles: 382 us with them, 275 without).
 // ------------------------------------------------------------------------------------------------
-template <bool ROW_IN_LDS, bool QUADS>
+template <bool ROW_IN_LDS, bool QUADS, bool PRES>
 __global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int nq, const int *__restrict__ order,
                                                      const uint8_t *__restrict__ color, int ncolors, double extra,
                                                      double *__restrict__ T, double *__restrict__ G,
@@ -730,6 +731,7 @@ __global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int n
   const bool qrow = r >= nn;
   const int erow = r - nn;
   const size_t mstrT = (size_t)nrows * nn, mstrG = (size_t)nrows * ne;
+  constexpr int NT = PRES ? 9 : 6;
   double s[3];
   if (!qrow)
     for (int j = 0; j < 3; ++j) s[j] = g.xyz[3 * r + j];
@@ -740,7 +742,7 @@ __global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int n
     if (ROW_IN_LDS) return lds + (size_t)k * nn;
     return k < 6 ? T + k * mstrT + (size_t)ro * nn : prT + (k - 6) * mstrT + (size_t)ro * nn;
   };
-  for (int k = 0; k < 9; ++k) {
+  for (int k = 0; k < NT; ++k) {
     double *p = trow(k);
     for (int i = threadIdx.x; i < nn; i += blockDim.x) p[i] = 0.0;
   }
@@ -749,9 +751,9 @@ __global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int n
   for (int i0 = 0; i0 < ne; i0 += blockDim.x) {
     const int idx = i0 + threadIdx.x;
     int col = -1, nno = 3, vv[NV] = {0};
-    double t[9][NV];  // T (6) and prT (3) at the element's nodes
+    double t[NT][NV];  // T (6) and prT (3) at the element's nodes
 #pragma unroll
-    for (int k = 0; k < 9; ++k)
+    for (int k = 0; k < NT; ++k)
 #pragma unroll
       for (int v = 0; v < NV; ++v) t[k][v] = 0.0;
     if (idx < ne) {
@@ -778,7 +780,7 @@ __global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int n
           quad_stokes_pair(x1, x2, x3, g.xyz + 3 * vv[3], s, g.mul[e], g.iquad, qs, acc);
           for (int k = 0; k < 6; ++k) Gs[k] = acc[k];
           for (int k = 0; k < 3; ++k) pG[k] = acc[6 + k];
-          for (int k = 0; k < 9; ++k)
+          for (int k = 0; k < NT; ++k)
             for (int v = 0; v < 4; ++v) t[k][v] = acc[9 + 4 * k + v];
         }
       } else {
@@ -794,8 +796,9 @@ __global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int n
           for (int v = 0; v < 3; ++v) {
 #pragma unroll
             for (int k = 0; k < 6; ++k) t[k][v] = Tv[k][v];
+            if constexpr (PRES)
 #pragma unroll
-            for (int k = 0; k < 3; ++k) t[6 + k][v] = pT[k][v];
+              for (int k = 0; k < 3; ++k) t[6 + k][v] = pT[k][v];
           }
         } else {
           andr_sing_stk(x1, x2, x3, s, isrc, Gs);  // T, prT, prG of a singular pair are zero
@@ -803,13 +806,14 @@ __global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int n
       }
 #pragma unroll
       for (int k = 0; k < 6; ++k) G[k * mstrG + (size_t)ro * ne + e] = Gs[k];
+      if constexpr (PRES)
 #pragma unroll
-      for (int k = 0; k < 3; ++k) prG[k * mstrG + (size_t)ro * ne + e] = pG[k];
+        for (int k = 0; k < 3; ++k) prG[k * mstrG + (size_t)ro * ne + e] = pG[k];
     }
     for (int c = 0; c < ncolors; ++c) {
       if (col == c) {
 #pragma unroll
-        for (int k = 0; k < 9; ++k) {
+        for (int k = 0; k < NT; ++k) {
           double *p = trow(k);
 #pragma unroll
           for (int v = 0; v < NV; ++v)
@@ -827,11 +831,13 @@ __global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int n
   }
   block_sum<6>(sums, red);
   double psum[3] = {0, 0, 0};
-  for (int k = 0; k < 3; ++k) {
-    const double *p = trow(6 + k);
-    for (int i = threadIdx.x; i < nn; i += blockDim.x) psum[k] += p[i];
+  if constexpr (PRES) {
+    for (int k = 0; k < 3; ++k) {
+      const double *p = trow(6 + k);
+      for (int i = threadIdx.x; i < nn; i += blockDim.x) psum[k] += p[i];
+    }
+    block_sum<3>(psum, red);
   }
-  block_sum<3>(psum, red);
   const double osemPi = (double)(atanf(1.0f)) * 4.0 * 8.0;  // REAL(4) ATAN(1.0) (src/lib_Stokes.f90:1596)
   double err = -9.99;
   const double cx = -sums[0], cy = -sums[3], cz = -sums[5];
@@ -871,13 +877,14 @@ __global__ __launch_bounds__(256) void k_stokes_rows(BodyGeom g, int qoff, int n
         trow(5)[cn[v]] += shpf * (cz + extra);
       }
       // pressure correction (src/lib_Stokes.f90:1851-1863)
-      for (int v = 0; v < nno; ++v)
-        for (int k = 0; k < 3; ++k) trow(6 + k)[cn[v]] -= psum[k] / nno;
+      if constexpr (PRES)
+        for (int v = 0; v < nno; ++v)
+          for (int k = 0; k < 3; ++k) trow(6 + k)[cn[v]] -= psum[k] / nno;
     }
   }
   __syncthreads();
   if (ROW_IN_LDS) {
-    for (int k = 0; k < 9; ++k) {
+    for (int k = 0; k < NT; ++k) {
       double *out = k < 6 ? T + k * mstrT + (size_t)ro * nn : prT + (k - 6) * mstrT + (size_t)ro * nn;
       const double *p = lds + (size_t)k * nn;
       for (int i = threadIdx.x; i < nn; i += blockDim.x) out[i] = p[i];
@@ -1160,16 +1167,20 @@ int andr_launch_stokes_rows(andr_ctx *ctx, DevBody &b, double extra, double *T, 
                             double *err_rows, int r0, int nrows) {
   QuadRule qr = andr_rule(b.itri);
   const int nsp = nrows < 0 ? b.g.nn + b.g.ne - r0 : nrows;  // rows r0 .. r0 + nsp - 1
-  const size_t lds = sizeof(double) * 9 * (size_t)b.g.nn;
+  const bool pres = prT != nullptr;  // with prG: both or neither
+  const int nm = pres ? 9 : 6;
+  const size_t lds = sizeof(double) * nm * (size_t)b.g.nn;
   const double evals = (double)nsp * b.g.ne * qr.npts;
-  const int tok = andr_prof_begin(ctx, "stokes_rows", 8.0 * 9 * nsp * ((double)b.g.nn + b.g.ne),
+  const int tok = andr_prof_begin(ctx, "stokes_rows", 8.0 * nm * nsp * ((double)b.g.nn + b.g.ne),
                                   evals * ANDR_FLOPS_PER_STOKES_EVAL);
   const bool in_lds = lds <= 144 * 1024, quads = b.g.nv == 4;
   using Kern = void (*)(BodyGeom, int, int, const int *, const uint8_t *, int, double, double *, double *, double *,
                         double *, double *, int, int);
-  const Kern kerns[4] = {k_stokes_rows<false, false>, k_stokes_rows<false, true>, k_stokes_rows<true, false>,
-                         k_stokes_rows<true, true>};
-  const Kern kern = kerns[(in_lds ? 2 : 0) + (quads ? 1 : 0)];
+  const Kern kerns[8] = {k_stokes_rows<false, false, false>, k_stokes_rows<false, false, true>,
+                         k_stokes_rows<false, true, false>,  k_stokes_rows<false, true, true>,
+                         k_stokes_rows<true, false, false>,  k_stokes_rows<true, false, true>,
+                         k_stokes_rows<true, true, false>,   k_stokes_rows<true, true, true>};
+  const Kern kern = kerns[(in_lds ? 4 : 0) + (quads ? 2 : 0) + (pres ? 1 : 0)];
   if (in_lds) ANDR_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   hipLaunchKernelGGL(kern, dim3(nsp), dim3(row_threads(b.g.ne)), in_lds ? lds : 0, ctx->stream, b.g, qr.offset, qr.npts,
                      b.order, b.color, b.ncolors, extra, T, G, prT, prG, err_rows, r0, nsp);

@@ -269,7 +269,9 @@ extern "C" int andr_assemble_stokes_rows(andr_ctx *ctx, const andr_mesh *mesh, i
   const int nn = b.g.nn, ne = b.g.ne, nr = row_end - row_begin;
   const size_t sT = (size_t)nr * nn, sG = (size_t)nr * ne;
   DevBuf<double> dT, dG, dpT, dpG, dE;
-  if (dT.alloc(6 * sT, ctx) || dG.alloc(6 * sG, ctx) || dpT.alloc(3 * sT, ctx) || dpG.alloc(3 * sG, ctx) ||
+  bool pres = false;  // any pressure matrix wanted
+  for (int k = 0; k < 3; ++k) pres = pres || (prT && prT[k]) || (prG && prG[k]);
+  if (dT.alloc(6 * sT, ctx) || dG.alloc(6 * sG, ctx) || (pres && (dpT.alloc(3 * sT, ctx) || dpG.alloc(3 * sG, ctx))) ||
       dE.alloc(nr, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "Stokes integral matrices (%zu doubles)", 9 * (sT + sG));
   if ((rc = andr_launch_stokes_rows(ctx, b, extra_free_term, dT.p, dG.p, dpT.p, dpG.p, dE.p, row_begin, nr))) return rc;
@@ -278,7 +280,7 @@ extern "C" int andr_assemble_stokes_rows(andr_ctx *ctx, const andr_mesh *mesh, i
     out.push_back({dT.p + k * sT, nr, nn, T ? T[k] : nullptr});
     out.push_back({dG.p + k * sG, nr, ne, G ? G[k] : nullptr});
   }
-  for (int k = 0; k < 3; ++k) {
+  for (int k = 0; k < 3 && pres; ++k) {
     out.push_back({dpT.p + k * sT, nr, nn, prT ? prT[k] : nullptr});
     out.push_back({dpG.p + k * sG, nr, ne, prG ? prG[k] : nullptr});
   }

@@ -95,6 +95,18 @@ void andr_pinned_release(andr_ctx *ctx, void *slot);
 // device to host behind the work on the context's stream; the copies are done when it returns
 int andr_copy_to_host(andr_ctx *ctx, const std::vector<andr_copy> &copies);
 
+// a point of a stream, for times from the device's clock
+struct andr_mark {
+  hipEvent_t ev = nullptr;
+  andr_mark() = default;
+  andr_mark(const andr_mark &) = delete;
+  andr_mark &operator=(const andr_mark &) = delete;
+  ~andr_mark() {
+    if (ev) (void)hipEventDestroy(ev);
+  }
+  bool record(hipStream_t st) { return (!ev && hipEventCreate(&ev) != hipSuccess) || hipEventRecord(ev, st) != hipSuccess; }
+};
+
 // RAII device buffer; with a context it draws on the context's memory cache
 template <class T>
 struct DevBuf {

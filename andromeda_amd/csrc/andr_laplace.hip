@@ -207,12 +207,38 @@ std::vector<double> g_factors(const andr_subdomain &sd, const SdLists &l) {
   return gm;
 }
 
-template <class T>
-int upload(andr_ctx *ctx, DevBuf<T> &d, const std::vector<T> &h) {
-  if (d.alloc(std::max<size_t>(h.size(), 1), ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "Laplace maps");
-  if (!h.empty())
-    ANDR_HIP(ctx, hipMemcpyAsync(d.p, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice, ctx->stream));
-  return ANDR_OK;
+// Tables that go up together: one copy, some 7 us each otherwise, while the device still integrates
+struct Tables {
+  std::vector<char> host;
+  DevBuf<char> dev;
+  template <class T>
+  size_t put(const T *src, size_t n) {  // its place; on a 256-byte boundary
+    const size_t at = host.size();
+    host.resize(at + (sizeof(T) * n + 255) / 256 * 256);
+    if (n) std::memcpy(host.data() + at, src, sizeof(T) * n);
+    return at;
+  }
+  template <class T>
+  size_t put(const std::vector<T> &v) {
+    return put(v.data(), v.size());
+  }
+  int upload(andr_ctx *ctx) {
+    if (dev.alloc(std::max<size_t>(host.size(), 1), ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "Laplace maps");
+    if (!host.empty())
+      ANDR_HIP(ctx, hipMemcpyAsync(dev.p, host.data(), host.size(), hipMemcpyHostToDevice, ctx->stream));
+    return ANDR_OK;
+  }
+  template <class T>
+  T *at(size_t o) const {
+    return (T *)(dev.p + o);
+  }
+};
+// largest self-check errors of node rows and of all rows (rows below nn are nodes')
+void max_row_errors(const std::vector<double> &e, int nn, double &errU, double &errQ) {
+  for (int i = 0; i < (int)e.size(); ++i) {
+    if (i < nn) errU = std::max(errU, e[i]);
+    else errQ = std::max(errQ, e[i]);
+  }
 }
 
 }  // namespace
@@ -262,10 +288,10 @@ int laplace_solve(andr_ctx *ctx, const andr_mesh *mesh, int32_t nsd, const andr_
   // ---- integral matrices of every subdomain (kept on the device) ---------------------------------
   struct SdDev {
     DevBuf<double> H, G, E;
+    std::vector<double> he;  // the rows' self-checks
     int nn = 0, ne = 0;
   };
   std::vector<SdDev> D(nsd);
-  double errU = 0.0, errQ = 0.0;
   for (int s = 0; s < nsd; ++s) {
     SubMesh sub;
     make_submesh(mesh, sds[s], L[s], sub);
@@ -279,15 +305,11 @@ int laplace_solve(andr_ctx *ctx, const andr_mesh *mesh, int32_t nsd, const andr_
     if (d.H.alloc((size_t)nsp * d.nn, ctx) || d.G.alloc((size_t)nsp * d.ne, ctx) || d.E.alloc(nsp, ctx))
       return andr_fail(ctx, ANDR_ERR_ALLOC, "integral matrices of subdomain %d", s);
     if ((rc = andr_launch_laplace_rows(ctx, body, d.H.p, d.G.p, d.E.p, 0, -1, mixed))) return rc;
-    std::vector<double> he(nsp);
-    ANDR_HIP(ctx, hipMemcpyAsync(he.data(), d.E.p, sizeof(double) * nsp, hipMemcpyDeviceToHost, st));
-    ANDR_HIP(ctx, hipStreamSynchronize(st));  // the body's buffers go back to the cache after this
-    for (int i = 0; i < nsp; ++i) {
-      if (i < d.nn) errU = std::max(errU, he[i]);
-      else errQ = std::max(errQ, he[i]);
-    }
+    d.he.resize(nsp);
   }
-  const double t1 = andr_now();
+  double errU = 0.0, errQ = 0.0, t_assemble = 0.0;
+  andr_mark assembled, finished;  // the host goes on with the first equation's maps meanwhile
+  if (assembled.record(st)) return andr_fail(ctx, ANDR_ERR_HIP, "event");
   // mesh geometry for the wall fluxes (areas, wall ids)
   DevBody whole;
   if (wall_flux && (rc = andr_body_upload(ctx, mesh, whole, false))) return rc;
@@ -354,10 +376,10 @@ int laplace_solve(andr_ctx *ctx, const andr_mesh *mesh, int32_t nsd, const andr_
     }
     // rows start on 128-byte lines (16 FP64 or 32 FP32 entries)
     const int64_t lda = mixed ? ((int64_t)nx + 31) / 32 * 32 : ((int64_t)nx + 15) / 16 * 16;
-    DevBuf<double> sys, B, X, db, qs, du, dq;
+    DevBuf<double> sys, B, qs;
     DevBuf<float> sys32;
     if ((mixed ? sys32.alloc((size_t)neq * lda, ctx) : sys.alloc((size_t)neq * lda, ctx)) ||
-        B.alloc((size_t)neq * ANDR_NB, ctx) || X.alloc((size_t)nx * ANDR_NB, ctx) || qs.alloc(nx, ctx))
+        B.alloc((size_t)neq * ANDR_NB, ctx) || qs.alloc(nx, ctx))
       return andr_fail(ctx, ANDR_ERR_ALLOC, "Laplace system %d x %d", neq, nx);
     if (mixed)
       hipLaunchKernelGGL(k_lap_fill<float>, dim3(((size_t)neq * lda + 255) / 256), dim3(256), 0, st, (size_t)neq * lda,
@@ -367,11 +389,17 @@ int laplace_solve(andr_ctx *ctx, const andr_mesh *mesh, int32_t nsd, const andr_
                          (size_t)neq * lda, sys.p);
     hipLaunchKernelGGL(k_lap_fill<double>, dim3(((size_t)neq * ANDR_NB + 255) / 256), dim3(256), 0, st,
                        (size_t)neq * ANDR_NB, B.p);
+    Tables tb;
+    std::vector<double> xp((size_t)nx * ANDR_NB, 0.0);
+    for (int i = 0; i < nx; ++i) xp[(size_t)i * ANDR_NB] = x0[i];
+    const size_t o_x = tb.put(xp), o_b = tb.put(b), o_su = tb.put(src_u), o_sq = tb.put(src_q), o_u = tb.put(ue, nn),
+                 o_q = tb.put(qe, ne);
+    struct Maps {
+      size_t rr, nc, qc, nk, qk, gm;
+      int row, rows;
+    };
+    std::vector<Maps> maps(nsd);
     {
-      std::vector<double> xp((size_t)nx * ANDR_NB, 0.0);
-      for (int i = 0; i < nx; ++i) xp[(size_t)i * ANDR_NB] = x0[i];
-      ANDR_HIP(ctx, hipMemcpyAsync(X.p, xp.data(), sizeof(double) * xp.size(), hipMemcpyHostToDevice, st));
-      if ((rc = upload(ctx, db, b))) return rc;
       // sdSetUpSysMrhsM_CRS: rows of flux / contact nodes, then of function / contact elements
       int row = 0;
       for (int s = 0; s < nsd; ++s) {
@@ -402,24 +430,24 @@ int laplace_solve(andr_ctx *ctx, const andr_mesh *mesh, int32_t nsd, const andr_
           if (qc[k] < 0 || qc[k] >= (qk[k] ? nb : nx))
             return andr_fail(ctx, ANDR_ERR_ARG, "element %d: conditions of different kinds in two subdomains",
                              l.elems[k]);
-        if (rr.empty()) continue;
-        DevBuf<int> drr, dnc, dqc;
-        DevBuf<uint8_t> dnk, dqk;
-        DevBuf<double> dgm;
-        if ((rc = upload(ctx, drr, rr)) || (rc = upload(ctx, dnc, nc)) || (rc = upload(ctx, dqc, qc)) ||
-            (rc = upload(ctx, dnk, nk)) || (rc = upload(ctx, dqk, qk)) || (rc = upload(ctx, dgm, gm)))
-          return rc;
-        if (mixed)
-          hipLaunchKernelGGL(k_lap_system<float>, dim3((int)rr.size()), dim3(256), 0, st, D[s].nn, D[s].ne, D[s].H.p,
-                             D[s].G.p, drr.p, row, dnc.p, dnk.p, dqc.p, dqk.p, dgm.p, db.p, sys32.p, lda, B.p);
-        else
-          hipLaunchKernelGGL(k_lap_system<double>, dim3((int)rr.size()), dim3(256), 0, st, D[s].nn, D[s].ne, D[s].H.p,
-                             D[s].G.p, drr.p, row, dnc.p, dnk.p, dqc.p, dqk.p, dgm.p, db.p, sys.p, lda, B.p);
-        ANDR_HIP(ctx, hipGetLastError());
-        ANDR_HIP(ctx, hipStreamSynchronize(st));  // the maps go back to the cache after this
+        maps[s] = {tb.put(rr), tb.put(nc), tb.put(qc), tb.put(nk), tb.put(qk), tb.put(gm), row, (int)rr.size()};
         row += (int)rr.size();
       }
       if (row != neq) return andr_fail(ctx, ANDR_ERR_STATE, "system rows %d, expected %d", row, neq);
+    }
+    if ((rc = tb.upload(ctx))) return rc;
+    double *dX = tb.at<double>(o_x), *du = tb.at<double>(o_u), *dq = tb.at<double>(o_q);
+    for (int s = 0; s < nsd; ++s) {
+      const Maps &m = maps[s];
+      if (m.rows == 0) continue;
+      auto system = [&](auto kernel, auto *a) {
+        hipLaunchKernelGGL(kernel, dim3(m.rows), dim3(256), 0, st, D[s].nn, D[s].ne, D[s].H.p, D[s].G.p,
+                           tb.at<int>(m.rr), m.row, tb.at<int>(m.nc), tb.at<uint8_t>(m.nk), tb.at<int>(m.qc),
+                           tb.at<uint8_t>(m.qk), tb.at<double>(m.gm), tb.at<double>(o_b), a, lda, B.p);
+      };
+      if (mixed) system(k_lap_system<float>, sys32.p);
+      else system(k_lap_system<double>, sys.p);
+      ANDR_HIP(ctx, hipGetLastError());
     }
     // lsqr_precon + lsqr_solve (column scaling in place, hot start, the reference's stopping rules)
     const int maxit = opts ? opts[en].maxit : 0;
@@ -427,26 +455,34 @@ int laplace_solve(andr_ctx *ctx, const andr_mesh *mesh, int32_t nsd, const andr_
     void *A = mixed ? (void *)sys32.p : (void *)sys.p;
     if ((rc = andr_colscale(ctx, A, mixed, lda, neq, nx, qs.p))) return rc;
     int nit = 0, istop = 0;
-    if ((rc = andr_lsqr_device(ctx, A, mixed, lda, neq, nx, qs.p, B.p, X.p, 1, maxit, eps, &nit, &istop)))
+    if ((rc = andr_lsqr_device(ctx, A, mixed, lda, neq, nx, qs.p, B.p, dX, 1, maxit, eps, &nit, &istop)))
       return rc;
     // the solution back to u and q, then the wall fluxes
-    DevBuf<int> dsu, dsq;
-    if (du.alloc(nn, ctx) || dq.alloc(ne, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "boundary values");
-    ANDR_HIP(ctx, hipMemcpyAsync(du.p, ue, sizeof(double) * nn, hipMemcpyHostToDevice, st));
-    ANDR_HIP(ctx, hipMemcpyAsync(dq.p, qe, sizeof(double) * ne, hipMemcpyHostToDevice, st));
-    if ((rc = upload(ctx, dsu, src_u)) || (rc = upload(ctx, dsq, src_q))) return rc;
-    hipLaunchKernelGGL(k_lap_scatter, dim3((nn + 255) / 256), dim3(256), 0, st, nn, dsu.p, X.p, du.p);
-    hipLaunchKernelGGL(k_lap_scatter, dim3((ne + 255) / 256), dim3(256), 0, st, ne, dsq.p, X.p, dq.p);
+    hipLaunchKernelGGL(k_lap_scatter, dim3((nn + 255) / 256), dim3(256), 0, st, nn, tb.at<int>(o_su), dX, du);
+    hipLaunchKernelGGL(k_lap_scatter, dim3((ne + 255) / 256), dim3(256), 0, st, ne, tb.at<int>(o_sq), dX, dq);
     DevBuf<double> dflux;
     if (wall_flux) {
       if (dflux.alloc(nw, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "wall fluxes");
-      hipLaunchKernelGGL(k_wall_flux, dim3(nw), dim3(256), 0, st, ne, whole.g.bcid, whole.g.area, dq.p, dflux.p);
+      hipLaunchKernelGGL(k_wall_flux, dim3(nw), dim3(256), 0, st, ne, whole.g.bcid, whole.g.area, dq, dflux.p);
       ANDR_HIP(ctx, hipMemcpyAsync(wall_flux + (size_t)en * nw, dflux.p, sizeof(double) * nw, hipMemcpyDeviceToHost, st));
     }
     ANDR_HIP(ctx, hipGetLastError());
-    ANDR_HIP(ctx, hipMemcpyAsync(ue, du.p, sizeof(double) * nn, hipMemcpyDeviceToHost, st));
-    ANDR_HIP(ctx, hipMemcpyAsync(qe, dq.p, sizeof(double) * ne, hipMemcpyDeviceToHost, st));
+    ANDR_HIP(ctx, hipMemcpyAsync(ue, du, sizeof(double) * nn, hipMemcpyDeviceToHost, st));
+    ANDR_HIP(ctx, hipMemcpyAsync(qe, dq, sizeof(double) * ne, hipMemcpyDeviceToHost, st));
+    if (en == 0) {
+      for (int s = 0; s < nsd; ++s)
+        ANDR_HIP(ctx, hipMemcpyAsync(D[s].he.data(), D[s].E.p, sizeof(double) * D[s].he.size(), hipMemcpyDeviceToHost, st));
+      if (finished.record(st)) return andr_fail(ctx, ANDR_ERR_HIP, "event");
+    }
     ANDR_HIP(ctx, hipStreamSynchronize(st));
+    double t_solve = andr_now() - ts;
+    if (en == 0) {  // from the end of the integration on
+      float ms = 0.f;
+      ANDR_HIP(ctx, hipEventElapsedTime(&ms, assembled.ev, finished.ev));
+      t_solve = ms * 1e-3;
+      t_assemble = std::max(0.0, andr_now() - t0 - t_solve);
+      for (int s = 0; s < nsd; ++s) max_row_errors(D[s].he, D[s].nn, errU, errQ);
+    }
     if (reports) {
       andr_laplace_report &R = reports[en];
       R.neq = neq;
@@ -456,8 +492,8 @@ int laplace_solve(andr_ctx *ctx, const andr_mesh *mesh, int32_t nsd, const andr_
       R.istop = istop;
       R.err[0] = errU;
       R.err[1] = std::max(errU, errQ);
-      R.t_assemble = t1 - t0;
-      R.t_solve = andr_now() - ts;
+      R.t_assemble = t_assemble;
+      R.t_solve = t_solve;
     }
   }
   return ANDR_OK;
@@ -547,22 +583,12 @@ extern "C" int andr_stokes_solve(andr_ctx *ctx, const andr_mesh *mesh, const and
   if ((rc = andr_body_upload(ctx, &sub.m, body, true))) return rc;
   const int nns = sub.m.nnodes, nes = sub.m.nelem, nsp = nns + nes;
   const size_t sT = (size_t)nsp * nns, sG = (size_t)nsp * nes;
-  DevBuf<double> dT, dG, dpT, dpG, dE;
-  if (dT.alloc(6 * sT, ctx) || dG.alloc(6 * sG, ctx) || dpT.alloc(3 * sT, ctx) || dpG.alloc(3 * sG, ctx) ||
-      dE.alloc(nsp, ctx))
+  DevBuf<double> dT, dG, dE;
+  if (dT.alloc(6 * sT, ctx) || dG.alloc(6 * sG, ctx) || dE.alloc(nsp, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "Stokes integral matrices of the subdomain");
-  if ((rc = andr_launch_stokes_rows(ctx, body, 0.0, dT.p, dG.p, dpT.p, dpG.p, dE.p))) return rc;
-  std::vector<double> he(nsp);
-  ANDR_HIP(ctx, hipMemcpyAsync(he.data(), dE.p, sizeof(double) * nsp, hipMemcpyDeviceToHost, st));
-  ANDR_HIP(ctx, hipStreamSynchronize(st));
-  dpT.release();
-  dpG.release();
-  double errU = 0.0, errQ = 0.0;
-  for (int i = 0; i < nsp; ++i) {
-    if (i < nns) errU = std::max(errU, he[i]);
-    else errQ = std::max(errQ, he[i]);
-  }
-  const double t1 = andr_now();
+  if ((rc = andr_launch_stokes_rows(ctx, body, 0.0, dT.p, dG.p, nullptr, nullptr, dE.p))) return rc;
+  andr_mark assembled, finished;  // the host goes on with the system's maps meanwhile
+  if (assembled.record(st)) return andr_fail(ctx, ANDR_ERR_HIP, "event");
   // ---- sdSetUpXandB per component, stacked as StokesBigSystemXB ---------------------------------------
   std::vector<int> ncol(3 * (size_t)nns), qcol(3 * (size_t)nes);
   std::vector<uint8_t> nknown(3 * (size_t)nns), qknown(3 * (size_t)nes);
@@ -617,49 +643,52 @@ extern "C" int andr_stokes_solve(andr_ctx *ctx, const andr_mesh *mesh, const and
     }
   }
   const int64_t lda = ((int64_t)nx + 15) / 16 * 16;
-  DevBuf<double> sys, B, X, db, qs, dgm, du, dq;
-  DevBuf<int2> drows;
-  DevBuf<int> dnc, dqc, dsu, dsq;
-  DevBuf<uint8_t> dnk, dqk;
-  if (sys.alloc((size_t)neq * lda, ctx) || B.alloc((size_t)neq * ANDR_NB, ctx) || X.alloc((size_t)nx * ANDR_NB, ctx) ||
-      qs.alloc(nx, ctx) || du.alloc(3 * (size_t)nn, ctx) || dq.alloc(3 * (size_t)ne, ctx))
+  DevBuf<double> sys, B, qs;
+  if (sys.alloc((size_t)neq * lda, ctx) || B.alloc((size_t)neq * ANDR_NB, ctx) || qs.alloc(nx, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "Stokes system %d x %d", neq, nx);
-  if ((rc = upload(ctx, db, b)) || (rc = upload(ctx, dgm, g_factors(*sd, l))) || (rc = upload(ctx, drows, rows)) ||
-      (rc = upload(ctx, dnc, ncol)) || (rc = upload(ctx, dqc, qcol)) || (rc = upload(ctx, dnk, nknown)) ||
-      (rc = upload(ctx, dqk, qknown)) || (rc = upload(ctx, dsu, src_u)) || (rc = upload(ctx, dsq, src_q)))
-    return rc;
-  ANDR_HIP(ctx, hipMemcpyAsync(X.p, xp.data(), sizeof(double) * xp.size(), hipMemcpyHostToDevice, st));
+  Tables tb;
+  const size_t o_b = tb.put(b), o_gm = tb.put(g_factors(*sd, l)), o_rows = tb.put(rows), o_nc = tb.put(ncol),
+               o_qc = tb.put(qcol), o_nk = tb.put(nknown), o_qk = tb.put(qknown), o_su = tb.put(src_u),
+               o_sq = tb.put(src_q), o_x = tb.put(xp), o_u = tb.put(u, 3 * (size_t)nn), o_q = tb.put(q, 3 * (size_t)ne);
+  if ((rc = tb.upload(ctx))) return rc;
+  double *dX = tb.at<double>(o_x), *du = tb.at<double>(o_u), *dq = tb.at<double>(o_q);
+  DevBody whole;
+  if (wall_force && (rc = andr_body_upload(ctx, mesh, whole, false))) return rc;
   hipLaunchKernelGGL(k_lap_fill<double>, dim3(((size_t)neq * lda + 255) / 256), dim3(256), 0, st, (size_t)neq * lda, sys.p);
   hipLaunchKernelGGL(k_lap_fill<double>, dim3(((size_t)neq * ANDR_NB + 255) / 256), dim3(256), 0, st, (size_t)neq * ANDR_NB,
                      B.p);
-  hipLaunchKernelGGL(k_stk_system, dim3(neq), dim3(256), 0, st, nns, nes, nsp, dT.p, dG.p, drows.p, dnc.p, dnk.p,
-                     dqc.p, dqk.p, dgm.p, db.p, sys.p, lda, B.p);
+  hipLaunchKernelGGL(k_stk_system, dim3(neq), dim3(256), 0, st, nns, nes, nsp, dT.p, dG.p, tb.at<int2>(o_rows),
+                     tb.at<int>(o_nc), tb.at<uint8_t>(o_nk), tb.at<int>(o_qc), tb.at<uint8_t>(o_qk),
+                     tb.at<double>(o_gm), tb.at<double>(o_b), sys.p, lda, B.p);
   ANDR_HIP(ctx, hipGetLastError());
   const int maxit = opts ? opts->maxit : 0;
   const double eps = opts && opts->eps > 0.0 ? opts->eps : 1e-15;
   if ((rc = andr_colscale(ctx, sys.p, false, lda, neq, nx, qs.p))) return rc;
   int nit = 0, istop = 0;
-  if ((rc = andr_lsqr_device(ctx, sys.p, false, lda, neq, nx, qs.p, B.p, X.p, 1, maxit, eps, &nit, &istop))) return rc;
+  if ((rc = andr_lsqr_device(ctx, sys.p, false, lda, neq, nx, qs.p, B.p, dX, 1, maxit, eps, &nit, &istop))) return rc;
   // StokesDistributeUnknowns, then the force on every wall (sum_e A_e q_e per component)
-  ANDR_HIP(ctx, hipMemcpyAsync(du.p, u, sizeof(double) * 3 * nn, hipMemcpyHostToDevice, st));
-  ANDR_HIP(ctx, hipMemcpyAsync(dq.p, q, sizeof(double) * 3 * ne, hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_lap_scatter, dim3((3 * nn + 255) / 256), dim3(256), 0, st, 3 * nn, dsu.p, X.p, du.p);
-  hipLaunchKernelGGL(k_lap_scatter, dim3((3 * ne + 255) / 256), dim3(256), 0, st, 3 * ne, dsq.p, X.p, dq.p);
-  DevBody whole;
+  hipLaunchKernelGGL(k_lap_scatter, dim3((3 * nn + 255) / 256), dim3(256), 0, st, 3 * nn, tb.at<int>(o_su), dX, du);
+  hipLaunchKernelGGL(k_lap_scatter, dim3((3 * ne + 255) / 256), dim3(256), 0, st, 3 * ne, tb.at<int>(o_sq), dX, dq);
   DevBuf<double> dforce;
   if (wall_force) {
-    if ((rc = andr_body_upload(ctx, mesh, whole, false))) return rc;
     if (dforce.alloc(3 * (size_t)nw, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "wall forces");
     for (int en = 0; en < 3; ++en)
-      hipLaunchKernelGGL(k_wall_flux, dim3(nw), dim3(256), 0, st, ne, whole.g.bcid, whole.g.area, dq.p + (size_t)en * ne,
+      hipLaunchKernelGGL(k_wall_flux, dim3(nw), dim3(256), 0, st, ne, whole.g.bcid, whole.g.area, dq + (size_t)en * ne,
                          dforce.p + (size_t)en * nw);
     ANDR_HIP(ctx, hipMemcpyAsync(wall_force, dforce.p, sizeof(double) * 3 * nw, hipMemcpyDeviceToHost, st));
   }
   ANDR_HIP(ctx, hipGetLastError());
-  ANDR_HIP(ctx, hipMemcpyAsync(u, du.p, sizeof(double) * 3 * nn, hipMemcpyDeviceToHost, st));
-  ANDR_HIP(ctx, hipMemcpyAsync(q, dq.p, sizeof(double) * 3 * ne, hipMemcpyDeviceToHost, st));
+  std::vector<double> he(nsp);
+  ANDR_HIP(ctx, hipMemcpyAsync(he.data(), dE.p, sizeof(double) * nsp, hipMemcpyDeviceToHost, st));
+  ANDR_HIP(ctx, hipMemcpyAsync(u, du, sizeof(double) * 3 * nn, hipMemcpyDeviceToHost, st));
+  ANDR_HIP(ctx, hipMemcpyAsync(q, dq, sizeof(double) * 3 * ne, hipMemcpyDeviceToHost, st));
+  if (finished.record(st)) return andr_fail(ctx, ANDR_ERR_HIP, "event");
   ANDR_HIP(ctx, hipStreamSynchronize(st));
   if (report) {
+    double errU = 0.0, errQ = 0.0;
+    max_row_errors(he, nns, errU, errQ);
+    float solve_ms = 0.f;
+    ANDR_HIP(ctx, hipEventElapsedTime(&solve_ms, assembled.ev, finished.ev));
     report->neq = neq;
     report->nx = nx;
     report->nb = nb;
@@ -667,8 +696,8 @@ extern "C" int andr_stokes_solve(andr_ctx *ctx, const andr_mesh *mesh, const and
     report->istop = istop;
     report->err[0] = errU;
     report->err[1] = std::max(errU, errQ);
-    report->t_assemble = t1 - t0;
-    report->t_solve = andr_now() - t1;
+    report->t_solve = solve_ms * 1e-3;
+    report->t_assemble = std::max(0.0, andr_now() - t0 - report->t_solve);
   }
   return ANDR_OK;
 }

@@ -176,14 +176,6 @@ size_t body_bytes(int ne, int nn, bool plain, bool learned, int restart) {
 // restart that fits the same buffers.
 constexpr int RESTART = 128, RESTART_MAX = 192;
 
-struct Mark {  // a point of the stream
-  hipEvent_t ev = nullptr;
-  ~Mark() {
-    if (ev) (void)hipEventDestroy(ev);
-  }
-  bool record(hipStream_t st) { return hipEventCreate(&ev) != hipSuccess || hipEventRecord(ev, st) != hipSuccess; }
-};
-
 // The resistance tensors of one wave of prepared bodies: assembly, solve, force and torque.
 // FT and reports point at the wave's first body; t_up is the wave's upload time (reported).
 int run_wave(andr_ctx *ctx, Prepared *const *P, int nb, const andr_resistance_opts *opts, int restart, bool timing,
@@ -282,7 +274,7 @@ int run_wave(andr_ctx *ctx, Prepared *const *P, int nb, const andr_resistance_op
   else
     rc = andr_launch_stokes_system(ctx, djobs, drow, (int)nrows, !plain, !plain, alg_bytes, alg_flops, summed);
   if (rc) return rc;
-  Mark assembled, finished;  // the reported times come from the device's clock: the host runs on
+  andr_mark assembled, finished;  // the reported times come from the device's clock: the host runs on
   if (assembled.record(ctx->stream)) return andr_fail(ctx, ANDR_ERR_HIP, "event");
   // ---- solve ----------------------------------------------------------------------------------
   std::vector<int> iters((size_t)nb * 6, 0), stops((size_t)nb * 6, 0);
