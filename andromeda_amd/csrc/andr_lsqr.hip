@@ -30,7 +30,8 @@
 // 84 -> 44 us; 1587^2, one 57 -> 18 us; 4897^2 in FP32, one 132 -> 40 us.
 //
 // The host reads the states of every LSQR_POLL-th iteration from pinned memory one poll late, so that
-// the device never waits for it; the iterations enqueued past the end return at once.
+// the device never waits for it; the iterations enqueued past the end return at once. Where there is no pinned
+// memory to be had it copies state B and waits.
 #include "andr_internal.h"
 #include "andr_solve.h"
 #include "andr_prof.h"
@@ -1239,7 +1240,7 @@ struct LsqrRun {
   DevBuf<double> U[2], V, W, Xl, Xs, P, PN, partU, partB, partV, partW;
   DevBuf<LsqrState> S;  // state A, state B
   LsqrState hs[NB];
-  LsqrState *slot = nullptr;  // two polls' states, pinned host memory of the context
+  LsqrState *slot = nullptr;  // two polls' states, pinned host memory of the context (null: none to be had)
   hipEvent_t ev[2] = {nullptr, nullptr};
   int polls = 0, read = 0;  // polls enqueued and read
   double abytes = 0, vbytes = 0, aflops = 0;
@@ -1248,10 +1249,8 @@ struct LsqrRun {
   LsqrRun(const LsqrRun &) = delete;
   LsqrRun &operator=(const LsqrRun &) = delete;
   ~LsqrRun() {
-    if (slot) {
-      (void)hipStreamSynchronize(st);  // nothing in flight writes the slot or the workspaces any more
-      andr_pinned_release(ctx, slot);
-    }
+    if (ctx) (void)hipStreamSynchronize(st);  // nothing in flight writes the slot or the workspaces any more
+    if (slot) andr_pinned_release(ctx, slot);
     for (auto e : ev)
       if (e) (void)hipEventDestroy(e);
   }
@@ -1417,7 +1416,6 @@ struct LsqrRun {
       return andr_fail(ctx, ANDR_ERR_ALLOC, "LSQR workspace (m=%d n=%d)", m, n);
     static_assert(2 * NB * sizeof(LsqrState) <= ANDR_PINNED_SLOT, "two polls' states in a pinned slot");
     slot = (LsqrState *)andr_pinned_alloc(ctx);
-    if (!slot) return andr_fail(ctx, ANDR_ERR_ALLOC, "pinned memory for the LSQR states");
     for (auto &e : ev) ANDR_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     std::memset(hs, 0, sizeof(hs));
     itnlim = maxit > 0 ? maxit : 10 * (m + n + 50);
@@ -1493,7 +1491,7 @@ struct LsqrRun {
   }
   template <int WD>
   void iterate() {
-    LsqrState *host = slot + (polls % 2) * NB;
+    LsqrState *host = slot ? slot + (polls % 2) * NB : nullptr;
     bool last;
     do {
       LsqrVecs L = vecs();
@@ -1524,6 +1522,15 @@ struct LsqrRun {
   // reached. The device meanwhile works on the iterations after it, which are no-ops (the kernels
   // return on a stopped state) when that poll turns out to be the last.
   int poll_state() {
+    if (!slot) {  // state B of the last iteration enqueued; an update that k_lsqr_v has applied is still marked as owed
+                  // there until the next iteration's end, or the limit's, clears it: finish() must not see it
+      ANDR_HIP(ctx, hipMemcpyAsync(hs, sb(), sizeof(LsqrState) * wd, hipMemcpyDeviceToHost, st));
+      ANDR_HIP(ctx, hipStreamSynchronize(st));
+      bool any = false;
+      for (int k = 0; k < nrhs; ++k) any = any || hs[k].active || hs[k].upd;
+      done = !any || it >= itnlim;
+      return ANDR_OK;
+    }
     ANDR_HIP(ctx, hipEventSynchronize(ev[read % 2]));
     std::memcpy(hs, slot + (read % 2) * NB, sizeof(LsqrState) * wd);
     ++read;
