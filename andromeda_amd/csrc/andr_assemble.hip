@@ -1181,6 +1181,7 @@ int andr_launch_stokes_rows(andr_ctx *ctx, DevBody &b, double extra, double *T, 
                          k_stokes_rows<true, false, false>,  k_stokes_rows<true, false, true>,
                          k_stokes_rows<true, true, false>,   k_stokes_rows<true, true, true>};
   const Kern kern = kerns[(in_lds ? 4 : 0) + (quads ? 2 : 0) + (pres ? 1 : 0)];
+  if (quads) andr_pool_headroom(ctx);  // private arrays: others may have filled the device meanwhile
   if (in_lds) ANDR_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   hipLaunchKernelGGL(kern, dim3(nsp), dim3(row_threads(b.g.ne)), in_lds ? lds : 0, ctx->stream, b.g, qr.offset, qr.npts,
                      b.order, b.color, b.ncolors, extra, T, G, prT, prG, err_rows, r0, nsp);

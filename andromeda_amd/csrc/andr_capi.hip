@@ -105,7 +105,15 @@ void *andr_dev_alloc(andr_ctx *ctx, size_t bytes) {
     }
   }
   P.size_of[p] = want;
+  andr_pool_headroom(ctx);
   return p;
+}
+
+void andr_pool_headroom(andr_ctx *ctx) {
+  if (ctx->pool.free_blocks.empty()) return;
+  size_t free_b = 0, total_b = 0;
+  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) (void)hipGetLastError();
+  else if (free_b < ANDR_POOL_RESERVE) andr_pool_trim(ctx);
 }
 
 void andr_dev_release(andr_ctx *ctx, void *p) {

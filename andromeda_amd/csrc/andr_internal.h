@@ -25,7 +25,10 @@ __host__ __device__ constexpr int sym3(int i, int j) {
 // unmapping large blocks costs milliseconds each, which is most of a batched call's host time
 // otherwise. Every use of a block is ordered on the context's stream, so a block handed out again
 // is only touched by work queued after the work of its previous owner. The cache is emptied when
-// an allocation fails and on andr_destroy.
+// an allocation fails, when new memory leaves the device less than ANDR_POOL_RESERVE free (the runtime's scratch
+// memory of kernels with private arrays comes from there, and so do other contexts' and libraries' buffers) and
+// on andr_destroy.
+#define ANDR_POOL_RESERVE ((size_t)2 << 30)
 struct andr_pool {
   std::multimap<size_t, void *> free_blocks;  // size -> cached block
   std::unordered_map<void *, size_t> size_of;  // every block the pool owns (live or cached)
@@ -89,6 +92,7 @@ int andr_fail(andr_ctx *ctx, int code, const char *fmt, ...);
 
 void *andr_dev_alloc(andr_ctx *ctx, size_t bytes);  // from the context's cache or the driver; null on failure
 void andr_dev_release(andr_ctx *ctx, void *p);       // back to the context's cache
+void andr_pool_headroom(andr_ctx *ctx);              // empties the cache when little device memory is free
 void andr_pool_trim(andr_ctx *ctx);                  // return every cached block to the driver
 void *andr_pinned_alloc(andr_ctx *ctx);              // one slot; null on failure
 void andr_pinned_release(andr_ctx *ctx, void *slot);

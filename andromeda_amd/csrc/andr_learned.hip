@@ -763,11 +763,7 @@ static int labels_common(andr_ctx *ctx, const andr_mesh *mesh, double near_ratio
   DevBuf<int> dl, dfar;
   DevBuf<unsigned long long> cnt;
   const int64_t mp = mode == 0 ? std::max<int64_t>(max_pairs, 1) : 1;
-  // the label kernel needs scratch memory of the runtime's own, which a cache that fills the device leaves
-  // no room for
-  size_t free_b = 0, total_b = 0;
-  ANDR_HIP(ctx, hipMemGetInfo(&free_b, &total_b));
-  if (free_b < ((size_t)2 << 30)) andr_pool_trim(ctx);
+  andr_pool_headroom(ctx);  // the label kernel's private arrays: others may have filled the device meanwhile
   if (df.alloc((size_t)mp * 6, ctx) || dl.alloc(mp, ctx) || dfar.alloc(ANDR_FAR_BINS, ctx) || cnt.alloc(1, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "training pair buffers");
   uint32_t keep = 0xFFFFFFFFu;
