@@ -85,9 +85,10 @@ static size_t pool_round(size_t bytes) {
   return (bytes + g - 1) / g * g;
 }
 
-void *andr_dev_alloc(andr_ctx *ctx, size_t bytes) {
+void *andr_dev_alloc(andr_ctx *ctx, size_t bytes, bool *fresh) {
   andr_pool &P = ctx->pool;
   const size_t want = pool_round(bytes);
+  if (fresh) *fresh = false;
   auto it = P.free_blocks.lower_bound(want);
   if (it != P.free_blocks.end() && it->first <= want + want / 4 + (1u << 20)) {  // close enough: reuse
     void *p = it->second;
@@ -105,8 +106,14 @@ void *andr_dev_alloc(andr_ctx *ctx, size_t bytes) {
     }
   }
   P.size_of[p] = want;
+  if (fresh) *fresh = true;
   andr_pool_headroom(ctx);
   return p;
+}
+
+void andr_dev_free(andr_ctx *ctx, void *p) {
+  ctx->pool.size_of.erase(p);
+  (void)hipFree(p);  // waits for the device
 }
 
 void andr_pool_headroom(andr_ctx *ctx) {
@@ -529,7 +536,8 @@ int upload_csr(andr_ctx *ctx, int m, int n, int64_t nnz, const int64_t *ia, cons
   DevBuf<int32_t> dja;
   DevBuf<double> da;
   const int64_t ld = dense_ld(n);
-  if (c.D.alloc((size_t)m * ld) || dia.alloc(m + 1, ctx) || dja.alloc(nnz, ctx) || da.alloc(nnz, ctx))
+  if (c.D.alloc((size_t)m * ld) || dia.call_alloc(m + 1, ctx) || dja.call_alloc(nnz, ctx) ||
+      da.call_alloc(nnz, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "LSQR matrix %d x %d", m, n);
   ANDR_HIP(ctx, hipMemsetAsync(c.D.p, 0, sizeof(double) * (size_t)m * ld, st));
   ANDR_HIP(ctx, hipMemcpyAsync(dia.p, ia, sizeof(int64_t) * (m + 1), hipMemcpyHostToDevice, st));
@@ -610,8 +618,8 @@ extern "C" void lsqr_solve_(const int32_t *m, const int32_t *n, const int64_t *n
   if (*maxit == 0) *maxit = 10 * (*m + *n + 50);
   const int M = *m, N = *n;
   DevBuf<double> dq, dB, dX, tmp;
-  if (dq.alloc(N, ctx) || dB.alloc((size_t)M * ANDR_NB, ctx) || dX.alloc((size_t)N * ANDR_NB, ctx) ||
-      tmp.alloc(std::max(M, N), ctx)) {
+  if (dq.call_alloc(N, ctx) || dB.call_alloc((size_t)M * ANDR_NB, ctx) || dX.call_alloc((size_t)N * ANDR_NB, ctx) ||
+      tmp.call_alloc(std::max(M, N), ctx)) {
     *ierr = -3;
     return;
   }
@@ -686,8 +694,8 @@ extern "C" int andr_lsqr_dense(andr_ctx *ctx, int64_t m, int64_t n, const double
   andr_lsqr_opts o = opts ? *opts : andr_lsqr_opts{0, 1e-15, 1};
   DevBuf<double> dA, dq, dB, dX;
   const int64_t lda = (n + 15) / 16 * 16;  // rows start on 128-byte lines
-  if (dA.alloc((size_t)m * lda, ctx) || dq.alloc(n, ctx) || dB.alloc((size_t)m * ANDR_NB, ctx) ||
-      dX.alloc((size_t)n * ANDR_NB, ctx))
+  if (dA.call_alloc((size_t)m * lda, ctx) || dq.call_alloc(n, ctx) || dB.call_alloc((size_t)m * ANDR_NB, ctx) ||
+      dX.call_alloc((size_t)n * ANDR_NB, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "andr_lsqr_dense workspace");
   ANDR_HIP(ctx, hipMemcpy2DAsync(dA.p, sizeof(double) * lda, A, sizeof(double) * n, sizeof(double) * n, m,
                                  hipMemcpyHostToDevice, ctx->stream));

@@ -27,8 +27,11 @@ __host__ __device__ constexpr int sym3(int i, int j) {
 // is only touched by work queued after the work of its previous owner. The cache is emptied when
 // an allocation fails, when new memory leaves the device less than ANDR_POOL_RESERVE free (the runtime's scratch
 // memory of kernels with private arrays comes from there, and so do other contexts' and libraries' buffers) and
-// on andr_destroy.
+// on andr_destroy. Buffers of a user's own sizes (call_alloc below: the dense matrices of the solver seams, training
+// sets, transposes) stay up to ANDR_CALL_KEEP each: a driver's allocation of that size is some 1 % of the copy that
+// fills it.
 #define ANDR_POOL_RESERVE ((size_t)2 << 30)
+#define ANDR_CALL_KEEP ((size_t)128 << 20)
 struct andr_pool {
   std::multimap<size_t, void *> free_blocks;  // size -> cached block
   std::unordered_map<void *, size_t> size_of;  // every block the pool owns (live or cached)
@@ -90,8 +93,10 @@ int andr_fail(andr_ctx *ctx, int code, const char *fmt, ...);
                        hipGetErrorString(e_));                                                    \
   } while (0)
 
-void *andr_dev_alloc(andr_ctx *ctx, size_t bytes);  // from the context's cache or the driver; null on failure
+// from the context's cache or the driver (fresh); null on failure
+void *andr_dev_alloc(andr_ctx *ctx, size_t bytes, bool *fresh = nullptr);
 void andr_dev_release(andr_ctx *ctx, void *p);       // back to the context's cache
+void andr_dev_free(andr_ctx *ctx, void *p);          // back to the driver
 void andr_pool_headroom(andr_ctx *ctx);              // empties the cache when little device memory is free
 void andr_pool_trim(andr_ctx *ctx);                  // return every cached block to the driver
 void *andr_pinned_alloc(andr_ctx *ctx);              // one slot; null on failure
@@ -117,6 +122,7 @@ struct DevBuf {
   T *p = nullptr;
   size_t n = 0;
   andr_ctx *owner = nullptr;
+  bool give_back = false;  // to the driver on release
   DevBuf() = default;
   DevBuf(const DevBuf &) = delete;
   DevBuf &operator=(const DevBuf &) = delete;
@@ -136,14 +142,31 @@ struct DevBuf {
     }
     return hipMalloc(&p, sizeof(T) * count);
   }
+  // a buffer of a user's own size: what the cache did not have and is larger than `keep` goes back to the driver
+  hipError_t call_alloc(size_t count, andr_ctx *pool, size_t keep = ANDR_CALL_KEEP) {
+    release();
+    n = count;
+    if (count == 0) return hipSuccess;
+    bool fresh = false;
+    p = (T *)andr_dev_alloc(pool, sizeof(T) * count, &fresh);
+    if (!p) {
+      n = 0;
+      return hipErrorOutOfMemory;
+    }
+    owner = pool;
+    give_back = fresh && sizeof(T) * count > keep;
+    return hipSuccess;
+  }
   void release() {
     if (p) {
-      if (owner) andr_dev_release(owner, p);
+      if (owner && give_back) andr_dev_free(owner, p);
+      else if (owner) andr_dev_release(owner, p);
       else (void)hipFree(p);
     }
     p = nullptr;
     n = 0;
     owner = nullptr;
+    give_back = false;
   }
 };
 

@@ -437,7 +437,7 @@ struct MlpWork {
   MlpAct act{};
   int alloc(andr_ctx *ctx, int b) {
     const size_t B = ((size_t)b + 3) / 4 * 4;
-    if (buf.alloc(B * (NIN + 6 * NH + NOUT), ctx)) return 1;
+    if (buf.call_alloc(B * (NIN + 6 * NH + NOUT), ctx)) return 1;
     float *q = buf.p;
     for (float **h : {&act.H1, &act.H2, &act.H3, &act.D1, &act.D2, &act.D3}) {
       *h = q;
@@ -764,7 +764,8 @@ static int labels_common(andr_ctx *ctx, const andr_mesh *mesh, double near_ratio
   DevBuf<unsigned long long> cnt;
   const int64_t mp = mode == 0 ? std::max<int64_t>(max_pairs, 1) : 1;
   andr_pool_headroom(ctx);  // the label kernel's private arrays: others may have filled the device meanwhile
-  if (df.alloc((size_t)mp * 6, ctx) || dl.alloc(mp, ctx) || dfar.alloc(ANDR_FAR_BINS, ctx) || cnt.alloc(1, ctx))
+  if (df.call_alloc((size_t)mp * 6, ctx) || dl.call_alloc(mp, ctx) || dfar.alloc(ANDR_FAR_BINS, ctx) ||
+      cnt.alloc(1, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "training pair buffers");
   uint32_t keep = 0xFFFFFFFFu;
   unsigned long long n = 0;
@@ -821,8 +822,8 @@ extern "C" int andr_mlp_loss_grad(andr_ctx *ctx, int64_t npairs, const float *fe
   MlpWork w;
   DevBuf<float> X, p, gr, dloss;
   DevBuf<int> L;
-  if (w.alloc(ctx, M) || X.alloc((size_t)M * NIN, ctx) || p.alloc(NPARAM, ctx) || gr.alloc(NPARAM, ctx) ||
-      dloss.alloc(M, ctx) || L.alloc(M, ctx))
+  if (w.alloc(ctx, M) || X.call_alloc((size_t)M * NIN, ctx) || p.alloc(NPARAM, ctx) || gr.alloc(NPARAM, ctx) ||
+      dloss.call_alloc(M, ctx) || L.call_alloc(M, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "MLP buffers");
   hipStream_t st = ctx->stream;
   ANDR_HIP(ctx, hipMemcpyAsync(X.p, features, sizeof(float) * M * NIN, hipMemcpyHostToDevice, st));
@@ -874,8 +875,9 @@ extern "C" int andr_mlp_train(andr_ctx *ctx, int64_t npairs, const float *featur
   MlpWork w;
   DevBuf<float> X, p, m, v, loss;
   DevBuf<int> L, idx;
-  if (w.alloc(ctx, B) || X.alloc((size_t)N * NIN, ctx) || p.alloc(NPARAM, ctx) || m.alloc(NPARAM, ctx) ||
-      v.alloc(NPARAM, ctx) || loss.alloc((size_t)(samples + 1) * B, ctx) || L.alloc(N, ctx) || idx.alloc(N, ctx))
+  if (w.alloc(ctx, B) || X.call_alloc((size_t)N * NIN, ctx) || p.alloc(NPARAM, ctx) || m.alloc(NPARAM, ctx) ||
+      v.alloc(NPARAM, ctx) || loss.call_alloc((size_t)(samples + 1) * B, ctx) || L.call_alloc(N, ctx) ||
+      idx.call_alloc(N, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "MLP training buffers");
   hipStream_t st = ctx->stream;
   ANDR_HIP(ctx, hipMemcpyAsync(X.p, features, sizeof(float) * (size_t)N * NIN, hipMemcpyHostToDevice, st));

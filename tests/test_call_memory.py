@@ -83,3 +83,17 @@ for left in (64 << 30, 1 << 30):
         grown.append(live() - n0)
 assert grown[1] < grown[0] - 7 * MB, grown
 """)
+
+
+@pytest.mark.gpu
+def test_gpu_large_dense_matrix_goes_back(tmp_path):
+    """A matrix of 200 MB: the driver has it again when the call returns, and the small ones stay."""
+    run(tmp_path, """
+with api.Context(0) as ctx:
+    solve(ctx, 300)
+    n0 = live()
+    solve(ctx, 300)
+    assert live() == n0
+    solve(ctx, 5000)
+    assert live() - n0 < 40 * MB, live() - n0
+""")
