@@ -386,7 +386,7 @@ __global__ void k_unpack_col(int n, const double *__restrict__ V, double *__rest
 }
 
 namespace {
-// The device copy of the last matrix, keyed on the array pointers, the sizes and a checksum of every
+// The device copy of the last matrix (never left in the context's memory cache), keyed on the array pointers, the sizes and a checksum of every
 // byte of ia, ja and a: a solve on a matrix whose values or pattern changed since the copy was made
 // uploads it again. The checksum is one streaming pass over the host arrays (threads over chunks),
 // cheaper than the upload it saves.
@@ -518,8 +518,9 @@ int upload_csr(andr_ctx *ctx, int m, int n, int64_t nnz, const int64_t *ia, cons
         tja[o] = i;
         tva[o] = a[p];
       }
-    if (c.cia.alloc(m + 1) || c.cja.alloc(std::max<int64_t>(nnz, 1)) || c.cva.alloc(std::max<int64_t>(nnz, 1)) ||
-        c.tia.alloc(n + 1) || c.tja.alloc(std::max<int64_t>(nnz, 1)) || c.tva.alloc(std::max<int64_t>(nnz, 1)))
+    const size_t nz = std::max<int64_t>(nnz, 1);
+    if (c.cia.call_alloc(m + 1, ctx, 0) || c.cja.call_alloc(nz, ctx, 0) || c.cva.call_alloc(nz, ctx, 0) ||
+        c.tia.call_alloc(n + 1, ctx, 0) || c.tja.call_alloc(nz, ctx, 0) || c.tva.call_alloc(nz, ctx, 0))
       return andr_fail(ctx, ANDR_ERR_ALLOC, "sparse LSQR matrix %d x %d (%lld entries)", m, n, (long long)nnz);
     ANDR_HIP(ctx, hipMemcpyAsync(c.cia.p, hia.data(), sizeof(int64_t) * (m + 1), hipMemcpyHostToDevice, st));
     ANDR_HIP(ctx, hipMemcpyAsync(c.tia.p, tia.data(), sizeof(int64_t) * (n + 1), hipMemcpyHostToDevice, st));
@@ -536,7 +537,7 @@ int upload_csr(andr_ctx *ctx, int m, int n, int64_t nnz, const int64_t *ia, cons
   DevBuf<int32_t> dja;
   DevBuf<double> da;
   const int64_t ld = dense_ld(n);
-  if (c.D.alloc((size_t)m * ld) || dia.call_alloc(m + 1, ctx) || dja.call_alloc(nnz, ctx) ||
+  if (c.D.call_alloc((size_t)m * ld, ctx, 0) || dia.call_alloc(m + 1, ctx) || dja.call_alloc(nnz, ctx) ||
       da.call_alloc(nnz, ctx))
     return andr_fail(ctx, ANDR_ERR_ALLOC, "LSQR matrix %d x %d", m, n);
   ANDR_HIP(ctx, hipMemsetAsync(c.D.p, 0, sizeof(double) * (size_t)m * ld, st));

@@ -57,6 +57,16 @@ def solve(ctx, n):
     A, b = _system(n, n, 1)
     X, _ = ctx.lsqr_dense(A, b, eps=1e-12)
     assert np.linalg.norm(A @ X - b) < 1e-9 * np.linalg.norm(b)
+def csr(n, fill):
+    A = _system(n, n, 1)[0]
+    A[:, : n - fill] *= np.eye(n)[:, : n - fill]
+    i, j = np.nonzero(A)
+    ia = np.concatenate([[1], 1 + np.cumsum(np.bincount(i, minlength=n))]).astype(np.int64)
+    a, b, x = A[i, j], A @ np.ones(n), np.zeros(n)
+    ja = (j + 1).astype(np.int32)
+    q = api.lsqr_precon(n, n, ia, ja, a)
+    r = api.lsqr_solve(n, n, ia, ja, a, q, b, x, eps=1e-12)
+    assert r["ierr"] == 0 and np.abs(x - 1.0).max() < 1e-8
 """
 
 
@@ -96,4 +106,18 @@ with api.Context(0) as ctx:
     assert live() == n0
     solve(ctx, 5000)
     assert live() - n0 < 40 * MB, live() - n0
+""")
+
+
+@pytest.mark.gpu
+def test_gpu_csr_behind_a_larger_one(tmp_path):
+    """36.9 MB of device memory: a CSR whose dense copy, 24 MB, and staging fit them alone, behind another
+    whose staging and workspaces, 14 MB, the cache holds."""
+    run(tmp_path, """
+cell("limit").value = 36900000
+csr(1000, 1000)
+csr(1700, 570)
+n0 = live()
+api.lsqr_forget()
+assert n0 - live() >= 8 * 1700 * 1712
 """)
