@@ -25,9 +25,10 @@
 //      previous iteration still owes; starts with the scalars after A V (state A).
 // With more than LSQR_FUSE_SEG column segments every panel's own sum over them would cost more than a
 // launch (per row WD * 8 bytes a segment in each column panel against 1 KB of A), and
-// k_lsqr_u forms U once, as for CSR matrices. Measured per iteration with seven launches and
-// eight columns throughout against this: 3120^2, 6 right-hand sides 73 -> 41 us; 4881 x 2717, one
-// 84 -> 44 us; 1587^2, one 57 -> 18 us; 4897^2 in FP32, one 132 -> 40 us.
+// k_lsqr_u forms U once, as for CSR matrices and for several right-hand sides of a large A (fuse_u below).
+// Measured per iteration with seven launches and eight columns throughout against this: 3120^2, 6
+// right-hand sides 73 -> 41 us; 4881 x 2717, one 84 -> 44 us; 1587^2, one 57 -> 18 us; 4897^2 in FP32, one
+// 132 -> 40 us.
 //
 // The host reads the states of every LSQR_POLL-th iteration from pinned memory one poll late, so that
 // the device never waits for it; the iterations enqueued past the end return at once. Where there is no pinned
@@ -530,14 +531,16 @@ __global__ __launch_bounds__(256) void k_lsqr_av1(const ST *__restrict__ A, int6
 // A lane holds the columns of one 16-byte load of a row and their sums; the first rows are requested before
 // U is formed. Bound by the matrix stream; 3120^2 with 6 right-hand sides 22.6 -> 20.0 us, and an
 // eighth of the partial results for k_lsqr_v (13.8 -> 4.8 us); 4881 x 2717 with one 24.3 -> 19.4 us.
-constexpr int AT_WAVES = 8, AT_MAXRW = 32;
+// Rows per wave at most: 32 where U is formed, 64 where it is given (its 512 rows in LDS are 32 KB, which two blocks
+// of a CU still have room for): half the partial results of a large A.
+constexpr int AT_WAVES = 8, AT_MAXRW = 32, AT_MAXRW_GIVEN = 64;
 constexpr int at_cols(size_t elem) { return 64 * 16 / (int)elem; }  // a 16-byte load per lane
 
 template <class ST, int WD, bool FORM, bool KEEP>
 __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restrict__ A, int64_t lda, int m, int n, int rw,
                                                             LsqrVecs L, double *__restrict__ P) {
   constexpr int BS = 64 * AT_WAVES, CW = at_cols(sizeof(ST)), LV = CW / 64;  // columns per lane
-  constexpr int RMAX = AT_WAVES * AT_MAXRW;
+  constexpr int RMAX = AT_WAVES * (FORM ? AT_MAXRW : AT_MAXRW_GIVEN);
   typedef ST vec __attribute__((ext_vector_type(LV)));
   typedef const vec __attribute__((address_space(1))) *gvp;
   __shared__ __attribute__((aligned(16))) double ul[RMAX * WD];
@@ -1171,6 +1174,17 @@ constexpr int LSQR_POLL = 8;  // iterations between reads of the convergence sta
 // columns sums them again, WD * 8 bytes a row and segment (L2) against 1 KB of A.
 constexpr int LSQR_FUSE_SEG = 2, LSQR_FUSE_SEG1 = 16;
 
+// Whether k_lsqr_atu forms U. With several right-hand sides and an A beyond the 256 MB cache the panels' own sums
+// and the 256-row splits that they allow cost more than k_lsqr_u's launch. Six columns, an iteration formed in the
+// product against apart with 512-row splits: 8000^2 216 and 207 us, 12000^2 464 and 435, 16000^2 765 and 729; bodies
+// of 2400 elements (288 MB) 129 and 126 ms a solve of three, of 8000 (4.6 GB) 2303 and 2133 of two; but of 1620
+// (189 MB) 82 and 85, and below eight panels (200000 x 200) 199 and 209 us.
+constexpr int LSQR_FUSE_PANELS = 8;
+bool fuse_u(int m, int n, int64_t lda, bool fp32, int wd, int nseg, int panels) {
+  if (nseg > (wd == 1 ? LSQR_FUSE_SEG1 : LSQR_FUSE_SEG)) return false;
+  return wd == 1 || panels < LSQR_FUSE_PANELS || (double)m * lda * (fp32 ? 4 : 8) <= KEEP_BYTES;
+}
+
 // How A X splits its columns, a function of the shape alone (so that the tile count never changes the
 // sums): nseg column segments of AV_WAVES * wcols columns. Two segments while there are fewer than 128
 // 64-row tiles, else one wave per SIMD or less would be in flight; no more than AV_MAXCOLS columns per wave.
@@ -1382,19 +1396,20 @@ struct LsqrRun {
     } else if (wd == 1) {
       // a wave per eight rows: segments (of whole 1 KB loads) while there are fewer than 2048 waves
       const int rowwaves = (m + 7) / 8;
-        const int want = std::min(std::max(1, (2048 + rowwaves - 1) / rowwaves), std::max(1, n / 256));
+      const int want = std::min(std::max(1, (2048 + rowwaves - 1) / rowwaves), std::max(1, n / 256));
       av.wcols = ((n + want - 1) / want + 255) / 256 * 256;
       av.nseg = (n + av.wcols - 1) / av.wcols;
     } else {
       av = av_shape(m, n);
     }
-    fuse = !cia && av.nseg <= (wd == 1 ? LSQR_FUSE_SEG1 : LSQR_FUSE_SEG);
     const int cols = at_cols(fp32 ? 4 : 8), panels = (n + cols - 1) / cols;
+    fuse = !cia && fuse_u(m, n, lda, fp32, wd, av.nseg, panels);
     // Rows per wave of A^T U: the fewest (16, the finest split that keeps two register sets busy) whose
     // blocks run at once, two on each CU; a second, nearly empty round of blocks costs more than the
     // longer waves (3120^2, 6 right-hand sides: 650 blocks of 16 rows a wave 25.2 us, 425 of 24 20.0).
     rw = 16;
-    while (rw < AT_MAXRW && panels * ((m + AT_WAVES * rw - 1) / (AT_WAVES * rw) + 1) > 512) rw += wd == 1 ? 16 : 8;
+    const int maxrw = fuse || wd == 1 ? AT_MAXRW : AT_MAXRW_GIVEN;
+    while (rw < maxrw && panels * ((m + AT_WAVES * rw - 1) / (AT_WAVES * rw) + 1) > 512) rw += wd == 1 ? 16 : 8;
     splits = cia ? 1 : (m + AT_WAVES * rw - 1) / (AT_WAVES * rw);
     // one pass over A where a block's threads hold whole rows (4881 x 2717, with k_lsqr_v: 24 us an iteration, 44
     // with a kernel for each product)
