@@ -12,7 +12,8 @@
 // separate scaling passes of the reference (dscal at :947, :974, :980).
 //
 // A single right-hand side of at most 8192 unknowns takes two launches an iteration and reads A once: k_lsqr_pass
-// does the work of 1. and 2. below on rows that stay in registers. Otherwise
+// does the work of 1. and 2. below on rows that stay in registers (not where they are narrow and many, PASS_MIN_COLS).
+// Otherwise
 // an iteration is three launches. A small system (an A of the order of the 256 MB cache) spends its
 // time in the gaps and the latency of small kernels, not in the products, so the recurrences' scalar
 // work and the vector updates ride along in the products' own kernels:
@@ -683,7 +684,12 @@ __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restr
 // then sums the sixteen waves' shares for itself. One block per CU, each with its part of A^T u for
 // k_lsqr_v. A block's rows, and its XCD, are the same in every iteration. Bound by the matrix stream: 4881 x
 // 2717 18.8 us where the two products took 20.3 and 19.4, 1587^2 7.5 (6.2 + 8.2), 4897^2 in FP32 20.5 (17.5 + 16.2).
-constexpr int PASS_BS = 1024, PASS_BLOCKS = 255, PASS_CHUNKS = 4, PASS_LV = 2;
+// A set of eight rows takes a block some 2 us however narrow they are, as most of its threads have no columns; so
+// fewer than PASS_MIN_COLS columns go this way only while a block has no more than two sets (m <= 4080), where the
+// launch that it saves counts. Kernels of an iteration, one pass against two products: 128 columns, 4000 rows 13.3
+// and 13.6 us, 6000 15.6 and 13.7, 64000 68 and 36, 200000 188 and 82; 32 columns 200000 185 and 47; 320 columns
+// 64000 70 and 60; 384 70 and 65; 448 71 and 76; 512 86 and 107.
+constexpr int PASS_BS = 1024, PASS_BLOCKS = 255, PASS_CHUNKS = 4, PASS_LV = 2, PASS_MIN_COLS = 400;
 // rows of a register set: 128 bytes a thread in both
 constexpr int pass_rows(size_t elem, int ch) { return (ch == 1 ? 8 : ch == 2 ? 4 : 2) * (elem == 4 && ch > 1 ? 2 : 1); }
 
@@ -1412,12 +1418,15 @@ struct LsqrRun {
     while (rw < maxrw && panels * ((m + AT_WAVES * rw - 1) / (AT_WAVES * rw) + 1) > 512) rw += wd == 1 ? 16 : 8;
     splits = cia ? 1 : (m + AT_WAVES * rw - 1) / (AT_WAVES * rw);
     // one pass over A where a block's threads hold whole rows (4881 x 2717, with k_lsqr_v: 24 us an iteration, 44
-    // with a kernel for each product)
+    // with a kernel for each product) and narrow rows are few (PASS_MIN_COLS)
     chunks = (n + PASS_BS * PASS_LV - 1) / (PASS_BS * PASS_LV);
     if (wd == 1 && !cia && chunks <= PASS_CHUNKS) {
       const int R = pass_rows(fp32 ? 4 : 8, chunks);  // whole register sets: a shorter last one loads as much
-      rpb = ((m + PASS_BLOCKS - 1) / PASS_BLOCKS + R - 1) / R * R;
-      blocksP = (m + rpb - 1) / rpb;
+      const int rows = ((m + PASS_BLOCKS - 1) / PASS_BLOCKS + R - 1) / R * R;
+      if (n >= PASS_MIN_COLS || rows <= 2 * R) {
+        rpb = rows;
+        blocksP = (m + rpb - 1) / rpb;
+      }
     }
     const int vv = v_values(blocksP ? 16 : 4);
     blocksV = std::min((n * wd + vv - 1) / vv, V_MAXBLOCKS);
