@@ -411,48 +411,54 @@ __device__ __forceinline__ void quad_laplace_pair(const double *x1, const double
     }
     const int off = c_gl_off[iq], N = c_gl_n[iq];
     const double hx = 1.0 / ndx, hy = 1.0 / ndy;  // half cell widths
-    for (int ix = 0; ix < ndx; ++ix)
-      for (int i = 0; i < N; ++i) {
-        const double gi = -1.0 + (2 * ix + 1) * hx + c_gl[off + i][0] * hx;
-        double r0[3], et[3], n0[3], n1[3];  // r = r0 - gj et, normal n0 + gj n1
+    auto points = [&](auto ends) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          r0[k] = sc0[k] - gi * c1[k];
-          et[k] = c2[k] + gi * c3[k];
-        }
-        n0[0] = c1[1] * et[2] - c1[2] * et[1];
-        n0[1] = c1[2] * et[0] - c1[0] * et[2];
-        n0[2] = c1[0] * et[1] - c1[1] * et[0];
-        n1[0] = c3[1] * et[2] - c3[2] * et[1];
-        n1[1] = c3[2] * et[0] - c3[0] * et[2];
-        n1[2] = c3[0] * et[1] - c3[1] * et[0];
-        const double ra = r0[0] * n0[0] + r0[1] * n0[1] + r0[2] * n0[2];
-        const double rb = r0[0] * n1[0] + r0[1] * n1[1] + r0[2] * n1[2];
-        double sg = 0.0, h0 = 0.0, h1 = 0.0;
-        for (int iy = 0; iy < ndy; ++iy) {
-          const double gc = -1.0 + (2 * iy + 1) * hy;
-          for (int j = 0; j < N; ++j) {
-            const double gj = gc + c_gl[off + j][0] * hy, w = c_gl[off + j][1];
-            const double rx = r0[0] - gj * et[0], ry = r0[1] - gj * et[1], rz = r0[2] - gj * et[2];
-            const double ax = n0[0] + gj * n1[0], ay = n0[1] + gj * n1[1], az = n0[2] + gj * n1[2];
-            const double l2 = ax * ax + ay * ay + az * az;
-            const double len = l2 > 0.0 ? l2 * rsqrt64(l2) : 0.0;
-            const double ir = rsqrt64(rx * rx + ry * ry + rz * rz);
-            const double wi = w * ir;
-            sg += wi * len;
-            const double wh = wi * (ir * ir) * (ra + gj * rb);
-            h0 += wh;
-            h1 += wh * gj;
+      for (int k = 0; k < 5; ++k) out[k] = 0.0;
+      for (int ix = 0; ix < ndx; ++ix)
+        for (int i = 0; i < N; ++i) {
+          const double gi = -1.0 + (2 * ix + 1) * hx + c_gl[off + i][0] * hx;
+          double r0[3], et[3], n0[3], n1[3];  // r = r0 - gj et, normal n0 + gj n1
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            r0[k] = sc0[k] - gi * c1[k];
+            et[k] = c2[k] + gi * c3[k];
           }
+          n0[0] = c1[1] * et[2] - c1[2] * et[1];
+          n0[1] = c1[2] * et[0] - c1[0] * et[2];
+          n0[2] = c1[0] * et[1] - c1[1] * et[0];
+          n1[0] = c3[1] * et[2] - c3[2] * et[1];
+          n1[1] = c3[2] * et[0] - c3[0] * et[2];
+          n1[2] = c3[0] * et[1] - c3[1] * et[0];
+          const double ra = r0[0] * n0[0] + r0[1] * n0[1] + r0[2] * n0[2];
+          const double rb = r0[0] * n1[0] + r0[1] * n1[1] + r0[2] * n1[2];
+          double sg = 0.0, h0 = 0.0, h1 = 0.0;
+          for (int iy = 0; iy < ndy; ++iy) {
+            const double gc = -1.0 + (2 * iy + 1) * hy;
+            for (int j = 0; j < N; ++j) {
+              const double gj = gc + c_gl[off + j][0] * hy, w = c_gl[off + j][1];
+              const double rx = r0[0] - gj * et[0], ry = r0[1] - gj * et[1], rz = r0[2] - gj * et[2];
+              const double ax = n0[0] + gj * n1[0], ay = n0[1] + gj * n1[1], az = n0[2] + gj * n1[2];
+              const double l2 = ax * ax + ay * ay + az * az;
+              const double len = l2 > 0.0 ? l2 * rsqrt64(l2) : 0.0;
+              const double ir = rsqrt64<decltype(ends)::value>(rx * rx + ry * ry + rz * rz);
+              const double wi = w * ir;
+              sg += wi * len;
+              const double wh = wi * (ir * ir) * (ra + gj * rb);
+              h0 += wh;
+              h1 += wh * gj;
+            }
+          }
+          const double wi = c_gl[off + i][1];
+          out[0] += wi * sg;
+          const double hm = wi * (h0 - h1), hp = wi * (h0 + h1);
+          out[1] += (1.0 - gi) * hm;
+          out[2] += (1.0 + gi) * hm;
+          out[3] += (1.0 + gi) * hp;
+          out[4] += (1.0 - gi) * hp;
         }
-        const double wi = c_gl[off + i][1];
-        out[0] += wi * sg;
-        const double hm = wi * (h0 - h1), hp = wi * (h0 + h1);
-        out[1] += (1.0 - gi) * hm;
-        out[2] += (1.0 + gi) * hm;
-        out[3] += (1.0 + gi) * hp;
-        out[4] += (1.0 - gi) * hp;
-      }
+    };
+    points(std::false_type{});
+    if (out[0] != out[0]) points(std::true_type{});  // a point at the source, or too far away for its square
     const double sc = (0.25 / ANDR_PI) * hx * hy;
     out[0] *= sc;
 #pragma unroll
@@ -613,19 +619,24 @@ __global__ __launch_bounds__(256) void k_laplace_rows(BodyGeom g, int qoff, int 
             xb[c] = x2[c] - x3[c];
             rn += d[c] * g.nrm[3 * e + c];
           }
-          double gs = 0.0, f1 = 0.0, f2 = 0.0, f3 = 0.0;
-          for (int q = 0; q < nq; ++q) {
-            const double l1 = c_qd[qoff + q][0], l2 = c_qd[qoff + q][1], l3 = c_qd[qoff + q][2], w = c_qd[qoff + q][3];
-            const double rx = d[0] - l1 * xa[0] - l2 * xb[0];
-            const double ry = d[1] - l1 * xa[1] - l2 * xb[1];
-            const double rz = d[2] - l1 * xa[2] - l2 * xb[2];
-            const double ir = rsqrt64(rx * rx + ry * ry + rz * rz);
-            const double w1 = w * ir, w3 = w1 * (ir * ir);
-            gs += w1;
-            f1 += w3 * l1;
-            f2 += w3 * l2;
-            f3 += w3 * l3;
-          }
+          double gs, f1, f2, f3;
+          auto points = [&](auto ends) {
+            gs = f1 = f2 = f3 = 0.0;
+            for (int q = 0; q < nq; ++q) {
+              const double l1 = c_qd[qoff + q][0], l2 = c_qd[qoff + q][1], l3 = c_qd[qoff + q][2], w = c_qd[qoff + q][3];
+              const double rx = d[0] - l1 * xa[0] - l2 * xb[0];
+              const double ry = d[1] - l1 * xa[1] - l2 * xb[1];
+              const double rz = d[2] - l1 * xa[2] - l2 * xb[2];
+              const double ir = rsqrt64<decltype(ends)::value>(rx * rx + ry * ry + rz * rz);
+              const double w1 = w * ir, w3 = w1 * (ir * ir);
+              gs += w1;
+              f1 += w3 * l1;
+              f2 += w3 * l2;
+              f3 += w3 * l3;
+            }
+          };
+          points(std::false_type{});
+          if (gs != gs) points(std::true_type{});  // a point at the source, or too far away for its square
           gv = k4pi * g.area[e] * gs;
           const double ch = k4pi * g.area[e] * (g.mul[e] * rn);
           h[0] = ch * f1;

@@ -14,12 +14,15 @@ static inline int andr_upload_rules_here(andr_ctx *ctx, const double *tab, const
 }
 
 
-// 1 / sqrt(x) in FP64 for x > 0: the hardware estimate (v_rsq_f64, error e below 2^-20) and one step of
+// 1 / sqrt(x) in FP64 for 0 < x < infinity: the hardware estimate (v_rsq_f64, error e below 2^-20) and one step of
 // third order (Householder), which leaves e^3: five operations against the some twenty of a division and
-// a square root in their general forms.
+// a square root in their general forms. ENDS: 0 and infinity too, whose estimates, infinity and 0, stand (e is no
+// number there, its minimum with anything the other).
+template <bool ENDS = false>
 __device__ inline double rsqrt64(double x) {
   const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-x * y, y, 1.0);
+  double e = fma(-x * y, y, 1.0);
+  if constexpr (ENDS) e = fmin(e, 0.5);
   return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
