@@ -1569,15 +1569,8 @@ void launch_bround(hipStream_t st, int nsys, int L, const GSys *sys, const TileM
       hipLaunchKernelGGL(kb_bupdate, dim3(ntiles), dim3(256), 0, st, sys, tmap, j + 1, 1, all);
     }
   };
-  switch (L) {
-    case 1: go(std::integral_constant<int, 1>{}); break;
-    case 2: go(std::integral_constant<int, 2>{}); break;
-    case 3: go(std::integral_constant<int, 3>{}); break;
-    case 4: go(std::integral_constant<int, 4>{}); break;
-    case 5: go(std::integral_constant<int, 5>{}); break;
-    case 6: go(std::integral_constant<int, 6>{}); break;
-    default: go(std::integral_constant<int, 7>{}); break;
-  }
+  if (L == 3) go(std::integral_constant<int, 3>{});
+  else go(std::integral_constant<int, 6>{});
 }
 
 // block per system of the cycle: Y = R^-1 g over the rounds used, the solution blocks Y_b[l][k] into C1, from
@@ -1686,15 +1679,7 @@ int launch_bsolve_l(andr_ctx *ctx, int nsys, const GSys *sys, int steps) {
   return ANDR_OK;
 }
 int launch_bsolve(andr_ctx *ctx, int nsys, int L, const GSys *sys, int steps) {
-  switch (L) {
-    case 1: return launch_bsolve_l<1>(ctx, nsys, sys, steps);
-    case 2: return launch_bsolve_l<2>(ctx, nsys, sys, steps);
-    case 3: return launch_bsolve_l<3>(ctx, nsys, sys, steps);
-    case 4: return launch_bsolve_l<4>(ctx, nsys, sys, steps);
-    case 5: return launch_bsolve_l<5>(ctx, nsys, sys, steps);
-    case 6: return launch_bsolve_l<6>(ctx, nsys, sys, steps);
-    default: return launch_bsolve_l<7>(ctx, nsys, sys, steps);
-  }
+  return L == 3 ? launch_bsolve_l<3>(ctx, nsys, sys, steps) : launch_bsolve_l<6>(ctx, nsys, sys, steps);
 }
 
 }  // namespace
@@ -1724,10 +1709,10 @@ int andr_gmres_batch(andr_ctx *ctx, const GmresSys *in, int nsys, bool fp32, int
   }
   // per system: Hessenberg, rotations, g, coefficients; the per-rhs state (8 doubles per rhs) of all
   // systems sits in one separate array so that the host reads it with one copy
-  // Block GMRES (one Krylov space per system for its nrhs columns; the reflector window of its
-  // least-squares update holds nrhs + 1 rows in 8 lanes, so nrhs <= 7) unless
-  // ANDR_GMRES_INDEPENDENT=1, which runs one Krylov space per column.
-  const bool blk = getenv("ANDR_GMRES_INDEPENDENT") == nullptr && nrhs <= NB - 1;
+  // Block GMRES (one Krylov space per system for its nrhs columns) for the widths there are, three strain fields and
+  // six rigid-body problems (launch_bround, launch_bsolve); one Krylov space per column for others and with
+  // ANDR_GMRES_INDEPENDENT=1.
+  const bool blk = getenv("ANDR_GMRES_INDEPENDENT") == nullptr && (nrhs == 3 || nrhs == 6);
   const int L = nrhs;
   auto small_of = [&](int mc) {
     if (blk)  // Rp, hv, gB, C1, C2, Ri
