@@ -532,16 +532,18 @@ __global__ __launch_bounds__(256) void k_lsqr_av1(const ST *__restrict__ A, int6
 // A lane holds the columns of one 16-byte load of a row and their sums; the first rows are requested before
 // U is formed. Bound by the matrix stream; 3120^2 with 6 right-hand sides 22.6 -> 20.0 us, and an
 // eighth of the partial results for k_lsqr_v (13.8 -> 4.8 us); 4881 x 2717 with one 24.3 -> 19.4 us.
-// Rows per wave at most: 32 where U is formed, 64 where it is given (its 512 rows in LDS are 32 KB, which two blocks
-// of a CU still have room for): half the partial results of a large A.
-constexpr int AT_WAVES = 8, AT_MAXRW = 32, AT_MAXRW_GIVEN = 64;
+// Where U is given a wave takes AT_CHUNK rows of it at a time into its own part of the LDS, the next ones under way, so
+// that its rows may be many: the partial results of a large A, eight columns written and read again for every split,
+// are then nothing beside it (61440^2: 5.84 ms with U formed and 32 rows a wave, 5.21 with 64, 4.88 with 128, 4.47 with
+// 512, 6.76 TB/s).
+constexpr int AT_WAVES = 8, AT_MAXRW = 32, AT_MAXRW_GIVEN = 512, AT_CHUNK = 64;
 constexpr int at_cols(size_t elem) { return 64 * 16 / (int)elem; }  // a 16-byte load per lane
 
 template <class ST, int WD, bool FORM, bool KEEP>
 __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restrict__ A, int64_t lda, int m, int n, int rw,
                                                             LsqrVecs L, double *__restrict__ P) {
   constexpr int BS = 64 * AT_WAVES, CW = at_cols(sizeof(ST)), LV = CW / 64;  // columns per lane
-  constexpr int RMAX = AT_WAVES * (FORM ? AT_MAXRW : AT_MAXRW_GIVEN);
+  constexpr int RMAX = AT_WAVES * (FORM ? AT_MAXRW : AT_CHUNK);
   typedef ST vec __attribute__((ext_vector_type(LV)));
   typedef const vec __attribute__((address_space(1))) *gvp;
   __shared__ __attribute__((aligned(16))) double ul[RMAX * WD];
@@ -607,22 +609,21 @@ __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restr
       const double s = block_sum<WD, BS>(y2, red);
       if (tid < WD) L.partU[(size_t)blockIdx.y * WD + tid] = s;
     }
-  } else {
-    if (!any_active<WD>(L.sb)) return;
-    for (int e = tid; e < AT_WAVES * rw * WD; e += BS) ul[e] = e < nr * WD ? L.uin[(size_t)i0 * WD + e] : 0.0;
+    __syncthreads();
+  } else if (!any_active<WD>(L.sb)) {
+    return;
   }
-  __syncthreads();
   double acc[LV][WD];
 #pragma unroll
   for (int q = 0; q < LV; ++q)
 #pragma unroll
     for (int k = 0; k < WD; ++k) acc[q][k] = 0.0;
-  auto step = [&](int r, const Set &s) {
+  auto step = [&](const double *uw, const Set &s) {  // uw: U of the set's rows, zero past the last row
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
       double uv[WD];
 #pragma unroll
-      for (int k = 0; k < WD; ++k) uv[k] = ul[(r0 + r + u) * WD + k];  // zero past the last row
+      for (int k = 0; k < WD; ++k) uv[k] = uw[u * WD + k];
 #pragma unroll
       for (int q = 0; q < LV; ++q) {
         const double av = (double)s.a[u][q];
@@ -633,17 +634,46 @@ __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restr
       if (WD > 1 && u % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // rw is a multiple of 2 UN: two register sets in turn, the last loads repeat the last row
+  // two register sets in turn over rows r .. r1 - 1 (rw and AT_CHUNK are multiples of 2 UN); the last loads repeat the
+  // last row
+  auto rows = [&](int r, int r1, const double *uw) {
 #pragma unroll 1
-  for (int r = 0; r < rn; r += 2 * UN) {
-    load(r + UN, s1);
-    __builtin_amdgcn_sched_barrier(0);
-    step(r, s0);
-    __builtin_amdgcn_sched_barrier(0);
-    load(r + 2 * UN, s0);
-    __builtin_amdgcn_sched_barrier(0);
-    step(r + UN, s1);
-    __builtin_amdgcn_sched_barrier(0);
+    for (; r < r1; r += 2 * UN, uw += 2 * UN * WD) {
+      load(r + UN, s1);
+      __builtin_amdgcn_sched_barrier(0);
+      step(uw, s0);
+      __builtin_amdgcn_sched_barrier(0);
+      load(r + 2 * UN, s0);
+      __builtin_amdgcn_sched_barrier(0);
+      step(uw + UN * WD, s1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if constexpr (FORM) {
+    rows(0, rn, ul + r0 * WD);
+  } else {
+    static_assert(AT_CHUNK == 64, "WD values of a chunk of U per lane");
+    double un[WD], *uw = ul + wid * AT_CHUNK * WD;
+    const double *ug = L.uin + (size_t)(i0 + r0) * WD;
+    auto given = [&](int r) {
+#pragma unroll
+      for (int k = 0; k < WD; ++k) {
+        const int e = lane + 64 * k;
+        un[k] = r + e / WD < rn ? ug[(size_t)r * WD + e] : 0.0;
+      }
+    };
+    given(0);
+#pragma unroll 1
+    for (int r = 0; r < rn; r += AT_CHUNK) {
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      __builtin_amdgcn_wave_barrier();  // the last chunk is read
+#pragma unroll
+      for (int k = 0; k < WD; ++k) uw[lane + 64 * k] = un[k];
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      given(r + AT_CHUNK);
+      rows(r, min(r + AT_CHUNK, rn), uw);
+    }
   }
   // the waves' sums: (0 + 4) (1 + 5) (2 + 6) (3 + 7), then (0 + 2) (1 + 3), then (0 + 1)
 #pragma unroll
@@ -1181,10 +1211,10 @@ constexpr int LSQR_POLL = 8;  // iterations between reads of the convergence sta
 constexpr int LSQR_FUSE_SEG = 2, LSQR_FUSE_SEG1 = 16;
 
 // Whether k_lsqr_atu forms U. With several right-hand sides and an A beyond the 256 MB cache the panels' own sums
-// and the 256-row splits that they allow cost more than k_lsqr_u's launch. Six columns, an iteration formed in the
-// product against apart with 512-row splits: 8000^2 216 and 207 us, 12000^2 464 and 435, 16000^2 765 and 729; bodies
-// of 2400 elements (288 MB) 129 and 126 ms a solve of three, of 8000 (4.6 GB) 2303 and 2133 of two; but of 1620
-// (189 MB) 82 and 85, and below eight panels (200000 x 200) 199 and 209 us.
+// and the short splits that they need cost more than k_lsqr_u's launch: plain tensors of bodies of 2420 elements
+// (422 MB) 200 ms a solve of three formed in the product, 179 apart; of 5120 (1.9 GB) 1170 and 1009; of 8000 (4.6 GB)
+// 2264 of two and 1954; but of 1620 (189 MB) 79 and 82, and below eight panels (200000 x 200) 199 and 209 us an
+// iteration.
 constexpr int LSQR_FUSE_PANELS = 8;
 bool fuse_u(int m, int n, int64_t lda, bool fp32, int wd, int nseg, int panels) {
   if (nseg > (wd == 1 ? LSQR_FUSE_SEG1 : LSQR_FUSE_SEG)) return false;

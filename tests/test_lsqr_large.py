@@ -1,5 +1,6 @@
-"""LSQR with several right-hand sides of a matrix beyond the 256 MB cache: U is formed once and A^T U goes
-over splits of up to 512 rows; at fewer than eight column panels U is formed in the product, over 256 rows."""
+"""LSQR with several right-hand sides of a matrix beyond the 256 MB cache: U is formed once and A^T U goes over
+splits as long as leave one round of blocks; at fewer than eight column panels U is formed in the product, over 256
+rows. Splits that end within a wave's rows and within the pieces of 64 rows in which U is staged."""
 import numpy as np
 import pytest
 
@@ -7,11 +8,16 @@ from test_lsqr_shapes import _system
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,nrhs,rows", [(5700, 5700, 3, 512), (33000, 1025, 6, 512), (36000, 896, 2, 256)])
+@pytest.mark.parametrize("m,n,nrhs,rows", [(5700, 5700, 3, 576), (33000, 1025, 6, 640), (36000, 896, 2, 256),
+                                           (2100, 16500, 2, 1088)])
 def test_gpu_lsqr_large(ctx, m, n, nrhs, rows):
     A, B = _system(m, n, nrhs)
-    want = B[:n]
-    b = A @ want
+    if m >= n:
+        want = B[:n]
+        b = A @ want
+    else:  # the solution of least norm
+        b = B
+        want = A.T @ np.linalg.solve(A @ A.T, b)
     ctx.profile(True)
     try:
         X, st = ctx.lsqr_dense(A, b, eps=1e-13, precon=False)
