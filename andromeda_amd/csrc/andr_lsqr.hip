@@ -618,12 +618,12 @@ __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restr
   for (int q = 0; q < LV; ++q)
 #pragma unroll
     for (int k = 0; k < WD; ++k) acc[q][k] = 0.0;
-  auto step = [&](const double *uw, const Set &s) {  // uw: U of the set's rows, zero past the last row
+  auto step = [&](int r, const Set &s) {  // r: the set's first row in the LDS
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
       double uv[WD];
 #pragma unroll
-      for (int k = 0; k < WD; ++k) uv[k] = uw[u * WD + k];
+      for (int k = 0; k < WD; ++k) uv[k] = ul[(r + u) * WD + k];  // zero past the last row
 #pragma unroll
       for (int q = 0; q < LV; ++q) {
         const double av = (double)s.a[u][q];
@@ -634,23 +634,23 @@ __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restr
       if (WD > 1 && u % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // two register sets in turn over rows r .. r1 - 1 (rw and AT_CHUNK are multiples of 2 UN); the last loads repeat the
+  // two register sets in turn over rows first .. end - 1 (rw and AT_CHUNK are multiples of 2 UN); the last loads repeat the
   // last row
-  auto rows = [&](int r, int r1, const double *uw) {
+  auto rows = [&](int first, int end, int o) {  // row r of the wave is row o + r of the LDS
 #pragma unroll 1
-    for (; r < r1; r += 2 * UN, uw += 2 * UN * WD) {
+    for (int r = first; r < end; r += 2 * UN) {
       load(r + UN, s1);
       __builtin_amdgcn_sched_barrier(0);
-      step(uw, s0);
+      step(o + r, s0);
       __builtin_amdgcn_sched_barrier(0);
       load(r + 2 * UN, s0);
       __builtin_amdgcn_sched_barrier(0);
-      step(uw + UN * WD, s1);
+      step(o + r + UN, s1);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
   if constexpr (FORM) {
-    rows(0, rn, ul + r0 * WD);
+    rows(0, rn, r0);
   } else {
     static_assert(AT_CHUNK == 64, "WD values of a chunk of U per lane");
     double un[WD], *uw = ul + wid * AT_CHUNK * WD;
@@ -672,7 +672,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restr
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       __builtin_amdgcn_wave_barrier();
       given(r + AT_CHUNK);
-      rows(r, min(r + AT_CHUNK, rn), uw);
+      rows(r, min(r + AT_CHUNK, rn), wid * AT_CHUNK - r);
     }
   }
   // the waves' sums: (0 + 4) (1 + 5) (2 + 6) (3 + 7), then (0 + 2) (1 + 3), then (0 + 1)
