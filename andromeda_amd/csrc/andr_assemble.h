@@ -52,12 +52,17 @@ int andr_launch_stokes_domain(andr_ctx *ctx, DevBody &b, int npts, const double 
 // Surface pressure at the element centres (device arrays u[3 nn], q[3 ne], p[ne]); triangle meshes.
 int andr_launch_stokes_surface_pressure(andr_ctx *ctx, DevBody &b, const double *u, const double *q, double diff,
                                         double *p);
-// algorithmic work of a pair evaluation: Stokes G + T kernels 107 flops (per-vertex stresslet
-// moments), 60 flops with the vertex-summed moments of the fast form's rigid-body problems
-// (stokes_pair_sum); Laplace G + H 50 flops
+// algorithmic work of a pair evaluation (FMA as 2, square root, division and rsqrt as 1): Stokes G + T of the resistance
+// systems 107 flops (per-vertex stresslet moments), 60 flops with the vertex-summed moments of the fast form's
+// rigid-body problems (stokes_pair_sum)
 #define ANDR_FLOPS_PER_STOKES_EVAL 107.0
 #define ANDR_FLOPS_PER_STOKES_EVAL_SUM 60.0
-#define ANDR_FLOPS_PER_LAPLACE_EVAL 50.0
+// the same for the integral rows, from the loops over a triangle's points: Stokes in moment form (stokes_tri_full) with
+// and without the pressure integrals, Laplace in FP64 and FP32 (k_laplace_rows)
+#define ANDR_FLOPS_PER_STOKES_ROW_PRESSURE 107.0
+#define ANDR_FLOPS_PER_STOKES_ROW 77.0
+#define ANDR_FLOPS_PER_LAPLACE_ROW 28.0
+#define ANDR_FLOPS_PER_LAPLACE_ROW_FP32 36.0
 // velocity and pressure at a domain point (k_stokes_domain), surface pressure (FMA as 2, rsqrt as 1)
 #define ANDR_FLOPS_PER_DOMAIN_EVAL 92.0
 #define ANDR_FLOPS_PER_SURFACE_EVAL 55.0

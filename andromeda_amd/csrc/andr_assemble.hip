@@ -705,8 +705,9 @@ int andr_launch_laplace_rows(andr_ctx *ctx, DevBody &b, double *H, double *G, do
   const int nsp = nrows < 0 ? b.g.nn + b.g.ne - r0 : nrows;  // rows r0 .. r0 + nsp - 1
   const size_t lds = sizeof(double) * b.g.nn;
   const double evals = (double)nsp * b.g.ne * qr.npts;
+  const double flops = fp32_quad ? ANDR_FLOPS_PER_LAPLACE_ROW_FP32 : ANDR_FLOPS_PER_LAPLACE_ROW;
   const int tok = andr_prof_begin(ctx, fp32_quad ? "laplace_rows_fp32" : "laplace_rows",
-                                  8.0 * nsp * ((double)b.g.nn + b.g.ne), evals * ANDR_FLOPS_PER_LAPLACE_EVAL);
+                                  8.0 * nsp * ((double)b.g.nn + b.g.ne), evals * flops);
   const bool in_lds = lds <= 128 * 1024, quads = b.g.nv == 4;
   using Kern = void (*)(BodyGeom, int, int, const int *, const uint8_t *, int, double *, double *, double *, int);
   const Kern kerns[8] = {k_laplace_rows<false, false, false>, k_laplace_rows<false, false, true>,
@@ -1183,7 +1184,7 @@ int andr_launch_stokes_rows(andr_ctx *ctx, DevBody &b, double extra, double *T, 
   const size_t lds = sizeof(double) * nm * (size_t)b.g.nn;
   const double evals = (double)nsp * b.g.ne * qr.npts;
   const int tok = andr_prof_begin(ctx, "stokes_rows", 8.0 * nm * nsp * ((double)b.g.nn + b.g.ne),
-                                  evals * ANDR_FLOPS_PER_STOKES_EVAL);
+                                  evals * (pres ? ANDR_FLOPS_PER_STOKES_ROW_PRESSURE : ANDR_FLOPS_PER_STOKES_ROW));
   const bool in_lds = lds <= 144 * 1024, quads = b.g.nv == 4;
   using Kern = void (*)(BodyGeom, int, int, const int *, const uint8_t *, int, double, double *, double *, double *,
                         double *, double *, int, int);

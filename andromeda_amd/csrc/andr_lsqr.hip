@@ -62,7 +62,8 @@ typedef double d4v __attribute__((ext_vector_type(4)));
 // is left in an L2 from the product before, and the second half of a line that two rows share, are then hits.
 // A larger one is streamed past them. Measured: one pass over 106 MB 21.6 us streamed, 18.8 kept, 20 MB 9.9 and
 // 7.5, FP32 96 MB 25.8 and 20.5; A^T U of 78 MB 20.0 and 17.2, A V 15.5 and 13.5; but 512 MB 84 and 90, 1.15 GB 173
-// and 188.
+// and 188. Each system of a batch is judged by itself, although four are solved at a time: four of 69 MB take 36 ms
+// streamed and 30 kept, of 118 MB 60 and 53, three of 189 MB 85 and 82; only four of 189 MB 103 and 104.5.
 constexpr double KEEP_BYTES = 256e6;
 template <bool KEEP, class P>
 __device__ inline auto stream_load(P p) {
