@@ -1820,7 +1820,7 @@ int andr_copy_out(andr_ctx *ctx, int32_t layout, const std::vector<andr_matrix_o
       continue;
     }
     DevBuf<double> t;  // one transposed matrix at a time
-    if (t.call_alloc((size_t)o.m * o.n, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "transpose buffer");
+    if (t.alloc((size_t)o.m * o.n, ctx)) return andr_fail(ctx, ANDR_ERR_ALLOC, "transpose buffer");
     dim3 grid((unsigned)((o.n + 31) / 32), (unsigned)((o.m + 31) / 32));
     hipLaunchKernelGGL(k_transpose, grid, dim3(32, 8), 0, ctx->stream, o.d, t.p, o.m, o.n);
     ANDR_HIP(ctx, hipGetLastError());

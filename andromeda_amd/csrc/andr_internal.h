@@ -28,8 +28,8 @@ __host__ __device__ constexpr int sym3(int i, int j) {
 // an allocation fails, when new memory leaves the device less than ANDR_POOL_RESERVE free (the runtime's scratch
 // memory of kernels with private arrays comes from there, and so do other contexts' and libraries' buffers) and
 // on andr_destroy. Buffers of a user's own sizes (call_alloc below: the dense matrices of the solver seams, training
-// sets, transposes) stay up to ANDR_CALL_KEEP each: a driver's allocation of that size is some 1 % of the copy that
-// fills it.
+// sets) stay up to ANDR_CALL_KEEP each: the driver's allocation and release of a larger one, some 5 us a MB, are
+// 2 % of the copy that fills it.
 #define ANDR_POOL_RESERVE ((size_t)2 << 30)
 #define ANDR_CALL_KEEP ((size_t)128 << 20)
 struct andr_pool {
