@@ -386,9 +386,9 @@ __global__ void k_unpack_col(int n, const double *__restrict__ V, double *__rest
 }
 
 namespace {
-// The device copy of the last matrix (never left in the context's memory cache), keyed on the array pointers, the sizes and a checksum of every
-// byte of ia, ja and a: a solve on a matrix whose values or pattern changed since the copy was made
-// uploads it again. The checksum is one streaming pass over the host arrays (threads over chunks),
+// The device copy of the last matrix (the driver has it again when it is dropped), keyed on the array
+// pointers, the sizes and a checksum of every byte of ia, ja and a: a solve on a matrix whose values or
+// pattern changed since the copy was made uploads it again. The checksum is one streaming pass over the host arrays (threads over chunks),
 // cheaper than the upload it saves.
 struct LsqrCache {
   const double *key_a = nullptr;

@@ -535,8 +535,8 @@ __global__ __launch_bounds__(256) void k_lsqr_av1(const ST *__restrict__ A, int6
 // eighth of the partial results for k_lsqr_v (13.8 -> 4.8 us); 4881 x 2717 with one 24.3 -> 19.4 us.
 // Where U is given a wave takes AT_CHUNK rows of it at a time into its own part of the LDS, the next ones under way, so
 // that its rows may be many: the partial results of a large A, eight columns written and read again for every split,
-// are then nothing beside it (61440^2: 5.84 ms with U formed and 32 rows a wave, 5.21 with 64, 4.88 with 128, 4.47 with
-// 512, 6.76 TB/s).
+// are then nothing beside it (61440^2: 5.84 ms with 32 rows a wave, 5.21 with 64, 4.88 with 128, 4.47 with 512, 6.76
+// TB/s).
 constexpr int AT_WAVES = 8, AT_MAXRW = 32, AT_MAXRW_GIVEN = 512, AT_CHUNK = 64;
 constexpr int at_cols(size_t elem) { return 64 * 16 / (int)elem; }  // a 16-byte load per lane
 
@@ -635,8 +635,8 @@ __global__ __launch_bounds__(64 * AT_WAVES, 4) void k_lsqr_atu(const ST *__restr
       if (WD > 1 && u % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // two register sets in turn over rows first .. end - 1 (rw and AT_CHUNK are multiples of 2 UN); the last loads repeat the
-  // last row
+  // two register sets in turn over rows first .. end - 1 (rw and AT_CHUNK are multiples of 2 UN); the last loads
+  // repeat the last row
   auto rows = [&](int first, int end, int o) {  // row r of the wave is row o + r of the LDS
 #pragma unroll 1
     for (int r = first; r < end; r += 2 * UN) {
@@ -1212,10 +1212,9 @@ constexpr int LSQR_POLL = 8;  // iterations between reads of the convergence sta
 constexpr int LSQR_FUSE_SEG = 2, LSQR_FUSE_SEG1 = 16;
 
 // Whether k_lsqr_atu forms U. With several right-hand sides and an A beyond the 256 MB cache the panels' own sums
-// and the short splits that they need cost more than k_lsqr_u's launch: plain tensors of bodies of 2420 elements
-// (422 MB) 200 ms a solve of three formed in the product, 179 apart; of 5120 (1.9 GB) 1170 and 1009; of 8000 (4.6 GB)
-// 2264 of two and 1954; but of 1620 (189 MB) 79 and 82, and below eight panels (200000 x 200) 199 and 209 us an
-// iteration.
+// and the short splits that they need cost more than k_lsqr_u's launch: three plain tensors of bodies of 2420 elements
+// (422 MB) 200 ms formed in the product, 177 apart; of 5120 (1.9 GB) 1170 and 1002; but of 1620 (189 MB) 79 and 82,
+// and below eight panels (200000 x 200) 199 and 209 us an iteration.
 constexpr int LSQR_FUSE_PANELS = 8;
 bool fuse_u(int m, int n, int64_t lda, bool fp32, int wd, int nseg, int panels) {
   if (nseg > (wd == 1 ? LSQR_FUSE_SEG1 : LSQR_FUSE_SEG)) return false;

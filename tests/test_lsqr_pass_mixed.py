@@ -19,7 +19,8 @@ def _solve(ctx, nu, precision):
     u, q = m.xyz @ g, -(n @ g)  # the flux of unit diffusivity
     known = np.zeros(m.nnodes, dtype=bool)
     known[np.unique(m.con[m.bcid == 1])] = True
-    r = ctx.laplace_solve(m, [api.Subdomain([1, 2], [1.0, 1.0], 1.0)], np.array([[api.BC_FUNCTION, api.BC_FLUX]], dtype=np.int32),
+    bc = np.array([[api.BC_FUNCTION, api.BC_FLUX]], dtype=np.int32)
+    r = ctx.laplace_solve(m, [api.Subdomain([1, 2], [1.0, 1.0], 1.0)], bc,
                           np.where(known, u, 0.0)[None], np.where(m.bcid == 2, q, 0.0)[None], eps=1e-13, maxit=0,
                           precision=precision)[0]
     return r, u
